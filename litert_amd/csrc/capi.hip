@@ -71,13 +71,14 @@ constexpr int kGemmMinBatches = 128;
 // streams the filter once.
 constexpr int kPackedGemmMinBatches = 16;
 
-// Workspace layout for the hybrid paths (kernels.h).
+// Workspace layout for the hybrid paths on re-tiled filters (kernels.h): rows padded to whole
+// 16-byte pieces.
 using Workspace = lrtfc::ActivationWorkspace;
 size_t WorkspaceBytes(int batches, int depth) {
-  return lrtfc::ActivationWorkspaceBytes(batches, depth);
+  return lrtfc::ActivationWorkspaceBytes(batches, lrtfc::PaddedDepth(depth));
 }
 Workspace SplitWorkspace(void* base, int batches, int depth) {
-  return lrtfc::SplitActivationWorkspace(base, batches, depth);
+  return lrtfc::SplitActivationWorkspace(base, batches, lrtfc::PaddedDepth(depth));
 }
 
 }  // namespace
@@ -501,6 +502,15 @@ int FcHybridInt8Packed(const int8_t* quantized_input, const float* scaling_facto
                                                LRTFC_QUANT_PORTABLE, AsStream(stream)),
                  "packed hybrid GEMV");
 }
+
+// BatchQuantizeFloats into a workspace whose rows are padded (kernels.h).
+int BatchQuantizePadded(const float* values, int batches, int depth, const Workspace& w,
+                        int do_asymmetric, int variant, void* stream) {
+  LRTFC_REQUIRE(variant >= 0 && variant <= LRTFC_QUANT_NEON_LEGACY, "unknown quantizer variant");
+  return FromHip(lrtfc::LaunchBatchQuantize(values, batches, depth, lrtfc::PaddedDepth(depth), w.q,
+                                            w.sf, w.zp, do_asymmetric, variant, AsStream(stream)),
+                 "batch quantize");
+}
 }  // namespace
 
 int lrtfc_fc_hybrid_int8_packed(const int8_t* quantized_input, const float* scaling_factors,
@@ -531,12 +541,13 @@ int lrtfc_fc_hybrid_packed_workspace(const float* input, const int8_t* packed_fi
   LRTFC_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255) == 0,
                 "workspace must be 256-byte aligned");
   const Workspace w = SplitWorkspace(workspace, batches, depth);
-  int rc = lrtfc_batch_quantize_floats(input, batches, depth, w.q, w.sf, w.zp,
-                                       asymmetric_quantize_inputs, quant_variant, stream);
+  int rc = BatchQuantizePadded(input, batches, depth, w, asymmetric_quantize_inputs, quant_variant,
+                               stream);
   if (rc != LRTFC_OK) return rc;
   return FcHybridInt8Packed(w.q, w.sf, asymmetric_quantize_inputs ? w.zp : nullptr, packed_filter,
                             per_channel_scales, filter_scale, filter_row_sums, bias, output,
-                            batches, depth, out_depth, activation, /*zero_input_exit=*/1, stream);
+                            batches, lrtfc::PaddedDepth(depth), out_depth, activation,
+                            /*zero_input_exit=*/1, stream);
 }
 
 namespace {
@@ -600,8 +611,8 @@ int lrtfc_batch_matmul_hybrid_packed_nd(const float* lhs, const int* lhs_batch_d
   // BatchQuantizeFloats over every row of the float operand (batch_matmul.cc:472-497); symmetric
   // quantization leaves the offsets at zero (:487-489).
   const Workspace w = SplitWorkspace(quant_space, static_cast<int>(quant_rows), depth);
-  int rc = lrtfc_batch_quantize_floats(lhs, static_cast<int>(quant_rows), depth, w.q, w.sf, w.zp,
-                                       asymmetric_quantize_inputs, quant_variant, stream);
+  int rc = BatchQuantizePadded(lhs, static_cast<int>(quant_rows), depth, w,
+                               asymmetric_quantize_inputs, quant_variant, stream);
   if (rc != LRTFC_OK) return rc;
   const int32_t* zp = asymmetric_quantize_inputs ? w.zp : nullptr;
   // Output matrix (b0, b1, b2) pairs the left matrix and the weight matrix whose indices keep
@@ -628,12 +639,13 @@ int lrtfc_batch_matmul_hybrid_packed_nd(const float* lhs, const int* lhs_batch_d
       ++run;
     }
     const size_t row0 = static_cast<size_t>(l0) * rows;
-    rc = FcHybridInt8Packed(w.q + row0 * depth, w.sf + row0, zp ? zp + row0 : nullptr,
+    rc = FcHybridInt8Packed(w.q + row0 * lrtfc::PaddedDepth(depth), w.sf + row0, zp ? zp + row0 : nullptr,
                             packed_weights + static_cast<size_t>(w0) * matrix_bytes,
                             per_channel_scales, filter_scale,
                             row_sums + static_cast<size_t>(w0) * units, nullptr,
                             output + static_cast<size_t>(o) * rows * units,
-                            static_cast<int>(run * rows), depth, units, LRTFC_ACT_NONE, 0, stream,
+                            static_cast<int>(run * rows), lrtfc::PaddedDepth(depth), units,
+                            LRTFC_ACT_NONE, 0, stream,
                             /*batch_matmul=*/1);
     if (rc != LRTFC_OK) return rc;
     o += run;
@@ -670,8 +682,8 @@ int lrtfc_batch_quantize_floats(const float* values, int n_batch, int n_data, in
   LRTFC_REQUIRE(!do_asymmetric || zero_points, "zero_points is required for asymmetric mode");
   LRTFC_REQUIRE(variant >= 0 && variant <= LRTFC_QUANT_NEON_LEGACY, "unknown quantizer variant");
   LRTFC_REQUIRE(n_data > 0, "empty rows cannot be quantized");
-  return FromHip(lrtfc::LaunchBatchQuantize(values, n_batch, n_data, quantized, scaling_factors,
-                                            zero_points, do_asymmetric, variant,
+  return FromHip(lrtfc::LaunchBatchQuantize(values, n_batch, n_data, n_data, quantized,
+                                            scaling_factors, zero_points, do_asymmetric, variant,
                                             AsStream(stream)),
                  "batch quantize");
 }
@@ -744,12 +756,13 @@ int lrtfc_fc_hybrid(const float* input, const int8_t* filter, const float* per_c
                    "zero fill");
   }
   LRTFC_REQUIRE(input && workspace, "null pointer");
-  LRTFC_REQUIRE(workspace_bytes >= WorkspaceBytes(batches, depth),
-                "workspace too small: %zu < %zu bytes", workspace_bytes,
-                WorkspaceBytes(batches, depth));
+  // The row-major kernels take the rows without padding, as they take the filter.
+  const size_t need = lrtfc::ActivationWorkspaceBytes(batches, depth);
+  LRTFC_REQUIRE(workspace_bytes >= need, "workspace too small: %zu < %zu bytes", workspace_bytes,
+                need);
   LRTFC_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255) == 0,
                 "workspace must be 256-byte aligned");
-  const Workspace w = SplitWorkspace(workspace, batches, depth);
+  const Workspace w = lrtfc::SplitActivationWorkspace(workspace, batches, depth);
   int rc = lrtfc_batch_quantize_floats(input, batches, depth, w.q, w.sf, w.zp,
                                        asymmetric_quantize_inputs, quant_variant, stream);
   if (rc != LRTFC_OK) return rc;
@@ -771,10 +784,11 @@ int lrtfc_fc_hybrid_static_scratch(const float* input, const int8_t* filter,
   if (int rc = RequireInit()) return rc;
   LRTFC_REQUIRE(batches >= 0 && depth >= 0 && out_depth >= 0, "negative dimension");
   if (batches == 0 || out_depth == 0) return LRTFC_OK;
-  LRTFC_REQUIRE(WorkspaceBytes(batches, depth) <= LRTFC_STATIC_SCRATCH_BYTES,
+  LRTFC_REQUIRE(lrtfc::ActivationWorkspaceBytes(batches, depth) <= LRTFC_STATIC_SCRATCH_BYTES,
                 "%d rows of depth %d need %zu bytes of activation scratch; the static scratch "
                 "holds %d (use lrtfc_fc_hybrid with a workspace of the caller's)",
-                batches, depth, WorkspaceBytes(batches, depth), LRTFC_STATIC_SCRATCH_BYTES);
+                batches, depth, lrtfc::ActivationWorkspaceBytes(batches, depth),
+                LRTFC_STATIC_SCRATCH_BYTES);
   int device = -1;
   if (hipError_t err = hipGetDevice(&device)) return FromHip(err, "hipGetDevice");
   void* ptr = (device >= 0 && device < kMaxDevices) ? g_scratch_ptr[device].load() : nullptr;
@@ -899,7 +913,7 @@ int lrtfc_batch_quantize_floats_4bit(const float* values, int n_batch, int n_dat
   if (n_batch == 0) return LRTFC_OK;
   LRTFC_REQUIRE(values && quantized && scaling_factors && input_offsets, "null pointer");
   LRTFC_REQUIRE(n_data > 0, "empty rows cannot be quantized");
-  return FromHip(lrtfc::LaunchBatchQuantize4Bit(values, n_batch, n_data, quantized,
+  return FromHip(lrtfc::LaunchBatchQuantize4Bit(values, n_batch, n_data, n_data, quantized,
                                                 scaling_factors, input_offsets, AsStream(stream)),
                  "4-bit path row quantizer");
 }
@@ -924,13 +938,15 @@ int lrtfc_fc_hybrid_int4_per_channel_packed(const float* input, const int8_t* pa
   LRTFC_REQUIRE((reinterpret_cast<uintptr_t>(packed_filter) & 15) == 0,
                 "packed filter must be 16-byte aligned");
   const Workspace w = SplitWorkspace(workspace, batches, depth);
-  int rc = lrtfc_batch_quantize_floats_4bit(input, batches, depth, w.q, w.sf, w.zp, stream);
+  int rc = FromHip(lrtfc::LaunchBatchQuantize4Bit(input, batches, depth, lrtfc::PaddedDepth(depth),
+                                                  w.q, w.sf, w.zp, AsStream(stream)),
+                   "4-bit path row quantizer");
   if (rc != LRTFC_OK) return rc;
   lrtfc::FcInt8Args a{};
   a.input = w.q;
   a.filter = packed_filter;
   a.batches = batches;
-  a.depth = depth;
+  a.depth = lrtfc::PaddedDepth(depth);
   a.out_depth = out_depth;
   a.scaling_factors = w.sf;
   a.zero_points = w.zp;  // the rows' input offsets on this path
@@ -998,12 +1014,14 @@ int lrtfc_fc_hybrid_int4_per_channel_nibbles(const float* input, const uint8_t* 
                    "per-channel int4 hybrid GEMV (nibble layout, fused quantizer)");
   }
   const Workspace w = SplitWorkspace(workspace, batches, depth);
-  int rc = lrtfc_batch_quantize_floats_4bit(input, batches, depth, w.q, w.sf, w.zp, stream);
+  int rc = FromHip(lrtfc::LaunchBatchQuantize4Bit(input, batches, depth, lrtfc::PaddedDepth(depth),
+                                                  w.q, w.sf, w.zp, AsStream(stream)),
+                   "4-bit path row quantizer");
   if (rc != LRTFC_OK) return rc;
   return FromHip(lrtfc::LaunchFcInt4PerChannelGemv(retiled_filter, nullptr, w.q, w.sf, w.zp,
                                                    per_channel_scales, filter_scale, bias, output,
-                                                   batches, depth, out_depth, activation,
-                                                   AsStream(stream)),
+                                                   batches, lrtfc::PaddedDepth(depth), out_depth,
+                                                   activation, AsStream(stream)),
                  "per-channel int4 hybrid GEMV (nibble layout)");
 }
 

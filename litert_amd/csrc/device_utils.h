@@ -15,6 +15,11 @@ constexpr int kWaveSize = 64;
 // 128-bit register quad: the unit of every weight load (global_load_dwordx4).
 using i32x4 = int __attribute__((ext_vector_type(4)));
 using i32x2 = int __attribute__((ext_vector_type(2)));
+// The same loads and stores where nothing is known about the address but that it is that of an
+// int8 (or a float): one global_load_dwordx4 each, as gfx9 takes global accesses on any byte.
+typedef int i32x4_unaligned __attribute__((ext_vector_type(4), aligned(1)));
+typedef int32_t i32_unaligned __attribute__((aligned(1)));
+typedef float f32x4_unaligned __attribute__((ext_vector_type(4), aligned(4)));
 
 // ---- integer requantization -------------------------------------------------
 
@@ -167,6 +172,35 @@ __device__ __forceinline__ float WaveMaxF32(float v) {
   v = fmaxf(v, DppMoveF32<kDppRowMirror>(v));
   return fmaxf(fmaxf(ReadLaneF32(v, 0), ReadLaneF32(v, 16)),
                fmaxf(ReadLaneF32(v, 32), ReadLaneF32(v, 48)));
+}
+
+// Four floats from any float's address.
+__device__ __forceinline__ float4 LoadFloat4(const float* at) {
+  const f32x4_unaligned v = *reinterpret_cast<const f32x4_unaligned*>(at);
+  return make_float4(v.x, v.y, v.z, v.w);
+}
+
+// The bytes of v from byte `skip` (0 .. 15) on, zeros behind them. With it a row of int8 values of
+// any length is read in whole 16-byte pieces: the piece that would reach past the row's end is
+// read 16 bytes before that end and shifted down (RowPieceSkip).
+__device__ __forceinline__ i32x4 ShiftBytesDown(const i32x4 v, int skip) {
+  const bool one = skip & 4, two = skip & 8;
+  const int a0 = one ? v[1] : v[0], a1 = one ? v[2] : v[1], a2 = one ? v[3] : v[2],
+            a3 = one ? 0 : v[3];
+  const int b0 = two ? a2 : a0, b1 = two ? a3 : a1, b2 = two ? 0 : a2, b3 = two ? 0 : a3;
+  const int by = skip & 3;
+  return i32x4{static_cast<int>(__builtin_amdgcn_alignbyte(b1, b0, by)),
+               static_cast<int>(__builtin_amdgcn_alignbyte(b2, b1, by)),
+               static_cast<int>(__builtin_amdgcn_alignbyte(b3, b2, by)),
+               static_cast<int>(__builtin_amdgcn_alignbyte(0, b3, by))};
+}
+// How far a piece at depth `at` of a row of `depth` >= 16 values has to be shifted when it was read
+// at min(at, depth - 16). (A piece wholly past the end: any bytes, the caller drops them.)
+__device__ __forceinline__ int RowPieceSkip(int at, int depth) {
+  return min(max(at + 16 - depth, 0), 15);
+}
+__device__ __forceinline__ i32x4 LoadRowPiece(const int8_t* row, int at, int depth) {
+  return *reinterpret_cast<const i32x4_unaligned*>(row + min(at, depth - 16));
 }
 
 // 4-way int8 dot product with int32 accumulate (v_dot4_i32_i8).

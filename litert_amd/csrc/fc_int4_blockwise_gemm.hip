@@ -113,7 +113,7 @@ __global__ __launch_bounds__(kQuantizeThreads) void QuantizeRowsTiledKernel(
   const Tile16x64Placement place{m % kTile};
   if (m < batches) {
     // EvalBlockwise4Bit always quantizes asymmetrically (fully_connected.cc:1044-1047).
-    QuantizeRow<VARIANT>(input + static_cast<size_t>(m) * depth, depth, tile_row,
+    QuantizeRow<VARIANT>(input + static_cast<size_t>(m) * depth, depth, tile_row, depth,
                          scaling_factors + m, zero_points + m, /*do_asymmetric=*/1, place);
   } else {
     for (int k = threadIdx.x * 8; k < depth; k += kQuantizeThreads * 8) {
@@ -761,7 +761,7 @@ __global__ __launch_bounds__(THREADS) void QuantizeNibbleGroupRowsKernel(
   const NibbleQuadArgs& a = table->node[node];
   QuantizeRow<VARIANT, RowMajorPlacement, THREADS>(
                        table->input_f32[node] + static_cast<size_t>(row) * a.depth, a.depth,
-                       const_cast<int8_t*>(a.rows) + static_cast<size_t>(row) * a.depth,
+                       const_cast<int8_t*>(a.rows) + static_cast<size_t>(row) * a.depth, a.depth,
                        const_cast<float*>(a.scaling_factors) + row,
                        const_cast<int32_t*>(a.zero_points) + row, /*do_asymmetric=*/1);
 }
@@ -920,7 +920,7 @@ hipError_t LaunchFcInt4BlockwiseNibbleGemm(const float* input, int variant,
   const int channel_tiles = (out_depth + kTile - 1) / kTile;
   if (batches <= 4) {
     // Row-major quantized rows (they fit where the tiled rows of a 16-row tile would lie).
-    if (hipError_t err = LaunchBatchQuantize(input, batches, depth, static_cast<int8_t*>(tiled_rows),
+    if (hipError_t err = LaunchBatchQuantize(input, batches, depth, depth, static_cast<int8_t*>(tiled_rows),
                                              scaling_factors, zero_points, /*do_asymmetric=*/1,
                                              variant, stream)) {
       return err;

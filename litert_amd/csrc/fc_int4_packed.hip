@@ -670,7 +670,7 @@ __global__ __launch_bounds__(THREADS) void QuantizeGroupRowsKernel(
   const Int4PackedArgs& a = table->node[node];
   QuantizeRow<VARIANT, RowMajorPlacement, THREADS>(
                        a.input_f32 + static_cast<size_t>(row) * a.depth, a.depth,
-                       const_cast<int8_t*>(a.input_q) + static_cast<size_t>(row) * a.depth,
+                       const_cast<int8_t*>(a.input_q) + static_cast<size_t>(row) * a.depth, a.depth,
                        const_cast<float*>(a.scaling_factors) + row,
                        const_cast<int32_t*>(a.zero_points) + row, /*do_asymmetric=*/1);
 }

@@ -74,13 +74,11 @@ struct NibbleArgs {
   int slabs;                    // padded depth / 128
 };
 
-constexpr int kFusedRows = 4;                        // rows the fused prologue quantizes
-constexpr int kFusedDepth = 4 * kThreads * 4;        // ... of at most this depth (in registers)
-constexpr int kRowStateBytes = kFusedRows * (kWaves * 3 + 4) * 4;
+constexpr int kFusedRows = 4;  // rows the fused prologue of the register-resident form quantizes
 
 size_t SharedBytes(int bt, int qstride) {
   return ((static_cast<size_t>(bt) * qstride + 15) & ~static_cast<size_t>(15)) +
-         kWaves * 64 * sizeof(i32x4) + kRowStateBytes;
+         kWaves * 64 * sizeof(i32x4);
 }
 
 // Even-position and odd-position bytes of 16 consecutive int8.
@@ -91,11 +89,7 @@ __device__ __forceinline__ void Deinterleave16(const i32x4 v, i32x2* even, i32x2
   (*odd)[1] = static_cast<int>(__builtin_amdgcn_perm(v[3], v[2], 0x07050301u));
 }
 
-// FUSED: the rows arrive as floats and the 4-bit path's row quantizer
-// (ReferenceBatchQuantizeFloats4Bit, optimized/4bit/fully_connected_reference.cc:121-180) runs
-// in the prologue of every workgroup: at most kFusedRows rows of at most kFusedDepth values,
-// depth a multiple of 4, 16-byte aligned.
-template <bool FUSED>
+// Rows arrive quantized, depth a multiple of 16 (padded rows, kernels.h) on 16-byte boundaries.
 __global__ __launch_bounds__(kThreads) void FcInt4PerChannelGemvKernel(NibbleArgs a, int batch0,
                                                                        int bt, int ksplit) {
   extern __shared__ __align__(16) int8_t smem[];
@@ -111,13 +105,6 @@ __global__ __launch_bounds__(kThreads) void FcInt4PerChannelGemvKernel(NibbleArg
   int8_t* q = smem;
   i32x4* partial = reinterpret_cast<i32x4*>(
       smem + ((static_cast<size_t>(bt) * qstride + 15) & ~static_cast<size_t>(15)));
-  // Row state of the fused form: per row and wavefront min, max and sum(q); then per row the
-  // multiplier, the stored scale and the input offset.
-  float* row_mm = reinterpret_cast<float*>(partial + kWaves * 64);  // [rows][waves][2]
-  int32_t* row_sum = reinterpret_cast<int32_t*>(row_mm + kFusedRows * kWaves * 2);  // [rows][waves]
-  float* row_mult = reinterpret_cast<float*>(row_sum + kFusedRows * kWaves);        // [rows]
-  float* row_sf = row_mult + kFusedRows;
-  int32_t* row_offset = reinterpret_cast<int32_t*>(row_sf + kFusedRows);
   const int tiles = (a.out_depth + kTileRows - 1) / kTileRows;
   const int tiles_per_wg = kWaves / ksplit;
   const int tile = blockIdx.x * tiles_per_wg + wave / ksplit;  // may run past the last group
@@ -132,8 +119,7 @@ __global__ __launch_bounds__(kThreads) void FcInt4PerChannelGemvKernel(NibbleArg
   // thread in registers, else staged before anything else) go out ahead of the weights.
   constexpr int kQRegs = 4;
   const int chunks_per_row = padded / 16;
-  const bool vec_ok = (depth % 16 == 0) && ((reinterpret_cast<uintptr_t>(a.input) & 15) == 0);
-  const bool in_regs = vec_ok && bt * chunks_per_row <= kQRegs * kThreads;
+  const bool in_regs = bt * chunks_per_row <= kQRegs * kThreads;
   // Chunk c of a row (depth 16 c .. +16): its even bytes go to slab base + 8 * (c % 8), its odd
   // bytes 64 further on.
   auto park = [&](int b, int c, const i32x4 v) {
@@ -144,18 +130,7 @@ __global__ __launch_bounds__(kThreads) void FcInt4PerChannelGemvKernel(NibbleArg
     *reinterpret_cast<i32x2*>(base + 64) = odd;
   };
   i32x4 qr[kQRegs];
-  float4 xr[FUSED ? kFusedRows : 1][4];
-  if (FUSED) {
-#pragma unroll
-    for (int b = 0; b < kFusedRows; ++b) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int i = (j * kThreads + tid) * 4;  // raw, clamped; consumed after the ring is out
-        xr[b][j] = *reinterpret_cast<const float4*>(
-            a.input_f32 + static_cast<size_t>(batch0 + min(b, bt - 1)) * depth + min(i, depth - 4));
-      }
-    }
-  } else if (in_regs) {
+  if (in_regs) {
 #pragma unroll
     for (int j = 0; j < kQRegs; ++j) {
       const int c = j * kThreads + tid;
@@ -165,17 +140,11 @@ __global__ __launch_bounds__(kThreads) void FcInt4PerChannelGemvKernel(NibbleArg
           a.input + static_cast<size_t>(batch0 + min(b, bt - 1)) * depth + min(i, depth - 16));
     }
   } else {
-    for (int b = 0; b < bt; ++b) {  // (never reached by the fused form)
+    for (int b = 0; b < bt; ++b) {
       const int8_t* x = a.input + static_cast<size_t>(batch0 + b) * depth;
       for (int c = tid; c < chunks_per_row; c += kThreads) {
         i32x4 v = {0, 0, 0, 0};
-        if (vec_ok) {
-          if (c * 16 < depth) v = *reinterpret_cast<const i32x4*>(x + c * 16);
-        } else {
-          int8_t bytes[16];
-          for (int t = 0; t < 16; ++t) bytes[t] = c * 16 + t < depth ? x[c * 16 + t] : 0;
-          v = *reinterpret_cast<const i32x4*>(bytes);
-        }
+        if (c * 16 < depth) v = *reinterpret_cast<const i32x4*>(x + c * 16);
         park(b, c, v);
       }
     }
@@ -200,77 +169,7 @@ __global__ __launch_bounds__(kThreads) void FcInt4PerChannelGemvKernel(NibbleArg
   for (int u = 0; u < kRing; ++u) {
     ring[u] = __builtin_nontemporal_load(wbase + static_cast<size_t>(min(s0 + u, slabs - 1)) * 64);
   }
-  if (FUSED) {
-#pragma unroll
-    for (int b = 0; b < kFusedRows; ++b) {
-      if (b < bt) {
-        float mn = 0.0f, mx = 0.0f;  // clamped duplicates past the row are harmless here
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float4 t = xr[b][j];
-          mn = fminf(fminf(mn, t.x), fminf(fminf(t.y, t.z), t.w));
-          mx = fmaxf(fmaxf(mx, t.x), fmaxf(fmaxf(t.y, t.z), t.w));
-        }
-        mn = WaveMinF32(mn);
-        mx = WaveMaxF32(mx);
-        if (lane == 0) {
-          row_mm[(b * kWaves + wave) * 2] = mn;
-          row_mm[(b * kWaves + wave) * 2 + 1] = mx;
-        }
-      }
-    }
-    __syncthreads();
-    if (tid < bt) {
-      float mn = row_mm[tid * kWaves * 2], mx = row_mm[tid * kWaves * 2 + 1];
-#pragma unroll
-      for (int w = 1; w < kWaves; ++w) {
-        mn = fminf(mn, row_mm[(tid * kWaves + w) * 2]);
-        mx = fmaxf(mx, row_mm[(tid * kWaves + w) * 2 + 1]);
-      }
-      float scale_denom = fmaxf(fabsf(mn), fabsf(mx));
-      if (scale_denom == 0.0f) scale_denom = 127.0f;
-      row_mult[tid] = static_cast<float>(127.0 / static_cast<double>(scale_denom));
-      row_sf[tid] = static_cast<float>(static_cast<double>(scale_denom) / 127.0);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int b = 0; b < kFusedRows; ++b) {
-      if (b < bt) {
-        const float mult = row_mult[b];
-        int32_t sum = 0;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int i = (j * kThreads + tid) * 4;  // depth of the first of four values
-          if (i < padded) {
-            int32_t o[4] = {0, 0, 0, 0};
-            if (i < depth) {
-              const float4 t = xr[b][j];
-              o[0] = static_cast<int8_t>(RoundHalfAway(__fmul_rn(t.x, mult)));
-              o[1] = static_cast<int8_t>(RoundHalfAway(__fmul_rn(t.y, mult)));
-              o[2] = static_cast<int8_t>(RoundHalfAway(__fmul_rn(t.z, mult)));
-              o[3] = static_cast<int8_t>(RoundHalfAway(__fmul_rn(t.w, mult)));
-              sum += (o[0] + o[1]) + (o[2] + o[3]);
-            }
-            // even depths to the first half of the slab's 128 bytes, odd depths to the second
-            int8_t* base = q + b * qstride + (i >> 7) * kSlabDepth + ((i & 127) >> 1);
-            *reinterpret_cast<int16_t*>(base) =
-                static_cast<int16_t>((o[0] & 0xFF) | ((o[2] & 0xFF) << 8));
-            *reinterpret_cast<int16_t*>(base + 64) =
-                static_cast<int16_t>((o[1] & 0xFF) | ((o[3] & 0xFF) << 8));
-          }
-        }
-        sum = WaveSumI32(sum);
-        if (lane == 0) row_sum[b * kWaves + wave] = sum;
-      }
-    }
-    __syncthreads();
-    if (tid < bt) {
-      int32_t total = 0;
-#pragma unroll
-      for (int w = 0; w < kWaves; ++w) total += row_sum[tid * kWaves + w];
-      row_offset[tid] = total * -7;
-    }
-  } else if (in_regs) {
+  if (in_regs) {
 #pragma unroll
     for (int j = 0; j < kQRegs; ++j) {
       const int c = j * kThreads + tid;
@@ -326,8 +225,8 @@ __global__ __launch_bounds__(kThreads) void FcInt4PerChannelGemvKernel(NibbleArg
   // Epilogue. Accumulator register i holds channel 4 * (L / 16) + i, column L % 16.
   if (col >= bt || tile >= tiles) return;
   const int b = batch0 + col;
-  const float batch_scale = FUSED ? row_sf[col] : a.scaling_factors[b];
-  const int32_t input_offset = FUSED ? row_offset[col] : a.input_offsets[b];
+  const float batch_scale = a.scaling_factors[b];
+  const int32_t input_offset = a.input_offsets[b];
   const int32_t sum_q = -(input_offset / 7);  // exact: the offset is -7 * sum(q)
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -369,18 +268,6 @@ static_assert(3 * sizeof(void*) + 7 * sizeof(int) <= kResidentArgsOffset &&
 size_t ResidentSharedBytes(int bt, int qstride) {
   return ((static_cast<size_t>(bt) * qstride + 15) & ~static_cast<size_t>(15)) + 128 +
          kWaves * 64 * sizeof(i32x4) + kFusedRows * 8;
-}
-
-// Four values of a row times its multiplier, rounded half away from zero, as four bytes (the
-// saturation of v_cvt_pk_u8_f32 on value + 128 never binds: |v * mult| < 127.5).
-__device__ __forceinline__ uint32_t QuantizeSymmetricPack4(float a, float b, float c, float d,
-                                                           float mult) {
-  uint32_t w = 0;
-  w = __builtin_amdgcn_cvt_pk_u8_f32(__fadd_rn(RoundHalfAway(__fmul_rn(a, mult)), 128.0f), 0, w);
-  w = __builtin_amdgcn_cvt_pk_u8_f32(__fadd_rn(RoundHalfAway(__fmul_rn(b, mult)), 128.0f), 1, w);
-  w = __builtin_amdgcn_cvt_pk_u8_f32(__fadd_rn(RoundHalfAway(__fmul_rn(c, mult)), 128.0f), 2, w);
-  w = __builtin_amdgcn_cvt_pk_u8_f32(__fadd_rn(RoundHalfAway(__fmul_rn(d, mult)), 128.0f), 3, w);
-  return w ^ 0x80808080u;
 }
 
 template <bool FUSED, int TILES, int QREGS>
@@ -533,8 +420,8 @@ void FcInt4PerChannelResidentKernel(const uint8_t* early_packed, const float* ea
 #pragma unroll
       for (int j = 0; j < kPieces; ++j) {
         const int i = (j * kWaveSize + lane) * 8;
-        xr[j][0] = *reinterpret_cast<const float4*>(x + min(i, depth - 4));
-        xr[j][1] = *reinterpret_cast<const float4*>(x + min(i + 4, depth - 4));
+        xr[j][0] = LoadFloat4(x + min(i, depth - 4));
+        xr[j][1] = LoadFloat4(x + min(i + 4, depth - 4));
       }
       __builtin_amdgcn_sched_barrier(0);
       // Every wavefront of a workgroup with four rows has one: some weights go out ahead of the
@@ -563,14 +450,17 @@ void FcInt4PerChannelResidentKernel(const uint8_t* early_packed, const float* ea
 #pragma unroll
       for (int j = 0; j < kPieces; ++j) {
         const int i = (j * kWaveSize + lane) * 8;  // depth of the first of eight values
-        const float4 a = xr[j][0], b = xr[j][1];
+        float4 a = xr[j][0], b = xr[j][1];
+        if (i + 8 > depth) {
+          // The row ends in this piece or before it. A depth of 4 n + 2 leaves two values in its
+          // last four, read two places early; values past the row are zeros.
+          const float4 none = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+          if (i + 4 > depth) a = i < depth ? make_float4(a.z, a.w, 0.0f, 0.0f) : none;
+          b = i + 4 < depth ? make_float4(b.z, b.w, 0.0f, 0.0f) : none;
+        }
         // Even depths to the first half of the slab's 128 bytes, odd depths to the second.
         uint32_t even = QuantizeSymmetricPack4(a.x, a.z, b.x, b.z, mult);
         uint32_t odd = QuantizeSymmetricPack4(a.y, a.w, b.y, b.w, mult);
-        if (i + 4 >= depth) {  // the second four (or all eight) lie past the row
-          even &= i < depth ? 0x0000FFFFu : 0u;
-          odd &= i < depth ? 0x0000FFFFu : 0u;
-        }
         sum = __builtin_amdgcn_sdot4(static_cast<int>(even), 0x01010101, sum, false);
         sum = __builtin_amdgcn_sdot4(static_cast<int>(odd), 0x01010101, sum, false);
         if (i < staged) {
@@ -698,14 +588,11 @@ hipError_t TryLaunchResident(const NibbleArgs& a, int batch0, int bt, hipStream_
   const int staged = ksplit * per_part * kSlabDepth;
   if (FUSED) {
     if (bt > kFusedRows || a.depth > kResidentRowDepth || staged > kResidentRowDepth ||
-        a.depth % 4 != 0 || a.depth < 4 || (reinterpret_cast<uintptr_t>(a.input_f32) & 15) != 0) {
+        a.depth < 4) {
       return hipSuccess;
     }
   } else {
-    if (a.depth % 16 != 0 || a.depth < 16 || (reinterpret_cast<uintptr_t>(a.input) & 15) != 0 ||
-        static_cast<int64_t>(bt) * (staged / 16) > 16 * kThreads) {
-      return hipSuccess;
-    }
+    if (static_cast<int64_t>(bt) * (staged / 16) > 16 * kThreads) return hipSuccess;
   }
   if (ResidentSharedBytes(bt, staged + kQPad) > 150 * 1024) return hipSuccess;
   *launched = true;
@@ -792,7 +679,8 @@ hipError_t LaunchFcInt4PerChannelGemv(const uint8_t* packed, const float* input_
       continue;
     }
     const size_t lds = SharedBytes(bt, qstride);
-    auto kernel = fused ? FcInt4PerChannelGemvKernel<true> : FcInt4PerChannelGemvKernel<false>;
+    if (fused) return hipErrorNotSupported;  // FcInt4PerChannelGemvFuses admits only what fits above
+    auto kernel = FcInt4PerChannelGemvKernel;
     if (hipError_t err = EnsureDynamicLds(reinterpret_cast<const void*>(kernel), lds)) return err;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), lds, stream, a, batch0, bt, ksplit);
     if (hipError_t err = hipGetLastError()) return err;
@@ -802,8 +690,7 @@ hipError_t LaunchFcInt4PerChannelGemv(const uint8_t* packed, const float* input_
 }
 
 bool FcInt4PerChannelGemvFuses(const float* input_f32, int batches, int depth) {
-  return batches <= kFusedRows && depth <= kFusedDepth && depth % 4 == 0 &&
-         (reinterpret_cast<uintptr_t>(input_f32) & 15) == 0;
+  return input_f32 != nullptr && batches <= kFusedRows && depth >= 4 && depth <= kResidentRowDepth;
 }
 
 }  // namespace lrtfc

@@ -22,8 +22,8 @@
 // (batches of a few dozen to a few hundred rows) run the same kernel with 64 rows x 128
 // channels per workgroup (32 channels per wavefront).
 //
-// The int8 outputs of an interior tile are put together in LDS (the row buffers, free by then)
-// and stored in 16-byte pieces, whole cache lines per row.
+// The outputs of a tile are put together in LDS (the row buffers, free by then) and stored in
+// 16-byte pieces, whole cache lines per row.
 //
 // int32 accumulation is exact, so tiling cannot change the accumulator; bit-exactness rests
 // on the epilogues, which are the ones of the GEMV kernels (fc_epilogues.h).
@@ -54,8 +54,10 @@ __device__ __forceinline__ void ForEachConst(std::integer_sequence<int, Is...>, 
 }
 
 // BM: batch rows per workgroup (128, or 64 for launches the large tile would leave with few
-// workgroups); kWaveTiles: 32-channel MFMA tiles per wavefront (2 or 1).
-template <Int8Epilogue EPI, int BM, int kWaveTiles>
+// workgroups); kWaveTiles: 32-channel MFMA tiles per wavefront (2 or 1); kRagged: the depth is no
+// multiple of 16, so the last piece of every row is shifted into place on its way to LDS (a
+// form of its own: a test for it inside the steps would break their straight line).
+template <Int8Epilogue EPI, int BM, int kWaveTiles, bool kRagged>
 __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args a) {
   constexpr int BN = kWaves * kWaveTiles * 32;  // output channels per workgroup
   constexpr int kStageBytes = BM * kXStride;
@@ -144,6 +146,9 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
   // An odd number of slabs leaves the second half of the last step without a filter tile: the
   // weight addresses are clamped to the last tile and the rows' half is staged as zeros.
   const bool upper_chunk = ld_chunk >= 4;
+  // The piece a row ends in lies in this step and is shifted by this many bytes (kRagged).
+  const int ragged_step = K / kStep;
+  const int ragged_skip = RowPieceSkip(ragged_step * kStep + ld_chunk * 16, K);
   const int half_step = (slabs & 1) ? steps - 1 : -1;
 
   // Weights: wring[step % 2] holds a step's operands; a piece is requested again, for two steps
@@ -163,11 +168,12 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
     // zeros when staged, or is never used.
     const int k = min(min(step, steps - 1) * kStep + ld_chunk * 16, K - 16);
     xr[decltype(set)::value][decltype(piece)::value] =
-        *reinterpret_cast<const i32x4*>(xp[decltype(piece)::value] + k);
+        *reinterpret_cast<const i32x4_unaligned*>(xp[decltype(piece)::value] + k);
   };
   auto store_x_piece = [&](int step, auto set, auto piece) {
     constexpr int p = decltype(piece)::value;
     i32x4 v = xr[decltype(set)::value][p];
+    if (kRagged) v = ShiftBytesDown(v, step == ragged_step ? ragged_skip : 0);
     if (upper_chunk && step == half_step) v = i32x4{0, 0, 0, 0};
     *reinterpret_cast<i32x4*>(smem + decltype(set)::value * kStageBytes + st_off +
                               p * 32 * kXStride) = v;
@@ -285,29 +291,27 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
   // the wavefront's 64 and batch row 32 j + L % 32 of the workgroup's 128: four groups (g) of
   // four consecutive channels per lane and tile.
   const int row_in_tile = lane & 31;
-  const bool vec_ok = (N & 3) == 0;
   // The clamp bounds in vector registers: v_med3_i32 takes at most one scalar operand.
   int32_t act_lo = a.act_min, act_hi = a.act_max;
   asm volatile("" : "+v"(act_lo), "+v"(act_hi));
-  // Interior tiles (the common case) store whole dwords without any bounds test.
-  // kStaged (int8 outputs of an interior tile): the tile is put together in LDS and leaves in
-  // 16-byte pieces, sixteen lanes to a row, i.e. in whole cache lines. Stored from the
-  // accumulator layout a store instruction touches 32 rows with 8 bytes each, and the 8 MB of
-  // config 4's output reach L2 as a million partial-line writes behind the last MFMA.
+  // The outputs of a tile are put together in LDS (the row buffers, free by now) and leave in
+  // 16-byte pieces, neighbouring lanes on neighbouring pieces of a row, i.e. in whole cache
+  // lines. Stored from the accumulator layout a store instruction touches 32 rows with 8 bytes
+  // each, and the 8 MB of config 4's output reach L2 as a million partial-line writes behind the
+  // last MFMA. kFull: an interior tile, no bounds test; tiles at the edge store what lies inside,
+  // the last piece of a row value by value. Rows of any length start on any byte (an int8 output
+  // of an odd channel count): the pieces' addresses need no alignment.
   constexpr int kOutStride = BN + 16;
   static_assert(BM * kOutStride <= 2 * kStageBytes, "output tile does not fit the row buffers");
-  auto epilogue = [&](auto full_tag, auto short_tag, auto staged_tag) {
-  constexpr bool kFull = decltype(full_tag)::value;
-  constexpr bool kShort = decltype(short_tag)::value;
-  constexpr bool kStaged = decltype(staged_tag)::value;
-  if (kStaged) __syncthreads();  // every wavefront has read its last row operands
+  auto epilogue_int8 = [&](auto full_tag, auto short_tag) {
+    constexpr bool kFull = decltype(full_tag)::value;
+    constexpr bool kShort = decltype(short_tag)::value;
+    __syncthreads();  // every wavefront has read its last row operands
 #pragma unroll
-  for (int i = 0; i < kWaveTiles; ++i) {
+    for (int i = 0; i < kWaveTiles; ++i) {
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int c0 = n0 + (wave * kWaveTiles + i) * 32 + 8 * g + 4 * (lane >> 5);
-      const int local = (wave * kWaveTiles + i) * 32 + 8 * g + 4 * (lane >> 5);
-      if (EPI == Int8Epilogue::kRequantize) {
+      for (int g = 0; g < 4; ++g) {
+        const int local = (wave * kWaveTiles + i) * 32 + 8 * g + 4 * (lane >> 5);
         int32_t mult[4], shift[4], addend[4], half[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -319,7 +323,6 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
         }
 #pragma unroll
         for (int j = 0; j < kBatchTiles; ++j) {
-          const int m = m0 + j * 32 + row_in_tile;
           int32_t q[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
@@ -328,83 +331,37 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
                           : RequantizeCore(acc[i][j][4 * g + r] + addend[r], mult[r], shift[r],
                                            a.output_offset, a.act_min, a.act_max);
           }
-          if (kStaged) {
-            *reinterpret_cast<int32_t*>(smem + (j * 32 + row_in_tile) * kOutStride + local) =
-                PackLowBytes(q[0], q[1], q[2], q[3]);
-          } else if (kFull || m < M) {
-            int8_t* dst = a.output_i8 + static_cast<size_t>(m) * N + c0;
-            if (kFull || (vec_ok && c0 + 3 < N)) {
-              *reinterpret_cast<int32_t*>(dst) = PackLowBytes(q[0], q[1], q[2], q[3]);
-            } else {
-#pragma unroll
-              for (int r = 0; r < 4; ++r) {
-                if (c0 + r < N) dst[r] = static_cast<int8_t>(q[r]);
-              }
-            }
-          }
-        }
-      } else {
-        float cscale[4], base[4];
-        int32_t rsum[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const i32x4 p = chan_params[local + r];
-          cscale[r] = __int_as_float(p[0]);
-          base[r] = __int_as_float(p[1]);
-          rsum[r] = p[2];
-        }
-#pragma unroll
-        for (int j = 0; j < kBatchTiles; ++j) {
-          const int m = m0 + j * 32 + row_in_tile;
-          const int mc = min(m, M - 1);
-          const float bscale = a.scaling_factors[mc];
-          const int32_t bzp = a.zero_points ? a.zero_points[mc] : 0;
-          float v[4];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            v[r] = EPI == Int8Epilogue::kHybrid4Bit
-                       ? Hybrid4BitCore(acc[i][j][4 * g + r], bscale, cscale[r], bzp, base[r],
-                                        a.bias_f32 != nullptr, a.activation)
-                       : HybridCoreSelect(acc[i][j][4 * g + r], bscale, cscale[r], bzp, rsum[r],
-                                          base[r], a.activation, a.batch_matmul != 0, zero_input);
-          }
-          if (kFull || m < M) {
-            float* dst = a.output_f32 + static_cast<size_t>(m) * N + c0;
-            if (kFull || (vec_ok && c0 + 3 < N)) {
-              *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
-            } else {
-#pragma unroll
-              for (int r = 0; r < 4; ++r) {
-                if (c0 + r < N) dst[r] = v[r];
-              }
-            }
-          }
+          *reinterpret_cast<int32_t*>(smem + (j * 32 + row_in_tile) * kOutStride + local) =
+              PackLowBytes(q[0], q[1], q[2], q[3]);
         }
       }
     }
-  }
-  if (kStaged) {
     __syncthreads();
     constexpr int kPiecesPerRow = BN / 16;
 #pragma unroll
     for (int k = 0; k < BM * kPiecesPerRow / kThreads; ++k) {
       const int piece = k * kThreads + tid;
       const int row = piece / kPiecesPerRow, at = (piece % kPiecesPerRow) * 16;
-      *reinterpret_cast<i32x4*>(a.output_i8 + static_cast<size_t>(m0 + row) * N + n0 + at) =
-          *reinterpret_cast<const i32x4*>(smem + row * kOutStride + at);
+      const int8_t* from = smem + row * kOutStride + at;
+      int8_t* to = a.output_i8 + static_cast<size_t>(m0 + row) * N + n0 + at;
+      const int inside = kFull ? 16 : (m0 + row < M ? N - (n0 + at) : 0);
+      if (inside >= 16) {
+        *reinterpret_cast<i32x4_unaligned*>(to) = *reinterpret_cast<const i32x4*>(from);
+      } else {
+        for (int b = 0; b < inside; ++b) to[b] = from[b];
+      }
     }
-  }
   };
-  // The float outputs of an interior tile take the same way, 32 rows (one batch tile) at a time:
-  // a wavefront then stores one row's whole kilobyte per instruction instead of 32 bytes in each
-  // of 32 rows.
-  auto epilogue_float_staged = [&]() {
+  // Float outputs go 32 rows (one batch tile) at a time: a wavefront then stores one row's whole
+  // kilobyte per instruction instead of 32 bytes in each of 32 rows.
+  auto epilogue_float = [&](auto full_tag) {
+    constexpr bool kFull = decltype(full_tag)::value;
     constexpr int kRowBytes = BN * 4 + 16;
     static_assert(32 * kRowBytes <= 2 * kStageBytes, "a batch tile of floats does not fit");
     constexpr int kPiecesPerRow = BN / 4;
 #pragma unroll
     for (int j = 0; j < kBatchTiles; ++j) {
-      const int m = m0 + j * 32 + row_in_tile;
+      const int m = kFull ? m0 + j * 32 + row_in_tile : min(m0 + j * 32 + row_in_tile, M - 1);
       const float bscale = a.scaling_factors[m];
       const int32_t bzp = a.zero_points ? a.zero_points[m] : 0;
       __syncthreads();  // the buffer's last readers (main loop, previous batch tile) are through
@@ -432,49 +389,55 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
 #pragma unroll
       for (int k = 0; k < 32 * kPiecesPerRow / kThreads; ++k) {
         const int piece = k * kThreads + tid;
-        const int row = piece / kPiecesPerRow, at = (piece % kPiecesPerRow) * 16;
-        *reinterpret_cast<i32x4*>(reinterpret_cast<int8_t*>(a.output_f32) +
-                                  (static_cast<size_t>(m0 + j * 32 + row) * N + n0) * 4 + at) =
-            *reinterpret_cast<const i32x4*>(smem + row * kRowBytes + at);
+        const int row = piece / kPiecesPerRow, at = (piece % kPiecesPerRow) * 4;
+        const float* from = reinterpret_cast<const float*>(smem + row * kRowBytes) + at;
+        float* to = a.output_f32 + static_cast<size_t>(m0 + j * 32 + row) * N + n0 + at;
+        const int inside = kFull ? 4 : (m0 + j * 32 + row < M ? N - (n0 + at) : 0);
+        if (inside >= 4) {
+          *reinterpret_cast<f32x4_unaligned*>(to) = *reinterpret_cast<const f32x4_unaligned*>(from);
+        } else {
+          for (int c = 0; c < inside; ++c) to[c] = from[c];
+        }
       }
     }
   };
-  const bool interior = vec_ok && m0 + BM <= M && n0 + BN <= N;
-  if (EPI != Int8Epilogue::kRequantize && interior &&
-      (reinterpret_cast<uintptr_t>(a.output_f32) & 15) == 0) {
-    epilogue_float_staged();
-    return;
-  }
-  if (EPI == Int8Epilogue::kRequantize && !general_requantize) {
-    const bool staged =
-        interior && (N & 15) == 0 && (reinterpret_cast<uintptr_t>(a.output_i8) & 15) == 0;
-    if (staged) {
-      epilogue(std::true_type{}, std::true_type{}, std::true_type{});
-    } else if (interior) {
-      epilogue(std::true_type{}, std::true_type{}, std::false_type{});
+  const bool interior = m0 + BM <= M && n0 + BN <= N;
+  if (EPI != Int8Epilogue::kRequantize) {
+    if (interior) {
+      epilogue_float(std::true_type{});
     } else {
-      epilogue(std::false_type{}, std::true_type{}, std::false_type{});
+      epilogue_float(std::false_type{});
     }
-  } else if (interior) {
-    epilogue(std::true_type{}, std::false_type{}, std::false_type{});
+  } else if (!general_requantize) {
+    if (interior) {
+      epilogue_int8(std::true_type{}, std::true_type{});
+    } else {
+      epilogue_int8(std::false_type{}, std::true_type{});
+    }
   } else {
-    epilogue(std::false_type{}, std::false_type{}, std::false_type{});
+    epilogue_int8(std::false_type{}, std::false_type{});
   }
+}
+
+template <int BM, int kWaveTiles, bool kRagged>
+hipError_t LaunchForm(const FcInt8Args& a, Int8Epilogue epilogue, int grid, hipStream_t stream) {
+  if (epilogue == Int8Epilogue::kRequantize) {
+    hipLaunchKernelGGL((FcInt8PackedGemmKernel<Int8Epilogue::kRequantize, BM, kWaveTiles, kRagged>),
+                       dim3(grid), dim3(kThreads), 0, stream, a);
+  } else if (epilogue == Int8Epilogue::kHybrid) {
+    hipLaunchKernelGGL((FcInt8PackedGemmKernel<Int8Epilogue::kHybrid, BM, kWaveTiles, kRagged>),
+                       dim3(grid), dim3(kThreads), 0, stream, a);
+  } else {
+    hipLaunchKernelGGL((FcInt8PackedGemmKernel<Int8Epilogue::kHybrid4Bit, BM, kWaveTiles, kRagged>),
+                       dim3(grid), dim3(kThreads), 0, stream, a);
+  }
+  return hipGetLastError();
 }
 
 template <int BM, int kWaveTiles>
 hipError_t LaunchShape(const FcInt8Args& a, Int8Epilogue epilogue, int grid, hipStream_t stream) {
-  if (epilogue == Int8Epilogue::kRequantize) {
-    hipLaunchKernelGGL((FcInt8PackedGemmKernel<Int8Epilogue::kRequantize, BM, kWaveTiles>),
-                       dim3(grid), dim3(kThreads), 0, stream, a);
-  } else if (epilogue == Int8Epilogue::kHybrid) {
-    hipLaunchKernelGGL((FcInt8PackedGemmKernel<Int8Epilogue::kHybrid, BM, kWaveTiles>),
-                       dim3(grid), dim3(kThreads), 0, stream, a);
-  } else {
-    hipLaunchKernelGGL((FcInt8PackedGemmKernel<Int8Epilogue::kHybrid4Bit, BM, kWaveTiles>),
-                       dim3(grid), dim3(kThreads), 0, stream, a);
-  }
-  return hipGetLastError();
+  return a.depth % 16 ? LaunchForm<BM, kWaveTiles, true>(a, epilogue, grid, stream)
+                      : LaunchForm<BM, kWaveTiles, false>(a, epilogue, grid, stream);
 }
 
 constexpr int kMinLargeTiles = 128;
@@ -482,9 +445,8 @@ constexpr int kMinLargeTiles = 128;
 }  // namespace
 
 bool FcInt8PackedGemmSupports(const FcInt8Args& a) {
-  return a.depth >= 16 && a.depth % 16 == 0 && a.filter_offset == 0 && a.batches > 0 &&
-         a.out_depth > 0 && ((reinterpret_cast<uintptr_t>(a.filter) & 15) == 0) &&
-         ((reinterpret_cast<uintptr_t>(a.input) & 15) == 0);
+  return a.depth >= 16 && a.filter_offset == 0 && a.batches > 0 && a.out_depth > 0 &&
+         (reinterpret_cast<uintptr_t>(a.filter) & 15) == 0;
 }
 
 hipError_t LaunchFcInt8PackedGemm(const FcInt8Args& a, Int8Epilogue epilogue, hipStream_t stream) {

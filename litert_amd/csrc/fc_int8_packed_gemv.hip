@@ -60,6 +60,12 @@ __global__ __launch_bounds__(kThreads) void PackInt8FilterKernel(const int8_t* _
   *reinterpret_cast<i32x4*>(dst + c * 16) = *reinterpret_cast<const i32x4*>(out);
 }
 
+// Four quantized values of which the first `over` belong to the piece before (a row's last piece,
+// read four values before the row's end): the others, zeros behind them.
+__device__ __forceinline__ int32_t DropBytes(int32_t packed, int over) {
+  return static_cast<int32_t>(static_cast<uint32_t>(packed) >> (8 * min(max(over, 0), 3)));
+}
+
 struct PackedArgs {
   FcInt8Args a;            // a.filter is the packed filter; a.input the int8 rows (unfused)
   const float* input_f32;  // fused form: float rows to quantize in the prologue
@@ -154,8 +160,7 @@ __global__ __launch_bounds__(kThreads) void FcInt8PackedGemvKernel(
   i32x4 qr[kQRegs];
   bool in_regs = false;
   if (FUSED) {
-    const bool vec_ok =
-        (depth % 4 == 0) && ((reinterpret_cast<uintptr_t>(early_input_f32) & 15) == 0);
+    const bool vec_ok = depth >= 4;
     in_regs = vec_ok && bt <= REG_ROWS && depth <= kXRegs * kThreads * 4;
     if (in_regs) {
 #pragma unroll
@@ -164,9 +169,9 @@ __global__ __launch_bounds__(kThreads) void FcInt8PackedGemvKernel(
         for (int j = 0; j < kXRegs; ++j) {
           const int i = (j * kThreads + tid) * 4;
           // Raw, clamped load; nothing may consume it before the weight loads are out.
-          xr[b][j] = *reinterpret_cast<const float4*>(
-              early_input_f32 + static_cast<size_t>(batch0 + min(b, bt - 1)) * depth +
-              min(i, depth - 4));
+          xr[b][j] = LoadFloat4(early_input_f32 +
+                                static_cast<size_t>(batch0 + min(b, bt - 1)) * depth +
+                                min(i, depth - 4));
         }
       }
     } else {
@@ -176,7 +181,7 @@ __global__ __launch_bounds__(kThreads) void FcInt8PackedGemvKernel(
         float mn = 0.0f, mx = 0.0f;
         if (vec_ok) {
           for (int i = tid * 4; i < depth; i += kThreads * 4) {
-            const float4 t = *reinterpret_cast<const float4*>(x + i);
+            const float4 t = LoadFloat4(x + min(i, depth - 4));
             mn = fminf(fminf(mn, t.x), fminf(fminf(t.y, t.z), t.w));
             mx = fmaxf(fmaxf(mx, t.x), fmaxf(fmaxf(t.y, t.z), t.w));
           }
@@ -195,7 +200,7 @@ __global__ __launch_bounds__(kThreads) void FcInt8PackedGemvKernel(
       }
     }
   } else {
-    const bool vec_ok = (depth % 16 == 0) && ((reinterpret_cast<uintptr_t>(a.input) & 15) == 0);
+    const bool vec_ok = depth >= 16;
     in_regs = vec_ok && bt * (padded / 16) <= kQRegs * kThreads;
     if (in_regs) {
       const int chunks_per_row = padded / 16;
@@ -204,8 +209,8 @@ __global__ __launch_bounds__(kThreads) void FcInt8PackedGemvKernel(
         const int c = j * kThreads + tid;
         const int b = c / chunks_per_row;
         const int i = (c - b * chunks_per_row) * 16;
-        qr[j] = *reinterpret_cast<const i32x4*>(
-            a.input + static_cast<size_t>(batch0 + min(b, bt - 1)) * depth + min(i, depth - 16));
+        qr[j] = LoadRowPiece(a.input + static_cast<size_t>(batch0 + min(b, bt - 1)) * depth, i,
+                             depth);
       }
     } else {
       for (int b = 0; b < bt; ++b) {
@@ -214,7 +219,7 @@ __global__ __launch_bounds__(kThreads) void FcInt8PackedGemvKernel(
         if (vec_ok) {
           for (int i = tid * 16; i < padded; i += kThreads * 16) {
             i32x4 v = {0, 0, 0, 0};
-            if (i < depth) v = *reinterpret_cast<const i32x4*>(x + i);
+            if (i < depth) v = ShiftBytesDown(LoadRowPiece(x, i, depth), RowPieceSkip(i, depth));
             *reinterpret_cast<i32x4*>(qrow + i) = v;
           }
         } else {
@@ -326,7 +331,8 @@ __global__ __launch_bounds__(kThreads) void FcInt8PackedGemvKernel(
               if (i < depth) {
                 const float4 t = xr[b][j];
                 const bool tail = i >= vector_end;
-                packed = QuantizePack4<VARIANT>(t.x, t.y, t.z, t.w, qp, tail);
+                packed = DropBytes(QuantizePack4<VARIANT>(t.x, t.y, t.z, t.w, qp, tail),
+                                   i + 4 - depth);
               }
               *reinterpret_cast<int32_t*>(qrow + i) = packed;
             }
@@ -334,8 +340,7 @@ __global__ __launch_bounds__(kThreads) void FcInt8PackedGemvKernel(
         }
       }
     } else {
-      const bool vec_ok =
-          (depth % 4 == 0) && ((reinterpret_cast<uintptr_t>(p.input_f32) & 15) == 0);
+      const bool vec_ok = depth >= 4;
       for (int b = 0; b < bt; ++b) {
         const float* x = p.input_f32 + static_cast<size_t>(batch0 + b) * depth;
         RowQuantParams qp;
@@ -348,9 +353,10 @@ __global__ __launch_bounds__(kThreads) void FcInt8PackedGemvKernel(
           for (int i = tid * 4; i < padded; i += kThreads * 4) {
             int32_t packed = 0;
             if (i < depth) {
-              const float4 t = *reinterpret_cast<const float4*>(x + i);
+              const float4 t = LoadFloat4(x + min(i, depth - 4));
               const bool tail = i >= vector_end;
-              packed = QuantizePack4<VARIANT>(t.x, t.y, t.z, t.w, qp, tail);
+              packed = DropBytes(QuantizePack4<VARIANT>(t.x, t.y, t.z, t.w, qp, tail),
+                                 i + 4 - depth);
             }
             *reinterpret_cast<int32_t*>(qrow + i) = packed;
           }
@@ -371,7 +377,8 @@ __global__ __launch_bounds__(kThreads) void FcInt8PackedGemvKernel(
       const int b = c / chunks_per_row;
       const int i = (c - b * chunks_per_row) * 16;
       if (b < bt) {
-        *reinterpret_cast<i32x4*>(sh.q + b * qstride + i) = i < depth ? qr[j] : i32x4{0, 0, 0, 0};
+        *reinterpret_cast<i32x4*>(sh.q + b * qstride + i) =
+            i < depth ? ShiftBytesDown(qr[j], RowPieceSkip(i, depth)) : i32x4{0, 0, 0, 0};
       }
     }
   }
@@ -729,7 +736,7 @@ void FcInt8ResidentGemvKernel(
 #pragma unroll
       for (int j = 0; j < kPieces; ++j) {
         const int i = (j * kWaveSize + lane) * 4;
-        xr[j] = *reinterpret_cast<const float4*>(x + min(i, depth - 4));
+        xr[j] = LoadFloat4(x + min(i, depth - 4));
       }
       __builtin_amdgcn_sched_barrier(0);
       if (EARLY) {
@@ -768,7 +775,7 @@ void FcInt8ResidentGemvKernel(
           const float4 t = xr[j];
           int32_t packed =
               QuantizePack4<VARIANT>(t.x, t.y, t.z, t.w, qp, kWhole ? false : i >= vector_end);
-          if (!kWhole) packed = i < depth ? packed : 0;
+          if (!kWhole) packed = i < depth ? DropBytes(packed, i + 4 - depth) : 0;
           if (kWhole || i < staged) *reinterpret_cast<int32_t*>(qrow + i) = packed;
         }
       };
@@ -802,20 +809,30 @@ void FcInt8ResidentGemvKernel(
       const int c = j * (WAVES * kWaveSize) + tid;
       const int b = min(c / chunks_per_row, bt - 1);
       const int i = (c % chunks_per_row) * 16;
-      qr[j] = *reinterpret_cast<const i32x4*>(
-          early_input_i8 + static_cast<size_t>(batch0 + b) * depth + min(i, depth - 16));
+      qr[j] = LoadRowPiece(early_input_i8 + static_cast<size_t>(batch0 + b) * depth, i, depth);
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < kFirst; ++u) request(u);
+    auto stage_rows = [&](auto ragged_c) {
 #pragma unroll
-    for (int j = 0; j < kQRegs; ++j) {
-      const int c = j * (WAVES * kWaveSize) + tid;
-      const int b = c / chunks_per_row;
-      const int i = (c % chunks_per_row) * 16;
-      if (b < bt) {
-        *reinterpret_cast<i32x4*>(sh.q + b * qstride + i) = i < depth ? qr[j] : i32x4{0, 0, 0, 0};
+      for (int j = 0; j < kQRegs; ++j) {
+        const int c = j * (WAVES * kWaveSize) + tid;
+        const int b = c / chunks_per_row;
+        const int i = (c % chunks_per_row) * 16;
+        i32x4 piece = qr[j];
+        if (decltype(ragged_c)::value) piece = ShiftBytesDown(piece, RowPieceSkip(i, depth));
+        if (b < bt) {
+          *reinterpret_cast<i32x4*>(sh.q + b * qstride + i) = i < depth ? piece : i32x4{0, 0, 0, 0};
+        }
       }
+    };
+    // Rows that end inside a piece need it shifted; the test stands outside the loop, so that the
+    // pieces of the others still go out side by side.
+    if (depth & 15) {
+      stage_rows(std::true_type{});
+    } else {
+      stage_rows(std::false_type{});
     }
     __builtin_amdgcn_sched_barrier(0);
     stream(integral_constant<int, kFirst>{}, integral_constant<int, kStreamAhead>{});
@@ -974,7 +991,7 @@ hipError_t LaunchResidentSized(const PackedArgs& p, int batch0, int bt, int kspl
 // image (32 x depth) fits one compute unit. *ksplit receives the depth split.
 bool ResidentTwoRowTilesFit(const PackedArgs& p, int bt, int* ksplit_out) {
   if (bt <= 16 || bt > 32) return false;
-  if (p.a.depth % 16 != 0 || (reinterpret_cast<uintptr_t>(p.a.input) & 15) != 0) return false;
+  if (p.a.depth < 16) return false;
   // The rows' image leaves room for one workgroup per compute unit, and every workgroup stages
   // the whole image: the fewest workgroups that still cover the chip in one round win (measured
   // at 14336 x 4096, 32 rows: shares of 32 tiles, 224 workgroups, 17.6 us for quantizer +
@@ -1019,9 +1036,7 @@ hipError_t TryLaunchResident(const PackedArgs& p, int batch0, int bt, hipStream_
     }
   }
   if (FUSED) {
-    const bool vec_ok =
-        (depth % 4 == 0) && ((reinterpret_cast<uintptr_t>(p.input_f32) & 15) == 0);
-    if (!vec_ok || depth > kFusedRowMaxDepth || depth < 4 || bt > kFusedMaxRows) return hipSuccess;
+    if (depth > kFusedRowMaxDepth || depth < 4 || bt > kFusedMaxRows) return hipSuccess;
     if (bt > 1) {
       int ksplit = 1;
       while ((p.slabs + ksplit - 1) / ksplit > 16) ksplit *= 2;  // depth <= 4096: at most 4
@@ -1043,9 +1058,8 @@ hipError_t TryLaunchResident(const PackedArgs& p, int batch0, int bt, hipStream_
   if (per_part > 32) return hipSuccess;
   bool many_rows = false;
   if (!FUSED) {
-    const bool vec_ok = (depth % 16 == 0) && ((reinterpret_cast<uintptr_t>(p.a.input) & 15) == 0);
     const int64_t chunks = static_cast<int64_t>(bt) * (ksplit * per_part * kSlabDepth / 16);
-    if (!vec_ok || chunks > 16 * kThreads) return hipSuccess;
+    if (depth < 16 || chunks > 16 * kThreads) return hipSuccess;
     many_rows = chunks > 4 * kThreads;
   }
   *launched = true;
@@ -1152,7 +1166,7 @@ hipError_t LaunchPackInt8Filter(const int8_t* filter, int out_depth, int depth, 
 int FcInt8PackedGemvFusedMaxRows(int depth) {
   // Eight rows where a wavefront can hold a whole row (the register-resident form: one wavefront
   // of eight per row); four on deeper rows, which every wavefront of a workgroup quantizes.
-  return (depth % 4 == 0 && depth <= kFusedRowMaxDepth) ? kFusedMaxRows : 4;
+  return (depth >= 4 && depth <= kFusedRowMaxDepth) ? kFusedMaxRows : 4;
 }
 
 bool FcInt8PackedGemvTakesRowsInOnePass(const FcInt8Args& a) {

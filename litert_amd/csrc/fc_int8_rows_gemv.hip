@@ -45,7 +45,8 @@ struct RowsShape {
   static_assert(kRowsWaves * 2 * RT * 1024 <= 2 * kBufferBytes, "partial sums do not fit");
 };
 
-template <Int8Epilogue EPI, int RT>
+// RAGGED: the depth is no multiple of 16, and the rows' last pieces are shifted into place.
+template <Int8Epilogue EPI, int RT, bool RAGGED>
 __global__ __launch_bounds__(kRowsThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void FcInt8RowsGemvKernel(FcInt8Args a, int slabs, int batch0, int bt) {
   using S = RowsShape<RT>;
@@ -87,7 +88,7 @@ void FcInt8RowsGemvKernel(FcInt8Args a, int slabs, int batch0, int bt) {
       const int at = c * S::kChunkSlabs * kSlabDepth + (p % kPiecesPerRow) * 16;
       const size_t from = c < chunks ? static_cast<size_t>(batch0 + row) * depth + min(at, depth - 16)
                                      : static_cast<size_t>(batch0) * depth;
-      staged[j] = *reinterpret_cast<const i32x4*>(a.input + from);
+      staged[j] = *reinterpret_cast<const i32x4_unaligned*>(a.input + from);
     }
   };
   auto store_rows = [&](int c, int8_t* buffer) {
@@ -96,8 +97,10 @@ void FcInt8RowsGemvKernel(FcInt8Args a, int slabs, int batch0, int bt) {
       const int p = j * kRowsThreads + tid;
       const int piece = p % kPiecesPerRow;
       const int at = c * S::kChunkSlabs * kSlabDepth + piece * 16;
+      i32x4 v = staged[j];
+      if (RAGGED) v = ShiftBytesDown(v, RowPieceSkip(at, depth));
       *reinterpret_cast<i32x4*>(buffer + (p / kPiecesPerRow) * S::kStride + piece * 16) =
-          at < depth ? staged[j] : i32x4{0, 0, 0, 0};
+          at < depth ? v : i32x4{0, 0, 0, 0};
     }
   };
 
@@ -268,10 +271,10 @@ void FcInt8RowsGemvKernel(FcInt8Args a, int slabs, int batch0, int bt) {
   }
 }
 
-template <Int8Epilogue EPI, int RT>
+template <Int8Epilogue EPI, int RT, bool RAGGED>
 hipError_t LaunchRows(const FcInt8Args& a, int batch0, int bt, hipStream_t stream) {
   const size_t lds = 2 * static_cast<size_t>(RowsShape<RT>::kBufferBytes);
-  auto kernel = FcInt8RowsGemvKernel<EPI, RT>;
+  auto kernel = FcInt8RowsGemvKernel<EPI, RT, RAGGED>;
   if (hipError_t err = EnsureDynamicLds(reinterpret_cast<const void*>(kernel), lds)) return err;
   const int tiles = (a.out_depth + kTileRows - 1) / kTileRows;
   const int slabs = (a.depth + kSlabDepth - 1) / kSlabDepth;
@@ -285,8 +288,11 @@ hipError_t LaunchRowsEpilogue(const FcInt8Args& a, hipStream_t stream) {
   // Passes of at most 128 rows; a pass of up to 64 rows takes four row tiles per weight tile.
   for (int batch0 = 0; batch0 < a.batches; batch0 += 128) {
     const int bt = min(128, a.batches - batch0);
-    const hipError_t err = bt <= 64 ? LaunchRows<EPI, 4>(a, batch0, bt, stream)
-                                    : LaunchRows<EPI, 8>(a, batch0, bt, stream);
+    const bool ragged = a.depth % 16 != 0;
+    const hipError_t err = bt <= 64 ? (ragged ? LaunchRows<EPI, 4, true>(a, batch0, bt, stream)
+                                              : LaunchRows<EPI, 4, false>(a, batch0, bt, stream))
+                                    : (ragged ? LaunchRows<EPI, 8, true>(a, batch0, bt, stream)
+                                              : LaunchRows<EPI, 8, false>(a, batch0, bt, stream));
     if (err != hipSuccess) return err;
   }
   return hipSuccess;
@@ -299,8 +305,7 @@ bool FcInt8RowsGemvTakes(const FcInt8Args& a) {
   // workgroups, and the chunked walk wants a few chunks of depth.
   const int tiles = (a.out_depth + kTileRows - 1) / kTileRows;
   return a.batches > 32 && a.batches <= 128 && a.filter_offset == 0 && a.depth >= 1024 &&
-         a.depth % 16 == 0 && tiles >= 4 * 160 &&
-         (reinterpret_cast<uintptr_t>(a.input) & 15) == 0 &&
+         tiles >= 4 * 160 &&
          (reinterpret_cast<uintptr_t>(a.filter) & 15) == 0;
 }
 

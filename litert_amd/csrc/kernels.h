@@ -19,21 +19,25 @@ hipError_t EnsureDynamicLds(const void* kernel, size_t bytes);
 
 // Layout of the activation workspace of lrtfc_activation_workspace_bytes(batches, depth):
 // quantized rows, then scaling factors, then zero points, each region on a 256-byte boundary.
+// The kernels on re-tiled filters find the rows PaddedDepth(depth) bytes apart, zeros behind the
+// row's last value: they then read whole aligned 16-byte pieces at any depth, as if the depth
+// were PaddedDepth(depth) (the re-tiled filters are padded with zero weights beyond that).
+inline int PaddedDepth(int depth) { return (depth + 15) / 16 * 16; }
 struct ActivationWorkspace {
   int8_t* q;
   float* sf;
   int32_t* zp;
 };
 inline size_t AlignUp256(size_t v) { return (v + 255) / 256 * 256; }
-inline size_t ActivationWorkspaceBytes(int batches, int depth) {
-  return AlignUp256(static_cast<size_t>(batches) * depth) +
+inline size_t ActivationWorkspaceBytes(int batches, int row_stride) {
+  return AlignUp256(static_cast<size_t>(batches) * row_stride) +
          2 * AlignUp256(static_cast<size_t>(batches) * 4);
 }
-inline ActivationWorkspace SplitActivationWorkspace(void* base, int batches, int depth) {
+inline ActivationWorkspace SplitActivationWorkspace(void* base, int batches, int row_stride) {
   char* p = static_cast<char*>(base);
   ActivationWorkspace w;
   w.q = reinterpret_cast<int8_t*>(p);
-  p += AlignUp256(static_cast<size_t>(batches) * depth);
+  p += AlignUp256(static_cast<size_t>(batches) * row_stride);
   w.sf = reinterpret_cast<float*>(p);
   p += AlignUp256(static_cast<size_t>(batches) * 4);
   w.zp = reinterpret_cast<int32_t*>(p);
@@ -73,13 +77,14 @@ struct FcInt8Args {
 // holds the rows' input offsets (-7 * sum(q)) and a.filter_row_sums is unused.
 enum class Int8Epilogue { kRequantize, kHybrid, kHybrid4Bit };
 
-hipError_t LaunchBatchQuantize(const float* values, int n_batch, int n_data, int8_t* quantized,
-                               float* scaling_factors, int32_t* zero_points, int do_asymmetric,
-                               int variant, hipStream_t stream);
+// Rows of n_data floats -> int8 rows row_stride >= n_data bytes apart, zeros in between.
+hipError_t LaunchBatchQuantize(const float* values, int n_batch, int n_data, int row_stride,
+                               int8_t* quantized, float* scaling_factors, int32_t* zero_points,
+                               int do_asymmetric, int variant, hipStream_t stream);
 
-hipError_t LaunchBatchQuantize4Bit(const float* values, int n_batch, int n_data, int8_t* quantized,
-                                   float* scaling_factors, int32_t* input_offsets,
-                                   hipStream_t stream);
+hipError_t LaunchBatchQuantize4Bit(const float* values, int n_batch, int n_data, int row_stride,
+                                   int8_t* quantized, float* scaling_factors,
+                                   int32_t* input_offsets, hipStream_t stream);
 // `matrices` row-major [in_rows, in_cols] float32 matrices -> [in_cols, in_rows] each.
 hipError_t LaunchTransposeLastTwoF32(const float* src, int matrices, int in_rows, int in_cols,
                                      float* dst, hipStream_t stream);

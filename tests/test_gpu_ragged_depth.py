@@ -1,0 +1,80 @@
+"""Depths and channel counts off every vector size, on each kernel that reads rows in 16-byte
+pieces: the last piece of a row is read early and shifted into place, and nothing behind a row's
+last value may reach a result. Bit-exact against the CPU oracle, as everywhere on these paths."""
+import numpy as np
+import pytest
+
+import oracle
+from litert_amd import workloads as wl
+from tests.test_gpu_parity import _bits_equal, _cuda, _run_int8, fc  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+# rows: ring / resident GEMV (1, 5, 16), two row tiles (17, 32), GEMM (77, 150), rows kernel on
+# >= 640 channel tiles (33, 128), large GEMM tiles (1100 x 4099)
+SHAPES = [(1, 17, 19), (1, 2999, 530), (5, 2049, 67), (16, 1030, 33), (3, 20001, 9), (17, 2047, 301),
+          (32, 4093, 515), (77, 1999, 261), (150, 21, 130), (257, 1283, 515), (40, 1027, 10243),
+          (128, 1037, 10241), (1100, 131, 4099)]
+
+
+@pytest.mark.parametrize("B,K,N", SHAPES)
+@pytest.mark.parametrize("activation", ["none", "relu6"])
+def test_int8_ragged_depth_bit_exact(fc, B, K, N, activation):  # noqa: F811
+    y, want = _run_int8(fc, wl.int8_fc(B, K, N, seed=B + K + N), activation)
+    assert np.array_equal(y, want)
+
+
+def test_int8_rows_that_end_with_their_allocation(fc):  # noqa: F811
+    """Rows on odd addresses: the tensor starts one byte into its memory."""
+    import torch
+    for B, K, N in ((1, 2999, 40), (33, 259, 40), (140, 1021, 70)):
+        c = wl.int8_fc(B, K, N, seed=K)
+        op = fc.FullyConnectedInt8(c["w"], c["bias"], float(c["in_scale"]), c["in_zp"], c["w_scale"],
+                                   float(c["out_scale"]), c["out_zp"])
+        memory = torch.zeros(B * K + 1, dtype=torch.int8, device="cuda")
+        memory[1:] = _cuda(c["x"]).reshape(-1)
+        out = torch.zeros(B * N + 3, dtype=torch.int8, device="cuda")
+        op(memory[1:].view(B, K), out=out[3:].view(B, N))
+        _, want = _run_int8(fc, c)
+        assert np.array_equal(out[3:].view(B, N).cpu().numpy(), want)
+        assert not out[:3].any()
+
+
+@pytest.mark.parametrize("B,K,N", SHAPES + [(8, 4095, 66), (2, 4, 9), (7, 3, 5), (900, 7396, 33)])
+@pytest.mark.parametrize("asym", [True, False])
+def test_hybrid_ragged_depth_matches_oracle(fc, B, K, N, asym):  # noqa: F811
+    c = wl.hybrid_fc(B, K, N, seed=B + K + N)
+    bias = np.random.default_rng(K).standard_normal(N).astype(np.float32)
+    op = fc.FullyConnectedHybrid(c["w"], c["pcs"], bias=bias, asymmetric_quantize_inputs=asym,
+                                 activation="relu")
+    want = oracle.fc_hybrid(c["x"], c["w"], c["pcs"], bias=bias, asymmetric=asym,
+                            activation=oracle.ACT_RELU)
+    assert _bits_equal(op(_cuda(c["x"])).cpu().numpy(), want)
+    assert _bits_equal(op.call_split(_cuda(c["x"])).cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("variant", [0, 1, 2])
+@pytest.mark.parametrize("K", [3, 4, 5, 7, 255, 4097, 16385, 20003])
+def test_quantizer_ragged_rows_bit_exact(fc, variant, K):  # noqa: F811
+    x = np.random.default_rng(K).standard_normal((3, K)).astype(np.float32)
+    for asym in (True, False):
+        q, sf, zp = fc.batch_quantize_floats(_cuda(x), asym, variant)
+        want = oracle.batch_quantize_floats(x, asym, variant)
+        assert np.array_equal(q.cpu().numpy(), want[0])
+        assert _bits_equal(sf.cpu().numpy(), want[1])
+        if asym:
+            assert np.array_equal(zp.cpu().numpy(), want[2])
+
+
+@pytest.mark.parametrize("B,K,N", [(1, 4094, 70), (4, 2998, 33), (2, 6, 5), (3, 4098, 40), (18, 1062, 67),
+                                   (40, 2998, 101), (300, 1030, 259), (5, 20002, 9)])
+def test_int4_per_channel_ragged_depth_matches_oracle(fc, B, K, N):  # noqa: F811
+    rng = np.random.default_rng(B + K + N)
+    x = rng.standard_normal((B, K)).astype(np.float32)
+    packed = wl.pack_int4(rng.integers(-7, 8, (N, K)).astype(np.int8))
+    scales = rng.uniform(0.01, 0.1, N).astype(np.float32)
+    bias = rng.standard_normal(N).astype(np.float32)
+    want = oracle.fc_hybrid_int4_per_channel(x, packed, N, scales, bias)
+    op = fc.FullyConnectedHybridInt4PerChannel(packed, K, scales, bias=bias)
+    assert _bits_equal(op(_cuda(x)).cpu().numpy(), want)
+    assert _bits_equal(op(_cuda(x), force_int8=True).cpu().numpy(), want)
