@@ -5,24 +5,38 @@
 // which is right for one to a few rows and hopeless for hundreds. Here every (row, channel)
 // output keeps its float32 accumulator in a register and walks the blocks of 32 depth
 // positions in order: one v_mfma_i32_16x16x32_i8 per block and 16 x 16 tile gives the exact
-// int32 block sums (its K is exactly one block), and three vector operations per output add
-// `float(sum) * scale[channel][block]` to the accumulator -- the reference's own order of
-// float operations (:1069-1077), unfused, so the results are bit-identical to the decode
-// kernel's and the oracle's. Those three operations per output and block, not the matrix
-// cores, bound the kernel (the MFMA of a block takes 16 cycles, its 4 outputs per lane 48).
+// int32 block sums (its K is exactly one block), and `float(sum) * scale[channel][block]` is
+// added to the accumulator unfused, the reference's own order of float operations (:1069-1077),
+// so the results are bit-identical to the decode kernel's and the oracle's.
+//
+// The vector operations per output and block bound the kernel, not the matrix cores (the MFMA of a
+// block takes 16 cycles of its SIMD, three operations on its 4 outputs per lane 48). Two suffice:
+//   * The accumulator input of every MFMA is the bit pattern of 1.5 * 2^23, so its integer result
+//     READ AS A FLOAT is 1.5 * 2^23 + sum, exactly (|sum| <= 32 * 8 * 128 < 2^22): no conversion.
+//   * fma(that, scale, -1.5 * 2^23 * scale) rounds the exact product sum * scale once, which is
+//     what converting and multiplying gives: 1.5 * 2^23 * scale is exact in float32 for a scale
+//     of eleven significant bits.
+//   * The batch rows are the A operand and the channels the B operand, so that a lane's four results
+//     are four rows of ONE channel: one scale per lane and block (and its product with -1.5 * 2^23)
+//     serves every row tile, where four channels per lane took four broadcasts per block.
+// 2048 x 4096 -> 14336: 2 x 4 x 14.7 M wavefront operations of 4 cycles on 1024 SIMDs, 191 us at
+// 2.4 GHz.
 //
 // Layouts, made once at prepare (filter) or per call (activations):
-//   filter `tile16x32s`: for channel tile t (16 channels) and block b, 512 bytes: lane L's 8
-//     bytes are channel 16 t + L % 16, depths 32 b + 8 (L / 16) ... + 8, sign-extended to
-//     int8 -- the A operand of the MFMA as one 8-byte load per lane; after all tiles, the block
-//     scales as float32, 16 per (t, b): a lane's 16-byte load is the scales of its four output
-//     channels for one block, and a wavefront fetches those of 16 blocks in one instruction.
-//   activations `tile16x64`: batch rows in place of channels (B operand), with the 8 bytes of
-//     blocks 2 p and 2 p + 1 side by side in a lane's 16 bytes; written in that order by the
-//     row quantizer itself.
-// No LDS: a wavefront owns CT x RT tiles (16 to 32 channels x 16 to 64 rows, by batch size)
-// and requests the operands of the next blocks while it works on the current ones (a ring of
-// pairs of blocks in registers); both operands are re-read by other wavefronts from L2.
+//   filter `tile32x32s`: for channel tile t (32 channels) and block b, 1 KiB: lane L's 16 bytes are
+//     channel 32 t + L % 32, depths 16 (L / 32) ... + 16 of the block, sign-extended to int8: an
+//     operand of v_mfma_i32_32x32x32_i8. After all tiles, the block scales as float32, 32 channels x
+//     4 blocks per tile and quad of blocks: a lane's 16-byte load is its channel's scales of four
+//     blocks.
+//   activations: batch rows in place of channels, either in the same form (`tile32x32`) or, for the
+//     small forms, `tile16x64`: 16 rows and a pair of blocks in 1 KiB, lane L's 16 bytes row L % 16,
+//     depths 8 (L / 16) ... + 8 of the first block, then of the second. The row quantizer writes
+//     either order itself.
+// No LDS: a wavefront owns CT x RT tiles and requests the operands of the next blocks while it works
+// on the current ones (a ring in registers); both operands are re-read by other wavefronts from L1
+// and L2. Two kernels: FcInt4BlockwiseGemmLargeKernel on 32 x 32 tiles, whose one MFMA per block and
+// tile does four times the work of a 16 x 16 one in twice the time; and FcInt4BlockwiseGemmKernel on
+// 16 x 16 tiles for launches that the large tiles would cut into too few wavefronts.
 #include <mutex>
 
 #include "kernels.h"
@@ -47,20 +61,23 @@ __device__ __forceinline__ int SignedNibble(uint32_t byte, int high) {
   return (n ^ 8) - 8;
 }
 
+constexpr int kWide = 32;  // channels / rows per tile of the large form
+
 // Model layout (rows of depth / 2 bytes, low nibble = even depth; fp16 scales [N, nb]) ->
-// tile16x32s + float32 scales. One thread per 8-byte lane slot of the tile array.
+// tile32x32s + float32 scales. One thread per 8-byte half of a lane slot of the tile array.
 __global__ __launch_bounds__(kThreads) void PackInt4BlockwiseGemmKernel(
     const uint8_t* __restrict__ filter, const uint16_t* __restrict__ scales_f16, int out_depth,
     int depth, int tiles, int nb, uint8_t* __restrict__ dst) {
   const int64_t slot = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-  const int64_t slots = static_cast<int64_t>(tiles) * nb * 64;
+  const int quads = (nb + 3) / 4;
+  const int64_t slots = static_cast<int64_t>(tiles) * nb * 128;
   if (slot < slots) {
-    const int lane = static_cast<int>(slot & 63);
-    const int64_t tb = slot >> 6;
+    const int lane = static_cast<int>((slot >> 1) & 63);
+    const int64_t tb = slot >> 7;
     const int b = static_cast<int>(tb % nb);
     const int t = static_cast<int>(tb / nb);
-    const int n = t * kTile + (lane & 15);
-    const int k0 = b * kBlock + 8 * (lane >> 4);
+    const int n = t * kWide + (lane & 31);
+    const int k0 = b * kBlock + 16 * (lane >> 5) + 8 * static_cast<int>(slot & 1);
     uint32_t lo = 0, hi = 0;
     if (n < out_depth) {
       const uint8_t* src = filter + static_cast<size_t>(n) * (depth / 2) + k0 / 2;
@@ -78,16 +95,17 @@ __global__ __launch_bounds__(kThreads) void PackInt4BlockwiseGemmKernel(
     }
     reinterpret_cast<uint2*>(dst)[slot] = make_uint2(lo, hi);
   }
-  // scales: one thread per (tile, block, channel)
-  const int64_t scale_slots = static_cast<int64_t>(tiles) * nb * kTile;
+  // scales: one thread per (tile, quad of blocks, channel, block)
+  const int64_t scale_slots = static_cast<int64_t>(tiles) * quads * (kWide * 4);
   if (slot < scale_slots) {
-    const int c = static_cast<int>(slot & 15);
-    const int64_t tb = slot >> 4;
-    const int b = static_cast<int>(tb % nb);
-    const int t = static_cast<int>(tb / nb);
-    const int n = t * kTile + c;
+    const int c = static_cast<int>((slot >> 2) & 31);
+    const int64_t tq = slot >> 7;
+    const int b = 4 * static_cast<int>(tq % quads) + static_cast<int>(slot & 3);
+    const int t = static_cast<int>(tq / quads);
+    const int n = t * kWide + c;
     float* out = reinterpret_cast<float*>(dst + slots * 8);
-    out[slot] = n < out_depth ? HalfBitsToFloatFast(scales_f16[static_cast<size_t>(n) * nb + b]) : 0.0f;
+    out[slot] = n < out_depth && b < nb
+                    ? HalfBitsToFloatFast(scales_f16[static_cast<size_t>(n) * nb + b]) : 0.0f;
   }
 }
 
@@ -101,20 +119,29 @@ struct Tile16x64Placement {
   }
 };
 
-// BatchQuantizeFloats of float rows [batches, depth] straight into tile16x64: one workgroup
+// The same within a tile of 32 rows of the tile32x32 layout.
+struct Tile32x32Placement {
+  int row_in_tile;
+  __device__ __forceinline__ size_t operator()(int k) const {
+    return static_cast<size_t>(k >> 5) * 1024 + ((k & 31) >> 4) * 512 + row_in_tile * 16 + (k & 15);
+  }
+};
+
+// BatchQuantizeFloats of float rows [batches, depth] straight into tiles of ROWS rows: one workgroup
 // per row of the padded batch (rows past the batch are zero). `tile_bytes`: one row tile.
-template <int VARIANT>
+template <int VARIANT, int ROWS>
 __global__ __launch_bounds__(kQuantizeThreads) void QuantizeRowsTiledKernel(
     const float* __restrict__ input, int batches, int depth, size_t tile_bytes,
     int8_t* __restrict__ tiled, float* __restrict__ scaling_factors,
     int32_t* __restrict__ zero_points) {
+  using Placement = std::conditional_t<ROWS == kWide, Tile32x32Placement, Tile16x64Placement>;
   const int m = blockIdx.x;
-  int8_t* tile_row = tiled + static_cast<size_t>(m / kTile) * tile_bytes;
-  const Tile16x64Placement place{m % kTile};
+  int8_t* tile_row = tiled + static_cast<size_t>(m / ROWS) * tile_bytes;
+  const Placement place{m % ROWS};
   if (m < batches) {
     // EvalBlockwise4Bit always quantizes asymmetrically (fully_connected.cc:1044-1047).
-    QuantizeRow<VARIANT>(input + static_cast<size_t>(m) * depth, depth, tile_row, depth,
-                         scaling_factors + m, zero_points + m, /*do_asymmetric=*/1, place);
+    QuantizeRow<VARIANT, Placement>(input + static_cast<size_t>(m) * depth, depth, tile_row, depth,
+                                    scaling_factors + m, zero_points + m, /*do_asymmetric=*/1, place);
   } else {
     for (int k = threadIdx.x * 8; k < depth; k += kQuantizeThreads * 8) {
       *reinterpret_cast<uint2*>(tile_row + place(k)) = make_uint2(0, 0);
@@ -123,24 +150,16 @@ __global__ __launch_bounds__(kQuantizeThreads) void QuantizeRowsTiledKernel(
 }
 
 struct GemmArgs {
-  const i64* filter;        // tile16x32s
-  const float4* scales;     // float32 [tiles][nb][16] viewed as float4
-  const i64x2* activations;  // tile16x64
+  const char* filter;       // tile32x32s
+  const char* scales;       // float32 [tiles][quads of blocks][32 channels][4 blocks]
+  const char* activations;  // tile16x64 or tile32x32
   const float* scaling_factors;  // [batches]
   const int32_t* zero_points;    // [batches]
   const float* kfsum;            // [out_depth]
   const float* bias;             // [out_depth] or nullptr
   float* output;                 // [batches, out_depth]
   int batches, out_depth, nb;
-  int channel_tiles, row_tiles;  // of 16
-  int vector_store;              // rows of the output start on 16-byte boundaries
-};
-
-// One pair of consecutive blocks of a wavefront's operands.
-template <int CT, int RT>
-struct Stage {
-  i64 w[2][CT];  // channel tiles of the two blocks
-  i64x2 x[RT];   // row tiles, both blocks
+  int channel_tiles, row_tiles;  // of the kernel's tile size
 };
 
 // Lane j of every 16 lanes to all 16 (row_newbcast:j).
@@ -151,77 +170,108 @@ __device__ __forceinline__ float RowBroadcast(float v) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x150 + J, 0xF, 0xF, true));
 }
 
-// WROWS: wavefronts of a workgroup along the batch rows (1 or 2); the others along the channels.
-// PAIRS: pairs of blocks in flight per wavefront. The count of outstanding vector loads a
-//   wavefront can wait on selectively is 63, so depth comes from few, wide loads: a row tile's
-//   two blocks in one 16-byte load, and the scales of 16 blocks in one load (lane = block
-//   16 g + lane % 16, its float4 = channels 4 (lane / 16) ... + 4), handed to the lanes of a
-//   block by a row broadcast.
+// A block sum that an MFMA left on top of the bit pattern of kSumBase is, read as a float,
+// kSumBase + sum; see the head of this file.
+constexpr float kSumBase = 12582912.0f;  // 1.5 * 2^23
+constexpr int kSumBaseBits = 0x4B400000;
+// float(sum) * scale, rounded once; `offset` is -kSumBase * scale.
+__device__ __forceinline__ float ScaleBlockSum(int biased_sum, float scale, float offset) {
+  return __fmaf_rn(__int_as_float(biased_sum), scale, offset);
+}
+
+// fully_connected.cc:1078-1082: zero-point term, row scale, bias.
+__device__ __forceinline__ float FinishOutput(float sum, float zero_point, float kfsum,
+                                              float row_scale, bool has_bias, float bias) {
+  const float v = __fmul_rn(__fsub_rn(sum, __fmul_rn(zero_point, kfsum)), row_scale);
+  return has_bias ? __fadd_rn(v, bias) : v;
+}
+
+// Workgroups are dealt round-robin to the 8 XCDs: each XCD gets a contiguous range of ids, and ids
+// walk rectangles of 8 workgroup rows x all channels, the rows fastest, so that the workgroups
+// resident on an XCD share their operands in its L2.
+__device__ __forceinline__ void WorkgroupTile(int wgs_c, int wgs_r, int* wg_c, int* wg_r) {
+  const int total = wgs_c * wgs_r;
+  int id = blockIdx.x;
+  if (total % 8 == 0) id = (id % 8) * (total / 8) + id / 8;
+  const int band = id / (8 * wgs_c);
+  const int band_rows = min(8, wgs_r - 8 * band);
+  const int in_band = id - band * 8 * wgs_c;
+  *wg_r = 8 * band + in_band % band_rows;
+  *wg_c = in_band / band_rows;
+}
+
+// CT x RT: tiles of 16 channels x 16 rows per wavefront. WROWS: wavefronts of a workgroup along the
+// batch rows (1 or 2); the others along the channels. PAIRS: pairs of blocks in flight.
 template <int CT, int RT, int WROWS, int PAIRS>
-__global__ __launch_bounds__(kThreads) void FcInt4BlockwiseGemmKernel(GemmArgs a) {
+__global__ __launch_bounds__(kThreads, 2) void FcInt4BlockwiseGemmKernel(GemmArgs a, int wgs_c,
+                                                                         int wgs_r) {
   constexpr int WCH = 4 / WROWS;
   const int lane = threadIdx.x & 63;
   // The wavefront index as a scalar: tile addresses then stay in scalar registers and every
   // load is "scalar base + lane offset".
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // Workgroups walk the channel direction fastest: neighbours share activation tiles in L2.
-  const int wg_c = blockIdx.x, wg_r = blockIdx.y;
+  int wg_c, wg_r;
+  WorkgroupTile(wgs_c, wgs_r, &wg_c, &wg_r);
   const int ct0 = (wg_c * WCH + wave % WCH) * CT;
   const int rt0 = (wg_r * WROWS + wave / WCH) * RT;
   if (ct0 >= a.channel_tiles || rt0 >= a.row_tiles) return;
-  // Tiles past the edge re-read the last valid one; their outputs are never stored.
-  int ct[CT], rt[RT];
-#pragma unroll
-  for (int j = 0; j < CT; ++j) ct[j] = min(ct0 + j, a.channel_tiles - 1);
-#pragma unroll
-  for (int j = 0; j < RT; ++j) rt[j] = min(rt0 + j, a.row_tiles - 1);
   const int nb = a.nb;
-  const int pairs = (nb + 1) / 2;
-  const i64* wp[CT];
-  const float4* sp[CT];
-  const i64x2* xp[RT];
+  const int pairs = (nb + 1) / 2, quads = (nb + 3) / 4;
+  const char* wp[CT];
+  const char* sp[CT];
+  const char* xp[RT];
+  // Tiles past the edge re-read the last valid one; their outputs are never stored.
 #pragma unroll
   for (int j = 0; j < CT; ++j) {
-    wp[j] = a.filter + static_cast<size_t>(ct[j]) * nb * 64 + lane;
-    sp[j] = a.scales + static_cast<size_t>(ct[j]) * nb * 4 + (lane >> 4);
+    const int ct = min(ct0 + j, a.channel_tiles - 1);
+    // Half of a tile of 32 channels, by lane offsets: 8 bytes of each of the pair's blocks.
+    wp[j] = a.filter + static_cast<size_t>(ct >> 1) * nb * 1024 + (ct & 1) * 256;
+    sp[j] = a.scales + static_cast<size_t>(ct >> 1) * quads * 512 + (ct & 1) * 256;
   }
 #pragma unroll
   for (int j = 0; j < RT; ++j) {
-    xp[j] = a.activations + static_cast<size_t>(rt[j]) * pairs * 64 + lane;
+    xp[j] = a.activations + static_cast<size_t>(min(rt0 + j, a.row_tiles - 1)) * pairs * 1024;
   }
-  auto fetch = [&](int p) {
-    const int pp = min(p, pairs - 1);  // past the end: a hot line, result unused
-    Stage<CT, RT> st;
+  // Operands of pair p in slot p % PAIRS, scales of quad q (four blocks) in slot q % kSlots. A slot
+  // is requested again right behind the last operation that reads it, so that the loads land in
+  // the registers they are read from. Past the end: a hot line, result unused.
+  constexpr int kSlots = PAIRS <= 4 ? 2 : PAIRS / 2;
+  i64 w[PAIRS][CT][2];
+  i64x2 x[PAIRS][RT];
+  float4 sg[kSlots][CT];
+  uint32_t lane16 = lane * 16, channel16 = (lane & 15) * 16;
+  uint32_t weight8 = channel16 + (lane >> 5) * 512 + ((lane >> 4) & 1) * 8;
+  auto fetch = [&](auto slot, int p) {
+    constexpr int s = decltype(slot)::value;
+    const int pp = min(p, pairs - 1);
+    const size_t at = static_cast<size_t>(pp) * 1024;
+#pragma unroll
+    for (int j = 0; j < RT; ++j) x[s][j] = *reinterpret_cast<const i64x2*>(xp[j] + at + lane16);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int bb = min(2 * pp + h, nb - 1);
+      // An odd block count: the last pair's second block is the first again, under zero scales.
+      const size_t block = static_cast<size_t>(min(2 * pp + h, nb - 1)) * 1024;
 #pragma unroll
-      for (int j = 0; j < CT; ++j) {
-        st.w[h][j] = wp[j][static_cast<size_t>(bb) * 64];
-      }
+      for (int j = 0; j < CT; ++j) w[s][j][h] = *reinterpret_cast<const i64*>(wp[j] + block + weight8);
     }
-#pragma unroll
-    for (int j = 0; j < RT; ++j) st.x[j] = xp[j][static_cast<size_t>(pp) * 64];
-    return st;
   };
-  // Scale groups (16 blocks = 8 pairs) held per wavefront: the current one and as many ahead
-  // as the ring of pairs reaches, so that a group is always requested before its blocks'
-  // weights; a power of two, group g in slot g % kGroups.
-  constexpr int kGroups = PAIRS > 8 ? 4 : 2;
-  static_assert((kGroups - 1) * 8 >= PAIRS, "scale groups must lead the ring");
-  float4 sg[kGroups][CT];
-  auto fetch_scales = [&](int g, float4 (&dst)[CT]) {
-    const int bb = min(16 * g + (lane & 15), nb - 1);
+  auto fetch_scales = [&](auto slot, int q) {
+    constexpr int s = decltype(slot)::value;
+    const size_t at = static_cast<size_t>(min(q, quads - 1)) * 512;
 #pragma unroll
-    for (int j = 0; j < CT; ++j) dst[j] = sp[j][static_cast<size_t>(bb) * 4];
+    for (int j = 0; j < CT; ++j) sg[s][j] = *reinterpret_cast<const float4*>(sp[j] + at + channel16);
   };
-#pragma unroll
-  for (int g = 0; g + 1 < kGroups; ++g) fetch_scales(g, sg[g]);
-  Stage<CT, RT> ring[PAIRS];
-#pragma unroll
-  for (int s = 0; s < PAIRS; ++s) ring[s] = fetch(s);
+  // One request at a time, in this order: waits count from the newest.
+  StaticFor<kSlots>([&](auto q) {
+    fetch_scales(q, decltype(q)::value);
+    __builtin_amdgcn_sched_barrier(0);
+  });
+  StaticFor<PAIRS>([&](auto s) {
+    fetch(s, decltype(s)::value);
+    __builtin_amdgcn_sched_barrier(0);
+  });
 
-  // out[cj][rj][i]: channel 16 ct[cj] + 4 (lane / 16) + i, batch row 16 rt[rj] + lane % 16.
+  // out[cj][rj][i]: channel 16 (ct0 + cj) + lane % 16, batch row 16 (rt0 + rj) + 4 (lane / 16) + i.
   float out[CT][RT][4];
 #pragma unroll
   for (int cj = 0; cj < CT; ++cj)
@@ -230,74 +280,253 @@ __global__ __launch_bounds__(kThreads) void FcInt4BlockwiseGemmKernel(GemmArgs a
 #pragma unroll
       for (int i = 0; i < 4; ++i) out[cj][rj][i] = 0.0f;
 
-  const i32x4 zero = {0, 0, 0, 0};
-  // One trip covers whole turns of the ring and of the scale slots, so that ring slots,
-  // scale slots and broadcast lanes are compile-time constants.
-  constexpr int kTrip = PAIRS > 8 * kGroups ? PAIRS : 8 * kGroups;
-  static_assert(kTrip % PAIRS == 0 && kTrip % (8 * kGroups) == 0, "trip");
-  for (int base = 0; base < pairs; base += kTrip) {
-    StaticFor<kTrip>([&](auto u_const) {
-      constexpr int u = decltype(u_const)::value;
-      constexpr int s = u % PAIRS;
-      constexpr int cur = (u / 8) % kGroups;  // slot of this pair's scale group
-      if constexpr (u % 8 == 0) {
-        // A new group of 16 blocks starts: the slot of the one before it takes the farthest.
-        fetch_scales((base + u) / 8 + kGroups - 1, sg[(cur + kGroups - 1) % kGroups]);
-      }
-      const Stage<CT, RT> st = ring[s];
-      ring[s] = fetch(base + u + PAIRS);
-      StaticFor<2>([&](auto h_const) {
-        constexpr int h = decltype(h_const)::value;
-        if (2 * (base + u) + h < nb) {
-#pragma unroll
-          for (int cj = 0; cj < CT; ++cj) {
-            constexpr int j = (2 * u + h) % 16;  // this block within its scale group
-            const float sc[4] = {RowBroadcast<j>(sg[cur][cj].x), RowBroadcast<j>(sg[cur][cj].y),
-                                 RowBroadcast<j>(sg[cur][cj].z), RowBroadcast<j>(sg[cur][cj].w)};
-#pragma unroll
-            for (int rj = 0; rj < RT; ++rj) {
-              const i32x4 acc =
-                  __builtin_amdgcn_mfma_i32_16x16x32_i8(st.w[h][cj], st.x[rj][h], zero, 0, 0, 0);
-#pragma unroll
-              for (int i = 0; i < 4; ++i) {
-                out[cj][rj][i] =
-                    __fadd_rn(out[cj][rj][i], __fmul_rn(static_cast<float>(acc[i]), sc[i]));
-              }
-            }
-          }
+  i32x4 base_bits = {kSumBaseBits, kSumBaseBits, kSumBaseBits, kSumBaseBits};
+  asm volatile("" : "+v"(base_bits));  // in registers for good
+  // The vector work on a tile trails its MFMA by kLag tiles, in this order (the fences keep it): the
+  // matrix core works on the next tiles meanwhile.
+  constexpr int kTiles = CT * RT;       // tiles per block
+  constexpr int kLag = 3;
+  // The tiles of pairs first .. first + COUNT - 1 (first a multiple of the slot counts; pair u of
+  // them in slots u % PAIRS and u / 2 % kSlots).
+  auto walk = [&](auto count_c, auto from_c, auto refill_c, int first) {
+    constexpr int kCount = decltype(count_c)::value, kFrom = decltype(from_c)::value;
+    constexpr bool kRefill = decltype(refill_c)::value;
+    constexpr int kAll = kCount * 2 * kTiles;
+    // (Opaque here, or the lane's offset is folded into every pointer outside the loop and each
+    // load pays a 64-bit vector addition for the pair's instead.)
+    asm volatile("" : "+v"(lane16), "+v"(channel16), "+v"(weight8));
+    i32x4 acc[kLag + 1];
+    StaticFor<kAll + kLag>([&](auto t_const) {
+      constexpr int t = decltype(t_const)::value;
+      if constexpr (t < kAll) {
+        constexpr int u = kFrom + t / (2 * kTiles), at = t % (2 * kTiles);
+        constexpr int h = at / kTiles, cj = at % kTiles / RT, rj = at % RT;
+        constexpr int s = u % PAIRS;
+        acc[t % (kLag + 1)] = __builtin_amdgcn_mfma_i32_16x16x32_i8(x[s][rj][h], w[s][cj][h],
+                                                                    base_bits, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (kRefill && at == 2 * kTiles - 1) {
+          fetch(std::integral_constant<int, s>{}, first + u + PAIRS);
+          __builtin_amdgcn_sched_barrier(0);
         }
-      });
-    });
-  }
-
-  // fully_connected.cc:1078-1082: zero-point term, row scale, bias.
-#pragma unroll
-  for (int rj = 0; rj < RT; ++rj) {
-    if (rt0 + rj >= a.row_tiles) break;
-    const int m = rt[rj] * kTile + (lane & 15);
-    if (m >= a.batches) continue;
-    const float zp = static_cast<float>(a.zero_points[m]);
-    const float row_scale = a.scaling_factors[m];
-#pragma unroll
-    for (int cj = 0; cj < CT; ++cj) {
-      if (ct0 + cj >= a.channel_tiles) break;
-      const int n0 = ct[cj] * kTile + 4 * (lane >> 4);
-      float o[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int n = min(n0 + i, a.out_depth - 1);
-        float v = __fsub_rn(out[cj][rj][i], __fmul_rn(zp, a.kfsum[n]));
-        v = __fmul_rn(v, row_scale);
-        if (a.bias) v = __fadd_rn(v, a.bias[n]);
-        o[i] = v;
       }
-      float* dst = a.output + static_cast<size_t>(m) * a.out_depth + n0;
-      if (n0 + 3 < a.out_depth && a.vector_store) {
-        *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]);
-      } else {
+      if constexpr (t >= kLag) {
+        constexpr int d = t - kLag;
+        constexpr int u = kFrom + d / (2 * kTiles), at = d % (2 * kTiles);
+        constexpr int h = at / kTiles, cj = at % kTiles / RT, rj = at % RT;
+        constexpr int b = 2 * (u % 2) + h, cur = u / 2 % kSlots;  // block of which quad
+        const float4& q = sg[cur][cj];
+        const float scale = b == 0 ? q.x : b == 1 ? q.y : b == 2 ? q.z : q.w;
+        const float offset = __fmul_rn(-kSumBase, scale);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          if (n0 + i < a.out_depth) dst[i] = o[i];
+          out[cj][rj][i] = __fadd_rn(out[cj][rj][i],
+                                     ScaleBlockSum(acc[d % (kLag + 1)][i], scale, offset));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (kRefill && u % 2 == 1 && at == 2 * kTiles - 1) {
+          fetch_scales(std::integral_constant<int, cur>{}, (first + u) / 2 + kSlots);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    });
+  };
+  // Whole turns of both rings are straight lines (slots are compile-time constants, and there is no
+  // branch to move registers at); what is left of the depth goes pair by pair.
+  constexpr int kTrip = PAIRS > 2 * kSlots ? PAIRS : 2 * kSlots;
+  static_assert(kTrip % PAIRS == 0 && kTrip % (2 * kSlots) == 0, "trip");
+  using std::integral_constant;
+  int first = 0;
+  for (; first + kTrip <= pairs; first += kTrip) {
+    walk(integral_constant<int, kTrip>{}, integral_constant<int, 0>{}, std::true_type{}, first);
+  }
+  StaticFor<kTrip - 1>([&](auto u_const) {
+    constexpr int u = decltype(u_const)::value;
+    if (first + u < pairs) {
+      walk(integral_constant<int, 1>{}, integral_constant<int, u>{}, std::false_type{}, first);
+      // Beyond the slots that a whole turn leaves filled (a ring shorter than the trip).
+      if constexpr (u + PAIRS < kTrip - 1) fetch(integral_constant<int, u % PAIRS>{}, first + u + PAIRS);
+    }
+  });
+
+#pragma unroll
+  for (int rj = 0; rj < RT; ++rj) {
+    const int m0 = (rt0 + rj) * kTile + 4 * (lane >> 4);
+    float zp[4], row_scale[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int m = min(m0 + i, a.batches - 1);
+      zp[i] = static_cast<float>(a.zero_points[m]);
+      row_scale[i] = a.scaling_factors[m];
+    }
+#pragma unroll
+    for (int cj = 0; cj < CT; ++cj) {
+      const int n = (ct0 + cj) * kTile + (lane & 15);
+      if (n >= a.out_depth) continue;
+      const float kfsum = a.kfsum[n];
+      const float bias = a.bias ? a.bias[n] : 0.0f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float v = FinishOutput(out[cj][rj][i], zp[i], kfsum, row_scale[i], a.bias != nullptr,
+                                     bias);
+        if (m0 + i < a.batches) a.output[static_cast<size_t>(m0 + i) * a.out_depth + n] = v;
+      }
+    }
+  }
+}
+
+
+// The large form: CT x RT tiles of 32 channels x 32 rows per wavefront, four wavefronts in WROWS x
+// 4 / WROWS; BLOCKS blocks in flight. Per tile and block one MFMA (32 cycles of the matrix core) and
+// 32 vector operations on its 16 results per lane (128 cycles of the SIMD).
+template <int CT, int RT, int WROWS, int BLOCKS>
+__global__ __launch_bounds__(kThreads, 2) void FcInt4BlockwiseGemmLargeKernel(GemmArgs a, int wgs_c,
+                                                                              int wgs_r) {
+  using i32x16 = int __attribute__((ext_vector_type(16)));
+  constexpr int WCH = 4 / WROWS;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int wg_c, wg_r;
+  WorkgroupTile(wgs_c, wgs_r, &wg_c, &wg_r);
+  const int ct0 = (wg_c * WCH + wave % WCH) * CT;
+  const int rt0 = (wg_r * WROWS + wave / WCH) * RT;
+  if (ct0 >= a.channel_tiles || rt0 >= a.row_tiles) return;
+  const int nb = a.nb;
+  const int quads = (nb + 3) / 4;
+  const char* wp[CT];
+  const char* sp[CT];
+  const char* xp[RT];
+#pragma unroll
+  for (int j = 0; j < CT; ++j) {
+    const int ct = min(ct0 + j, a.channel_tiles - 1);
+    wp[j] = a.filter + static_cast<size_t>(ct) * nb * 1024;
+    sp[j] = a.scales + static_cast<size_t>(ct) * quads * 512;
+  }
+#pragma unroll
+  for (int j = 0; j < RT; ++j) {
+    xp[j] = a.activations + static_cast<size_t>(min(rt0 + j, a.row_tiles - 1)) * nb * 1024;
+  }
+  // Operands of block b in slot b % BLOCKS, scales of quad q in slot q % 2; requested again behind
+  // the last operation that reads them, as above.
+  i32x4 w[BLOCKS][CT], x[BLOCKS][RT];
+  float4 sg[2][CT];
+  uint32_t lane16 = lane * 16, channel16 = (lane & 31) * 16;
+  auto fetch = [&](auto slot, int b) {
+    constexpr int s = decltype(slot)::value;
+    const size_t at = static_cast<size_t>(min(b, nb - 1)) * 1024;
+#pragma unroll
+    for (int j = 0; j < RT; ++j) x[s][j] = *reinterpret_cast<const i32x4*>(xp[j] + at + lane16);
+#pragma unroll
+    for (int j = 0; j < CT; ++j) w[s][j] = *reinterpret_cast<const i32x4*>(wp[j] + at + lane16);
+  };
+  auto fetch_scales = [&](auto slot, int q) {
+    constexpr int s = decltype(slot)::value;
+    const size_t at = static_cast<size_t>(min(q, quads - 1)) * 512;
+#pragma unroll
+    for (int j = 0; j < CT; ++j) sg[s][j] = *reinterpret_cast<const float4*>(sp[j] + at + channel16);
+  };
+  StaticFor<2>([&](auto q) {
+    fetch_scales(q, decltype(q)::value);
+    __builtin_amdgcn_sched_barrier(0);
+  });
+  StaticFor<BLOCKS>([&](auto s) {
+    fetch(s, decltype(s)::value);
+    __builtin_amdgcn_sched_barrier(0);
+  });
+
+  // out[cj][rj][e]: channel 32 (ct0 + cj) + lane % 32,
+  // batch row 32 (rt0 + rj) + 8 (e / 4) + 4 (lane / 32) + e % 4.
+  float out[CT][RT][16];
+#pragma unroll
+  for (int cj = 0; cj < CT; ++cj)
+#pragma unroll
+    for (int rj = 0; rj < RT; ++rj)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) out[cj][rj][e] = 0.0f;
+
+  i32x16 base_bits;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) base_bits[e] = kSumBaseBits;
+  asm volatile("" : "+v"(base_bits));  // in registers for good
+  constexpr int kTiles = CT * RT;
+  // The tiles of blocks first + kFrom ... (kCount of them), the vector work one tile behind the MFMAs.
+  auto walk = [&](auto count_c, auto from_c, auto refill_c, int first) {
+    constexpr int kCount = decltype(count_c)::value, kFrom = decltype(from_c)::value;
+    constexpr bool kRefill = decltype(refill_c)::value;
+    constexpr int kAll = kCount * kTiles;
+    asm volatile("" : "+v"(lane16), "+v"(channel16));
+    i32x16 acc[2];
+    StaticFor<kAll + 1>([&](auto t_const) {
+      constexpr int t = decltype(t_const)::value;
+      if constexpr (t < kAll) {
+        constexpr int u = kFrom + t / kTiles, cj = t % kTiles / RT, rj = t % RT;
+        constexpr int s = u % BLOCKS;
+        acc[t % 2] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x[s][rj], w[s][cj], base_bits, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (kRefill && t % kTiles == kTiles - 1) {
+          fetch(std::integral_constant<int, s>{}, first + u + BLOCKS);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      if constexpr (t >= 1) {
+        constexpr int d = t - 1;
+        constexpr int u = kFrom + d / kTiles, cj = d % kTiles / RT, rj = d % RT;
+        constexpr int b = u % 4, cur = u / 4 % 2;
+        const float4& q = sg[cur][cj];
+        const float scale = b == 0 ? q.x : b == 1 ? q.y : b == 2 ? q.z : q.w;
+        const float offset = __fmul_rn(-kSumBase, scale);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          out[cj][rj][e] = __fadd_rn(out[cj][rj][e], ScaleBlockSum(acc[d % 2][e], scale, offset));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (kRefill && b == 3 && d % kTiles == kTiles - 1) {
+          fetch_scales(std::integral_constant<int, cur>{}, (first + u) / 4 + 2);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    });
+  };
+  constexpr int kTrip = 8;
+  static_assert(kTrip % BLOCKS == 0, "trip");
+  using std::integral_constant;
+  int first = 0;
+  for (; first + kTrip <= nb; first += kTrip) {
+    walk(integral_constant<int, kTrip>{}, integral_constant<int, 0>{}, std::true_type{}, first);
+  }
+  StaticFor<kTrip - 1>([&](auto u_const) {
+    constexpr int u = decltype(u_const)::value;
+    if (first + u < nb) {
+      walk(integral_constant<int, 1>{}, integral_constant<int, u>{}, std::false_type{}, first);
+      if constexpr (u + BLOCKS < kTrip - 1) {
+        fetch(integral_constant<int, u % BLOCKS>{}, first + u + BLOCKS);
+      }
+    }
+  });
+
+#pragma unroll
+  for (int rj = 0; rj < RT; ++rj) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int m0 = (rt0 + rj) * kWide + 8 * g + 4 * (lane >> 5);
+      float zp[4], row_scale[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int m = min(m0 + i, a.batches - 1);
+        zp[i] = static_cast<float>(a.zero_points[m]);
+        row_scale[i] = a.scaling_factors[m];
+      }
+#pragma unroll
+      for (int cj = 0; cj < CT; ++cj) {
+        const int n = (ct0 + cj) * kWide + (lane & 31);
+        if (n >= a.out_depth) continue;
+        const float kfsum = a.kfsum[n];
+        const float bias = a.bias ? a.bias[n] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float v = FinishOutput(out[cj][rj][4 * g + i], zp[i], kfsum, row_scale[i],
+                                       a.bias != nullptr, bias);
+          if (m0 + i < a.batches) a.output[static_cast<size_t>(m0 + i) * a.out_depth + n] = v;
         }
       }
     }
@@ -769,9 +998,9 @@ __global__ __launch_bounds__(THREADS) void QuantizeNibbleGroupRowsKernel(
 }  // namespace
 
 size_t GemmInt4BlockwiseBytes(int out_depth, int depth) {
-  const size_t tiles = (static_cast<size_t>(out_depth) + kTile - 1) / kTile;
+  const size_t tiles = (static_cast<size_t>(out_depth) + kWide - 1) / kWide;
   const size_t nb = static_cast<size_t>(depth) / kBlock;
-  return tiles * nb * (512 + kTile * sizeof(float));
+  return tiles * (nb * 1024 + (nb + 3) / 4 * kWide * 4 * sizeof(float));
 }
 
 bool FcInt4BlockwiseGemmSupports(int depth, int blocksize) {
@@ -782,25 +1011,47 @@ hipError_t LaunchPackInt4BlockwiseGemm(const uint8_t* filter, const uint16_t* sc
                                        int out_depth, int depth, uint8_t* packed,
                                        hipStream_t stream) {
   if (out_depth == 0 || depth == 0) return hipSuccess;
-  const int tiles = (out_depth + kTile - 1) / kTile;
+  const int tiles = (out_depth + kWide - 1) / kWide;
   const int nb = depth / kBlock;
-  const int64_t slots = static_cast<int64_t>(tiles) * nb * 64;
+  const int64_t slots = static_cast<int64_t>(tiles) * nb * 128;
   const unsigned grid = static_cast<unsigned>((slots + kThreads - 1) / kThreads);
   hipLaunchKernelGGL(PackInt4BlockwiseGemmKernel, dim3(grid), dim3(kThreads), 0, stream, filter,
                      scales_f16, out_depth, depth, tiles, nb, packed);
   return hipGetLastError();
 }
 
-// One row tile: 16 rows x the depth padded to whole pairs of blocks.
-static size_t RowTileBytes(int depth) {
-  return static_cast<size_t>(kTile) * ((static_cast<size_t>(depth) + 2 * kBlock - 1) /
-                                       (2 * kBlock) * (2 * kBlock));
+// One tile of 16 rows x the depth padded to whole pairs of blocks, or of 32 rows x the depth.
+static size_t RowTileBytes(int depth, int rows) {
+  return rows == kWide ? static_cast<size_t>(kWide) * depth
+                       : static_cast<size_t>(kTile) * ((static_cast<size_t>(depth) + 2 * kBlock - 1) /
+                                                       (2 * kBlock) * (2 * kBlock));
 }
 
 size_t TiledRowsBytes(int batches, int depth) {
-  const size_t row_tiles = (static_cast<size_t>(batches) + kTile - 1) / kTile;
-  return row_tiles * RowTileBytes(depth);
+  const size_t narrow = (static_cast<size_t>(batches) + kTile - 1) / kTile * RowTileBytes(depth, kTile);
+  const size_t wide = (static_cast<size_t>(batches) + kWide - 1) / kWide * RowTileBytes(depth, kWide);
+  return narrow > wide ? narrow : wide;
 }
+
+namespace {
+template <int ROWS>
+hipError_t LaunchTiledQuantizer(const float* input, int variant, int batches, int depth,
+                                void* tiled_rows, float* scaling_factors, int32_t* zero_points,
+                                hipStream_t stream) {
+  const dim3 grid((batches + ROWS - 1) / ROWS * ROWS), block(kQuantizeThreads);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, 0, stream, input, batches, depth,
+                       RowTileBytes(depth, ROWS), static_cast<int8_t*>(tiled_rows), scaling_factors,
+                       zero_points);
+    return hipGetLastError();
+  };
+  switch (variant) {
+    case LRTFC_QUANT_NEON_V8: return launch(QuantizeRowsTiledKernel<LRTFC_QUANT_NEON_V8, ROWS>);
+    case LRTFC_QUANT_NEON_LEGACY: return launch(QuantizeRowsTiledKernel<LRTFC_QUANT_NEON_LEGACY, ROWS>);
+    default: return launch(QuantizeRowsTiledKernel<LRTFC_QUANT_PORTABLE, ROWS>);
+  }
+}
+}  // namespace
 
 hipError_t LaunchFcInt4BlockwiseGemm(const float* input, int variant, float* scaling_factors,
                                      int32_t* zero_points, const uint8_t* gemm_filter,
@@ -809,34 +1060,10 @@ hipError_t LaunchFcInt4BlockwiseGemm(const float* input, int variant, float* sca
                                      hipStream_t stream) {
   if (batches == 0 || out_depth == 0) return hipSuccess;
   const int nb = depth / kBlock;
-  const int row_tiles = (batches + kTile - 1) / kTile;
-  const int channel_tiles = (out_depth + kTile - 1) / kTile;
-  {
-    const dim3 grid(row_tiles * kTile), block(kQuantizeThreads);
-    int8_t* tiled = static_cast<int8_t*>(tiled_rows);
-    const size_t tile_bytes = RowTileBytes(depth);
-    switch (variant) {
-      case LRTFC_QUANT_NEON_V8:
-        hipLaunchKernelGGL(QuantizeRowsTiledKernel<LRTFC_QUANT_NEON_V8>, grid, block, 0, stream,
-                           input, batches, depth, tile_bytes, tiled, scaling_factors, zero_points);
-        break;
-      case LRTFC_QUANT_NEON_LEGACY:
-        hipLaunchKernelGGL(QuantizeRowsTiledKernel<LRTFC_QUANT_NEON_LEGACY>, grid, block, 0,
-                           stream, input, batches, depth, tile_bytes, tiled, scaling_factors,
-                           zero_points);
-        break;
-      default:
-        hipLaunchKernelGGL(QuantizeRowsTiledKernel<LRTFC_QUANT_PORTABLE>, grid, block, 0, stream,
-                           input, batches, depth, tile_bytes, tiled, scaling_factors, zero_points);
-        break;
-    }
-    if (hipError_t err = hipGetLastError()) return err;
-  }
   GemmArgs a;
-  a.filter = reinterpret_cast<const i64*>(gemm_filter);
-  a.scales = reinterpret_cast<const float4*>(gemm_filter +
-                                             static_cast<size_t>(channel_tiles) * nb * 512);
-  a.activations = static_cast<const i64x2*>(tiled_rows);
+  a.filter = reinterpret_cast<const char*>(gemm_filter);
+  a.scales = a.filter + static_cast<size_t>((out_depth + kWide - 1) / kWide) * nb * 1024;
+  a.activations = static_cast<const char*>(tiled_rows);
   a.scaling_factors = scaling_factors;
   a.zero_points = zero_points;
   a.kfsum = kfsum;
@@ -845,35 +1072,44 @@ hipError_t LaunchFcInt4BlockwiseGemm(const float* input, int variant, float* sca
   a.batches = batches;
   a.out_depth = out_depth;
   a.nb = nb;
-  a.channel_tiles = channel_tiles;
-  a.row_tiles = row_tiles;
-  a.vector_store = (out_depth % 4 == 0) && (reinterpret_cast<uintptr_t>(output) % 16 == 0);
-  // Tiles per wavefront (channels x rows), the four wavefronts of a workgroup side by side
-  // along the channels. Measured at 14336 x 4096: up to 128 rows one channel tile per
-  // wavefront spreads the filter stream over the most wavefronts (128 rows: 42 us against 51 us
-  // with two; 256 rows: level); beyond, 2 x 4 tiles re-read the least.
-  const int CT = row_tiles <= 8 ? 1 : 2;
-  const int RT = row_tiles <= 1 ? 1 : row_tiles <= 2 ? 2 : 4;
-  const dim3 grid((channel_tiles + 4 * CT - 1) / (4 * CT), (row_tiles + RT - 1) / RT);
-  if (grid.y > 65535) return hipErrorInvalidValue;
-  // Pairs in flight: small tiles are bound by the filter stream and want many (16 rows: 19.5 us
-  // with 16 blocks in flight, 17.1 us with 32); the 2 x 4 form is bound by its arithmetic and
-  // runs best with one pair and 124 registers, four wavefronts per SIMD (2048 rows: 443 us
-  // against 462 us with two pairs and two wavefronts per SIMD).
-  if (CT == 2) {
-    hipLaunchKernelGGL((FcInt4BlockwiseGemmKernel<2, 4, 1, 1>), grid, dim3(kThreads), 0,
-                       stream, a);
-  } else if (RT == 4) {
-    hipLaunchKernelGGL((FcInt4BlockwiseGemmKernel<1, 4, 1, 4>), grid, dim3(kThreads), 0,
-                       stream, a);
-  } else if (RT == 2) {
-    hipLaunchKernelGGL((FcInt4BlockwiseGemmKernel<1, 2, 1, 8>), grid, dim3(kThreads), 0,
-                       stream, a);
-  } else {
-    hipLaunchKernelGGL((FcInt4BlockwiseGemmKernel<1, 1, 1, 16>), grid, dim3(kThreads), 0,
-                       stream, a);
-  }
-  return hipGetLastError();
+  auto launch = [&](auto kernel, auto tile_c, int ct, int rt, int wrows) {
+    constexpr int kRows = decltype(tile_c)::value;
+    if (hipError_t err = LaunchTiledQuantizer<kRows>(input, variant, batches, depth, tiled_rows,
+                                                     scaling_factors, zero_points, stream)) {
+      return err;
+    }
+    a.channel_tiles = (out_depth + kRows - 1) / kRows;
+    a.row_tiles = (batches + kRows - 1) / kRows;
+    const int wgs_c = (a.channel_tiles + 4 / wrows * ct - 1) / (4 / wrows * ct);
+    const int wgs_r = (a.row_tiles + wrows * rt - 1) / (wrows * rt);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(wgs_c) * wgs_r), dim3(kThreads), 0, stream,
+                       a, wgs_c, wgs_r);
+    return hipGetLastError();
+  };
+  using Narrow = std::integral_constant<int, kTile>;
+  using Wide = std::integral_constant<int, kWide>;
+  // Tiles per wavefront, by how many the launch has: a wavefront walks the whole depth, so a launch
+  // with few tiles wants them on as many wavefronts as there are SIMDs (1024), and one with many
+  // wants large ones, which re-read the least. Measured, us with the row quantizer's launch (S: 16 x
+  // 16 tiles, L: 32 x 32; channels x rows per wavefront):
+  //   rows x depth -> channels       S 1x1   S 1x2   L 1x1   L 1x2   L 2x2
+  //   64 x 4096 -> 4096               14.5    16.0    20.1    30.4    53
+  //   128 x 4096 -> 4096              22.8    17.6    20.9    31.4    53
+  //   200 x 2944 -> 2944              25.8    21.9    17.9    26.5    43
+  //   128 x 4096 -> 14336             57.7    43.5    28.8    33.2    55
+  //   512 x 4096 -> 4096              67.2    47.5    31.9    36.4    56
+  //   256 x 4096 -> 14336              110    71.4    51.5    44.9    58
+  //   512 x 4096 -> 14336              214     135    85.6    85.0    79
+  //   2048 x 4096 -> 14336             837     516     325     268    267
+  const int64_t narrow_tiles = static_cast<int64_t>((out_depth + kTile - 1) / kTile) *
+                               ((batches + kTile - 1) / kTile);
+  const int64_t wide_tiles = static_cast<int64_t>((out_depth + kWide - 1) / kWide) *
+                             ((batches + kWide - 1) / kWide);
+  if (narrow_tiles <= 1024) return launch(FcInt4BlockwiseGemmKernel<1, 1, 1, 8>, Narrow{}, 1, 1, 1);
+  if (narrow_tiles <= 2048) return launch(FcInt4BlockwiseGemmKernel<1, 2, 1, 4>, Narrow{}, 1, 2, 1);
+  if (wide_tiles <= 2560) return launch(FcInt4BlockwiseGemmLargeKernel<1, 1, 1, 8>, Wide{}, 1, 1, 1);
+  if (wide_tiles <= 6144) return launch(FcInt4BlockwiseGemmLargeKernel<1, 2, 1, 4>, Wide{}, 1, 2, 1);
+  return launch(FcInt4BlockwiseGemmLargeKernel<2, 2, 2, 2>, Wide{}, 2, 2, 2);
 }
 
 size_t GemmInt4BlockwiseNibbleBytes(int out_depth, int depth) {
@@ -895,18 +1131,6 @@ hipError_t LaunchPackInt4BlockwiseNibbles(const uint8_t* filter, const uint16_t*
                      filter, scales_f16, out_depth, depth, tiles, nb, nq, ng, packed);
   return hipGetLastError();
 }
-
-namespace {
-template <int VARIANT>
-void LaunchTiledQuantizer(const float* input, int batches, int depth, int row_tiles,
-                          void* tiled_rows, float* scaling_factors, int32_t* zero_points,
-                          hipStream_t stream) {
-  const dim3 grid(row_tiles * kTile), block(kQuantizeThreads);
-  hipLaunchKernelGGL(QuantizeRowsTiledKernel<VARIANT>, grid, block, 0, stream, input, batches,
-                     depth, RowTileBytes(depth), static_cast<int8_t*>(tiled_rows),
-                     scaling_factors, zero_points);
-}
-}  // namespace
 
 hipError_t LaunchFcInt4BlockwiseNibbleGemm(const float* input, int variant,
                                            float* scaling_factors, int32_t* zero_points,
@@ -945,21 +1169,10 @@ hipError_t LaunchFcInt4BlockwiseNibbleGemm(const float* input, int variant,
                        stream, q);
     return hipGetLastError();
   }
-  switch (variant) {
-    case LRTFC_QUANT_NEON_V8:
-      LaunchTiledQuantizer<LRTFC_QUANT_NEON_V8>(input, batches, depth, row_tiles, tiled_rows,
-                                                scaling_factors, zero_points, stream);
-      break;
-    case LRTFC_QUANT_NEON_LEGACY:
-      LaunchTiledQuantizer<LRTFC_QUANT_NEON_LEGACY>(input, batches, depth, row_tiles, tiled_rows,
-                                                    scaling_factors, zero_points, stream);
-      break;
-    default:
-      LaunchTiledQuantizer<LRTFC_QUANT_PORTABLE>(input, batches, depth, row_tiles, tiled_rows,
-                                                 scaling_factors, zero_points, stream);
-      break;
+  if (hipError_t err = LaunchTiledQuantizer<kTile>(input, variant, batches, depth, tiled_rows,
+                                                   scaling_factors, zero_points, stream)) {
+    return err;
   }
-  if (hipError_t err = hipGetLastError()) return err;
   NibbleGemmArgs a;
   a.filter = reinterpret_cast<const i32x4*>(nibble_filter);
   a.scales = reinterpret_cast<const uint2*>(
