@@ -66,10 +66,8 @@ bool FloatActivationOk(int activation) {
 
 // Batches from this size on go to the MFMA GEMM when its tiling fits.
 constexpr int kGemmMinBatches = 128;
-// On the re-tiled filter: up to this many rows the GEMV wins always (16 rows per pass over the
-// filter), and up to 32 rows where it can take them in one pass; beyond that the GEMM, which
-// streams the filter once.
-constexpr int kPackedGemmMinBatches = 16;
+// (On the re-tiled filter the GEMV takes what it streams the filter for once and fastest,
+// FcInt8PackedGemvTakesRowsInOnePass, the GEMMs everything else.)
 
 // Workspace layout for the hybrid paths on re-tiled filters (kernels.h): rows padded to whole
 // 16-byte pieces.
@@ -414,7 +412,7 @@ int lrtfc_fc_int8_packed(const int8_t* input, const int8_t* packed_filter, const
   a.act_min = act_min;
   a.act_max = act_max;
   a.output_i8 = output;
-  if (batches > kPackedGemmMinBatches && !lrtfc::FcInt8PackedGemvTakesRowsInOnePass(a) &&
+  if (!lrtfc::FcInt8PackedGemvTakesRowsInOnePass(a) &&
       lrtfc::FcInt8PackedGemmSupports(a)) {
     return FromHip(lrtfc::LaunchFcInt8PackedGemm(a, lrtfc::Int8Epilogue::kRequantize,
                                                  AsStream(stream)),
@@ -492,7 +490,7 @@ int FcHybridInt8Packed(const int8_t* quantized_input, const float* scaling_facto
   a.output_f32 = output;
   a.zero_input_exit = zero_input_exit;
   a.batch_matmul = batch_matmul;
-  if (batches > kPackedGemmMinBatches && !lrtfc::FcInt8PackedGemvTakesRowsInOnePass(a) &&
+  if (!lrtfc::FcInt8PackedGemvTakesRowsInOnePass(a) &&
       lrtfc::FcInt8PackedGemmSupports(a)) {
     return FromHip(lrtfc::LaunchFcInt8PackedGemm(a, lrtfc::Int8Epilogue::kHybrid,
                                                  AsStream(stream)),
@@ -955,7 +953,7 @@ int lrtfc_fc_hybrid_int4_per_channel_packed(const float* input, const int8_t* pa
   a.bias_f32 = bias;
   a.activation = activation;
   a.output_f32 = output;
-  if (batches > kPackedGemmMinBatches && !lrtfc::FcInt8PackedGemvTakesRowsInOnePass(a) &&
+  if (!lrtfc::FcInt8PackedGemvTakesRowsInOnePass(a) &&
       lrtfc::FcInt8PackedGemmSupports(a)) {
     return FromHip(lrtfc::LaunchFcInt8PackedGemm(a, lrtfc::Int8Epilogue::kHybrid4Bit,
                                                  AsStream(stream)),

@@ -452,11 +452,15 @@ bool FcInt8PackedGemmSupports(const FcInt8Args& a) {
 hipError_t LaunchFcInt8PackedGemm(const FcInt8Args& a, Int8Epilogue epilogue, hipStream_t stream) {
   if (!FcInt8PackedGemmSupports(a)) return hipErrorNotSupported;
   // 128 x 256 tiles move the fewest bytes per MFMA; a launch they would cut into fewer
-  // workgroups than half the chip's CUs takes 64 x 128 tiles instead (four times as many).
+  // workgroups than half the chip's CUs takes 64 x 128 tiles instead (four times as many), or,
+  // where those leave it idle too, small tiles with the depth split over the wavefronts.
   const int large = ((a.batches + 127) / 128) * ((a.out_depth + 255) / 256);
   if (large >= kMinLargeTiles) return LaunchShape<128, 2>(a, epilogue, large, stream);
-  return LaunchShape<64, 1>(a, epilogue, ((a.batches + 63) / 64) * ((a.out_depth + 127) / 128),
-                            stream);
+  const int small = ((a.batches + 63) / 64) * ((a.out_depth + 127) / 128);
+  if (FcInt8SplitGemmBeatsTiles(a, small)) {
+    return LaunchFcInt8SplitGemm(a, epilogue, stream);
+  }
+  return LaunchShape<64, 1>(a, epilogue, small, stream);
 }
 
 }  // namespace lrtfc

@@ -1170,8 +1170,10 @@ int FcInt8PackedGemvFusedMaxRows(int depth) {
 }
 
 bool FcInt8PackedGemvTakesRowsInOnePass(const FcInt8Args& a) {
-  if (a.batches <= 16) return FcInt8PackedGemvSupports(a);
-  if (!FcInt8PackedGemvSupports(a)) return false;
+  // (A depth that this kernel cannot take is refused here up to 16 rows, and goes to the GEMM above.)
+  if (!FcInt8PackedGemvSupports(a)) return a.batches <= 16;
+  if (FcInt8SplitGemmBeatsOnePass(a)) return false;
+  if (a.batches <= 16) return true;
   if (a.batches > 32) return FcInt8RowsGemvTakes(a);
   PackedArgs p;
   p.a = a;

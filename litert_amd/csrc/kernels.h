@@ -137,8 +137,9 @@ hipError_t LaunchFcInt4PerChannelGemv(const uint8_t* packed, const float* input_
 // Prefill batches on the same re-tiled filter: int8 MFMA GEMM (a.filter = packed, a.input =
 // int8 rows; the hybrid epilogue reads a.scaling_factors / a.zero_points). Any batch count,
 // any out_depth; depth a multiple of 16.
-// Whether the GEMV streams the filter once for all of a.batches rows (up to 16 always; 17 to 32
-// rows that arrive quantized when their LDS image fits a compute unit).
+// Whether a.batches rows that arrive quantized go to LaunchFcInt8PackedGemv: where it streams the
+// filter once for all of them (up to 16 rows, 17 to 32 when their LDS image fits a compute unit, up
+// to 128 on wide filters) and small GEMM tiles do not beat it (FcInt8SplitGemmBeatsOnePass).
 bool FcInt8PackedGemvTakesRowsInOnePass(const FcInt8Args& a);
 // 33 to 128 quantized rows on wide re-tiled filters: the filter streamed once, the rows through
 // LDS in depth chunks (fc_int8_rows_gemv.hip). FcInt8RowsGemvTakes: the shapes it is meant for.
@@ -146,6 +147,12 @@ bool FcInt8RowsGemvTakes(const FcInt8Args& a);
 hipError_t LaunchFcInt8RowsGemv(const FcInt8Args& a, Int8Epilogue epilogue, hipStream_t stream);
 bool FcInt8PackedGemmSupports(const FcInt8Args& a);
 hipError_t LaunchFcInt8PackedGemm(const FcInt8Args& a, Int8Epilogue epilogue, hipStream_t stream);
+// The same for launches that leave the chip idle in those tiles (fc_int8_split_gemm.hip): small tiles,
+// the depth dealt to the wavefronts of a workgroup. LaunchFcInt8PackedGemm takes it by itself.
+// BeatsOnePass: against LaunchFcInt8PackedGemv, for rows that it would take in one pass.
+bool FcInt8SplitGemmBeatsOnePass(const FcInt8Args& a);
+bool FcInt8SplitGemmBeatsTiles(const FcInt8Args& a, long workgroups_64x128);
+hipError_t LaunchFcInt8SplitGemm(const FcInt8Args& a, Int8Epilogue epilogue, hipStream_t stream);
 
 struct FcInt4Args {
   const int8_t* input;           // [batches, depth] quantized activations
