@@ -567,6 +567,7 @@ struct FcNode {
 // more than a separate quantization launch; deep int4 rows fuse at most two batch rows.
 constexpr int kInt4FusedMaxDepth = 4096;
 constexpr int kInt4DeepFusedMaxBatches = 2;
+constexpr int kInt4GroupedMaxOutDepth = 511 * 16;  // wider ones fill the chip by themselves from five rows on
 // Up to this many rows a per-channel int4 node streams its filter as nibbles (one pass per 16
 // rows); above, the MFMA GEMM on the int8 expansion streams it once.
 constexpr int kInt4PerChannelNibbleMaxBatches = 32;
@@ -1130,9 +1131,12 @@ TfLiteStatus PrepareNode(TfLiteContext* ctx, PartitionKernel* k, FcNode* n) {
     n->use_retiled = weights > 0 && lrtfc_fc_blockwise_int4_preferred_layout(
                                         n->depth, n->blocksize) == LRTFC_LAYOUT_PACKED;
     n->split_quantize = n->depth > kInt4FusedMaxDepth && n->batches > kInt4DeepFusedMaxBatches;
-    const int form = n->use_retiled ? lrtfc_fc_blockwise_int4_preferred_form(
-                                          n->batches, n->depth, n->out_depth)
-                                    : LRTFC_INT4_FORM_DECODE;
+    int form = n->use_retiled ? lrtfc_fc_blockwise_int4_preferred_form(n->batches, n->depth,
+                                                                       n->out_depth)
+                              : LRTFC_INT4_FORM_DECODE;
+    // The form picked for a call of its own. Narrow nodes of fewer than sixteen rows keep the
+    // decode tiling here: it runs several independent nodes as one launch.
+    if (n->batches < 16 && n->out_depth <= kInt4GroupedMaxOutDepth) form = LRTFC_INT4_FORM_DECODE;
     const bool want_nibbles = form == LRTFC_INT4_FORM_GEMM_NIBBLES;
     n->gemm_layout = form != LRTFC_INT4_FORM_DECODE;
     if (n->gemm_layout && n->have_gemm && want_nibbles != n->gemm_nibbles) n->have_gemm = false;

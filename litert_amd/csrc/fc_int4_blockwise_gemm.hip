@@ -620,11 +620,11 @@ struct NibbleGemmArgs {
   int vector_store;
 };
 
-// WQ: quads of weights in flight per wavefront; XQ: quads of activations in flight (they come
-// from L2 and cost 8 registers per row tile and quad, so this ring is shorter). Measured at
-// 14336 x 4096, 16 rows: 8 and 4 quads 16.9 us for quantizer + product; 16 weight quads 18.1 us
-// -- a wavefront is alone on its SIMD here (896 wavefronts), and what bounds it is its own
-// chain of about 15 vector operations per block, not the loads.
+// A wavefront alone on its SIMD issues a vector operation every 8 cycles or so, and a block takes
+// 15 of them; with a branch per block, behind which each MFMA waited for the conversions and
+// additions of the one before, 14336 x 4096 at 16 rows took 16.9 us with the row quantizer, now
+// 14.1 us. One, two and four groups of 16 blocks in flight measure the same. Row tiles are
+// wavefronts of their own for the same reason (32 rows 19.0 us, as two tiles of one wavefront 22.3).
 // The wavefronts of the 4-bit-resident kernels share nothing (no LDS image, no barrier), so each is
 // a workgroup of its own: the dispatcher then spreads them one by one over the compute units.
 // In workgroups of four, a launch of 2304 wavefronts leaves 64 compute units with three
@@ -632,142 +632,243 @@ struct NibbleGemmArgs {
 // rows: 84 us; as single wavefronts 71 us; 28672 x 16384: 59.6 -> 54.5 us).
 constexpr int kLoneWave = 64;
 
-template <int RT, int WQ, int XQ>
+template <int QUADS>  // of blocks in flight
 __global__ __launch_bounds__(kLoneWave) void FcInt4NibbleGemmKernel(NibbleGemmArgs a) {
   const int lane = threadIdx.x & 63;
   const int ct0 = blockIdx.x;
-  const int rt0 = blockIdx.y * RT;
+  const int rt0 = blockIdx.y;
   if (ct0 >= a.channel_tiles || rt0 >= a.row_tiles) return;
-  int rt[RT];
-#pragma unroll
-  for (int j = 0; j < RT; ++j) rt[j] = min(rt0 + j, a.row_tiles - 1);
   const int nb = a.nb;
   const int pairs = (nb + 1) / 2;
   const int nq = (nb + 3) / 4;
   const int ng = (nb + 15) / 16;
   const i32x4* wp = a.filter + static_cast<size_t>(ct0) * nq * 64 + lane;
   const uint2* sp = a.scales + static_cast<size_t>(ct0) * ng * 64 + lane;
-  const i64x2* xp[RT];
-#pragma unroll
-  for (int j = 0; j < RT; ++j) {
-    xp[j] = a.activations + static_cast<size_t>(rt[j]) * pairs * 64 + lane;
-  }
+  const i64x2* xp = a.activations + static_cast<size_t>(rt0) * pairs * 64 + lane;
   // Past the end: a hot line, result unused.
   auto fetch_w = [&](int q) {
     return __builtin_nontemporal_load(wp + static_cast<size_t>(min(q, nq - 1)) * 64);
   };
   struct XStage {
-    i64x2 x[RT][2];  // row tiles: blocks 0-1, blocks 2-3 of the quad
+    i64x2 x[2];  // blocks 0-1, blocks 2-3 of the quad
   };
   auto fetch_x = [&](int q) {
     const int qq = min(q, nq - 1);
     XStage st;
-#pragma unroll
-    for (int j = 0; j < RT; ++j) {
-      st.x[j][0] = xp[j][static_cast<size_t>(min(2 * qq, pairs - 1)) * 64];
-      st.x[j][1] = xp[j][static_cast<size_t>(min(2 * qq + 1, pairs - 1)) * 64];
-    }
+    st.x[0] = xp[static_cast<size_t>(min(2 * qq, pairs - 1)) * 64];
+    st.x[1] = xp[static_cast<size_t>(min(2 * qq + 1, pairs - 1)) * 64];
     return st;
   };
-  // Scale groups (16 blocks = 4 quads): the current one and as many ahead as the weight ring
-  // reaches, so that a group is requested before its blocks' weights.
-  constexpr int kGroups = WQ / 4 + 1 <= 2 ? 2 : (WQ / 4 + 1 <= 4 ? 4 : 8);
-  static_assert((kGroups - 1) * 4 >= WQ, "scale groups must lead the weight ring");
-  uint2 sg[kGroups];
   auto fetch_scales = [&](int g) { return sp[static_cast<size_t>(min(g, ng - 1)) * 64]; };
+  constexpr int kGroups = QUADS / 4;  // scale groups per trip
+  uint2 sg[kGroups];
+  i32x4 wring[QUADS];
+  XStage xring[QUADS];
 #pragma unroll
-  for (int g = 0; g + 1 < kGroups; ++g) sg[g] = fetch_scales(g);
-  i32x4 wring[WQ];
-  XStage xring[XQ];
-#pragma unroll
-  for (int s = 0; s < WQ; ++s) wring[s] = fetch_w(s);
-#pragma unroll
-  for (int s = 0; s < XQ; ++s) xring[s] = fetch_x(s);
+  for (int s = 0; s < QUADS; ++s) {
+    if (s % 4 == 0) sg[s / 4] = fetch_scales(s / 4);
+    wring[s] = fetch_w(s);
+    xring[s] = fetch_x(s);
+  }
 
-  // out[rj][i]: channel 16 ct0 + 4 (lane / 16) + i, batch row 16 rt[rj] + lane % 16, times 16.
-  float out[RT][4];
-#pragma unroll
-  for (int rj = 0; rj < RT; ++rj)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) out[rj][i] = 0.0f;
-
+  // out[i]: channel 16 ct0 + 4 (lane / 16) + i, batch row 16 rt0 + lane % 16, times 16.
+  float out[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  // Whole groups without a branch: the blocks that pad the last group have scales of zero, and
+  // adding the zero product leaves a running sum, which is never -0, as it is. A quad's MFMAs are
+  // issued ahead of the conversions, products and additions of the quad before it.
   const i32x4 zero = {0, 0, 0, 0};
-  constexpr int kTrip = WQ > 4 * kGroups ? WQ : 4 * kGroups;
-  static_assert(kTrip % WQ == 0 && kTrip % XQ == 0 && kTrip % (4 * kGroups) == 0, "trip");
-  float4 cur_scales = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  for (int base = 0; base < nq; base += kTrip) {
-    StaticFor<kTrip>([&](auto u_const) {
-      constexpr int u = decltype(u_const)::value;
-      constexpr int cur = (u / 4) % kGroups;
-      if constexpr (u % 4 == 0) {
-        // A new group of 16 blocks starts: its scales become float32, and the slot of the group
-        // before it takes the farthest one.
-        const uint2 raw = sg[cur];
-        cur_scales = make_float4(HalfBitsToFloatFast(static_cast<uint16_t>(raw.x & 0xFFFF)),
-                                 HalfBitsToFloatFast(static_cast<uint16_t>(raw.x >> 16)),
-                                 HalfBitsToFloatFast(static_cast<uint16_t>(raw.y & 0xFFFF)),
-                                 HalfBitsToFloatFast(static_cast<uint16_t>(raw.y >> 16)));
-        sg[(cur + kGroups - 1) % kGroups] = fetch_scales((base + u) / 4 + kGroups - 1);
+  float4 scales = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  i32x4 acc[2][4] = {{zero, zero, zero, zero}, {zero, zero, zero, zero}};
+  auto add_quad = [&](auto u_const) {  // quad u of its group
+    constexpr int u = decltype(u_const)::value;
+    StaticFor<4>([&](auto h_const) {
+      constexpr int h = decltype(h_const)::value;
+      constexpr int j = 4 * u + h;  // this block within its scale group
+      const float sc[4] = {RowBroadcast<j>(scales.x), RowBroadcast<j>(scales.y),
+                           RowBroadcast<j>(scales.z), RowBroadcast<j>(scales.w)};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        out[i] = __fadd_rn(out[i], __fmul_rn(static_cast<float>(acc[u % 2][h][i]), sc[i]));
       }
-      const i32x4 w = wring[u % WQ];
-      wring[u % WQ] = fetch_w(base + u + WQ);
-      const XStage st = xring[u % XQ];
-      xring[u % XQ] = fetch_x(base + u + XQ);
-      StaticFor<4>([&](auto h_const) {
-        constexpr int h = decltype(h_const)::value;
-        if (4 * (base + u) + h < nb) {
-          constexpr int j = (4 * u + h) % 16;  // this block within its scale group
-          const float sc[4] = {RowBroadcast<j>(cur_scales.x), RowBroadcast<j>(cur_scales.y),
-                               RowBroadcast<j>(cur_scales.z), RowBroadcast<j>(cur_scales.w)};
+    });
+  };
+  for (int g = 0; g < ng; g += kGroups) {
+    StaticFor<kGroups>([&](auto g_const) {
+      constexpr int gi = decltype(g_const)::value;
+      if (gi > 0 && g + gi >= ng) return;
+      StaticFor<4>([&](auto u_const) {
+        constexpr int u = decltype(u_const)::value;  // quad of the group
+        constexpr int slot = 4 * gi + u;
+        const int next = 4 * (g + gi + kGroups) + u;
+        const i32x4 w = wring[slot];
+        const XStage st = xring[slot];
+        StaticFor<4>([&](auto h_const) {
+          constexpr int h = decltype(h_const)::value;
           const uint32_t d = static_cast<uint32_t>(w[h]);
           const uint32_t lo = (d << 4) & 0xF0F0F0F0u;
           const uint32_t hi = d & 0xF0F0F0F0u;
           const i64 wa = static_cast<i64>(static_cast<uint64_t>(lo) |
                                           (static_cast<uint64_t>(hi) << 32));
-#pragma unroll
-          for (int rj = 0; rj < RT; ++rj) {
-            const i32x4 acc =
-                __builtin_amdgcn_mfma_i32_16x16x32_i8(wa, st.x[rj][h >> 1][h & 1], zero, 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              out[rj][i] = __fadd_rn(out[rj][i], __fmul_rn(static_cast<float>(acc[i]), sc[i]));
-            }
-          }
+          acc[u % 2][h] =
+              __builtin_amdgcn_mfma_i32_16x16x32_i8(wa, st.x[h >> 1][h & 1], zero, 0, 0, 0);
+        });
+        wring[slot] = fetch_w(next);
+        xring[slot] = fetch_x(next);
+        __builtin_amdgcn_sched_barrier(0);
+        add_quad(std::integral_constant<int, (u + 3) % 4>{});  // of the quad before
+        if constexpr (u == 0) {
+          const uint2 raw = sg[gi];
+          scales = make_float4(HalfBitsToFloatFast(static_cast<uint16_t>(raw.x & 0xFFFF)),
+                               HalfBitsToFloatFast(static_cast<uint16_t>(raw.x >> 16)),
+                               HalfBitsToFloatFast(static_cast<uint16_t>(raw.y & 0xFFFF)),
+                               HalfBitsToFloatFast(static_cast<uint16_t>(raw.y >> 16)));
+          sg[gi] = fetch_scales(g + gi + kGroups);
         }
+        __builtin_amdgcn_sched_barrier(0);
       });
     });
   }
+  add_quad(std::integral_constant<int, 3>{});
 
   // fully_connected.cc:1078-1082: zero-point term, row scale, bias -- after taking the factor
   // 16 back out (exact).
+  const int m = rt0 * kTile + (lane & 15);
+  if (m >= a.batches) return;
+  const float zp = static_cast<float>(a.zero_points[m]);
+  const float row_scale = a.scaling_factors[m];
+  const int n0 = ct0 * kTile + 4 * (lane >> 4);
+  float o[4];
 #pragma unroll
-  for (int rj = 0; rj < RT; ++rj) {
-    if (rt0 + rj >= a.row_tiles) break;
-    const int m = rt[rj] * kTile + (lane & 15);
-    if (m >= a.batches) continue;
-    const float zp = static_cast<float>(a.zero_points[m]);
-    const float row_scale = a.scaling_factors[m];
-    const int n0 = ct0 * kTile + 4 * (lane >> 4);
-    float o[4];
+  for (int i = 0; i < 4; ++i) {
+    const int n = min(n0 + i, a.out_depth - 1);
+    o[i] = FinishOutput(__fmul_rn(out[i], 0.0625f), zp, a.kfsum[n], row_scale, a.bias != nullptr,
+                        a.bias ? a.bias[n] : 0.0f);
+  }
+  float* dst = a.output + static_cast<size_t>(m) * a.out_depth + n0;
+  if (n0 + 3 < a.out_depth && a.vector_store) {
+    *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]);
+  } else {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int n = min(n0 + i, a.out_depth - 1);
-      float v = __fsub_rn(__fmul_rn(out[rj][i], 0.0625f), __fmul_rn(zp, a.kfsum[n]));
-      v = __fmul_rn(v, row_scale);
-      if (a.bias) v = __fadd_rn(v, a.bias[n]);
-      o[i] = v;
-    }
-    float* dst = a.output + static_cast<size_t>(m) * a.out_depth + n0;
-    if (n0 + 3 < a.out_depth && a.vector_store) {
-      *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (n0 + i < a.out_depth) dst[i] = o[i];
-      }
+      if (n0 + i < a.out_depth) dst[i] = o[i];
     }
   }
 }
+
+// The same product where tiles are few (narrow filters): the depth of a tile dealt to the four
+// wavefronts of a workgroup. One wavefront that walks it alone takes 46 ns a block, and only the
+// additions, a quarter of that, have to be in block order. So wavefront s takes blocks 16 s ...
+// + 16 of every 64, leaves their scaled sums in registers (4 per block), and the running outputs
+// go from wavefront to wavefront through LDS, four turns with a barrier each, in which a wavefront
+// only adds (16 blocks, 4 chains side by side); the operands of its next 16 blocks are requested
+// before the turns. Rows are the MFMA's A operand, so a lane's four sums share one channel and one
+// scale. Results are bit-identical to the other forms. With the row quantizer, one wavefront per tile -> here: 16 x 4096 -> 4096
+// 12.6 -> 10.5 us, 16 x 16384 -> 2048 33.4 -> 26.8 us (the int8-expanded GEMM 48.8). Rounds of 128
+// blocks (eight wavefronts, or 32 blocks each) were no faster, and products made in the slots
+// between a wavefront's turns slower (244 registers, loads waited for in each slot: 13.6 us).
+constexpr int kChainWaves = 4;
+constexpr int kChainBlocks = 16;  // per wavefront and round: one scale group, four quads
+
+__global__ __launch_bounds__(kChainWaves * 64, 2) void FcInt4NibbleChainKernel(NibbleGemmArgs a) {
+  constexpr int kScaleStride = kChainBlocks + 8;  // halves: 16-byte lines, spread over the banks
+  __shared__ float carry[4][64];
+  __shared__ __align__(16) uint16_t scale_lines[kChainWaves][kTile][kScaleStride];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ct0 = blockIdx.x, rt0 = blockIdx.y;
+  const int nb = a.nb;
+  const int pairs = (nb + 1) / 2, nq = (nb + 3) / 4, ng = (nb + 15) / 16;
+  const i32x4* wp = a.filter + static_cast<size_t>(ct0) * nq * 64 + lane;
+  const uint2* sp = a.scales + static_cast<size_t>(ct0) * ng * 64 + lane;
+  const i64x2* xp = a.activations + static_cast<size_t>(rt0) * pairs * 64 + lane;
+  uint2 sg;
+  i32x4 w[4];
+  i64x2 x[4][2];
+  auto request = [&](int group) {  // past the end: clamped addresses, results unused
+    sg = sp[static_cast<size_t>(min(group, ng - 1)) * 64];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int q = min(4 * group + u, nq - 1);
+      w[u] = __builtin_nontemporal_load(wp + static_cast<size_t>(q) * 64);
+      x[u][0] = xp[static_cast<size_t>(min(2 * q, pairs - 1)) * 64];
+      x[u][1] = xp[static_cast<size_t>(min(2 * q + 1, pairs - 1)) * 64];
+    }
+  };
+  request(wave);
+
+  // The output this lane finishes: register `wave` of the tile, i.e. row 4 (L / 16) + wave, channel
+  // L % 16.
+  const int m = rt0 * kTile + 4 * (lane >> 4) + wave;
+  const int n = ct0 * kTile + (lane & 15);
+  const int mc = min(m, a.batches - 1), nc = min(n, a.out_depth - 1);
+  const float zp = static_cast<float>(a.zero_points[mc]);
+  const float row_scale = a.scaling_factors[mc];
+  const float kfsum = a.kfsum[nc];
+  const float bias = a.bias ? a.bias[nc] : 0.0f;
+
+  const i32x4 zero = {0, 0, 0, 0};
+  uint16_t* const my_lines = &scale_lines[wave][0][0];
+  for (int group0 = 0; group0 < ng; group0 += kChainWaves) {
+    const int group = group0 + wave;
+    // Scales arrive as (block, four channels) per lane and are wanted as (channel, blocks): through
+    // LDS of the wavefront's own, whose operations stay in order.
+    uint16_t* to = my_lines + (lane >> 4) * 4 * kScaleStride + (lane & 15);
+    to[0] = static_cast<uint16_t>(sg.x);
+    to[kScaleStride] = static_cast<uint16_t>(sg.x >> 16);
+    to[2 * kScaleStride] = static_cast<uint16_t>(sg.y);
+    to[3 * kScaleStride] = static_cast<uint16_t>(sg.y >> 16);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+    float product[kChainBlocks][4];
+    StaticFor<2>([&](auto e_const) {
+      constexpr int e = decltype(e_const)::value;
+      const i32x4 raw = *reinterpret_cast<const i32x4*>(my_lines + (lane & 15) * kScaleStride + 8 * e);
+      StaticFor<8>([&](auto b_const) {
+        constexpr int b = 8 * e + decltype(b_const)::value;
+        const uint32_t pair = static_cast<uint32_t>(raw[(b % 8) / 2]);
+        const float scale = HalfBitsToFloatFast(static_cast<uint16_t>(b % 2 ? pair >> 16 : pair & 0xFFFF));
+        const uint32_t d = static_cast<uint32_t>(w[b / 4][b % 4]);
+        const uint32_t lo = (d << 4) & 0xF0F0F0F0u;
+        const uint32_t hi = d & 0xF0F0F0F0u;
+        const i64 wb = static_cast<i64>(static_cast<uint64_t>(lo) | (static_cast<uint64_t>(hi) << 32));
+        const i32x4 acc = __builtin_amdgcn_mfma_i32_16x16x32_i8(x[b / 4][(b % 4) / 2][b % 2], wb, zero, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          product[b][i] = __fmul_rn(static_cast<float>(acc[i]), scale);
+        }
+      });
+    });
+    const int valid = min(nb - group * kChainBlocks, kChainBlocks);
+    request(group + kChainWaves);
+    for (int turn = 0; turn < kChainWaves; ++turn) {
+      if (turn == wave && valid > 0) {
+        float out[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) out[i] = group == 0 ? 0.0f : carry[i][lane];
+        StaticFor<kChainBlocks>([&](auto b_const) {
+          constexpr int b = decltype(b_const)::value;
+          if (b < valid) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) out[i] = __fadd_rn(out[i], product[b][i]);
+          }
+        });
+#pragma unroll
+        for (int i = 0; i < 4; ++i) carry[i][lane] = out[i];
+      }
+      __syncthreads();
+    }
+  }
+  // fully_connected.cc:1078-1082, after taking the factor 16 back out (exact).
+  if (m < a.batches && n < a.out_depth) {
+    a.output[static_cast<size_t>(m) * a.out_depth + n] = FinishOutput(
+        __fmul_rn(carry[wave][lane], 0.0625f), zp, kfsum, row_scale, a.bias != nullptr, bias);
+  }
+}
+
+// The four-wavefront kernel up to this many tiles (two workgroups per CU); with more the chip is
+// busy enough that one wavefront per tile moves less (us, wavefronts: 16 x 2976 -> 5003, 313 tiles,
+// 10.9 / 11.1; 32 x 4096 -> 4096, 512 tiles, 12.3 / 13.2; 64 x 4096 -> 4096, 1024 tiles, 17.6 / 14.6).
+constexpr int kChainMaxTiles = 512;
 
 
 // ---- the same filter for one to four rows: four blocks per matrix-core tile ----------------
@@ -1003,6 +1104,11 @@ size_t GemmInt4BlockwiseBytes(int out_depth, int depth) {
   return tiles * (nb * 1024 + (nb + 3) / 4 * kWide * 4 * sizeof(float));
 }
 
+bool FcInt4NibbleGemmFewTiles(int batches, int out_depth) {
+  return static_cast<int64_t>((batches + kTile - 1) / kTile) * ((out_depth + kTile - 1) / kTile) <=
+         kChainMaxTiles;
+}
+
 bool FcInt4BlockwiseGemmSupports(int depth, int blocksize) {
   return blocksize == kBlock && depth > 0 && depth % kBlock == 0;
 }
@@ -1189,13 +1295,12 @@ hipError_t LaunchFcInt4BlockwiseNibbleGemm(const float* input, int variant,
   a.channel_tiles = channel_tiles;
   a.row_tiles = row_tiles;
   a.vector_store = (out_depth % 4 == 0) && (reinterpret_cast<uintptr_t>(output) % 16 == 0);
-  const int RT = row_tiles <= 1 ? 1 : 2;
-  const dim3 grid(channel_tiles, (row_tiles + RT - 1) / RT);
+  const dim3 grid(channel_tiles, row_tiles);
   if (grid.y > 65535) return hipErrorInvalidValue;
-  if (RT == 1) {
-    hipLaunchKernelGGL((FcInt4NibbleGemmKernel<1, 8, 4>), grid, dim3(kLoneWave), 0, stream, a);
+  if (FcInt4NibbleGemmFewTiles(batches, out_depth)) {
+    hipLaunchKernelGGL(FcInt4NibbleChainKernel, grid, dim3(kChainWaves * 64), 0, stream, a);
   } else {
-    hipLaunchKernelGGL((FcInt4NibbleGemmKernel<2, 8, 2>), grid, dim3(kLoneWave), 0, stream, a);
+    hipLaunchKernelGGL(FcInt4NibbleGemmKernel<8>, grid, dim3(kLoneWave), 0, stream, a);
   }
   return hipGetLastError();
 }

@@ -206,6 +206,8 @@ hipError_t LaunchFcInt4Packed(const FcInt4Args& q, const uint8_t* packed, const 
 // arrays of `batches` entries, by a launch ahead of the GEMM's.
 size_t GemmInt4BlockwiseBytes(int out_depth, int depth);
 bool FcInt4BlockwiseGemmSupports(int depth, int blocksize);
+// Whether the 4-bit-resident GEMM gives every output tile four wavefronts: its fastest form.
+bool FcInt4NibbleGemmFewTiles(int batches, int out_depth);
 hipError_t LaunchPackInt4BlockwiseGemm(const uint8_t* filter, const uint16_t* scales_f16,
                                        int out_depth, int depth, uint8_t* packed,
                                        hipStream_t stream);

@@ -48,3 +48,34 @@ def test_int4_gemm_extreme_scales_and_sums(fc, B):  # noqa: F811
     op = fc.FullyConnectedBlockwiseInt4(packed, scales, K, 32)
     assert _bits_equal(op.call_gemm(_cuda(x)).cpu().numpy(), want)
     assert _bits_equal(op.call_gemm_nibbles(_cuda(x)).cpu().numpy(), want)
+
+
+# Four wavefronts per tile up to 512 tiles, one beyond: (5, 8191) has 512 tiles, (5, 8193) 513.
+@pytest.mark.parametrize("B,N", [(5, 19), (16, 530), (17, 4096), (5, 8191), (5, 8193), (33, 3001)])
+@pytest.mark.parametrize("blocks", [1, 2, 15, 16, 17, 31, 63, 64, 65, 131])
+def test_int4_nibble_forms_match_oracle(fc, B, N, blocks):  # noqa: F811
+    K = 32 * blocks
+    if B * N * K > 2.5e8:
+        pytest.skip("the oracle takes long, and this form's rounds are covered at narrower filters")
+    c = wl.blockwise_int4_fc(B, K, N, seed=B + N + K, lo=-8, hi=7)
+    bias = np.random.default_rng(K).standard_normal(N).astype(np.float32) if blocks % 2 else None
+    op = fc.FullyConnectedBlockwiseInt4(c["packed"], c["scales"], K, 32, bias=bias)
+    want = oracle.fc_blockwise_int4(c["x"], c["packed"], N, c["scales"].view(np.uint16), 32, bias=bias)
+    assert _bits_equal(op.call_gemm_nibbles(_cuda(c["x"])).cpu().numpy(), want)
+    assert _bits_equal(op(_cuda(c["x"])).cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("B,N", [(5, 70), (5, 8300)])
+def test_int4_nibble_infinite_scales(fc, B, N):  # noqa: F811
+    """A channel with an infinite block scale gives what float32 arithmetic gives, its neighbours what
+    they give without it."""
+    c = wl.blockwise_int4_fc(B, 544, N, seed=5)
+    scales = c["scales"].copy()
+    scales[3, 2] = np.inf
+    scales[N - 1, 16] = -np.inf
+    scales[7, 0] = np.nan
+    want = oracle.fc_blockwise_int4(c["x"], c["packed"], N, scales.view(np.uint16), 32)
+    op = fc.FullyConnectedBlockwiseInt4(c["packed"], scales, 544, 32)
+    got = op.call_gemm_nibbles(_cuda(c["x"])).cpu().numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[~np.isnan(got)], want[~np.isnan(want)])
