@@ -32,6 +32,7 @@ using f32x4 = float __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / kWaveSize;
+constexpr int kWideThreads = 512;  // single nodes of deep rows
 constexpr int kBlock = 32;       // weights per quantization block
 constexpr int kTileRows = 8;
 constexpr int kTileBlocks = 64;
@@ -121,7 +122,7 @@ __device__ __forceinline__ uint32_t UDot8(uint32_t a, uint32_t b, uint32_t acc) 
 // LDS map: [BT][padded depth] activations as nibble planes (per block of 32: four dwords of
 // high nibbles, then four of low nibbles); per wavefront [8 * BT][kPStride]
 // parked products; per-row quantization state.
-template <int BT>
+template <int BT, int THREADS = kThreads>
 struct Int4Shared {
   int32_t* q;   // dwords: per row padded_depth / 4
   float* p;     // [waves][8 * BT][kPStride]
@@ -136,12 +137,12 @@ struct Int4Shared {
   // alone; every tile of the group when `ksplit` wavefronts share it (the ordered walk then
   // needs them all).
   __host__ __device__ static size_t ProductFloats(int chunks, int ksplit) {
-    constexpr int waves = kWaves;
+    constexpr int waves = THREADS / kWaveSize;
     const size_t tile = static_cast<size_t>(8) * BT * kPStride;
     return ksplit == 1 ? waves * tile : (waves / ksplit) * static_cast<size_t>(chunks) * tile;
   }
   __device__ Int4Shared(int8_t* base, int padded, int chunks, int ksplit) {
-    constexpr int waves = kWaves;
+    constexpr int waves = THREADS / kWaveSize;
     q = reinterpret_cast<int32_t*>(base);
     size_t off = static_cast<size_t>(BT) * padded;
     p = reinterpret_cast<float*>(base + off);
@@ -155,7 +156,7 @@ struct Int4Shared {
     ob = kb + waves * 2 * 64;
   }
   static size_t Bytes(int padded, int ksplit) {
-    constexpr int waves = kWaves;
+    constexpr int waves = THREADS / kWaveSize;
     const int chunks = padded / (kTileBlocks * kBlock);
     return static_cast<size_t>(BT) * padded + ProductFloats(chunks, ksplit) * 4 + 4 * 8 * 4 +
            BT * waves * 2 * 4 + waves * 2 * 64 * 4 + waves * 64 * BT * 4;
@@ -183,9 +184,10 @@ __device__ __forceinline__ void StaticFor(F&& f) {
 // some tens of KiB of outstanding loads, and a wavefront whose load issue blocks cannot do its
 // share of the row quantizer (14336 x 4096, one row: two tiles per wavefront, one ahead, 8.3 us;
 // both ahead 9.0 us; four tiles per wavefront all ahead 9.9 us; the refilled ring of two 8.5 us).
-template <int BT, bool FUSED, int VARIANT, int GPT, int ALL = 0, int PRE = 0>
+template <int BT, bool FUSED, int VARIANT, int GPT, int ALL = 0, int PRE = 0, int THREADS = kThreads>
 __device__ __forceinline__ void FcInt4PackedBody(const Int4PackedArgs& a, int block, int batch0,
                                                  int bt, int ksplit, int gpw, int8_t* smem) {
+  constexpr int kThreads = THREADS, kWaves = THREADS / kWaveSize;
 
   // Every tensor is in global memory. Pointers that a kernel read from a table in memory
   // carry no address space, and accesses through them would go the flat path, whose waits
@@ -215,7 +217,7 @@ __device__ __forceinline__ void FcInt4PackedBody(const Int4PackedArgs& a, int bl
   const int first_group = min(group0, groups - 1);
   const LRTFC_GLOBAL i32x4* tbase = g_packed +
                        static_cast<size_t>(first_group) * chunks * kTileVecs + lane;
-  Int4Shared<BT> sh(smem, padded, chunks, ksplit);
+  Int4Shared<BT, THREADS> sh(smem, padded, chunks, ksplit);
   // Per-channel epilogue inputs of every channel this wavefront covers (lane = channel),
   // requested ahead of the weights and parked in LDS once the prologue is through.
   const int my_n = min(first_group * kTileRows + lane, a.out_depth - 1);
@@ -471,6 +473,35 @@ __device__ __forceinline__ void FcInt4PackedBody(const Int4PackedArgs& a, int bl
       for (int j = 0; j < count; ++j) out = __fadd_rn(out, line[j]);
     }
   };
+  // The same over all tiles of a group, half a tile read ahead of the additions: the reads of a
+  // tile take a third as long as its 64 dependent additions.
+  auto walk_whole_tiles = [&](const float* tiles) {
+    constexpr int kAhead = kTileBlocks / 8;  // float4 per half tile
+    const float* line = tiles + lane * kPStride;
+    auto read_half = [&](int half, float4* v) {
+      const float4* from = reinterpret_cast<const float4*>(
+          line + static_cast<size_t>(half >> 1) * kTileFloats + (half & 1) * (kTileBlocks / 2));
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j) v[j] = from[j];
+    };
+    auto add_half = [&](const float4* v) {
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j) {
+        out = __fadd_rn(out, v[j].x);
+        out = __fadd_rn(out, v[j].y);
+        out = __fadd_rn(out, v[j].z);
+        out = __fadd_rn(out, v[j].w);
+      }
+    };
+    float4 even[kAhead], odd[kAhead];
+    read_half(0, even);
+    for (int half = 0; half < 2 * chunks; half += 2) {
+      read_half(half + 1, odd);
+      add_half(even);
+      read_half(min(half + 2, 2 * chunks - 1), even);
+      add_half(odd);
+    }
+  };
   // fully_connected.cc:1078-1082 for the channel group at offset `goff` from the first. The
   // value is parked in LDS and leaves in one store at the end: a store inside the tile loop
   // would make the number of outstanding memory operations depend on the path taken, and
@@ -563,7 +594,7 @@ __device__ __forceinline__ void FcInt4PackedBody(const Int4PackedArgs& a, int bl
   int lin = kpart;
   if constexpr (ALL > 0) {
     StaticFor<ALL>([&](auto t) {
-      if (decltype(t)::value < ntiles) {
+      if (kpart + decltype(t)::value * ksplit < ntiles) {
         process(t, std::false_type{}, decltype(t)::value, c);
         LRTFC_INT4_ADVANCE();
       }
@@ -585,8 +616,12 @@ __device__ __forceinline__ void FcInt4PackedBody(const Int4PackedArgs& a, int bl
     // Every tile of the group is parked; its first wavefront walks them in depth order.
     __syncthreads();
     if (kpart == 0 && chain_lane && my_groups > 0) {
-      for (int cc = 0; cc < chunks; ++cc) {
-        walk_tile(pgroup + static_cast<size_t>(cc) * kTileFloats, cc);
+      if (ALL == 1 && nblk == chunks * kTileBlocks) {
+        walk_whole_tiles(pgroup);
+      } else {
+        for (int cc = 0; cc < chunks; ++cc) {
+          walk_tile(pgroup + static_cast<size_t>(cc) * kTileFloats, cc);
+        }
       }
       finish_group(0);
     }
@@ -608,8 +643,8 @@ __device__ __forceinline__ void FcInt4PackedBody(const Int4PackedArgs& a, int bl
 // shapes): the library is built with kernel-argument preloading, which hands the leading scalar
 // arguments to a wavefront in registers when it starts; the rest of the argument block is read
 // from memory as usual while the first loads are already under way.
-template <int BT, bool FUSED, int VARIANT, int GPT, int ALL, int PRE>
-__global__ __launch_bounds__(kThreads) void FcInt4PackedKernel(
+template <int BT, bool FUSED, int VARIANT, int GPT, int ALL, int PRE, int THREADS>
+__global__ __launch_bounds__(THREADS) void FcInt4PackedKernel(
     const uint8_t* early_packed, const float* early_input_f32, const int8_t* early_input_q,
     int early_depth, int early_out_depth, int early_chunks, int batch0, int bt, int ksplit,
     int gpw, Int4PackedArgs rest) {
@@ -621,7 +656,10 @@ __global__ __launch_bounds__(kThreads) void FcInt4PackedKernel(
   a.depth = early_depth;
   a.out_depth = early_out_depth;
   a.chunks = early_chunks;
-  FcInt4PackedBody<BT, FUSED, VARIANT, GPT, ALL, PRE>(a, blockIdx.x, batch0, bt, ksplit, gpw, smem);
+  // Slices of the grid (gridDim.y > 1) take bt rows each, side by side.
+  const int first_row = batch0 + static_cast<int>(blockIdx.y) * bt;
+  FcInt4PackedBody<BT, FUSED, VARIANT, GPT, ALL, PRE, THREADS>(
+      a, blockIdx.x, first_row, min(bt, a.batches - first_row), ksplit, gpw, smem);
 }
 
 // Several filters of the same depth in one launch (nodes of a graph that do not depend on
@@ -675,6 +713,12 @@ __global__ __launch_bounds__(THREADS) void QuantizeGroupRowsKernel(
                        const_cast<int32_t*>(a.zero_points) + row, /*do_asymmetric=*/1);
 }
 
+// Depth up to 4096 keeps two groups per thread; up to 16384, eight. A fused launch holds
+// the float rows (16 registers per group and row), so its deep form stops at two rows.
+constexpr int kShallowGpt = 2;
+constexpr int kShallowDepth = kShallowGpt * kThreads * 8;
+constexpr int kDeepDepth = 8 * kThreads * 8;
+
 // Wavefronts per channel group: one while that already gives the chip ~1000 wavefronts;
 // otherwise the depth is shared out, as long as each wavefront keeps at least two tiles.
 int ChooseKsplit(int out_depth, int chunks) {
@@ -682,6 +726,21 @@ int ChooseKsplit(int out_depth, int chunks) {
   int ksplit = 1;
   while (ksplit < kWaves && groups * ksplit < 1024 && chunks >= 4 * ksplit) ksplit *= 2;
   return ksplit;
+}
+
+// Single nodes of deep rows whose tiles make about one workgroup of eight wavefronts per CU, one tile
+// each: a wavefront alone on its SIMD issues a vector operation every 8 cycles or so, and the
+// prologue (16384 values quantized and split into nibble planes by every workgroup) is the larger
+// part of such a launch. Four wavefronts -> eight, us at 1 / 2 / 4 rows (4: int8 rows in, with
+// their quantizer): 16384 -> 2048 10.1 / 12.3 / 16.5 -> 9.5 / 11.0 / 14.1, 8192 -> 2048 8.3 / 9.7 /
+// 13.4 -> 7.0 / 8.3 / 11.5. With two tiles each it is no gain (11008 -> 4096 11.1 -> 11.5 at one
+// row), in more than one round a loss (4608 -> 12000 13.0 -> 17.3, 16384 -> 2050 14.4 -> 16.5).
+bool WideDeep(int depth, int out_depth, int chunks) {
+  constexpr int kWideWaves = kWideThreads / kWaveSize;
+  if (depth <= kShallowDepth || depth > kDeepDepth) return false;
+  if (chunks > kWideWaves || kWideWaves % chunks != 0) return false;
+  const int groups = (out_depth + kTileRows - 1) / kTileRows;
+  return groups <= kWideWaves / chunks * 256;
 }
 
 // Channel groups per wavefront. Measured on launches from 7 MB to 340 MB: a wavefront should
@@ -697,17 +756,17 @@ int ChooseGroupsPerWave(int total_groups, int chunks, int ksplit) {
   return gpw;
 }
 
-template <int BT, bool FUSED, int VARIANT, int GPT, int ALL, int PRE>
-hipError_t LaunchSized(const Int4PackedArgs& a, int batch0, int bt, int ksplit, int gpw,
+template <int BT, bool FUSED, int VARIANT, int GPT, int ALL, int PRE, int THREADS = kThreads>
+hipError_t LaunchSized(const Int4PackedArgs& a, int batch0, int bt, int slices, int ksplit, int gpw,
                        hipStream_t stream) {
   const int padded = a.chunks * kTileBlocks * kBlock;
-  const size_t lds = Int4Shared<BT>::Bytes(padded, ksplit);
-  auto kernel = FcInt4PackedKernel<BT, FUSED, VARIANT, GPT, ALL, PRE>;
+  const size_t lds = Int4Shared<BT, THREADS>::Bytes(padded, ksplit);
+  auto kernel = FcInt4PackedKernel<BT, FUSED, VARIANT, GPT, ALL, PRE, THREADS>;
   if (hipError_t err = EnsureDynamicLds(reinterpret_cast<const void*>(kernel), lds)) return err;
   const int groups = (a.out_depth + kTileRows - 1) / kTileRows;
-  const int groups_per_wg = kWaves / ksplit * gpw;
+  const int groups_per_wg = THREADS / kWaveSize / ksplit * gpw;
   const int grid = (groups + groups_per_wg - 1) / groups_per_wg;
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), lds, stream, a.packed, a.input_f32,
+  hipLaunchKernelGGL(kernel, dim3(grid, slices), dim3(THREADS), lds, stream, a.packed, a.input_f32,
                      a.input_q, a.depth, a.out_depth, a.chunks, batch0, bt, ksplit, gpw, a);
   return hipGetLastError();
 }
@@ -718,41 +777,42 @@ hipError_t LaunchSized(const Int4PackedArgs& a, int batch0, int bt, int ksplit, 
 constexpr int kStraightTiles = 2;
 
 template <int BT, bool FUSED, int VARIANT, int GPT>
-hipError_t LaunchOne(const Int4PackedArgs& a, int batch0, int bt, hipStream_t stream) {
+hipError_t LaunchOne(const Int4PackedArgs& a, int batch0, int bt, int slices, hipStream_t stream) {
+  if constexpr (GPT > kShallowGpt) {
+    if (WideDeep(a.depth, a.out_depth, a.chunks)) {
+      return LaunchSized<BT, FUSED, VARIANT, GPT * kThreads / kWideThreads, 1, 1, kWideThreads>(
+          a, batch0, bt, slices, /*ksplit=*/a.chunks, 1, stream);
+    }
+  }
   const int ksplit = ChooseKsplit(a.out_depth, a.chunks);
   const int groups = (a.out_depth + kTileRows - 1) / kTileRows;
   int gpw = ChooseGroupsPerWave(groups, a.chunks, ksplit);
   if constexpr (BT <= 2) {
     if (ksplit == 1 && a.chunks <= kStraightTiles) {
       gpw = min(gpw, kStraightTiles / a.chunks);
-      return LaunchSized<BT, FUSED, VARIANT, GPT, kStraightTiles, 1>(a, batch0, bt, ksplit, gpw,
-                                                                     stream);
+      return LaunchSized<BT, FUSED, VARIANT, GPT, kStraightTiles, 1>(a, batch0, bt, slices, ksplit,
+                                                                     gpw, stream);
     }
   }
-  return LaunchSized<BT, FUSED, VARIANT, GPT, 0, 0>(a, batch0, bt, ksplit, gpw, stream);
+  return LaunchSized<BT, FUSED, VARIANT, GPT, 0, 0>(a, batch0, bt, slices, ksplit, gpw, stream);
 }
 
 template <int BT, bool FUSED, int GPT>
-hipError_t LaunchVariant(const Int4PackedArgs& a, int variant, int batch0, int bt,
+hipError_t LaunchVariant(const Int4PackedArgs& a, int variant, int batch0, int bt, int slices,
                          hipStream_t stream) {
   if constexpr (!FUSED) {
-    return LaunchOne<BT, false, LRTFC_QUANT_PORTABLE, GPT>(a, batch0, bt, stream);
+    return LaunchOne<BT, false, LRTFC_QUANT_PORTABLE, GPT>(a, batch0, bt, slices, stream);
   } else {
     switch (variant) {
     case LRTFC_QUANT_NEON_V8:
-      return LaunchOne<BT, FUSED, LRTFC_QUANT_NEON_V8, GPT>(a, batch0, bt, stream);
+      return LaunchOne<BT, FUSED, LRTFC_QUANT_NEON_V8, GPT>(a, batch0, bt, slices, stream);
     case LRTFC_QUANT_NEON_LEGACY:
-      return LaunchOne<BT, FUSED, LRTFC_QUANT_NEON_LEGACY, GPT>(a, batch0, bt, stream);
+      return LaunchOne<BT, FUSED, LRTFC_QUANT_NEON_LEGACY, GPT>(a, batch0, bt, slices, stream);
     default:
-      return LaunchOne<BT, FUSED, LRTFC_QUANT_PORTABLE, GPT>(a, batch0, bt, stream);
+      return LaunchOne<BT, FUSED, LRTFC_QUANT_PORTABLE, GPT>(a, batch0, bt, slices, stream);
   }
   }
 }
-
-// Depth up to 4096 keeps two groups per thread; up to 16384, eight. A fused launch holds
-// the float rows (16 registers per group and row), so its deep form stops at two rows.
-constexpr int kShallowDepth = 2 * kThreads * 8;
-constexpr int kDeepDepth = 8 * kThreads * 8;
 
 template <bool FUSED>
 int MaxBatchTile(int depth) {
@@ -763,27 +823,31 @@ int MaxBatchTile(int depth) {
 constexpr size_t kLdsBudget = 150 * 1024;
 
 // Rows per launch: `want` (1, 2 or 4) cut down until the LDS map of that many rows fits.
-int FitBatchTile(int want, int padded, int ksplit) {
+int FitBatchTile(int want, int padded, int ksplit, bool wide = false) {
   int bt = want > 2 ? 4 : want;
-  while (bt > 1 && (bt > 2 ? Int4Shared<4>::Bytes(padded, ksplit)
-                           : Int4Shared<2>::Bytes(padded, ksplit)) > kLdsBudget) {
-    bt = bt > 2 ? 2 : 1;
-  }
+  auto bytes = [&](int rows) {
+    if (wide) {
+      return rows > 2 ? Int4Shared<4, kWideThreads>::Bytes(padded, ksplit)
+                      : Int4Shared<2, kWideThreads>::Bytes(padded, ksplit);
+    }
+    return rows > 2 ? Int4Shared<4>::Bytes(padded, ksplit) : Int4Shared<2>::Bytes(padded, ksplit);
+  };
+  while (bt > 1 && bytes(bt) > kLdsBudget) bt = bt > 2 ? 2 : 1;
   return bt;
 }
 
 template <bool FUSED>
-hipError_t LaunchTile(const Int4PackedArgs& a, int variant, int batch0, int bt,
+hipError_t LaunchTile(const Int4PackedArgs& a, int variant, int batch0, int bt, int slices,
                       hipStream_t stream) {
   if (a.depth > kShallowDepth && a.depth <= kDeepDepth) {
-    if (bt <= 1) return LaunchVariant<1, FUSED, 8>(a, variant, batch0, bt, stream);
-    if (bt <= 2) return LaunchVariant<2, FUSED, 8>(a, variant, batch0, bt, stream);
-    if (!FUSED) return LaunchVariant<4, false, 8>(a, variant, batch0, bt, stream);
+    if (bt <= 1) return LaunchVariant<1, FUSED, 8>(a, variant, batch0, bt, slices, stream);
+    if (bt <= 2) return LaunchVariant<2, FUSED, 8>(a, variant, batch0, bt, slices, stream);
+    if (!FUSED) return LaunchVariant<4, false, 8>(a, variant, batch0, bt, slices, stream);
     return hipErrorInvalidValue;  // MaxBatchTile keeps fused deep launches at two rows
   }
-  if (bt <= 1) return LaunchVariant<1, FUSED, 2>(a, variant, batch0, bt, stream);
-  if (bt <= 2) return LaunchVariant<2, FUSED, 2>(a, variant, batch0, bt, stream);
-  return LaunchVariant<4, FUSED, 2>(a, variant, batch0, bt, stream);
+  if (bt <= 1) return LaunchVariant<1, FUSED, 2>(a, variant, batch0, bt, slices, stream);
+  if (bt <= 2) return LaunchVariant<2, FUSED, 2>(a, variant, batch0, bt, slices, stream);
+  return LaunchVariant<4, FUSED, 2>(a, variant, batch0, bt, slices, stream);
 }
 
 }  // namespace
@@ -829,13 +893,25 @@ hipError_t LaunchFcInt4Packed(const FcInt4Args& q, const uint8_t* packed, const 
   a.out_depth = q.out_depth;
   a.chunks = (q.depth / kBlock + kTileBlocks - 1) / kTileBlocks;
   const int padded = a.chunks * kTileBlocks * kBlock;
+  const bool wide = WideDeep(q.depth, q.out_depth, a.chunks);
+  const int ksplit = wide ? a.chunks : ChooseKsplit(q.out_depth, a.chunks);
+  // Three or four fused rows of a small filter: two pairs side by side in one launch, as in small
+  // groups (PrepareInt4Group); us at four rows, one tile of four -> pairs: 2048 -> 2048 6.8 -> 4.8,
+  // 4096 -> 4096 8.7 -> 6.0.
+  const int groups_per_wg = kWaves / ksplit;
+  if (input_f32 && (q.batches == 3 || q.batches == 4) && q.depth <= kShallowDepth &&
+      ((q.out_depth + kTileRows - 1) / kTileRows + groups_per_wg - 1) / groups_per_wg <=
+          kSideBySideMaxBlocks &&
+      static_cast<int64_t>(q.out_depth) * q.depth / 2 <= kSideBySideMaxFilterBytes) {
+    return LaunchTile<true>(a, variant, 0, 2, 2, stream);
+  }
   const int tile = FitBatchTile(input_f32 ? MaxBatchTile<true>(q.depth) : MaxBatchTile<false>(q.depth),
-                                padded, ChooseKsplit(q.out_depth, a.chunks));
+                                padded, ksplit, wide);
   int batch0 = 0;
   while (batch0 < q.batches) {
     const int bt = min(tile, q.batches - batch0);
-    const hipError_t err = input_f32 ? LaunchTile<true>(a, variant, batch0, bt, stream)
-                                     : LaunchTile<false>(a, variant, batch0, bt, stream);
+    const hipError_t err = input_f32 ? LaunchTile<true>(a, variant, batch0, bt, 1, stream)
+                                     : LaunchTile<false>(a, variant, batch0, bt, 1, stream);
     if (err != hipSuccess) return err;
     batch0 += bt;
   }

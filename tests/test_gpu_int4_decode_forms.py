@@ -1,0 +1,33 @@
+"""Blockwise-int4 decode launches around their dispatch rules: eight wavefronts per workgroup on deep
+rows of four and eight tiles (whole and partial), one round of workgroups and one past it; three
+and four rows as two pairs side by side. Bit-identical to the CPU oracle."""
+import numpy as np
+import pytest
+
+import oracle
+from litert_amd import workloads as wl
+from tests.test_gpu_parity import _bits_equal, _cuda, fc  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B", [1, 2, 3, 4, 7])
+@pytest.mark.parametrize("K,N", [
+    (6176, 19), (8160, 130), (8192, 67),        # four tiles per channel group
+    (14368, 33), (16352, 9), (16384, 70),       # eight
+    (4128, 40), (6144, 40), (10240, 24), (16416, 9),  # three, five, and past the register form
+    (8192, 4096), (8192, 4104), (16384, 2048), (16384, 2056),  # 512 and 513 groups, 256 and 257
+    (2048, 8192), (2048, 8200), (4096, 515), (32, 9), (4096, 12000),  # pairs side by side, and past them
+])
+def test_int4_decode_forms_match_oracle(fc, B, K, N):  # noqa: F811
+    if B * K * N > 7e7 and B not in (1, 4):
+        pytest.skip("the oracle takes long")
+    c = wl.blockwise_int4_fc(B, K, N, seed=B + K + N, lo=-8, hi=7)
+    bias = np.random.default_rng(K).standard_normal(N).astype(np.float32) if B % 2 else None
+    op = fc.FullyConnectedBlockwiseInt4(c["packed"], c["scales"], K, 32, bias=bias)
+    op.FUSED_MAX_DEPTH = 1 << 30  # the fused launches at every row count ...
+    x = _cuda(c["x"])
+    want = oracle.fc_blockwise_int4(c["x"], c["packed"], N, c["scales"].view(np.uint16), 32, bias=bias)
+    if B <= 4:
+        assert _bits_equal(op(x).cpu().numpy(), want)
+    assert _bits_equal(op.call_split(x).cpu().numpy(), want)  # ... and those on quantized rows
