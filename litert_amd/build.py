@@ -9,6 +9,7 @@ import argparse
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -61,6 +62,16 @@ def build_fc():
     return out
 
 
+def build_python_calls():
+    """The per-call entry points as a CPython extension (host code only)."""
+    out = os.path.join(LIB, "litert_amd_calls.so")
+    _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+          "-I" + os.path.join(ROOT, "include"), "-I" + sysconfig.get_paths()["include"], "-o", out,
+          os.path.join(CSRC, "host", "python_calls.cc"), "-L" + LIB, "-llitert_amd_fc",
+          "-Wl,-rpath,$ORIGIN"])
+    return out
+
+
 def build_delegate():
     src_dir = os.path.join(CSRC, "delegate")
     if not os.path.isdir(src_dir):
@@ -83,7 +94,7 @@ def build_bench_probes():
 
 
 def build_all():
-    outs = [build_fc(), build_bench_probes()]
+    outs = [build_fc(), build_python_calls(), build_bench_probes()]
     d = build_delegate()
     if d:
         outs.append(d)
@@ -96,6 +107,7 @@ if __name__ == "__main__":
     args = ap.parse_args()
     if args.only == "fc":
         build_fc()
+        build_python_calls()
     elif args.only == "delegate":
         build_delegate()
     elif args.only == "probes":

@@ -6,6 +6,8 @@ fallback: if the library is missing, or no gfx950 device is visible, the calls
 raise.
 """
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -99,6 +101,27 @@ SYMBOLS = [
 ]
 
 _LIB = None
+
+
+_CALLS = None
+CALLS_PATH = os.path.join(_HERE, "lib", "litert_amd_calls.so")
+
+
+def calls():
+    """The entry points that ops call per invocation, under their C names, as functions of integer
+    addresses (or None), integers and floats: the same library without ctypes in between."""
+    global _CALLS
+    if _CALLS is None:
+        load()  # the extension binds to this library
+        if not os.path.exists(CALLS_PATH):
+            raise FileNotFoundError(
+                CALLS_PATH + " is missing: run `python -m litert_amd.build` first")
+        loader = importlib.machinery.ExtensionFileLoader("litert_amd_calls", CALLS_PATH)
+        spec = importlib.util.spec_from_file_location("litert_amd_calls", CALLS_PATH, loader=loader)
+        module = importlib.util.module_from_spec(spec)
+        loader.exec_module(module)
+        _CALLS = module
+    return _CALLS
 
 
 class LrtFcError(RuntimeError):

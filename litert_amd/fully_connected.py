@@ -26,6 +26,21 @@ def _stream():
     return C.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
+# Per-call forms of _stream() and _ptr() for capi.calls(): plain integers.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+
+
+def _call_stream():
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_current_device())
+
+
+def _addr(t):
+    return None if t is None else t.data_ptr()
+
+
 def _ptr(t):
     return None if t is None else C.c_void_p(t.data_ptr())
 
@@ -161,17 +176,17 @@ class FullyConnectedInt8:
         if out is None:
             out = torch.empty((batches, self.out_depth), dtype=torch.int8, device=x.device)
         if self.packed_filter is not None:
-            capi.check(capi.load().lrtfc_fc_int8_packed(
-                _ptr(x), _ptr(self.packed_filter), _ptr(self.bias), _ptr(self.multipliers),
-                _ptr(self.shifts), int(self.per_channel), _ptr(self.row_sums), _ptr(out), batches,
+            capi.check(capi.calls().lrtfc_fc_int8_packed(
+                _addr(x), _addr(self.packed_filter), _addr(self.bias), _addr(self.multipliers),
+                _addr(self.shifts), int(self.per_channel), _addr(self.row_sums), _addr(out), batches,
                 self.depth, self.out_depth, self.input_offset, self.output_offset, self.act_min,
-                self.act_max, _stream()))
+                self.act_max, _call_stream()))
             return out
-        capi.check(capi.load().lrtfc_fc_int8(
-            _ptr(x), _ptr(self.filter), _ptr(self.bias), _ptr(self.multipliers), _ptr(self.shifts),
-            int(self.per_channel), _ptr(self.row_sums), _ptr(out), batches, self.depth,
+        capi.check(capi.calls().lrtfc_fc_int8(
+            _addr(x), _addr(self.filter), _addr(self.bias), _addr(self.multipliers), _addr(self.shifts),
+            int(self.per_channel), _addr(self.row_sums), _addr(out), batches, self.depth,
             self.out_depth, self.input_offset, self.filter_offset, self.output_offset,
-            self.act_min, self.act_max, _stream()))
+            self.act_min, self.act_max, _call_stream()))
         return out
 
 
@@ -231,7 +246,7 @@ class FullyConnectedHybrid:
         self.packed_filter = _pack_int8(self.filter) if packed else None
 
     def _workspace(self, batches):
-        need = capi.load().lrtfc_activation_workspace_bytes(batches, self.depth)
+        need = capi.calls().lrtfc_activation_workspace_bytes(batches, self.depth)
         if self._ws is None or self._ws.numel() < need:
             self._ws = torch.empty(need, dtype=torch.uint8, device="cuda")
         return self._ws
@@ -244,16 +259,16 @@ class FullyConnectedHybrid:
         if self.packed_filter is not None and batches > self._fused_max():
             return self.call_split(x, out)
         if self.packed_filter is not None:
-            capi.check(capi.load().lrtfc_fc_hybrid_packed(
-                _ptr(x), _ptr(self.packed_filter), _ptr(self.pcs), self.filter_scale,
-                _ptr(self.row_sums), _ptr(self.bias), _ptr(out), batches, self.depth,
-                self.out_depth, int(self.asymmetric), self.activation, self.variant, _stream()))
+            capi.check(capi.calls().lrtfc_fc_hybrid_packed(
+                _addr(x), _addr(self.packed_filter), _addr(self.pcs), self.filter_scale,
+                _addr(self.row_sums), _addr(self.bias), _addr(out), batches, self.depth,
+                self.out_depth, int(self.asymmetric), self.activation, self.variant, _call_stream()))
             return out
         ws = self._workspace(batches)
-        capi.check(capi.load().lrtfc_fc_hybrid(
-            _ptr(x), _ptr(self.filter), _ptr(self.pcs), self.filter_scale, _ptr(self.row_sums),
-            _ptr(self.bias), _ptr(out), batches, self.depth, self.out_depth, int(self.asymmetric),
-            self.activation, self.variant, _ptr(ws), ws.numel(), _stream()))
+        capi.check(capi.calls().lrtfc_fc_hybrid(
+            _addr(x), _addr(self.filter), _addr(self.pcs), self.filter_scale, _addr(self.row_sums),
+            _addr(self.bias), _addr(out), batches, self.depth, self.out_depth, int(self.asymmetric),
+            self.activation, self.variant, _addr(ws), ws.numel(), _call_stream()))
         return out
 
 
@@ -264,7 +279,7 @@ class FullyConnectedHybrid:
     def _fused_max(self):
         if self.FUSED_MAX_BATCHES is not None:
             return self.FUSED_MAX_BATCHES
-        return capi.load().lrtfc_fc_hybrid_fused_max_batches(self.depth, self.out_depth)
+        return capi.calls().lrtfc_fc_hybrid_fused_max_batches(self.depth, self.out_depth)
 
     def call_split(self, x, out=None):
         """Two launches on the packed filter: the standalone row quantizer, then the
@@ -276,10 +291,10 @@ class FullyConnectedHybrid:
         if out is None:
             out = torch.empty((batches, self.out_depth), dtype=torch.float32, device=x.device)
         ws = self._workspace(batches)
-        capi.check(capi.load().lrtfc_fc_hybrid_packed_workspace(
-            _ptr(x), _ptr(self.packed_filter), _ptr(self.pcs), self.filter_scale,
-            _ptr(self.row_sums), _ptr(self.bias), _ptr(out), batches, self.depth, self.out_depth,
-            int(self.asymmetric), self.activation, self.variant, _ptr(ws), ws.numel(), _stream()))
+        capi.check(capi.calls().lrtfc_fc_hybrid_packed_workspace(
+            _addr(x), _addr(self.packed_filter), _addr(self.pcs), self.filter_scale,
+            _addr(self.row_sums), _addr(self.bias), _addr(out), batches, self.depth, self.out_depth,
+            int(self.asymmetric), self.activation, self.variant, _addr(ws), ws.numel(), _call_stream()))
         return out
 
 
@@ -327,7 +342,7 @@ class FullyConnectedBlockwiseInt4:
                                                      _ptr(self.retiled), _stream()))
 
     def _workspace(self, batches):
-        need = capi.load().lrtfc_activation_workspace_bytes(batches, self.depth)
+        need = capi.calls().lrtfc_activation_workspace_bytes(batches, self.depth)
         if self._ws is None or self._ws.numel() < need:
             self._ws = torch.empty(need, dtype=torch.uint8, device="cuda")
         return self._ws
@@ -353,13 +368,13 @@ class FullyConnectedBlockwiseInt4:
             capi.check(lib.lrtfc_pack_int4_blockwise_gemm(
                 _ptr(self.filter), _ptr(self.scales), self.out_depth, self.depth, 32,
                 _ptr(self._gemm_filter), _stream()))
-        need = lib.lrtfc_fc_blockwise_int4_gemm_workspace_bytes(batches, self.depth)
+        need = capi.calls().lrtfc_fc_blockwise_int4_gemm_workspace_bytes(batches, self.depth)
         if self._gemm_ws is None or self._gemm_ws.numel() < need:
             self._gemm_ws = torch.empty(need, dtype=torch.uint8, device="cuda")
-        capi.check(lib.lrtfc_fc_blockwise_int4_gemm(
-            _ptr(x), _ptr(self._gemm_filter), _ptr(self.kfsum), _ptr(self.bias), _ptr(out), batches,
-            self.depth, self.out_depth, self.variant, _ptr(self._gemm_ws), self._gemm_ws.numel(),
-            _stream()))
+        capi.check(capi.calls().lrtfc_fc_blockwise_int4_gemm(
+            _addr(x), _addr(self._gemm_filter), _addr(self.kfsum), _addr(self.bias), _addr(out), batches,
+            self.depth, self.out_depth, self.variant, _addr(self._gemm_ws), self._gemm_ws.numel(),
+            _call_stream()))
         return out
 
     def _nibble_filter_tensor(self):
@@ -387,21 +402,21 @@ class FullyConnectedBlockwiseInt4:
         if out is None:
             out = torch.empty((batches, self.out_depth), dtype=torch.float32, device=x.device)
         self._nibble_filter_tensor()
-        need = lib.lrtfc_fc_blockwise_int4_gemm_workspace_bytes(batches, self.depth)
+        need = capi.calls().lrtfc_fc_blockwise_int4_gemm_workspace_bytes(batches, self.depth)
         if self._gemm_ws is None or self._gemm_ws.numel() < need:
             self._gemm_ws = torch.empty(need, dtype=torch.uint8, device="cuda")
-        capi.check(lib.lrtfc_fc_blockwise_int4_gemm_nibbles(
-            _ptr(x), _ptr(self._nibble_filter), _ptr(self.kfsum), _ptr(self.bias), _ptr(out),
-            batches, self.depth, self.out_depth, self.variant, _ptr(self._gemm_ws),
-            self._gemm_ws.numel(), _stream()))
+        capi.check(capi.calls().lrtfc_fc_blockwise_int4_gemm_nibbles(
+            _addr(x), _addr(self._nibble_filter), _addr(self.kfsum), _addr(self.bias), _addr(out),
+            batches, self.depth, self.out_depth, self.variant, _addr(self._gemm_ws),
+            self._gemm_ws.numel(), _call_stream()))
         return out
 
     def __call__(self, x, out=None):
         x = x.contiguous()
         batches = x.numel() // self.depth
         if self.blocksize == 32 and self.depth % 32 == 0 and self.retiled is not None:
-            form = capi.load().lrtfc_fc_blockwise_int4_preferred_form(batches, self.depth,
-                                                                      self.out_depth)
+            form = capi.calls().lrtfc_fc_blockwise_int4_preferred_form(batches, self.depth,
+                                                                       self.out_depth)
             if form == capi.INT4_FORM_GEMM_NIBBLES:
                 return self.call_gemm_nibbles(x, out)
             if form == capi.INT4_FORM_GEMM_INT8:
@@ -412,9 +427,9 @@ class FullyConnectedBlockwiseInt4:
                 and batches > self.DEEP_FUSED_MAX_BATCHES):
             return self.call_split(x, out)
         if self.retiled is not None:
-            capi.check(capi.load().lrtfc_fc_blockwise_int4_packed(
-                _ptr(x), _ptr(self.retiled), _ptr(self.kfsum), _ptr(self.bias), _ptr(out), batches,
-                self.depth, self.out_depth, self.variant, _stream()))
+            capi.check(capi.calls().lrtfc_fc_blockwise_int4_packed(
+                _addr(x), _addr(self.retiled), _addr(self.kfsum), _addr(self.bias), _addr(out), batches,
+                self.depth, self.out_depth, self.variant, _call_stream()))
             return out
         ws = self._workspace(batches)
         capi.check(capi.load().lrtfc_fc_blockwise_int4(
@@ -486,7 +501,7 @@ class FullyConnectedHybridInt4PerChannel:
         batches = x.numel() // self.depth
         if out is None:
             out = torch.empty((batches, self.out_depth), dtype=torch.float32, device=x.device)
-        need = capi.load().lrtfc_activation_workspace_bytes(batches, self.depth)
+        need = capi.calls().lrtfc_activation_workspace_bytes(batches, self.depth)
         if self._ws is None or self._ws.numel() < need:
             self._ws = torch.empty(need, dtype=torch.uint8, device="cuda")
         lib = capi.load()
@@ -498,20 +513,20 @@ class FullyConnectedHybridInt4PerChannel:
                 capi.check(lib.lrtfc_pack_int4_per_channel(
                     _ptr(self._nibbles), self.out_depth, self.depth, _ptr(self._retiled_nibbles),
                     _stream()))
-            capi.check(lib.lrtfc_fc_hybrid_int4_per_channel_nibbles(
-                _ptr(x), _ptr(self._retiled_nibbles), _ptr(self.pcs), self.filter_scale,
-                _ptr(self.bias), _ptr(out), batches, self.depth, self.out_depth, self.activation,
-                _ptr(self._ws), self._ws.numel(), _stream()))
+            capi.check(capi.calls().lrtfc_fc_hybrid_int4_per_channel_nibbles(
+                _addr(x), _addr(self._retiled_nibbles), _addr(self.pcs), self.filter_scale,
+                _addr(self.bias), _addr(out), batches, self.depth, self.out_depth, self.activation,
+                _addr(self._ws), self._ws.numel(), _call_stream()))
             return out
         if self._packed_int8 is None:
             unpacked = torch.empty((self.out_depth, self.depth), dtype=torch.int8, device="cuda")
             capi.check(lib.lrtfc_unpack_int4(_ptr(self._nibbles), self.out_depth * self.depth,
                                              _ptr(unpacked), _stream()))
             self._packed_int8 = _pack_int8(unpacked)
-        capi.check(lib.lrtfc_fc_hybrid_int4_per_channel_packed(
-            _ptr(x), _ptr(self._packed_int8), _ptr(self.pcs), self.filter_scale, _ptr(self.bias),
-            _ptr(out), batches, self.depth, self.out_depth, self.activation, _ptr(self._ws),
-            self._ws.numel(), _stream()))
+        capi.check(capi.calls().lrtfc_fc_hybrid_int4_per_channel_packed(
+            _addr(x), _addr(self._packed_int8), _addr(self.pcs), self.filter_scale, _addr(self.bias),
+            _addr(out), batches, self.depth, self.out_depth, self.activation, _addr(self._ws),
+            self._ws.numel(), _call_stream()))
         return out
 
 
@@ -546,7 +561,7 @@ class GroupedBlockwiseInt4:
         # every filter is streamed once (same rule as FullyConnectedBlockwiseInt4.__call__).
         workspaces = None
         if batches > FullyConnectedBlockwiseInt4.DEEP_FUSED_MAX_BATCHES:
-            need = capi.load().lrtfc_activation_workspace_bytes(batches, self.depth)
+            need = capi.calls().lrtfc_activation_workspace_bytes(batches, self.depth)
             workspaces = torch.empty((len(self.ops), (need + 255) // 256 * 256), dtype=torch.uint8,
                                      device="cuda")
         out_depths = (C.c_int * len(self.ops))(*[op.out_depth for op in self.ops])
