@@ -123,6 +123,22 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
     }
   }
 
+  // Scale and zero point of the rows whose outputs this lane holds (row L % 32 of every batch tile).
+  float row_scale[kBatchTiles];
+  int32_t row_zero[kBatchTiles];
+  bool small_zero = true;  // |zero point| < 2^23
+#pragma unroll
+  for (int j = 0; j < kBatchTiles; ++j) {
+    row_scale[j] = 0.0f;
+    row_zero[j] = 0;
+    if (EPI != Int8Epilogue::kRequantize) {
+      const int m = min(m0 + j * 32 + (lane & 31), M - 1);
+      row_scale[j] = a.scaling_factors[m];
+      if (a.zero_points) row_zero[j] = a.zero_points[m];
+      small_zero = small_zero && row_zero[j] < (1 << 23) && row_zero[j] >= -(1 << 23);
+    }
+  }
+
   // Weight operands of this wavefront: lane L addresses channel L % 32 of MFMA tile i (tile
   // index clamped at the last 16-channel tile: duplicates are computed and never stored) and
   // the 16 bytes of depth half L / 32 within a 32-deep sub-step.
@@ -218,9 +234,13 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
   // The short requantization (RequantizeShort) needs every channel of the tile to shift right by
   // 1..31 bits and |accumulator + addend| < 2^30, which |addend| < 2^29 and a depth of at most
   // 32768 guarantee; one channel outside that sends the whole workgroup down the general form.
-  const bool general_requantize =
-      __syncthreads_or(EPI == Int8Epilogue::kRequantize &&
-                       ((tid < BN && !plain_channel) || K > 32768 || a.act_min > a.act_max));
+  // The short float epilogue multiplies zero point and row sum as 24-bit integers: |row sum| is at
+  // most 128 K.
+  const bool general_form =
+      EPI == Int8Epilogue::kRequantize
+          ? __syncthreads_or((tid < BN && !plain_channel) || K > 32768 || a.act_min > a.act_max)
+          : __syncthreads_or((EPI == Int8Epilogue::kHybrid && (!small_zero || K > 65535)) ||
+                             a.activation == 5 || a.batch_matmul || zero_input);
   i32x4 fa[kBatchTiles][kSub];
 #pragma unroll
   for (int j = 0; j < kBatchTiles; ++j) {
@@ -354,16 +374,31 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
   };
   // Float outputs go 32 rows (one batch tile) at a time: a wavefront then stores one row's whole
   // kilobyte per instruction instead of 32 bytes in each of 32 rows.
-  auto epilogue_float = [&](auto full_tag) {
+  // form_tag: 0 the general form; 1 and 2 a FULLY_CONNECTED product without and with a clamp. A
+  // wavefront alone on its SIMD issues a vector operation every 8 cycles or so, and the general
+  // form's 35 per output (both arithmetics, a 32-bit product at a quarter of the rate, a walk of
+  // the activations) for 128 outputs a lane were 10 us of a launch: 512 x 4096 -> 14336 53.8 us
+  // with the row quantizer, now 43.7.
+  const float clamp_lo = a.activation == 2 ? -1.0f : 0.0f;
+  const float clamp_hi =
+      a.activation == 2 ? 1.0f : (a.activation == 3 ? 6.0f : __builtin_inff());
+  auto epilogue_float = [&](auto full_tag, auto form_tag) {
     constexpr bool kFull = decltype(full_tag)::value;
+    constexpr int kForm = decltype(form_tag)::value;
+    // ApplyFloatActivation's clamps, one expression for all three.
+    auto activate = [&](float v) {
+      if (kForm == 0) return ApplyFloatActivation(v, a.activation);
+      if (kForm == 1) return v;
+      const float t = (clamp_hi < v) ? clamp_hi : v;
+      return (clamp_lo < t) ? t : clamp_lo;
+    };
     constexpr int kRowBytes = BN * 4 + 16;
     static_assert(32 * kRowBytes <= 2 * kStageBytes, "a batch tile of floats does not fit");
     constexpr int kPiecesPerRow = BN / 4;
 #pragma unroll
     for (int j = 0; j < kBatchTiles; ++j) {
-      const int m = kFull ? m0 + j * 32 + row_in_tile : min(m0 + j * 32 + row_in_tile, M - 1);
-      const float bscale = a.scaling_factors[m];
-      const int32_t bzp = a.zero_points ? a.zero_points[m] : 0;
+      const float bscale = row_scale[j];
+      const int32_t bzp = row_zero[j];
       __syncthreads();  // the buffer's last readers (main loop, previous batch tile) are through
 #pragma unroll
       for (int i = 0; i < kWaveTiles; ++i) {
@@ -374,12 +409,20 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const i32x4 p = chan_params[local + r];
-            v[r] = EPI == Int8Epilogue::kHybrid4Bit
-                       ? Hybrid4BitCore(acc[i][j][4 * g + r], bscale, __int_as_float(p[0]), bzp,
-                                        __int_as_float(p[1]), a.bias_f32 != nullptr, a.activation)
-                       : HybridCoreSelect(acc[i][j][4 * g + r], bscale, __int_as_float(p[0]), bzp,
-                                          p[2], __int_as_float(p[1]), a.activation,
-                                          a.batch_matmul != 0, zero_input);
+            const int32_t dot = acc[i][j][4 * g + r];
+            if (EPI == Int8Epilogue::kHybrid4Bit) {
+              v[r] = activate(Hybrid4BitCore(dot, bscale, __int_as_float(p[0]), bzp,
+                                             __int_as_float(p[1]), a.bias_f32 != nullptr, 0));
+            } else if (kForm != 0) {
+              v[r] = activate(__fadd_rn(
+                  __int_as_float(p[1]),
+                  __fmul_rn(static_cast<float>(dot - __mul24(p[2], bzp)),
+                            __fmul_rn(bscale, __int_as_float(p[0])))));
+            } else {
+              v[r] = HybridCoreSelect(dot, bscale, __int_as_float(p[0]), bzp, p[2],
+                                      __int_as_float(p[1]), a.activation, a.batch_matmul != 0,
+                                      zero_input);
+            }
           }
           *reinterpret_cast<float4*>(smem + row_in_tile * kRowBytes + local * 4) =
               make_float4(v[0], v[1], v[2], v[3]);
@@ -403,12 +446,23 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
   };
   const bool interior = m0 + BM <= M && n0 + BN <= N;
   if (EPI != Int8Epilogue::kRequantize) {
-    if (interior) {
-      epilogue_float(std::true_type{});
+    using General = std::integral_constant<int, 0>;
+    using Plain = std::integral_constant<int, 1>;
+    using Clamped = std::integral_constant<int, 2>;
+    if (general_form) {
+      epilogue_float(std::false_type{}, General{});
+    } else if (a.activation == 0) {
+      if (interior) {
+        epilogue_float(std::true_type{}, Plain{});
+      } else {
+        epilogue_float(std::false_type{}, Plain{});
+      }
+    } else if (interior) {
+      epilogue_float(std::true_type{}, Clamped{});
     } else {
-      epilogue_float(std::false_type{});
+      epilogue_float(std::false_type{}, Clamped{});
     }
-  } else if (!general_requantize) {
+  } else if (!general_form) {
     if (interior) {
       epilogue_int8(std::true_type{}, std::true_type{});
     } else {
