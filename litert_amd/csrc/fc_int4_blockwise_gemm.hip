@@ -179,6 +179,17 @@ __device__ __forceinline__ float ScaleBlockSum(int biased_sum, float scale, floa
   return __fmaf_rn(__int_as_float(biased_sum), scale, offset);
 }
 
+// Under an infinite scale (a model's own) that form gives NaN where the product is infinite. A
+// wavefront that ends its walk with a NaN therefore walks its tiles again with conversion and
+// product apart: only then, so the loop above pays nothing for it.
+template <int N>
+__device__ __forceinline__ bool AnyNaN(const float (&v)[N]) {
+  bool any = false;
+#pragma unroll
+  for (int i = 0; i < N; ++i) any = any || v[i] != v[i];
+  return any;
+}
+
 // fully_connected.cc:1078-1082: zero-point term, row scale, bias.
 __device__ __forceinline__ float FinishOutput(float sum, float zero_point, float kfsum,
                                               float row_scale, bool has_bias, float bias) {
@@ -348,6 +359,34 @@ __global__ __launch_bounds__(kThreads, 2) void FcInt4BlockwiseGemmKernel(GemmArg
       if constexpr (u + PAIRS < kTrip - 1) fetch(integral_constant<int, u % PAIRS>{}, first + u + PAIRS);
     }
   });
+  bool nan = false;
+#pragma unroll
+  for (int cj = 0; cj < CT; ++cj)
+#pragma unroll
+    for (int rj = 0; rj < RT; ++rj) nan = nan || AnyNaN(out[cj][rj]);
+  if (__ballot(nan) != 0) {
+    const i32x4 zero = {0, 0, 0, 0};
+#pragma unroll
+    for (int cj = 0; cj < CT; ++cj) {
+#pragma unroll
+      for (int rj = 0; rj < RT; ++rj) {
+        float again[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int b = 0; b < nb; ++b) {
+          const float scale = *reinterpret_cast<const float*>(sp[cj] + static_cast<size_t>(b / 4) * 512 +
+                                                              channel16 + (b % 4) * 4);
+          const i64 wb = *reinterpret_cast<const i64*>(wp[cj] + static_cast<size_t>(b) * 1024 + weight8);
+          const i64x2 xb = *reinterpret_cast<const i64x2*>(xp[rj] + static_cast<size_t>(b / 2) * 1024 + lane16);
+          const i32x4 acc = __builtin_amdgcn_mfma_i32_16x16x32_i8(b % 2 ? xb[1] : xb[0], wb, zero, 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            again[i] = __fadd_rn(again[i], __fmul_rn(static_cast<float>(acc[i]), scale));
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) out[cj][rj][i] = again[i];
+      }
+    }
+  }
 
 #pragma unroll
   for (int rj = 0; rj < RT; ++rj) {
@@ -503,6 +542,39 @@ __global__ __launch_bounds__(kThreads, 2) void FcInt4BlockwiseGemmLargeKernel(Ge
       }
     }
   });
+  bool nan = false;
+#pragma unroll
+  for (int cj = 0; cj < CT; ++cj)
+#pragma unroll
+    for (int rj = 0; rj < RT; ++rj) nan = nan || AnyNaN(out[cj][rj]);
+  if (__ballot(nan) != 0) {
+    i32x16 zero;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) zero[e] = 0;
+#pragma unroll
+    for (int cj = 0; cj < CT; ++cj) {
+#pragma unroll
+      for (int rj = 0; rj < RT; ++rj) {
+        float again[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) again[e] = 0.0f;
+        for (int b = 0; b < nb; ++b) {
+          const float scale = *reinterpret_cast<const float*>(sp[cj] + static_cast<size_t>(b / 4) * 512 +
+                                                              channel16 + (b % 4) * 4);
+          const size_t at = static_cast<size_t>(b) * 1024 + lane16;
+          const i32x16 acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(
+              *reinterpret_cast<const i32x4*>(xp[rj] + at), *reinterpret_cast<const i32x4*>(wp[cj] + at),
+              zero, 0, 0, 0);
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            again[e] = __fadd_rn(again[e], __fmul_rn(static_cast<float>(acc[e]), scale));
+          }
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) out[cj][rj][e] = again[e];
+      }
+    }
+  }
 
 #pragma unroll
   for (int rj = 0; rj < RT; ++rj) {

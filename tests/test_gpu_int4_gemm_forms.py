@@ -79,3 +79,18 @@ def test_int4_nibble_infinite_scales(fc, B, N):  # noqa: F811
     got = op.call_gemm_nibbles(_cuda(c["x"])).cpu().numpy()
     assert np.array_equal(np.isnan(got), np.isnan(want))
     assert np.array_equal(got[~np.isnan(got)], want[~np.isnan(want)])
+
+
+@pytest.mark.parametrize("B,N", [(33, 17), (49, 4099), (64, 8193), (1000, 6211)])
+def test_int4_gemm_infinite_scales(fc, B, N):  # noqa: F811
+    """The same on the int8-expanded forms, whose sums are scaled on top of 1.5 * 2^23."""
+    K = 224
+    c = wl.blockwise_int4_fc(B, K, N, seed=6)
+    scales = c["scales"].copy()
+    scales[3, 2] = np.inf
+    scales[N - 1, 6] = -np.inf
+    scales[7, 0] = np.nan
+    want = oracle.fc_blockwise_int4(c["x"], c["packed"], N, scales.view(np.uint16), 32)
+    got = fc.FullyConnectedBlockwiseInt4(c["packed"], scales, K, 32).call_gemm(_cuda(c["x"])).cpu().numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[~np.isnan(got)], want[~np.isnan(want)])
