@@ -135,7 +135,15 @@ __global__ __launch_bounds__(kQuantizeThreads) void QuantizeRowsTiledKernel(
     int8_t* __restrict__ tiled, float* __restrict__ scaling_factors,
     int32_t* __restrict__ zero_points) {
   using Placement = std::conditional_t<ROWS == kWide, Tile32x32Placement, Tile16x64Placement>;
-  const int m = blockIdx.x;
+  // Workgroups are dealt round-robin to the 8 XCDs: the rows of a tile go to one XCD, in whose L2
+  // their 16-byte pieces of a line meet (with a tile's rows on eight XCDs every line leaves as
+  // eight partial writes: 2048 rows of 4096 13.1 us, now 10.5). Whole rounds of 8 tiles; what is
+  // left of the grid keeps its order.
+  int m = blockIdx.x;
+  if (m < static_cast<int>(gridDim.x / (8 * ROWS) * (8 * ROWS))) {
+    const int in_round = m % (8 * ROWS);
+    m += (in_round % 8) * ROWS + in_round / 8 - in_round;
+  }
   int8_t* tile_row = tiled + static_cast<size_t>(m / ROWS) * tile_bytes;
   const Placement place{m % ROWS};
   if (m < batches) {
