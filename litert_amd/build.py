@@ -18,7 +18,7 @@ LIB = os.environ.get("LITERT_AMD_LIB_DIR", os.path.join(HERE, "lib"))
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 # -ffp-contract=off: several float steps reproduce the reference's unfused
-# multiply-then-add; packed-fp32 ops are disabled (they have misbehaved on this pool).
+# multiply-then-add; packed-fp32 ops are disabled (some of their forms have given wrong results).
 COMMON = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wall",
           "-Wno-unused-function", "-I" + os.path.join(ROOT, "include")]
