@@ -203,6 +203,13 @@ __device__ __forceinline__ i32x4 LoadRowPiece(const int8_t* row, int at, int dep
   return *reinterpret_cast<const i32x4_unaligned*>(row + min(at, depth - 16));
 }
 
+// The low bytes of four values as one dword, first value lowest.
+__device__ __forceinline__ int32_t PackLowBytes(int32_t q0, int32_t q1, int32_t q2, int32_t q3) {
+  const uint32_t lo = __builtin_amdgcn_perm(q1, q0, 0x0c0c0400u);
+  const uint32_t hi = __builtin_amdgcn_perm(q3, q2, 0x0c0c0400u);
+  return static_cast<int32_t>(__builtin_amdgcn_perm(hi, lo, 0x05040100u));
+}
+
 // 4-way int8 dot product with int32 accumulate (v_dot4_i32_i8).
 __device__ __forceinline__ int32_t Dot4(int32_t a, int32_t b, int32_t acc) {
   return __builtin_amdgcn_sdot4(a, b, acc, false);

@@ -34,13 +34,6 @@ __device__ __forceinline__ int32_t RequantizeShort(int32_t acc, int32_t multipli
   return out;
 }
 
-// The low bytes of four values as one dword, first value lowest.
-__device__ __forceinline__ int32_t PackLowBytes(int32_t q0, int32_t q1, int32_t q2, int32_t q3) {
-  const uint32_t lo = __builtin_amdgcn_perm(q1, q0, 0x0c0c0400u);
-  const uint32_t hi = __builtin_amdgcn_perm(q3, q2, 0x0c0c0400u);
-  return static_cast<int32_t>(__builtin_amdgcn_perm(hi, lo, 0x05040100u));
-}
-
 // Hybrid output value: reference/portable_tensor_utils.cc:186-203 after the bias
 // initialisation of fully_connected.cc:780-786, then ApplyActivationToVector.
 // channel_scale is the per-channel scale, or the per-tensor filter scale.

@@ -443,7 +443,7 @@ void FcInt4PerChannelResidentKernel(const uint8_t* early_packed, const float* ea
       mx = WaveMaxF32(mx);
       float scale_denom = fmaxf(fabsf(mn), fabsf(mx));
       if (scale_denom == 0.0f) scale_denom = 127.0f;
-      const float mult = static_cast<float>(127.0 / static_cast<double>(scale_denom));
+      const float mult = SymmetricMultiplier(scale_denom);
       const float sf = static_cast<float>(static_cast<double>(scale_denom) / 127.0);
       int8_t* qrow = q + wave * qstride;
       int32_t sum = 0;

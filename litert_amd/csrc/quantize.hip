@@ -65,7 +65,7 @@ __global__ __launch_bounds__(THREADS) void BatchQuantize4BitKernel(
   const RowRange range = BlockMinMax<THREADS>(mn, mx);
   float scale_denom = fmaxf(fabsf(range.mn), fabsf(range.mx));
   if (scale_denom == 0.0f) scale_denom = 127.0f;
-  const float multiplier = static_cast<float>(127.0 / static_cast<double>(scale_denom));
+  const float multiplier = SymmetricMultiplier(scale_denom);
   int32_t sum = 0;
   auto emit4 = [&](int i, const float4& t) {
     uint32_t word = QuantizeSymmetricPack4(t.x, t.y, t.z, t.w, multiplier);
@@ -88,7 +88,7 @@ __global__ __launch_bounds__(THREADS) void BatchQuantize4BitKernel(
     for (int i = threadIdx.x; i < n4; i += THREADS) emit4(i, load_piece(i));
   } else {
     for (int i = threadIdx.x; i < n_data; i += THREADS) {
-      const int32_t o = static_cast<int8_t>(RoundHalfAway(__fmul_rn(v[i], multiplier)));
+      const int32_t o = RoundHalfAwayToInt(__fmul_rn(v[i], multiplier));
       q[i] = static_cast<int8_t>(o);
       sum += o;
     }

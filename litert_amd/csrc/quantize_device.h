@@ -173,17 +173,33 @@ __device__ __forceinline__ int32_t QuantizePack4(float a, float b, float c, floa
   return static_cast<int32_t>(w ^ 0x80808080u);
 }
 
-// Four values of a row times its multiplier, rounded half away from zero, as four bytes: the row
-// quantizer of the per-channel int4 path (symmetric, no zero point). The saturation of
-// v_cvt_pk_u8_f32 on value + 128 never binds: |v * mult| < 127.5.
+// The row quantizer of the per-channel int4 path (symmetric, no zero point).
+//
+// RoundHalfAway as an integer: v_cvt_i32_f32 truncates by itself, and a NaN gives 0. (Written out
+// because the language leaves the conversion of a NaN open, and the compiler has made two values of
+// one such conversion.)
+__device__ __forceinline__ int32_t RoundHalfAwayToInt(float x) {
+  const float nudged = __fadd_rn(x, copysignf(0x1.fffffep-2f, x));
+  int32_t out;
+  asm("v_cvt_i32_f32 %0, %1" : "=v"(out) : "v"(nudged));
+  return out;
+}
+
+// 127 / the row's largest magnitude, divided in double. Below 3.8e-37 that is no float32: the
+// reference then multiplies by infinity and converts what comes out, infinities and (for a zero)
+// NaN, to int8, which gives 0 on x86. A NaN multiplier makes every value of the row such a 0.
+__device__ __forceinline__ float SymmetricMultiplier(float scale_denom) {
+  const float mult = static_cast<float>(127.0 / static_cast<double>(scale_denom));
+  return mult == __builtin_inff() ? __builtin_nanf("") : mult;
+}
+
+// Four values of a row times its multiplier, rounded half away from zero, as four bytes. With
+// SymmetricMultiplier every product is a NaN (one of the row's values is: 0) or less than 127.5.
 __device__ __forceinline__ uint32_t QuantizeSymmetricPack4(float a, float b, float c, float d,
                                                            float mult) {
-  uint32_t w = 0;
-  w = __builtin_amdgcn_cvt_pk_u8_f32(__fadd_rn(RoundHalfAway(__fmul_rn(a, mult)), 128.0f), 0, w);
-  w = __builtin_amdgcn_cvt_pk_u8_f32(__fadd_rn(RoundHalfAway(__fmul_rn(b, mult)), 128.0f), 1, w);
-  w = __builtin_amdgcn_cvt_pk_u8_f32(__fadd_rn(RoundHalfAway(__fmul_rn(c, mult)), 128.0f), 2, w);
-  w = __builtin_amdgcn_cvt_pk_u8_f32(__fadd_rn(RoundHalfAway(__fmul_rn(d, mult)), 128.0f), 3, w);
-  return w ^ 0x80808080u;
+  return static_cast<uint32_t>(
+      PackLowBytes(RoundHalfAwayToInt(__fmul_rn(a, mult)), RoundHalfAwayToInt(__fmul_rn(b, mult)),
+                   RoundHalfAwayToInt(__fmul_rn(c, mult)), RoundHalfAwayToInt(__fmul_rn(d, mult))));
 }
 
 // The multiplier the elementwise pass should use for a row.
