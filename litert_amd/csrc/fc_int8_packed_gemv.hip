@@ -123,7 +123,10 @@ constexpr int kRing = 16;  // weight tiles in flight per wavefront
 // 12.55 -> 12.28 us per launch at 14336 x 4096, B = 1).
 // XREGS: 16-byte pieces of a float row a thread holds between the two passes of the fused
 // prologue (4, 8 or 16: rows up to 4096, 8192, 16384 deep); REG_ROWS * XREGS stays at 16 or less.
-template <Int8Epilogue EPI, bool FUSED, int VARIANT, int REG_ROWS, int XREGS>
+// RAGGED: int8 rows of a depth that is no multiple of 16, whose last pieces are shifted into place. A
+// form of its own here and below: with both in one, the code for those rows cost all others up to
+// 0.9 us of a deep launch (4 x 16384 -> 1000 9.0 -> 9.9 us, 1 x 8192 -> 256 4.7 -> 5.0).
+template <Int8Epilogue EPI, bool FUSED, int VARIANT, int REG_ROWS, int XREGS, bool RAGGED>
 __global__ __launch_bounds__(kThreads) void FcInt8PackedGemvKernel(
     const int8_t* early_filter, const float* early_input_f32, int early_depth, int early_slabs,
     int early_out_depth, int batch0, int bt, int ksplit, PackedArgs p) {
@@ -219,7 +222,10 @@ __global__ __launch_bounds__(kThreads) void FcInt8PackedGemvKernel(
         if (vec_ok) {
           for (int i = tid * 16; i < padded; i += kThreads * 16) {
             i32x4 v = {0, 0, 0, 0};
-            if (i < depth) v = ShiftBytesDown(LoadRowPiece(x, i, depth), RowPieceSkip(i, depth));
+            if (i < depth) {
+              v = LoadRowPiece(x, i, depth);
+              if (RAGGED) v = ShiftBytesDown(v, RowPieceSkip(i, depth));
+            }
             *reinterpret_cast<i32x4*>(qrow + i) = v;
           }
         } else {
@@ -376,9 +382,10 @@ __global__ __launch_bounds__(kThreads) void FcInt8PackedGemvKernel(
       const int c = j * kThreads + tid;
       const int b = c / chunks_per_row;
       const int i = (c - b * chunks_per_row) * 16;
+      i32x4 piece = qr[j];
+      if (RAGGED) piece = ShiftBytesDown(piece, RowPieceSkip(i, depth));
       if (b < bt) {
-        *reinterpret_cast<i32x4*>(sh.q + b * qstride + i) =
-            i < depth ? ShiftBytesDown(qr[j], RowPieceSkip(i, depth)) : i32x4{0, 0, 0, 0};
+        *reinterpret_cast<i32x4*>(sh.q + b * qstride + i) = i < depth ? piece : i32x4{0, 0, 0, 0};
       }
     }
   }
@@ -519,7 +526,8 @@ constexpr size_t kResidentPackedArgsOffset =
     (sizeof(ResidentLeadingArgs) + alignof(PackedArgs) - 1) / alignof(PackedArgs) * alignof(PackedArgs);
 static_assert(kResidentPackedArgsOffset == 56, "argument layout of FcInt8ResidentGemvKernel");
 
-template <Int8Epilogue EPI, bool FUSED, int VARIANT, int TILES, bool EARLY, int WAVES, int RT = 1>
+template <Int8Epilogue EPI, bool FUSED, int VARIANT, int TILES, bool EARLY, int WAVES, int RT,
+          bool RAGGED>
 __global__ __launch_bounds__(WAVES * kWaveSize)
 __attribute__((amdgpu_waves_per_eu(WAVES / 2 / RT, WAVES / 2 / RT)))
 void FcInt8ResidentGemvKernel(
@@ -814,25 +822,16 @@ void FcInt8ResidentGemvKernel(
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < kFirst; ++u) request(u);
-    auto stage_rows = [&](auto ragged_c) {
 #pragma unroll
-      for (int j = 0; j < kQRegs; ++j) {
-        const int c = j * (WAVES * kWaveSize) + tid;
-        const int b = c / chunks_per_row;
-        const int i = (c % chunks_per_row) * 16;
-        i32x4 piece = qr[j];
-        if (decltype(ragged_c)::value) piece = ShiftBytesDown(piece, RowPieceSkip(i, depth));
-        if (b < bt) {
-          *reinterpret_cast<i32x4*>(sh.q + b * qstride + i) = i < depth ? piece : i32x4{0, 0, 0, 0};
-        }
+    for (int j = 0; j < kQRegs; ++j) {
+      const int c = j * (WAVES * kWaveSize) + tid;
+      const int b = c / chunks_per_row;
+      const int i = (c % chunks_per_row) * 16;
+      i32x4 piece = qr[j];
+      if (RAGGED) piece = ShiftBytesDown(piece, RowPieceSkip(i, depth));
+      if (b < bt) {
+        *reinterpret_cast<i32x4*>(sh.q + b * qstride + i) = i < depth ? piece : i32x4{0, 0, 0, 0};
       }
-    };
-    // Rows that end inside a piece need it shifted; the test stands outside the loop, so that the
-    // pieces of the others still go out side by side.
-    if (depth & 15) {
-      stage_rows(std::true_type{});
-    } else {
-      stage_rows(std::false_type{});
     }
     __builtin_amdgcn_sched_barrier(0);
     stream(integral_constant<int, kFirst>{}, integral_constant<int, kStreamAhead>{});
@@ -959,14 +958,14 @@ int ChooseKsplit(int slabs, int tiles, int waves = kWaves) {
   return ksplit;
 }
 
-template <Int8Epilogue EPI, bool FUSED, int VARIANT, int TILES, bool EARLY, int WAVES = kWaves,
-          int RT = 1>
+template <Int8Epilogue EPI, bool FUSED, int VARIANT, bool RAGGED, int TILES, bool EARLY,
+          int WAVES = kWaves, int RT = 1>
 hipError_t LaunchResidentSized(const PackedArgs& p, int batch0, int bt, int ksplit,
                               hipStream_t stream) {
   const int per_part = (p.slabs + ksplit - 1) / ksplit;
   const int qstride = ksplit * per_part * kSlabDepth + kQPad;
   const size_t lds = SharedBytes(bt, qstride, WAVES * RT);
-  auto kernel = FcInt8ResidentGemvKernel<EPI, FUSED, VARIANT, TILES, EARLY, WAVES, RT>;
+  auto kernel = FcInt8ResidentGemvKernel<EPI, FUSED, VARIANT, TILES, EARLY, WAVES, RT, RAGGED>;
   if (hipError_t err = EnsureDynamicLds(reinterpret_cast<const void*>(kernel), lds)) return err;
   const int tiles = (p.a.out_depth + kTileRows - 1) / kTileRows;
   const int tiles_per_wg = WAVES / ksplit;
@@ -1015,7 +1014,7 @@ bool ResidentTwoRowTilesFit(const PackedArgs& p, int bt, int* ksplit_out) {
   return true;
 }
 
-template <Int8Epilogue EPI, bool FUSED, int VARIANT>
+template <Int8Epilogue EPI, bool FUSED, int VARIANT, bool RAGGED>
 hipError_t TryLaunchResident(const PackedArgs& p, int batch0, int bt, hipStream_t stream,
                             bool* launched) {
   *launched = false;
@@ -1027,15 +1026,15 @@ hipError_t TryLaunchResident(const PackedArgs& p, int batch0, int bt, hipStream_
       if (!ResidentTwoRowTilesFit(p, bt, &ksplit)) return hipSuccess;
       *launched = true;
       if ((p.slabs + ksplit - 1) / ksplit <= 8) {
-        return LaunchResidentSized<EPI, false, VARIANT, 8, true, 8, 2>(p, batch0, bt, ksplit, stream);
+        return LaunchResidentSized<EPI, false, VARIANT, RAGGED, 8, true, 8, 2>(p, batch0, bt, ksplit, stream);
       }
       if ((p.slabs + ksplit - 1) / ksplit > 16) {
-        return LaunchResidentSized<EPI, false, VARIANT, 32, true, 8, 2>(p, batch0, bt, ksplit, stream);
+        return LaunchResidentSized<EPI, false, VARIANT, RAGGED, 32, true, 8, 2>(p, batch0, bt, ksplit, stream);
       }
-      return LaunchResidentSized<EPI, false, VARIANT, 16, true, 8, 2>(p, batch0, bt, ksplit, stream);
+      return LaunchResidentSized<EPI, false, VARIANT, RAGGED, 16, true, 8, 2>(p, batch0, bt, ksplit, stream);
     }
   }
-  if (FUSED) {
+  if constexpr (FUSED) {
     if (depth > kFusedRowMaxDepth || depth < 4 || bt > kFusedMaxRows) return hipSuccess;
     if (bt > 1) {
       int ksplit = 1;
@@ -1043,13 +1042,13 @@ hipError_t TryLaunchResident(const PackedArgs& p, int batch0, int bt, hipStream_
       const int per_part = (p.slabs + ksplit - 1) / ksplit;
       *launched = true;
       if (per_part <= 8) {
-        return bt > 4 ? LaunchResidentSized<EPI, FUSED, VARIANT, 8, true, 8>(p, batch0, bt, ksplit, stream)
-                      : LaunchResidentSized<EPI, FUSED, VARIANT, 8, false, 8>(p, batch0, bt, ksplit, stream);
+        return bt > 4 ? LaunchResidentSized<EPI, FUSED, VARIANT, RAGGED, 8, true, 8>(p, batch0, bt, ksplit, stream)
+                      : LaunchResidentSized<EPI, FUSED, VARIANT, RAGGED, 8, false, 8>(p, batch0, bt, ksplit, stream);
       }
       // Shares of 9 to 16 tiles: the quantizing wavefronts request four tiles ahead of their row's
       // arithmetic at any row count (14336 x 4096 at 2 / 3 / 4 rows: 11.2 / 11.5 / 11.9 us against
       // 11.3 / 11.6 / 12.0 us without).
-      return LaunchResidentSized<EPI, FUSED, VARIANT, 16, true, 8>(p, batch0, bt, ksplit, stream);
+      return LaunchResidentSized<EPI, FUSED, VARIANT, RAGGED, 16, true, 8>(p, batch0, bt, ksplit, stream);
     }
   }
   int ksplit = ChooseKsplit(p.slabs, tiles);
@@ -1064,22 +1063,22 @@ hipError_t TryLaunchResident(const PackedArgs& p, int batch0, int bt, hipStream_
   }
   *launched = true;
   if (per_part <= 8) {
-    return many_rows ? LaunchResidentSized<EPI, FUSED, VARIANT, 8, !FUSED>(p, batch0, bt, ksplit, stream)
-                     : LaunchResidentSized<EPI, FUSED, VARIANT, 8, false>(p, batch0, bt, ksplit, stream);
+    return many_rows ? LaunchResidentSized<EPI, FUSED, VARIANT, RAGGED, 8, !FUSED>(p, batch0, bt, ksplit, stream)
+                     : LaunchResidentSized<EPI, FUSED, VARIANT, RAGGED, 8, false>(p, batch0, bt, ksplit, stream);
   }
   if (per_part <= 16) {
-    return many_rows ? LaunchResidentSized<EPI, FUSED, VARIANT, 16, !FUSED>(p, batch0, bt, ksplit, stream)
-                     : LaunchResidentSized<EPI, FUSED, VARIANT, 16, false>(p, batch0, bt, ksplit, stream);
+    return many_rows ? LaunchResidentSized<EPI, FUSED, VARIANT, RAGGED, 16, !FUSED>(p, batch0, bt, ksplit, stream)
+                     : LaunchResidentSized<EPI, FUSED, VARIANT, RAGGED, 16, false>(p, batch0, bt, ksplit, stream);
   }
-  return many_rows ? LaunchResidentSized<EPI, FUSED, VARIANT, 32, !FUSED>(p, batch0, bt, ksplit, stream)
-                   : LaunchResidentSized<EPI, FUSED, VARIANT, 32, false>(p, batch0, bt, ksplit, stream);
+  return many_rows ? LaunchResidentSized<EPI, FUSED, VARIANT, RAGGED, 32, !FUSED>(p, batch0, bt, ksplit, stream)
+                   : LaunchResidentSized<EPI, FUSED, VARIANT, RAGGED, 32, false>(p, batch0, bt, ksplit, stream);
 }
 
-template <Int8Epilogue EPI, bool FUSED, int VARIANT, int REG_ROWS, int XREGS = 4>
+template <Int8Epilogue EPI, bool FUSED, int VARIANT, bool RAGGED, int REG_ROWS, int XREGS = 4>
 hipError_t LaunchSized(const PackedArgs& p, int batch0, int bt, hipStream_t stream) {
   const int qstride = p.slabs * kSlabDepth + kQPad;
   const size_t lds = SharedBytes(bt, qstride);
-  auto kernel = FcInt8PackedGemvKernel<EPI, FUSED, VARIANT, REG_ROWS, XREGS>;
+  auto kernel = FcInt8PackedGemvKernel<EPI, FUSED, VARIANT, REG_ROWS, XREGS, RAGGED>;
   if (hipError_t err = EnsureDynamicLds(reinterpret_cast<const void*>(kernel), lds)) return err;
   const int tiles = (p.a.out_depth + kTileRows - 1) / kTileRows;
   // How many wavefronts share one channel group's depth. What the memory system rewards is
@@ -1098,49 +1097,56 @@ hipError_t LaunchSized(const PackedArgs& p, int batch0, int bt, hipStream_t stre
   return hipGetLastError();
 }
 
-template <Int8Epilogue EPI, bool FUSED, int VARIANT>
+template <Int8Epilogue EPI, bool FUSED, int VARIANT, bool RAGGED = false>
 hipError_t LaunchOne(const PackedArgs& p, int batch0, int bt, hipStream_t stream) {
   {
     bool launched = false;
-    hipError_t err = TryLaunchResident<EPI, FUSED, VARIANT>(p, batch0, bt, stream, &launched);
+    hipError_t err = TryLaunchResident<EPI, FUSED, VARIANT, RAGGED>(p, batch0, bt, stream, &launched);
     if (launched || err != hipSuccess) return err;
   }
-  if (!FUSED) {
+  if constexpr (!FUSED) {
     // Quantized rows that fit the registers are requested before the weights and need no
     // wait of their own: up to 16 rows of depth 4096.
     const int64_t row_bytes = static_cast<int64_t>(bt) * p.slabs * kSlabDepth;
-    if (row_bytes <= 16 * kThreads * 4) return LaunchSized<EPI, false, VARIANT, 1>(p, batch0, bt, stream);
-    if (row_bytes <= 16 * kThreads * 8) return LaunchSized<EPI, false, VARIANT, 2>(p, batch0, bt, stream);
-    return LaunchSized<EPI, false, VARIANT, 4>(p, batch0, bt, stream);
+    if (row_bytes <= 16 * kThreads * 4) return LaunchSized<EPI, false, VARIANT, RAGGED, 1>(p, batch0, bt, stream);
+    if (row_bytes <= 16 * kThreads * 8) return LaunchSized<EPI, false, VARIANT, RAGGED, 2>(p, batch0, bt, stream);
+    return LaunchSized<EPI, false, VARIANT, RAGGED, 4>(p, batch0, bt, stream);
+  } else {
+    // Deep rows stay in registers through the prologue too, as long as rows x depth fits 16
+    // pieces per thread: a row that does not is read twice, with the weight loads behind the
+    // first pass instead of under it (2048 x 16384, B = 1: 15.6 us that way, 11.8 us from
+    // registers).
+    const int depth = p.a.depth;
+    if (bt <= 1) {
+      if (depth > 8192 && depth <= 16384) return LaunchSized<EPI, true, VARIANT, false, 1, 16>(p, batch0, bt, stream);
+      if (depth > 4096 && depth <= 8192) return LaunchSized<EPI, true, VARIANT, false, 1, 8>(p, batch0, bt, stream);
+      return LaunchSized<EPI, true, VARIANT, false, 1>(p, batch0, bt, stream);
+    }
+    if (bt <= 2) {
+      if (depth > 4096 && depth <= 8192) return LaunchSized<EPI, true, VARIANT, false, 2, 8>(p, batch0, bt, stream);
+      return LaunchSized<EPI, true, VARIANT, false, 2>(p, batch0, bt, stream);
+    }
+    return LaunchSized<EPI, true, VARIANT, false, 4>(p, batch0, bt, stream);
   }
-  // Deep rows stay in registers through the prologue too, as long as rows x depth fits 16
-  // pieces per thread: a row that does not is read twice, with the weight loads behind the
-  // first pass instead of under it (2048 x 16384, B = 1: 15.6 us that way, 11.8 us from
-  // registers).
-  const int depth = p.a.depth;
-  if (bt <= 1) {
-    if (depth > 8192 && depth <= 16384) return LaunchSized<EPI, FUSED, VARIANT, 1, 16>(p, batch0, bt, stream);
-    if (depth > 4096 && depth <= 8192) return LaunchSized<EPI, FUSED, VARIANT, 1, 8>(p, batch0, bt, stream);
-    return LaunchSized<EPI, FUSED, VARIANT, 1>(p, batch0, bt, stream);
-  }
-  if (bt <= 2) {
-    if (depth > 4096 && depth <= 8192) return LaunchSized<EPI, FUSED, VARIANT, 2, 8>(p, batch0, bt, stream);
-    return LaunchSized<EPI, FUSED, VARIANT, 2>(p, batch0, bt, stream);
-  }
-  return LaunchSized<EPI, FUSED, VARIANT, 4>(p, batch0, bt, stream);
 }
 
 template <Int8Epilogue EPI, bool FUSED>
 hipError_t LaunchVariant(const PackedArgs& p, int variant, int batch0, int bt,
                          hipStream_t stream) {
-  if (!FUSED) return LaunchOne<EPI, false, LRTFC_QUANT_PORTABLE>(p, batch0, bt, stream);
-  switch (variant) {
-    case LRTFC_QUANT_NEON_V8:
-      return LaunchOne<EPI, FUSED, LRTFC_QUANT_NEON_V8>(p, batch0, bt, stream);
-    case LRTFC_QUANT_NEON_LEGACY:
-      return LaunchOne<EPI, FUSED, LRTFC_QUANT_NEON_LEGACY>(p, batch0, bt, stream);
-    default:
-      return LaunchOne<EPI, FUSED, LRTFC_QUANT_PORTABLE>(p, batch0, bt, stream);
+  if constexpr (!FUSED) {
+    if (p.a.depth % 16 != 0) {
+      return LaunchOne<EPI, false, LRTFC_QUANT_PORTABLE, true>(p, batch0, bt, stream);
+    }
+    return LaunchOne<EPI, false, LRTFC_QUANT_PORTABLE>(p, batch0, bt, stream);
+  } else {
+    switch (variant) {
+      case LRTFC_QUANT_NEON_V8:
+        return LaunchOne<EPI, FUSED, LRTFC_QUANT_NEON_V8>(p, batch0, bt, stream);
+      case LRTFC_QUANT_NEON_LEGACY:
+        return LaunchOne<EPI, FUSED, LRTFC_QUANT_NEON_LEGACY>(p, batch0, bt, stream);
+      default:
+        return LaunchOne<EPI, FUSED, LRTFC_QUANT_PORTABLE>(p, batch0, bt, stream);
+    }
   }
 }
 
