@@ -145,6 +145,22 @@ int lrtfc_fc_blockwise_int4_preferred_layout(int depth, int blocksize);
  * for every batch size (tflite/kernels/fully_connected.cc:847-851). Pure host function. */
 int lrtfc_fc_hybrid_fused_max_batches(int depth, int out_depth);
 
+/* Which kernel the entry points on a re-tiled int8 filter run for `batches` rows that arrive
+ * quantized (lrtfc_fc_int8_packed, lrtfc_fc_hybrid_int8_packed, and what follows the row quantizer
+ * of lrtfc_fc_hybrid_packed_workspace): for profiles, and for tests that are meant for one of them.
+ * All give the same bits. The matrix-core GEMV takes 16 rows a pass, or up to 32 as two row tiles;
+ * ROWS streams the filter once for up to 128; SPLIT deals the depth of small tiles to the wavefronts
+ * of a workgroup; the rest are GEMM tiles of rows x channels. Pure host function. */
+enum {
+  LRTFC_INT8_KERNEL_GEMV = 0,
+  LRTFC_INT8_KERNEL_GEMV_TWO_TILES = 1,
+  LRTFC_INT8_KERNEL_ROWS = 2,
+  LRTFC_INT8_KERNEL_SPLIT = 3,
+  LRTFC_INT8_KERNEL_TILES_64X128 = 4,
+  LRTFC_INT8_KERNEL_TILES_128X256 = 5
+};
+int lrtfc_fc_int8_packed_kernel(int batches, int depth, int out_depth);
+
 /* Re-tiles a row-major int8 filter [out_depth, depth] for the matrix-core GEMV: tiles of
  * 16 output channels x 64 depth (1 KiB each, zero-padded at the edges), the 16 bytes of
  * lane L inside a tile being channel L % 16, depth 16 * (L / 16) .. +16; tiles of one

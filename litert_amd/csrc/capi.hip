@@ -361,6 +361,24 @@ int lrtfc_fc_hybrid_fused_max_batches(int depth, int out_depth) {
   return lrtfc::FcInt8PackedGemvFusedMaxRows(depth);
 }
 
+int lrtfc_fc_int8_packed_kernel(int batches, int depth, int out_depth) {
+  lrtfc::FcInt8Args a{};  // null pointers: aligned ones
+  a.batches = batches;
+  a.depth = depth;
+  a.out_depth = out_depth;
+  const bool gemm = !lrtfc::FcInt8PackedGemvTakesRowsInOnePass(a) && lrtfc::FcInt8PackedGemmSupports(a);
+  if (!gemm) {
+    // (More than 16 rows otherwise: 16 a pass.)
+    if (!lrtfc::FcInt8PackedGemvTakesRowsInOnePass(a) || batches <= 16) return LRTFC_INT8_KERNEL_GEMV;
+    return batches <= 32 ? LRTFC_INT8_KERNEL_GEMV_TWO_TILES : LRTFC_INT8_KERNEL_ROWS;
+  }
+  switch (lrtfc::FcInt8PackedGemmForm(a)) {
+    case lrtfc::Int8GemmForm::kSplit: return LRTFC_INT8_KERNEL_SPLIT;
+    case lrtfc::Int8GemmForm::kTiles64x128: return LRTFC_INT8_KERNEL_TILES_64X128;
+    default: return LRTFC_INT8_KERNEL_TILES_128X256;
+  }
+}
+
 int lrtfc_fc_blockwise_int4_preferred_layout(int depth, int blocksize) {
   return lrtfc::FcInt4PackedSupports(depth, blocksize) ? LRTFC_LAYOUT_PACKED
                                                        : LRTFC_LAYOUT_ROW_MAJOR;

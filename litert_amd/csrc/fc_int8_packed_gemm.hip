@@ -496,6 +496,13 @@ hipError_t LaunchShape(const FcInt8Args& a, Int8Epilogue epilogue, int grid, hip
 
 constexpr int kMinLargeTiles = 128;
 
+int LargeTiles(const FcInt8Args& a) {
+  return ((a.batches + 127) / 128) * ((a.out_depth + 255) / 256);
+}
+int SmallTiles(const FcInt8Args& a) {
+  return ((a.batches + 63) / 64) * ((a.out_depth + 127) / 128);
+}
+
 }  // namespace
 
 bool FcInt8PackedGemmSupports(const FcInt8Args& a) {
@@ -503,18 +510,22 @@ bool FcInt8PackedGemmSupports(const FcInt8Args& a) {
          (reinterpret_cast<uintptr_t>(a.filter) & 15) == 0;
 }
 
+// 128 x 256 tiles move the fewest bytes per MFMA; a launch they would cut into fewer workgroups than
+// half the chip's CUs takes 64 x 128 tiles instead (four times as many), or, where those leave it
+// idle too, small tiles with the depth split over the wavefronts.
+Int8GemmForm FcInt8PackedGemmForm(const FcInt8Args& a) {
+  if (LargeTiles(a) >= kMinLargeTiles) return Int8GemmForm::kTiles128x256;
+  return FcInt8SplitGemmBeatsTiles(a, SmallTiles(a)) ? Int8GemmForm::kSplit
+                                                     : Int8GemmForm::kTiles64x128;
+}
+
 hipError_t LaunchFcInt8PackedGemm(const FcInt8Args& a, Int8Epilogue epilogue, hipStream_t stream) {
   if (!FcInt8PackedGemmSupports(a)) return hipErrorNotSupported;
-  // 128 x 256 tiles move the fewest bytes per MFMA; a launch they would cut into fewer
-  // workgroups than half the chip's CUs takes 64 x 128 tiles instead (four times as many), or,
-  // where those leave it idle too, small tiles with the depth split over the wavefronts.
-  const int large = ((a.batches + 127) / 128) * ((a.out_depth + 255) / 256);
-  if (large >= kMinLargeTiles) return LaunchShape<128, 2>(a, epilogue, large, stream);
-  const int small = ((a.batches + 63) / 64) * ((a.out_depth + 127) / 128);
-  if (FcInt8SplitGemmBeatsTiles(a, small)) {
-    return LaunchFcInt8SplitGemm(a, epilogue, stream);
+  switch (FcInt8PackedGemmForm(a)) {
+    case Int8GemmForm::kSplit: return LaunchFcInt8SplitGemm(a, epilogue, stream);
+    case Int8GemmForm::kTiles128x256: return LaunchShape<128, 2>(a, epilogue, LargeTiles(a), stream);
+    default: return LaunchShape<64, 1>(a, epilogue, SmallTiles(a), stream);
   }
-  return LaunchShape<64, 1>(a, epilogue, small, stream);
 }
 
 }  // namespace lrtfc

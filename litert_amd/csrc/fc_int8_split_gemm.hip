@@ -326,10 +326,16 @@ bool FcInt8SplitGemmBeatsOnePass(const FcInt8Args& a) {
 // Against the GEMM on 64 x 128 tiles, in the same unit: 1 us and 0.25 us per 128 deep step and
 // round (77 x 2999 -> 5003 12.2 -> 7.1 us, 250 x 2048 -> 2048 9.2 -> 6.1 us, 400 x 8192 -> 2048
 // 27.6 -> 15.8 us; 400 x 2048 -> 4096 stays there: 8.1, here 11.4 us).
+// 64 x 64 tiles in three rounds and more keep all CUs at the L2 at once, which then gives each a third
+// of the 150 bytes per nanosecond: at all 66 measured sizes that Cost sends there they are the
+// slower ones, by 3 to 37 % (us, 64 x 128 tiles / here: 256 x 4096 -> 10240 20.3 / 27.5,
+// 400 x 6144 -> 5120 27.5 / 33.9, 640 x 16384 -> 6144 80 / 103).
 bool FcInt8SplitGemmBeatsTiles(const FcInt8Args& a, long workgroups_64x128) {
   const long theirs = (workgroups_64x128 + kCus - 1) / kCus *
                       (150000 + 37500 * ((static_cast<long>(a.depth) + kStep - 1) / kStep));
-  return Cost(kTiles[BestTile(a)], a) < theirs;
+  const Tile& tile = kTiles[BestTile(a)];
+  if (tile.rows * tile.channels == 64 * 64 && Workgroups(tile, a) > 2 * kCus) return false;
+  return Cost(tile, a) < theirs;
 }
 
 hipError_t LaunchFcInt8SplitGemm(const FcInt8Args& a, Int8Epilogue epilogue, hipStream_t stream) {

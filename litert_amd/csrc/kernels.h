@@ -136,7 +136,7 @@ hipError_t LaunchFcInt4PerChannelGemv(const uint8_t* packed, const float* input_
 
 // Prefill batches on the same re-tiled filter: int8 MFMA GEMM (a.filter = packed, a.input =
 // int8 rows; the hybrid epilogue reads a.scaling_factors / a.zero_points). Any batch count,
-// any out_depth; depth a multiple of 16.
+// any out_depth, depths from 16 on.
 // Whether a.batches rows that arrive quantized go to LaunchFcInt8PackedGemv: where it streams the
 // filter once for all of them (up to 16 rows, 17 to 32 when their LDS image fits a compute unit, up
 // to 128 on wide filters) and small GEMM tiles do not beat it (FcInt8SplitGemmBeatsOnePass).
@@ -146,6 +146,8 @@ bool FcInt8PackedGemvTakesRowsInOnePass(const FcInt8Args& a);
 bool FcInt8RowsGemvTakes(const FcInt8Args& a);
 hipError_t LaunchFcInt8RowsGemv(const FcInt8Args& a, Int8Epilogue epilogue, hipStream_t stream);
 bool FcInt8PackedGemmSupports(const FcInt8Args& a);
+enum class Int8GemmForm { kSplit, kTiles64x128, kTiles128x256 };
+Int8GemmForm FcInt8PackedGemmForm(const FcInt8Args& a);
 hipError_t LaunchFcInt8PackedGemm(const FcInt8Args& a, Int8Epilogue epilogue, hipStream_t stream);
 // The same for launches that leave the chip idle in those tiles (fc_int8_split_gemm.hip): small tiles,
 // the depth dealt to the wavefronts of a workgroup. LaunchFcInt8PackedGemm takes it by itself.

@@ -1,0 +1,32 @@
+"""Which kernel int8 rows on a re-tiled filter go to (lrtfc_fc_int8_packed_kernel, a host function):
+each line of the rule at sizes on both its sides, as measured."""
+import pytest
+
+from litert_amd import capi
+
+
+def _kernel(rows, depth, channels):
+    return capi.load().lrtfc_fc_int8_packed_kernel(rows, depth, channels)
+
+
+@pytest.mark.parametrize("rows,depth,channels", [
+    (129, 4096, 14336), (200, 4096, 10240), (256, 4096, 12288), (400, 6144, 5120), (512, 8192, 6144),
+    (640, 16384, 6144), (900, 4096, 3072)])
+def test_small_tiles_in_many_rounds_stay_with_the_gemm(rows, depth, channels):
+    assert _kernel(rows, depth, channels) == capi.INT8_KERNEL_TILES_64X128
+
+
+@pytest.mark.parametrize("rows,depth,channels", [
+    (77, 3008, 5003), (250, 2048, 2048), (400, 8192, 2048), (100, 16384, 512), (200, 4096, 4096),
+    (160, 6144, 6144), (300, 16384, 4096)])
+def test_small_tiles_in_one_or_two_rounds(rows, depth, channels):
+    assert _kernel(rows, depth, channels) == capi.INT8_KERNEL_SPLIT
+
+
+@pytest.mark.parametrize("rows,depth,channels,kernel", [
+    (1, 2048, 2048, capi.INT8_KERNEL_GEMV), (16, 4096, 14336, capi.INT8_KERNEL_GEMV),
+    (20, 8, 40, capi.INT8_KERNEL_GEMV),  # too shallow for a GEMM
+    (32, 4096, 14336, capi.INT8_KERNEL_GEMV_TWO_TILES), (128, 4096, 14336, capi.INT8_KERNEL_ROWS),
+    (400, 2048, 4096, capi.INT8_KERNEL_TILES_64X128), (2048, 4096, 4096, capi.INT8_KERNEL_TILES_128X256)])
+def test_the_other_kernels(rows, depth, channels, kernel):
+    assert _kernel(rows, depth, channels) == kernel
