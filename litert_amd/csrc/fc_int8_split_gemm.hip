@@ -40,7 +40,7 @@ __device__ __forceinline__ void LaneFence() {
 // RT x CT tiles of 32 rows x 32 channels per workgroup.
 template <Int8Epilogue EPI, int RT, int CT>
 __global__ __launch_bounds__(kThreads, RT * CT == 4 ? 2 : 4)
-void FcInt8SplitGemmKernel(FcInt8Args a, int tiles_m, int total, int per_xcd) {
+void FcInt8SplitGemmKernel(FcInt8Args a, int tiles, bool rows_inner, int total, int per_xcd) {
   constexpr int BM = RT * 32, BN = CT * 32;
   constexpr int kSumStride = BN + 1;  // 32 rows at one channel lie in 32 banks
   __shared__ __align__(16) int8_t rows[kWaves * BM * kRowStride];
@@ -50,12 +50,14 @@ void FcInt8SplitGemmKernel(FcInt8Args a, int tiles_m, int total, int per_xcd) {
   const int slabs = (K + kSlab - 1) / kSlab;
   const int steps = (slabs + 1) / 2;
 
-  // Workgroups are dealt round-robin to the 8 XCDs; each takes a contiguous range of tiles, the
-  // row tiles of one channel range next to each other, so that a filter tile is fetched into one
-  // L2 once.
+  // Workgroups are dealt round-robin to the 8 XCDs; each takes a contiguous range of tiles. With the
+  // row tiles of one channel range next to each other (rows_inner) a filter tile is fetched into one
+  // L2 once, and every L2 fetches the rows; where those are the larger operand it is the other way
+  // round (2048 x 3072 -> 512 8.6 us, rows inner 12.8; 1500 x 16384 -> 1024 52 and 57).
   const int id = static_cast<int>(blockIdx.x % 8) * per_xcd + static_cast<int>(blockIdx.x / 8);
   if (static_cast<int>(blockIdx.x / 8) >= per_xcd || id >= total) return;
-  const int m0 = (id % tiles_m) * BM, n0 = (id / tiles_m) * BN;
+  const int inner = id % tiles, outer = id / tiles;
+  const int m0 = (rows_inner ? inner : outer) * BM, n0 = (rows_inner ? outer : inner) * BN;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -258,18 +260,21 @@ void FcInt8SplitGemmKernel(FcInt8Args a, int tiles_m, int total, int per_xcd) {
 template <int RT, int CT>
 hipError_t LaunchTile(const FcInt8Args& a, Int8Epilogue epilogue, hipStream_t stream) {
   const int tiles_m = (a.batches + 32 * RT - 1) / (32 * RT);
-  const int total = tiles_m * ((a.out_depth + 32 * CT - 1) / (32 * CT));
+  const int tiles_n = (a.out_depth + 32 * CT - 1) / (32 * CT);
+  const int total = tiles_m * tiles_n;
+  const bool rows_inner = a.batches <= a.out_depth;
+  const int inner_tiles = rows_inner ? tiles_m : tiles_n;
   const int per_xcd = (total + 7) / 8;
   const dim3 grid(per_xcd * 8), block(kThreads);
   if (epilogue == Int8Epilogue::kRequantize) {
     hipLaunchKernelGGL((FcInt8SplitGemmKernel<Int8Epilogue::kRequantize, RT, CT>), grid, block, 0,
-                       stream, a, tiles_m, total, per_xcd);
+                       stream, a, inner_tiles, rows_inner, total, per_xcd);
   } else if (epilogue == Int8Epilogue::kHybrid) {
     hipLaunchKernelGGL((FcInt8SplitGemmKernel<Int8Epilogue::kHybrid, RT, CT>), grid, block, 0,
-                       stream, a, tiles_m, total, per_xcd);
+                       stream, a, inner_tiles, rows_inner, total, per_xcd);
   } else {
     hipLaunchKernelGGL((FcInt8SplitGemmKernel<Int8Epilogue::kHybrid4Bit, RT, CT>), grid, block, 0,
-                       stream, a, tiles_m, total, per_xcd);
+                       stream, a, inner_tiles, rows_inner, total, per_xcd);
   }
   return hipGetLastError();
 }

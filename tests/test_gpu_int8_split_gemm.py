@@ -14,6 +14,8 @@ SHAPES = [(9, 16, 5), (9, 63, 31), (12, 129, 33), (5, 2112, 67), (16, 4100, 255)
           # 32 x 32 tiles; 32 x 64; 64 x 64: one row or channel past and short of a tile
           (17, 1000, 1000), (33, 1023, 65), (64, 960, 2049), (31, 2048, 8257), (72, 2047, 4097),
           (129, 4096, 4030), (400, 4224, 1090), (128, 5000, 1985),
+          # more rows than channels: the tiles in the other order
+          (700, 1030, 70), (1500, 272, 515),
           # beside the rule: one workgroup more than a round of tiles
           (32, 2048, 16385), (65, 1024, 10241), (100, 16390, 40)]
 
