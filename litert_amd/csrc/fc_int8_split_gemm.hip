@@ -318,7 +318,8 @@ int BestTile(const FcInt8Args& a) {
 // 16 x 12000 -> 3000 29.8 -> 14.1, 32 x 2048 -> 2048 6.7 -> 4.5, 20 x 2048 -> 16384 9.9 -> 9.0,
 // 48 x 4096 -> 14336 16.5 -> 15.1, 48 x 2048 -> 16384 12.4 -> 9.9.
 bool FcInt8SplitGemmBeatsOnePass(const FcInt8Args& a) {
-  if (!FcInt8PackedGemmSupports(a)) return false;
+  // What the GEMM launches for the size is what the figures above are of.
+  if (!FcInt8PackedGemmSupports(a) || FcInt8PackedGemmForm(a) != Int8GemmForm::kSplit) return false;
   if (a.batches <= 16) {
     return a.batches >= (a.depth > 2048 ? 5 : 9) && Workgroups(kTiles[0], a) <= kCus;
   }
@@ -331,6 +332,8 @@ bool FcInt8SplitGemmBeatsOnePass(const FcInt8Args& a) {
 // Against the GEMM on 64 x 128 tiles, in the same unit: 1 us and 0.25 us per 128 deep step and
 // round (77 x 2999 -> 5003 12.2 -> 7.1 us, 250 x 2048 -> 2048 9.2 -> 6.1 us, 400 x 8192 -> 2048
 // 27.6 -> 15.8 us; 400 x 2048 -> 4096 stays there: 8.1, here 11.4 us).
+// What fits one round of tiles is faster here at all 640 sizes measured, or equal (64 x 64 tiles of
+// a depth about 1024: 64 x 1024 -> 16384 7.7 us for 8.7, 256 x 1024 -> 4096 1 % slower).
 // 64 x 64 tiles in three rounds and more keep all CUs at the L2 at once, which then gives each a third
 // of the 150 bytes per nanosecond: at all 66 measured sizes that Cost sends there they are the
 // slower ones, by 3 to 37 % (us, 64 x 128 tiles / here: 256 x 4096 -> 10240 20.3 / 27.5,
@@ -339,6 +342,7 @@ bool FcInt8SplitGemmBeatsTiles(const FcInt8Args& a, long workgroups_64x128) {
   const long theirs = (workgroups_64x128 + kCus - 1) / kCus *
                       (150000 + 37500 * ((static_cast<long>(a.depth) + kStep - 1) / kStep));
   const Tile& tile = kTiles[BestTile(a)];
+  if (Workgroups(tile, a) <= kCus) return true;
   if (tile.rows * tile.channels == 64 * 64 && Workgroups(tile, a) > 2 * kCus) return false;
   return Cost(tile, a) < theirs;
 }

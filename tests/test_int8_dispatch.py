@@ -30,3 +30,22 @@ def test_small_tiles_in_one_or_two_rounds(rows, depth, channels):
     (400, 2048, 4096, capi.INT8_KERNEL_TILES_64X128), (2048, 4096, 4096, capi.INT8_KERNEL_TILES_128X256)])
 def test_the_other_kernels(rows, depth, channels, kernel):
     assert _kernel(rows, depth, channels) == kernel
+
+
+@pytest.mark.parametrize("rows,depth,channels", [
+    (64, 1024, 16384), (33, 1037, 10243), (50, 1152, 14080), (40, 1370, 10240), (17, 128, 8200),
+    (32, 100, 14336)])
+def test_what_leaves_the_one_pass_kernels_runs_on_what_beat_them(rows, depth, channels):
+    assert _kernel(rows, depth, channels) == capi.INT8_KERNEL_SPLIT
+
+
+def test_no_row_count_falls_between_the_rules():
+    """Wherever a kernel takes all rows in one pass, the launch is that kernel's or the small tiles'."""
+    for rows in range(17, 129):
+        for depth in (16, 128, 1000, 1024, 1200, 1376, 1500, 2048, 3000, 4096):
+            for channels in (300, 2048, 8192, 10225, 12000, 14336, 16384, 20000):
+                one_pass = (capi.INT8_KERNEL_GEMV_TWO_TILES if rows <= 32 else
+                            capi.INT8_KERNEL_ROWS if depth >= 1024 and channels > 639 * 16 else None)
+                if one_pass is not None:
+                    assert _kernel(rows, depth, channels) in (one_pass, capi.INT8_KERNEL_SPLIT), \
+                        (rows, depth, channels)
