@@ -223,8 +223,11 @@ __global__ __launch_bounds__(kThreads) void FcInt8PackedGemvKernel(
           for (int i = tid * 16; i < padded; i += kThreads * 16) {
             i32x4 v = {0, 0, 0, 0};
             if (i < depth) {
-              v = LoadRowPiece(x, i, depth);
-              if (RAGGED) v = ShiftBytesDown(v, RowPieceSkip(i, depth));
+              if (RAGGED) {
+                v = ShiftBytesDown(LoadRowPiece(x, i, depth), RowPieceSkip(i, depth));
+              } else {
+                v = *reinterpret_cast<const i32x4_unaligned*>(x + i);
+              }
             }
             *reinterpret_cast<i32x4*>(qrow + i) = v;
           }
