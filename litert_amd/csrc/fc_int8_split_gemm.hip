@@ -310,18 +310,33 @@ int BestTile(const FcInt8Args& a) {
 
 }  // namespace
 
-// Against the kernels that take up to 128 rows in one pass over the filter (int8 rows in, cold
-// filters, microseconds there -> here): they keep what fills the chip by channel tiles alone
-// (20 x 4096 -> 14336 13.7 -> 13.9, 72 rows 19.2 -> 20.6), and the fewest rows, whose products
-// hide behind the filter's stream (8 x 2048 -> 2048 3.6 -> 4.3). What gains is whatever fits one
-// round of small tiles: 16 x 4096 -> 4096 6.3 -> 5.7, 8 x 2999 -> 5003 9.5 -> 6.9,
-// 16 x 12000 -> 3000 29.8 -> 14.1, 32 x 2048 -> 2048 6.7 -> 4.5, 20 x 2048 -> 16384 9.9 -> 9.0,
-// 48 x 4096 -> 14336 16.5 -> 15.1, 48 x 2048 -> 16384 12.4 -> 9.9.
+// Against the kernels that take up to 128 rows in one pass over the filter (int8 rows in,
+// microseconds there -> here; "cold": filters rotated through 700 MB, else the same one again).
+// Up to 16 rows the register-resident GEMV requests a wavefront's whole share of the filter at once,
+// where a wavefront here has one step ahead: on cold filters that weighs more than what these tiles
+// save. So the GEMV keeps
+//   - rows of at most 16 KB together (9 x 1024 -> 2048 3.6 -> 3.6, cold 3.2 -> 4.0),
+//   - shares of more than 24 of its 32 tiles, i.e. depths from 6145 to 8192 (8 x 8192 -> 256
+//     5.8 -> 6.3, cold 6.1 -> 8.7),
+// unless the tiles make 192 workgroups or more (8 x 4096 -> 6144 7.3 -> 4.8, cold 7.8 -> 7.4). Its rows
+// have to fit 64 KB; others, and depths beyond 8192, walk its refilled ring and gain here
+// (16 x 8192 -> 1024 11.4 -> 6.5, cold 11.1 -> 9.7). What is left gains on a filter in the cache about
+// what it loses on a cold one (16 x 2048 -> 2048 4.8 -> 3.9, cold 4.4 -> 4.8; 12 x 3072 -> 1024
+// 5.2 -> 4.3, cold 4.7 -> 5.5; 16 x 4096 -> 1024 5.5 -> 4.7, cold 4.9 -> 6.4).
+// Beyond 16 rows: whatever fits one round of small tiles (32 x 2048 -> 2048 6.7 -> 4.5,
+// 20 x 2048 -> 16384 9.9 -> 9.0, 48 x 4096 -> 14336 16.5 -> 15.1, 48 x 2048 -> 16384 12.4 -> 9.9);
+// the others keep what fills the chip by channel tiles alone (20 x 4096 -> 14336 13.7 -> 13.9,
+// 72 rows 19.2 -> 20.6).
 bool FcInt8SplitGemmBeatsOnePass(const FcInt8Args& a) {
   // What the GEMM launches for the size is what the figures above are of.
   if (!FcInt8PackedGemmSupports(a) || FcInt8PackedGemmForm(a) != Int8GemmForm::kSplit) return false;
   if (a.batches <= 16) {
-    return a.batches >= (a.depth > 2048 ? 5 : 9) && Workgroups(kTiles[0], a) <= kCus;
+    const long tiles = Workgroups(kTiles[0], a);
+    if (a.batches < 5 || tiles > kCus) return false;
+    const long image = static_cast<long>(a.batches) * ((a.depth + kSlab - 1) / kSlab * kSlab);
+    if (image > 65536 || a.depth > 8192) return true;
+    if (tiles >= 192) return a.depth > (a.batches < 9 ? 2048 : 1024);
+    return image > 16384 && a.depth <= 6144;
   }
   if (a.batches <= 32) {
     return Workgroups(kTiles[a.depth <= 2048 ? 1 : 0], a) <= kCus;

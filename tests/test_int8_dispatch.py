@@ -49,3 +49,17 @@ def test_no_row_count_falls_between_the_rules():
                 if one_pass is not None:
                     assert _kernel(rows, depth, channels) in (one_pass, capi.INT8_KERNEL_SPLIT), \
                         (rows, depth, channels)
+
+
+@pytest.mark.parametrize("rows,depth,channels,kernel", [
+    (8, 8192, 256, capi.INT8_KERNEL_GEMV), (5, 6145, 4096, capi.INT8_KERNEL_GEMV),
+    (8, 6144, 4096, capi.INT8_KERNEL_SPLIT),
+    (9, 8192, 256, capi.INT8_KERNEL_SPLIT), (8, 8193, 256, capi.INT8_KERNEL_SPLIT),  # past 64 KB, 8192
+    (16, 1024, 2048, capi.INT8_KERNEL_GEMV), (16, 1025, 2048, capi.INT8_KERNEL_SPLIT),  # 16 KB of rows
+    (8, 2048, 6144, capi.INT8_KERNEL_GEMV), (8, 2049, 6144, capi.INT8_KERNEL_SPLIT),  # 192 workgroups
+    (5, 3000, 6113, capi.INT8_KERNEL_SPLIT), (5, 3000, 6112, capi.INT8_KERNEL_GEMV),
+    (9, 1024, 6144, capi.INT8_KERNEL_GEMV), (9, 1025, 6144, capi.INT8_KERNEL_SPLIT),
+    (16, 4096, 8192, capi.INT8_KERNEL_SPLIT), (16, 4096, 8193, capi.INT8_KERNEL_GEMV),
+    (4, 16384, 256, capi.INT8_KERNEL_GEMV), (5, 16384, 256, capi.INT8_KERNEL_SPLIT)])
+def test_up_to_sixteen_rows(rows, depth, channels, kernel):
+    assert _kernel(rows, depth, channels) == kernel
