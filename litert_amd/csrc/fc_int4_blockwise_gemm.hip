@@ -704,7 +704,12 @@ struct NibbleGemmArgs {
 // 15 of them; with a branch per block, behind which each MFMA waited for the conversions and
 // additions of the one before, 14336 x 4096 at 16 rows took 16.9 us with the row quantizer, now
 // 14.1 us. One, two and four groups of 16 blocks in flight measure the same. Row tiles are
-// wavefronts of their own for the same reason (32 rows 19.0 us, as two tiles of one wavefront 22.3).
+// wavefronts of their own for the same reason (32 rows 19.0 us, as two tiles of one wavefront 22.3),
+// next to each other on one XCD, or the second fetches the filter from memory once more. Filters
+// that give every SIMD more than one wavefront by their channels alone (kPairedMinTiles) are bound
+// by that vector work itself, of which the expanded nibbles are shared by two tiles of one
+// wavefront (32 rows, filters not in the cache, us: one tile each in any order / on one XCD / two
+// tiles: 8192 -> 28672 68.5 / 61.5 / 49.6, 4096 -> 32000 39.6 / 34.2 / 29.3).
 // The wavefronts of the 4-bit-resident kernels share nothing (no LDS image, no barrier), so each is
 // a workgroup of its own: the dispatcher then spreads them one by one over the compute units.
 // In workgroups of four, a launch of 2304 wavefronts leaves 64 compute units with three
@@ -712,53 +717,76 @@ struct NibbleGemmArgs {
 // rows: 84 us; as single wavefronts 71 us; 28672 x 16384: 59.6 -> 54.5 us).
 constexpr int kLoneWave = 64;
 
-template <int QUADS>  // of blocks in flight
-__global__ __launch_bounds__(kLoneWave) void FcInt4NibbleGemmKernel(NibbleGemmArgs a) {
+// RT: row tiles per wavefront; WQ, XQ: quads of blocks whose weights / activations are in flight.
+template <int RT, int WQ, int XQ>
+__global__ __launch_bounds__(kLoneWave, 2) void FcInt4NibbleGemmKernel(NibbleGemmArgs a) {
   const int lane = threadIdx.x & 63;
-  const int ct0 = blockIdx.x;
-  const int rt0 = blockIdx.y;
-  if (ct0 >= a.channel_tiles || rt0 >= a.row_tiles) return;
+  // Workgroups are dealt round-robin to the 8 XCDs: the row tiles of a channel tile follow each other
+  // on one XCD, in whose L2 the second finds what the first has fetched.
+  const int in_xcd = static_cast<int>(blockIdx.x / 8);
+  const int row_groups = (a.row_tiles + RT - 1) / RT;
+  const int rt0 = in_xcd % row_groups * RT;
+  const int ct0 = in_xcd / row_groups * 8 + static_cast<int>(blockIdx.x % 8);
+  if (ct0 >= a.channel_tiles) return;
   const int nb = a.nb;
   const int pairs = (nb + 1) / 2;
   const int nq = (nb + 3) / 4;
   const int ng = (nb + 15) / 16;
   const i32x4* wp = a.filter + static_cast<size_t>(ct0) * nq * 64 + lane;
   const uint2* sp = a.scales + static_cast<size_t>(ct0) * ng * 64 + lane;
-  const i64x2* xp = a.activations + static_cast<size_t>(rt0) * pairs * 64 + lane;
+  const i64x2* xp[RT];  // a last group may be short: its last tile again, not stored
+#pragma unroll
+  for (int r = 0; r < RT; ++r) {
+    xp[r] = a.activations + static_cast<size_t>(min(rt0 + r, a.row_tiles - 1)) * pairs * 64 + lane;
+  }
   // Past the end: a hot line, result unused.
   auto fetch_w = [&](int q) {
     return __builtin_nontemporal_load(wp + static_cast<size_t>(min(q, nq - 1)) * 64);
   };
   struct XStage {
-    i64x2 x[2];  // blocks 0-1, blocks 2-3 of the quad
+    i64x2 x[RT][2];  // blocks 0-1, blocks 2-3 of the quad
   };
   auto fetch_x = [&](int q) {
     const int qq = min(q, nq - 1);
     XStage st;
-    st.x[0] = xp[static_cast<size_t>(min(2 * qq, pairs - 1)) * 64];
-    st.x[1] = xp[static_cast<size_t>(min(2 * qq + 1, pairs - 1)) * 64];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      st.x[r][0] = xp[r][static_cast<size_t>(min(2 * qq, pairs - 1)) * 64];
+      st.x[r][1] = xp[r][static_cast<size_t>(min(2 * qq + 1, pairs - 1)) * 64];
+    }
     return st;
   };
   auto fetch_scales = [&](int g) { return sp[static_cast<size_t>(min(g, ng - 1)) * 64]; };
-  constexpr int kGroups = QUADS / 4;  // scale groups per trip
+  constexpr int kGroups = WQ / 4;  // scale groups per trip
+  static_assert(WQ % 4 == 0 && WQ % XQ == 0, "trip");
   uint2 sg[kGroups];
-  i32x4 wring[QUADS];
-  XStage xring[QUADS];
+  i32x4 wring[WQ];
+  XStage xring[XQ];
 #pragma unroll
-  for (int s = 0; s < QUADS; ++s) {
+  for (int s = 0; s < WQ; ++s) {
     if (s % 4 == 0) sg[s / 4] = fetch_scales(s / 4);
     wring[s] = fetch_w(s);
-    xring[s] = fetch_x(s);
+    if (s < XQ) xring[s] = fetch_x(s);
   }
 
-  // out[i]: channel 16 ct0 + 4 (lane / 16) + i, batch row 16 rt0 + lane % 16, times 16.
-  float out[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  // out[r][i]: channel 16 ct0 + 4 (lane / 16) + i, batch row 16 (rt0 + r) + lane % 16, times 16.
+  float out[RT][4];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) out[r][i] = 0.0f;
   // Whole groups without a branch: the blocks that pad the last group have scales of zero, and
   // adding the zero product leaves a running sum, which is never -0, as it is. A quad's MFMAs are
   // issued ahead of the conversions, products and additions of the quad before it.
   const i32x4 zero = {0, 0, 0, 0};
   float4 scales = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  i32x4 acc[2][4] = {{zero, zero, zero, zero}, {zero, zero, zero, zero}};
+  i32x4 acc[2][4][RT];
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+#pragma unroll
+      for (int r = 0; r < RT; ++r) acc[u][h][r] = zero;
   auto add_quad = [&](auto u_const) {  // quad u of its group
     constexpr int u = decltype(u_const)::value;
     StaticFor<4>([&](auto h_const) {
@@ -767,8 +795,12 @@ __global__ __launch_bounds__(kLoneWave) void FcInt4NibbleGemmKernel(NibbleGemmAr
       const float sc[4] = {RowBroadcast<j>(scales.x), RowBroadcast<j>(scales.y),
                            RowBroadcast<j>(scales.z), RowBroadcast<j>(scales.w)};
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        out[i] = __fadd_rn(out[i], __fmul_rn(static_cast<float>(acc[u % 2][h][i]), sc[i]));
+      for (int r = 0; r < RT; ++r) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          out[r][i] =
+              __fadd_rn(out[r][i], __fmul_rn(static_cast<float>(acc[u % 2][h][r][i]), sc[i]));
+        }
       }
     });
   };
@@ -779,9 +811,9 @@ __global__ __launch_bounds__(kLoneWave) void FcInt4NibbleGemmKernel(NibbleGemmAr
       StaticFor<4>([&](auto u_const) {
         constexpr int u = decltype(u_const)::value;  // quad of the group
         constexpr int slot = 4 * gi + u;
-        const int next = 4 * (g + gi + kGroups) + u;
+        const int quad = 4 * (g + gi) + u;
         const i32x4 w = wring[slot];
-        const XStage st = xring[slot];
+        const XStage st = xring[slot % XQ];
         StaticFor<4>([&](auto h_const) {
           constexpr int h = decltype(h_const)::value;
           const uint32_t d = static_cast<uint32_t>(w[h]);
@@ -789,11 +821,14 @@ __global__ __launch_bounds__(kLoneWave) void FcInt4NibbleGemmKernel(NibbleGemmAr
           const uint32_t hi = d & 0xF0F0F0F0u;
           const i64 wa = static_cast<i64>(static_cast<uint64_t>(lo) |
                                           (static_cast<uint64_t>(hi) << 32));
-          acc[u % 2][h] =
-              __builtin_amdgcn_mfma_i32_16x16x32_i8(wa, st.x[h >> 1][h & 1], zero, 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < RT; ++r) {
+            acc[u % 2][h][r] =
+                __builtin_amdgcn_mfma_i32_16x16x32_i8(wa, st.x[r][h >> 1][h & 1], zero, 0, 0, 0);
+          }
         });
-        wring[slot] = fetch_w(next);
-        xring[slot] = fetch_x(next);
+        wring[slot] = fetch_w(quad + WQ);
+        xring[slot % XQ] = fetch_x(quad + XQ);
         __builtin_amdgcn_sched_barrier(0);
         add_quad(std::integral_constant<int, (u + 3) % 4>{});  // of the quad before
         if constexpr (u == 0) {
@@ -812,25 +847,28 @@ __global__ __launch_bounds__(kLoneWave) void FcInt4NibbleGemmKernel(NibbleGemmAr
 
   // fully_connected.cc:1078-1082: zero-point term, row scale, bias -- after taking the factor
   // 16 back out (exact).
-  const int m = rt0 * kTile + (lane & 15);
-  if (m >= a.batches) return;
-  const float zp = static_cast<float>(a.zero_points[m]);
-  const float row_scale = a.scaling_factors[m];
-  const int n0 = ct0 * kTile + 4 * (lane >> 4);
-  float o[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int n = min(n0 + i, a.out_depth - 1);
-    o[i] = FinishOutput(__fmul_rn(out[i], 0.0625f), zp, a.kfsum[n], row_scale, a.bias != nullptr,
-                        a.bias ? a.bias[n] : 0.0f);
-  }
-  float* dst = a.output + static_cast<size_t>(m) * a.out_depth + n0;
-  if (n0 + 3 < a.out_depth && a.vector_store) {
-    *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]);
-  } else {
+  for (int r = 0; r < RT; ++r) {
+    const int m = (rt0 + r) * kTile + (lane & 15);
+    if (m >= a.batches) return;
+    const float zp = static_cast<float>(a.zero_points[m]);
+    const float row_scale = a.scaling_factors[m];
+    const int n0 = ct0 * kTile + 4 * (lane >> 4);
+    float o[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      if (n0 + i < a.out_depth) dst[i] = o[i];
+      const int n = min(n0 + i, a.out_depth - 1);
+      o[i] = FinishOutput(__fmul_rn(out[r][i], 0.0625f), zp, a.kfsum[n], row_scale,
+                          a.bias != nullptr, a.bias ? a.bias[n] : 0.0f);
+    }
+    float* dst = a.output + static_cast<size_t>(m) * a.out_depth + n0;
+    if (n0 + 3 < a.out_depth && a.vector_store) {
+      *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (n0 + i < a.out_depth) dst[i] = o[i];
+      }
     }
   }
 }
@@ -949,6 +987,8 @@ __global__ __launch_bounds__(kChainWaves * 64, 2) void FcInt4NibbleChainKernel(N
 // busy enough that one wavefront per tile moves less (us, wavefronts: 16 x 2976 -> 5003, 313 tiles,
 // 10.9 / 11.1; 32 x 4096 -> 4096, 512 tiles, 12.3 / 13.2; 64 x 4096 -> 4096, 1024 tiles, 17.6 / 14.6).
 constexpr int kChainMaxTiles = 512;
+// Two row tiles per wavefront from this many channel tiles on.
+constexpr int kPairedMinTiles = 1536;
 
 
 // ---- the same filter for one to four rows: four blocks per matrix-core tile ----------------
@@ -1380,7 +1420,14 @@ hipError_t LaunchFcInt4BlockwiseNibbleGemm(const float* input, int variant,
   if (FcInt4NibbleGemmFewTiles(batches, out_depth)) {
     hipLaunchKernelGGL(FcInt4NibbleChainKernel, grid, dim3(kChainWaves * 64), 0, stream, a);
   } else {
-    hipLaunchKernelGGL(FcInt4NibbleGemmKernel<8>, grid, dim3(kLoneWave), 0, stream, a);
+    const unsigned columns = (channel_tiles + 7) / 8 * 8;
+    if (row_tiles > 1 && channel_tiles >= kPairedMinTiles) {
+      hipLaunchKernelGGL((FcInt4NibbleGemmKernel<2, 4, 4>), dim3(columns * ((row_tiles + 1) / 2)),
+                         dim3(kLoneWave), 0, stream, a);
+    } else {
+      hipLaunchKernelGGL((FcInt4NibbleGemmKernel<1, 8, 8>), dim3(columns * row_tiles),
+                         dim3(kLoneWave), 0, stream, a);
+    }
   }
   return hipGetLastError();
 }

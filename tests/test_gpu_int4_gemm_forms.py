@@ -94,3 +94,15 @@ def test_int4_gemm_infinite_scales(fc, B, N):  # noqa: F811
     got = fc.FullyConnectedBlockwiseInt4(c["packed"], scales, K, 32).call_gemm(_cuda(c["x"])).cpu().numpy()
     assert np.array_equal(np.isnan(got), np.isnan(want))
     assert np.array_equal(got[~np.isnan(got)], want[~np.isnan(want)])
+
+
+# Two row tiles per wavefront from 1536 channel tiles on: 17 to 32 rows, and a third tile left over.
+@pytest.mark.parametrize("B,N", [(17, 24561), (32, 24560), (40, 24590), (20, 24577)])
+@pytest.mark.parametrize("blocks", [1, 5, 16, 33])
+def test_int4_nibble_paired_row_tiles_match_oracle(fc, B, N, blocks):  # noqa: F811
+    K = 32 * blocks
+    c = wl.blockwise_int4_fc(B, K, N, seed=B + N + K, lo=-8, hi=7)
+    bias = np.random.default_rng(K).standard_normal(N).astype(np.float32) if blocks % 2 else None
+    op = fc.FullyConnectedBlockwiseInt4(c["packed"], c["scales"], K, 32, bias=bias)
+    want = oracle.fc_blockwise_int4(c["x"], c["packed"], N, c["scales"].view(np.uint16), 32, bias=bias)
+    assert _bits_equal(op.call_gemm_nibbles(_cuda(c["x"])).cpu().numpy(), want)
