@@ -46,6 +46,7 @@ constexpr int kMaxGroupsPerWave = 8;  // 64 channels: one lane each when their k
 constexpr int kSplitShallowMinBlocks = 1024;  // grouped launches: see PrepareInt4Group
 constexpr int kRowPairsSideBySide = 2;        // lrtfc_int4_group_launch.split_quantize
 constexpr int kSideBySideMaxBlocks = 256;
+constexpr int kPairRound = 256;  // workgroups of a round: one per CU
 constexpr int64_t kSideBySideMaxFilterBytes = 24 << 20;
 
 __global__ __launch_bounds__(kThreads) void PackInt4BlockwiseKernel(
@@ -897,13 +898,14 @@ hipError_t LaunchFcInt4Packed(const FcInt4Args& q, const uint8_t* packed, const 
   const int ksplit = wide ? a.chunks : ChooseKsplit(q.out_depth, a.chunks);
   // Three or four fused rows of a small filter: two pairs side by side in one launch, as in small
   // groups (PrepareInt4Group); us at four rows, one tile of four -> pairs: 2048 -> 2048 6.8 -> 4.8,
-  // 4096 -> 4096 8.7 -> 6.0.
-  const int groups_per_wg = kWaves / ksplit;
+  // 4096 -> 4096 8.7 -> 6.0. Both slices together are one round of a workgroup per CU; in two they read
+  // the filter from memory twice (filters not in the cache: 2976 -> 5003 9.0 -> 10.0, 2976 -> 8192
+  // 9.2 -> 9.9, 4096 -> 7700 9.2 -> 9.9; in it, 2048 -> 8192 6.9 -> 6.3).
   if (input_f32 && (q.batches == 3 || q.batches == 4) && q.depth <= kShallowDepth &&
-      ((q.out_depth + kTileRows - 1) / kTileRows + groups_per_wg - 1) / groups_per_wg <=
-          kSideBySideMaxBlocks &&
       static_cast<int64_t>(q.out_depth) * q.depth / 2 <= kSideBySideMaxFilterBytes) {
-    return LaunchTile<true>(a, variant, 0, 2, 2, stream);
+    const int groups_per_wg = kWaves / ksplit;  // (shallow rows: ksplit is at most kWaves)
+    const int blocks = ((q.out_depth + kTileRows - 1) / kTileRows + groups_per_wg - 1) / groups_per_wg;
+    if (2 * blocks <= kPairRound) return LaunchTile<true>(a, variant, 0, 2, 2, stream);
   }
   const int tile = FitBatchTile(input_f32 ? MaxBatchTile<true>(q.depth) : MaxBatchTile<false>(q.depth),
                                 padded, ksplit, wide);

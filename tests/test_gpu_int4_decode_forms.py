@@ -18,6 +18,7 @@ pytestmark = pytest.mark.gpu
     (4128, 40), (6144, 40), (10240, 24), (16416, 9),  # three, five, and past the register form
     (8192, 4096), (8192, 4104), (16384, 2048), (16384, 2056),  # 512 and 513 groups, 256 and 257
     (2048, 8192), (2048, 8200), (4096, 515), (32, 9), (4096, 12000),  # pairs side by side, and past them
+    (2048, 4096), (2048, 4104),  # 128 and 129 workgroups a pair
 ])
 def test_int4_decode_forms_match_oracle(fc, B, K, N):  # noqa: F811
     if B * K * N > 7e7 and B not in (1, 4):
