@@ -1136,7 +1136,14 @@ TfLiteStatus PrepareNode(TfLiteContext* ctx, PartitionKernel* k, FcNode* n) {
                               : LRTFC_INT4_FORM_DECODE;
     // The form picked for a call of its own. Narrow nodes of fewer than sixteen rows keep the
     // decode tiling here: it runs several independent nodes as one launch.
-    if (n->batches < 16 && n->out_depth <= kInt4GroupedMaxOutDepth) form = LRTFC_INT4_FORM_DECODE;
+    const bool narrow = n->out_depth <= kInt4GroupedMaxOutDepth;
+    if (n->batches < 16 && narrow) form = LRTFC_INT4_FORM_DECODE;
+    // A narrow node that has been resized past the 4-bit-resident form's row counts once keeps the
+    // int8 expansion below them too: the other form saves it 2 to 3 us a launch, and every crossing
+    // of that line would upload the model's filter again and re-tile it.
+    if (form == LRTFC_INT4_FORM_GEMM_NIBBLES && narrow && n->have_gemm && !n->gemm_nibbles) {
+      form = LRTFC_INT4_FORM_GEMM_INT8;
+    }
     const bool want_nibbles = form == LRTFC_INT4_FORM_GEMM_NIBBLES;
     n->gemm_layout = form != LRTFC_INT4_FORM_DECODE;
     if (n->gemm_layout && n->have_gemm && want_nibbles != n->gemm_nibbles) n->have_gemm = false;
@@ -2183,6 +2190,8 @@ int litert_amd_describe_partition(const void* user_data, char* out, size_t out_s
       // "n" behind the group: the member runs on the 4-bit-resident matrix-core form
       text += "/g" + std::to_string(n.group) + (n.group_nibbles_from ? "n" : "");
     }
+    // "m4" / "m8": blockwise int4 on the matrix-core GEMM, weights of 4 bits or expanded to 8
+    if (n.gemm_layout) text += n.gemm_nibbles ? "/m4" : "/m8";
   }
   std::snprintf(out, out_size, "%s", text.c_str());
   return static_cast<int>(k->groups.size());

@@ -969,6 +969,35 @@ def test_blockwise_int4_resize_between_decode_and_prefill():
                 assert np.array_equal(h.read(y).view(np.uint32), want.view(np.uint32)), (rows, n)
 
 
+def test_blockwise_int4_resized_prefill_packs_its_filter_once_more_at_most():
+    """A narrow node starts on 4-bit weights at 40 rows; a resize to more rows than that form is for
+    packs the int8 expansion, and the node then stays on it, whichever side of the line it is resized
+    to: no resize between prefill sizes re-tiles the filter again."""
+    K, N, most = 64, 2048, 200
+    c = wl.blockwise_int4_fc(most, K, N, seed=77, lo=-8, hi=7)
+    with FakeHost() as h:
+        x = h.tensor(FLOAT32, (40, K), data=c["x"][:40])
+        w = h.tensor(INT4, (N, K), data=c["packed"], const=True)
+        s_ = h.tensor(FLOAT16, (N, K // 32), data=c["scales"], const=True)
+        h.blockwise(w, s_, 32)
+        y = h.tensor(FLOAT32, (40, N))
+        h.fc(x, w, None, y)
+        assert h.load_delegate() == 0, h.errors()
+        assert h.modify_graph_with_delegate() == OK and h.allocate_tensors() == OK, h.errors()
+        forms = []
+        for rows in (40, 64, 200, 64, 100, 64):
+            h.resize(x, (rows, K))
+            h.resize(y, (rows, N))
+            h.write(x, c["x"][:rows])
+            assert h.allocate_tensors() == OK, h.errors()
+            forms.append(h.describe_partition(h.plan()[0][2])[1].split("/")[-1])
+            assert h.invoke() == OK, h.errors()
+            want = oracle.fc_blockwise_int4(c["x"][:rows], c["packed"], N,
+                                            c["scales"].view(np.uint16), 32)
+            assert np.array_equal(h.read(y).view(np.uint32), want.view(np.uint32)), rows
+        assert forms == ["m4", "m4", "m8", "m8", "m8", "m8"]
+
+
 def test_completion_mark_follows_the_work_enqueued_before_it():
     """lrtfc_mark_completion: the word turns into the value only after the kernel in front of it
     on the stream has written its output, so a host that has seen the value reads the output."""
