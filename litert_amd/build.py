@@ -63,10 +63,15 @@ def build_fc():
 
 
 def build_python_calls():
-    """The per-call entry points as a CPython extension (host code only)."""
-    out = os.path.join(LIB, "litert_amd_calls.so")
+    """The per-call entry points as a CPython extension (host code only), named for the interpreter it
+    is built for. Without that interpreter's headers there is none, and the ops use ctypes."""
+    include = sysconfig.get_paths()["include"]
+    if not os.path.exists(os.path.join(include, "Python.h")):
+        print("no Python.h in %s: litert_amd_calls is not built" % include, flush=True)
+        return None
+    out = os.path.join(LIB, "litert_amd_calls" + sysconfig.get_config_var("EXT_SUFFIX"))
     _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
-          "-I" + os.path.join(ROOT, "include"), "-I" + sysconfig.get_paths()["include"], "-o", out,
+          "-I" + os.path.join(ROOT, "include"), "-I" + include, "-o", out,
           os.path.join(CSRC, "host", "python_calls.cc"), "-L" + LIB, "-llitert_amd_fc",
           "-Wl,-rpath,$ORIGIN"])
     return out
@@ -94,11 +99,8 @@ def build_bench_probes():
 
 
 def build_all():
-    outs = [build_fc(), build_python_calls(), build_bench_probes()]
-    d = build_delegate()
-    if d:
-        outs.append(d)
-    return outs
+    outs = [build_fc(), build_python_calls(), build_bench_probes(), build_delegate()]
+    return [out for out in outs if out]
 
 
 if __name__ == "__main__":

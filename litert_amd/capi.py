@@ -9,6 +9,8 @@ import ctypes as C
 import importlib.machinery
 import importlib.util
 import os
+import sysconfig
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "liblitert_amd_fc.so")
@@ -107,18 +109,21 @@ _LIB = None
 
 
 _CALLS = None
-CALLS_PATH = os.path.join(_HERE, "lib", "litert_amd_calls.so")
+CALLS_PATH = os.path.join(_HERE, "lib", "litert_amd_calls" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 
 def calls():
     """The entry points that ops call per invocation, under their C names, as functions of integer
-    addresses (or None), integers and floats: the same library without ctypes in between."""
+    addresses (or None), integers and floats: the same library without ctypes in between, or with it
+    where the extension has not been built for this interpreter."""
     global _CALLS
     if _CALLS is None:
-        load()  # the extension binds to this library
+        library = load()  # the extension binds to this library
         if not os.path.exists(CALLS_PATH):
-            raise FileNotFoundError(
-                CALLS_PATH + " is missing: run `python -m litert_amd.build` first")
+            warnings.warn(CALLS_PATH + " is missing (`python -m litert_amd.build` makes it where "
+                          "Python.h is installed): calls go through ctypes, 2 to 4 us more each")
+            _CALLS = library
+            return _CALLS
         loader = importlib.machinery.ExtensionFileLoader("litert_amd_calls", CALLS_PATH)
         spec = importlib.util.spec_from_file_location("litert_amd_calls", CALLS_PATH, loader=loader)
         module = importlib.util.module_from_spec(spec)
