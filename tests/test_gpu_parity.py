@@ -230,10 +230,9 @@ def test_hybrid_packed_gemm_matches_oracle(fc, B, K, N, asym, per_channel):
                                    (17, 8192, 64), (30, 4100, 40)])
 @pytest.mark.parametrize("asym", [True, False])
 def test_hybrid_17_to_32_rows_in_one_pass_matches_oracle(fc, B, K, N, asym):
-    """17 to 32 rows whose LDS image fits a compute unit take the register-resident GEMV with two
-    row tiles per weight tile (depth shares of 8 and 16 tiles, depths that end inside a slab, one
-    or several channel tiles per workgroup, ragged channel counts); the last two shapes -- too
-    deep, and a depth that is no multiple of 16 -- go to the GEMM instead. Same bits either way."""
+    """17 to 32 rows, on small tiles with the depth split over the wavefronts at these sizes (the
+    register-resident GEMV with two row tiles per weight tile, which takes wider filters, gives the
+    same bits: test_gpu_int8_kernels.py)."""
     c = wl.hybrid_fc(B, K, N, seed=29 + B + K)
     bias = np.random.default_rng(5).standard_normal(N).astype(np.float32)
     bias[::5] = -0.0
@@ -266,11 +265,11 @@ ROWS_33_TO_128 = [(33, 1024, 10225), (40, 4096, 14336), (64, 1040, 10256), (100,
 @pytest.mark.parametrize("B,K,N", ROWS_33_TO_128)
 @pytest.mark.parametrize("asym", [True, False])
 def test_hybrid_33_to_128_rows_on_wide_filters_matches_oracle(fc, B, K, N, asym):
-    """33 to 128 rows against a filter of 640 or more channel tiles take the kernel that streams
-    the filter once and walks the rows through LDS in depth chunks: four and eight row tiles per
-    weight tile, odd and even chunk counts, depths that end 16 into a chunk, a ragged last channel
-    tile, a ragged last row tile, workgroups whose last tiles lie past the filter; 130 rows stay on
-    the GEMM. Same bits either way."""
+    """33 to 128 rows against a filter of 640 or more channel tiles: beyond 64 rows the kernel that
+    streams the filter once and walks the rows through LDS in depth chunks (eight row tiles per weight
+    tile, a ragged last channel tile, a ragged last row tile, workgroups whose last tiles lie past
+    the filter), up to 64 at these widths small tiles (test_gpu_int8_kernels.py has the first on
+    wider filters); 130 rows stay on the GEMM. Same bits either way."""
     c = wl.hybrid_fc(B, K, N, seed=41 + B + K)
     bias = np.random.default_rng(6).standard_normal(N).astype(np.float32)
     bias[::5] = -0.0

@@ -11,8 +11,8 @@ from tests.test_gpu_parity import _bits_equal, _cuda, _run_int8, fc  # noqa: F40
 
 pytestmark = pytest.mark.gpu
 
-# rows: ring / resident GEMV (1, 5, 16), two row tiles (17, 32), GEMM (77, 150), rows kernel on
-# >= 640 channel tiles (33, 128), large GEMM tiles (1100 x 4099)
+# GEMV (1, 3 and 5 rows), small tiles (16 to 77, 150 and 257 rows), the rows kernel (128 x 10241), large
+# GEMM tiles (1100 x 4099). test_gpu_int8_kernels.py has such depths for every kernel, by name.
 SHAPES = [(1, 17, 19), (1, 2999, 530), (5, 2049, 67), (16, 1030, 33), (3, 20001, 9), (17, 2047, 301),
           (32, 4093, 515), (77, 1999, 261), (150, 21, 130), (257, 1283, 515), (40, 1027, 10243),
           (128, 1037, 10241), (1100, 131, 4099)]
