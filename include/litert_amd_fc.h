@@ -236,8 +236,9 @@ int lrtfc_fc_hybrid_int8_packed(const int8_t* quantized_input, const float* scal
                                 int batches, int depth, int out_depth, int activation,
                                 void* stream);
 
-/* Bytes of device scratch lrtfc_fc_hybrid / lrtfc_fc_blockwise_int4 need for
- * (batches, depth): quantized activations, scaling factors and zero points. */
+/* Bytes of device scratch for (batches, depth): quantized activations, in rows padded to a multiple of
+ * 16 bytes, scaling factors and zero points. Enough for every entry point that asks for it;
+ * lrtfc_fc_hybrid and lrtfc_fc_blockwise_int4 need the rows without the padding only. */
 size_t lrtfc_activation_workspace_bytes(int batches, int depth);
 
 /* EvalHybridDense end to end (tflite/kernels/fully_connected.cc:763-858):
@@ -256,8 +257,8 @@ int lrtfc_fc_hybrid(const float* input, const int8_t* filter, const float* per_c
  * LRTFC_STATIC_SCRATCH_BYTES that the library holds on every device it was initialised on
  * (lrtfc_init looks its address up); the call allocates and frees nothing and enqueues the same
  * two launches as lrtfc_fc_hybrid, with bit-identical results. Fails with
- * LRTFC_INVALID_ARGUMENT when lrtfc_activation_workspace_bytes(batches, depth) exceeds
- * LRTFC_STATIC_SCRATCH_BYTES (64 rows of depth 16384 fit). All calls on one device share the
+ * LRTFC_INVALID_ARGUMENT when batches * depth bytes and twice batches * 4, each rounded up to a
+ * multiple of 256, exceed LRTFC_STATIC_SCRATCH_BYTES together (64 rows of depth 16384 fit). All calls on one device share the
  * one array: calls that overlap on a device (different streams or threads) race; calls ordered
  * on one stream do not. */
 #define LRTFC_STATIC_SCRATCH_BYTES (1024 * 1024 + 64 * 1024)

@@ -1112,7 +1112,9 @@ int lrtfc_fc_blockwise_int4_preferred_form(int batches, int depth, int out_depth
   // and 20 us on the int8 copy), and where output tiles are so few that it gives each four
   // wavefronts (us, streaming or int8-expanded form -> here: 5 x 4096 -> 4096 13.2 -> 10.4,
   // 16 x 8192 -> 2048 20.8 -> 16.2, 64 x 4096 -> 1024 13.5 -> 10.5, 128 x 1024 -> 1024 8.0 -> 7.2);
-  // the int8-expanded one from 16 rows on otherwise.
+  // the int8-expanded one from 16 rows on otherwise. Depths beyond 8192 keep the answer they had
+  // before the four-wavefront tiles: callers re-tile their filters for it, and it is part of what the
+  // tests of this function fix (16 x 16384 -> 2048: 26.8 us there, 48.8 on the int8 copy).
   const int channel_tiles = (out_depth + 15) / 16;
   if (batches <= 4) return LRTFC_INT4_FORM_DECODE;
   if (depth <= 8192 && ((batches <= 32 && channel_tiles >= 512) ||

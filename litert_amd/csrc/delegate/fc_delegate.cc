@@ -796,9 +796,10 @@ void KernelFree(TfLiteContext* /*ctx*/, void* buffer) {
   if (buffer && buffer != reinterpret_cast<void*>(-1)) delete static_cast<PartitionKernel*>(buffer);
 }
 
-// The workspace of lrtfc_activation_workspace_bytes(batches, depth) bytes, carved as the
-// library carves it: quantized rows, then scaling factors, then zero points, each region
-// starting on a 256-byte boundary.
+// The workspace of lrtfc_activation_workspace_bytes(batches, depth) bytes, carved for the calls that
+// quantize into it themselves (blockwise int4, whose depths are multiples of 32): quantized rows,
+// then scaling factors, then zero points, each region starting on a 256-byte boundary. The library
+// carves it like this for its own calls, with rows padded to 16 bytes.
 struct ActivationScratch {
   int8_t* q;
   float* sf;

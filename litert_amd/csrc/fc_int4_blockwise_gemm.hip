@@ -32,7 +32,7 @@
 //     small forms, `tile16x64`: 16 rows and a pair of blocks in 1 KiB, lane L's 16 bytes row L % 16,
 //     depths 8 (L / 16) ... + 8 of the first block, then of the second. The row quantizer writes
 //     either order itself.
-// No LDS: a wavefront owns CT x RT tiles and requests the operands of the next blocks while it works
+// No LDS: a wavefront owns a few tiles and requests the operands of the next blocks while it works
 // on the current ones (a ring in registers); both operands are re-read by other wavefronts from L1
 // and L2. Two kernels: FcInt4BlockwiseGemmLargeKernel on 32 x 32 tiles, whose one MFMA per block and
 // tile does four times the work of a 16 x 16 one in twice the time; and FcInt4BlockwiseGemmKernel on
@@ -50,8 +50,6 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kBlock = 32;    // depth positions per quantization block
 constexpr int kTile = 16;     // channels / rows per MFMA tile
-// A wavefront owns CT x RT tiles of 16 channels x 16 rows (template parameters of the kernel);
-// a workgroup is 2 x 2 wavefronts.
 
 using i64 = long;
 typedef long i64x2 __attribute__((ext_vector_type(2)));
@@ -222,34 +220,27 @@ __device__ __forceinline__ bool WorkgroupTile(int wgs_c, int wgs_r, int* wg_c, i
   return true;
 }
 
-// CT x RT: tiles of 16 channels x 16 rows per wavefront. WROWS: wavefronts of a workgroup along the
-// batch rows (1 or 2); the others along the channels. PAIRS: pairs of blocks in flight.
-template <int CT, int RT, int WROWS, int PAIRS>
+// RT tiles of 16 channels x 16 rows per wavefront, the four of a workgroup on four channel tiles. PAIRS:
+// pairs of blocks in flight.
+template <int RT, int PAIRS>
 __global__ __launch_bounds__(kThreads, 2) void FcInt4BlockwiseGemmKernel(GemmArgs a, int wgs_c,
                                                                          int wgs_r) {
-  constexpr int WCH = 4 / WROWS;
   const int lane = threadIdx.x & 63;
   // The wavefront index as a scalar: tile addresses then stay in scalar registers and every
   // load is "scalar base + lane offset".
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int wg_c, wg_r;
   if (!WorkgroupTile(wgs_c, wgs_r, &wg_c, &wg_r)) return;
-  const int ct0 = (wg_c * WCH + wave % WCH) * CT;
-  const int rt0 = (wg_r * WROWS + wave / WCH) * RT;
-  if (ct0 >= a.channel_tiles || rt0 >= a.row_tiles) return;
+  const int ct = wg_c * 4 + wave;
+  const int rt0 = wg_r * RT;
+  if (ct >= a.channel_tiles || rt0 >= a.row_tiles) return;
   const int nb = a.nb;
   const int pairs = (nb + 1) / 2, quads = (nb + 3) / 4;
-  const char* wp[CT];
-  const char* sp[CT];
+  // Half of a tile of 32 channels, by lane offsets: 8 bytes of each of the pair's blocks.
+  const char* const wp = a.filter + static_cast<size_t>(ct >> 1) * nb * 1024 + (ct & 1) * 256;
+  const char* const sp = a.scales + static_cast<size_t>(ct >> 1) * quads * 512 + (ct & 1) * 256;
   const char* xp[RT];
-  // Tiles past the edge re-read the last valid one; their outputs are never stored.
-#pragma unroll
-  for (int j = 0; j < CT; ++j) {
-    const int ct = min(ct0 + j, a.channel_tiles - 1);
-    // Half of a tile of 32 channels, by lane offsets: 8 bytes of each of the pair's blocks.
-    wp[j] = a.filter + static_cast<size_t>(ct >> 1) * nb * 1024 + (ct & 1) * 256;
-    sp[j] = a.scales + static_cast<size_t>(ct >> 1) * quads * 512 + (ct & 1) * 256;
-  }
+  // Row tiles past the edge re-read the last valid one; their outputs are never stored.
 #pragma unroll
   for (int j = 0; j < RT; ++j) {
     xp[j] = a.activations + static_cast<size_t>(min(rt0 + j, a.row_tiles - 1)) * pairs * 1024;
@@ -258,9 +249,9 @@ __global__ __launch_bounds__(kThreads, 2) void FcInt4BlockwiseGemmKernel(GemmArg
   // is requested again right behind the last operation that reads it, so that the loads land in
   // the registers they are read from. Past the end: a hot line, result unused.
   constexpr int kSlots = PAIRS <= 4 ? 2 : PAIRS / 2;
-  i64 w[PAIRS][CT][2];
+  i64 w[PAIRS][2];
   i64x2 x[PAIRS][RT];
-  float4 sg[kSlots][CT];
+  float4 sg[kSlots];
   uint32_t lane16 = lane * 16, channel16 = (lane & 15) * 16;
   uint32_t weight8 = channel16 + (lane >> 5) * 512 + ((lane >> 4) & 1) * 8;
   auto fetch = [&](auto slot, int p) {
@@ -273,15 +264,13 @@ __global__ __launch_bounds__(kThreads, 2) void FcInt4BlockwiseGemmKernel(GemmArg
     for (int h = 0; h < 2; ++h) {
       // An odd block count: the last pair's second block is the first again, under zero scales.
       const size_t block = static_cast<size_t>(min(2 * pp + h, nb - 1)) * 1024;
-#pragma unroll
-      for (int j = 0; j < CT; ++j) w[s][j][h] = *reinterpret_cast<const i64*>(wp[j] + block + weight8);
+      w[s][h] = *reinterpret_cast<const i64*>(wp + block + weight8);
     }
   };
   auto fetch_scales = [&](auto slot, int q) {
     constexpr int s = decltype(slot)::value;
     const size_t at = static_cast<size_t>(min(q, quads - 1)) * 512;
-#pragma unroll
-    for (int j = 0; j < CT; ++j) sg[s][j] = *reinterpret_cast<const float4*>(sp[j] + at + channel16);
+    sg[s] = *reinterpret_cast<const float4*>(sp + at + channel16);
   };
   // One request at a time, in this order: waits count from the newest.
   StaticFor<kSlots>([&](auto q) {
@@ -293,20 +282,18 @@ __global__ __launch_bounds__(kThreads, 2) void FcInt4BlockwiseGemmKernel(GemmArg
     __builtin_amdgcn_sched_barrier(0);
   });
 
-  // out[cj][rj][i]: channel 16 (ct0 + cj) + lane % 16, batch row 16 (rt0 + rj) + 4 (lane / 16) + i.
-  float out[CT][RT][4];
+  // out[rj][i]: channel 16 ct + lane % 16, batch row 16 (rt0 + rj) + 4 (lane / 16) + i.
+  float out[RT][4];
 #pragma unroll
-  for (int cj = 0; cj < CT; ++cj)
+  for (int rj = 0; rj < RT; ++rj)
 #pragma unroll
-    for (int rj = 0; rj < RT; ++rj)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) out[cj][rj][i] = 0.0f;
+    for (int i = 0; i < 4; ++i) out[rj][i] = 0.0f;
 
   i32x4 base_bits = {kSumBaseBits, kSumBaseBits, kSumBaseBits, kSumBaseBits};
   asm volatile("" : "+v"(base_bits));  // in registers for good
   // The vector work on a tile trails its MFMA by kLag tiles, in this order (the fences keep it): the
   // matrix core works on the next tiles meanwhile.
-  constexpr int kTiles = CT * RT;       // tiles per block
+  constexpr int kTiles = RT;  // tiles per block
   constexpr int kLag = 3;
   // The tiles of pairs first .. first + COUNT - 1 (first a multiple of the slot counts; pair u of
   // them in slots u % PAIRS and u / 2 % kSlots).
@@ -322,9 +309,9 @@ __global__ __launch_bounds__(kThreads, 2) void FcInt4BlockwiseGemmKernel(GemmArg
       constexpr int t = decltype(t_const)::value;
       if constexpr (t < kAll) {
         constexpr int u = kFrom + t / (2 * kTiles), at = t % (2 * kTiles);
-        constexpr int h = at / kTiles, cj = at % kTiles / RT, rj = at % RT;
+        constexpr int h = at / kTiles, rj = at % RT;
         constexpr int s = u % PAIRS;
-        acc[t % (kLag + 1)] = __builtin_amdgcn_mfma_i32_16x16x32_i8(x[s][rj][h], w[s][cj][h],
+        acc[t % (kLag + 1)] = __builtin_amdgcn_mfma_i32_16x16x32_i8(x[s][rj][h], w[s][h],
                                                                     base_bits, 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (kRefill && at == 2 * kTiles - 1) {
@@ -335,15 +322,15 @@ __global__ __launch_bounds__(kThreads, 2) void FcInt4BlockwiseGemmKernel(GemmArg
       if constexpr (t >= kLag) {
         constexpr int d = t - kLag;
         constexpr int u = kFrom + d / (2 * kTiles), at = d % (2 * kTiles);
-        constexpr int h = at / kTiles, cj = at % kTiles / RT, rj = at % RT;
+        constexpr int h = at / kTiles, rj = at % RT;
         constexpr int b = 2 * (u % 2) + h, cur = u / 2 % kSlots;  // block of which quad
-        const float4& q = sg[cur][cj];
+        const float4& q = sg[cur];
         const float scale = b == 0 ? q.x : b == 1 ? q.y : b == 2 ? q.z : q.w;
         const float offset = __fmul_rn(-kSumBase, scale);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          out[cj][rj][i] = __fadd_rn(out[cj][rj][i],
-                                     ScaleBlockSum(acc[d % (kLag + 1)][i], scale, offset));
+          out[rj][i] =
+              __fadd_rn(out[rj][i], ScaleBlockSum(acc[d % (kLag + 1)][i], scale, offset));
         }
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (kRefill && u % 2 == 1 && at == 2 * kTiles - 1) {
@@ -372,30 +359,25 @@ __global__ __launch_bounds__(kThreads, 2) void FcInt4BlockwiseGemmKernel(GemmArg
   });
   bool nan = false;
 #pragma unroll
-  for (int cj = 0; cj < CT; ++cj)
-#pragma unroll
-    for (int rj = 0; rj < RT; ++rj) nan = nan || AnyNaN(out[cj][rj]);
+  for (int rj = 0; rj < RT; ++rj) nan = nan || AnyNaN(out[rj]);
   if (__ballot(nan) != 0) {
     const i32x4 zero = {0, 0, 0, 0};
 #pragma unroll
-    for (int cj = 0; cj < CT; ++cj) {
+    for (int rj = 0; rj < RT; ++rj) {
+      float again[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+      for (int b = 0; b < nb; ++b) {
+        const float scale = *reinterpret_cast<const float*>(sp + static_cast<size_t>(b / 4) * 512 +
+                                                            channel16 + (b % 4) * 4);
+        const i64 wb = *reinterpret_cast<const i64*>(wp + static_cast<size_t>(b) * 1024 + weight8);
+        const i64x2 xb = *reinterpret_cast<const i64x2*>(xp[rj] + static_cast<size_t>(b / 2) * 1024 + lane16);
+        const i32x4 acc = __builtin_amdgcn_mfma_i32_16x16x32_i8(b % 2 ? xb[1] : xb[0], wb, zero, 0, 0, 0);
 #pragma unroll
-      for (int rj = 0; rj < RT; ++rj) {
-        float again[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int b = 0; b < nb; ++b) {
-          const float scale = *reinterpret_cast<const float*>(sp[cj] + static_cast<size_t>(b / 4) * 512 +
-                                                              channel16 + (b % 4) * 4);
-          const i64 wb = *reinterpret_cast<const i64*>(wp[cj] + static_cast<size_t>(b) * 1024 + weight8);
-          const i64x2 xb = *reinterpret_cast<const i64x2*>(xp[rj] + static_cast<size_t>(b / 2) * 1024 + lane16);
-          const i32x4 acc = __builtin_amdgcn_mfma_i32_16x16x32_i8(b % 2 ? xb[1] : xb[0], wb, zero, 0, 0, 0);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            again[i] = __fadd_rn(again[i], __fmul_rn(static_cast<float>(acc[i]), scale));
-          }
+        for (int i = 0; i < 4; ++i) {
+          again[i] = __fadd_rn(again[i], __fmul_rn(static_cast<float>(acc[i]), scale));
         }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) out[cj][rj][i] = again[i];
       }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) out[rj][i] = again[i];
     }
   }
 
@@ -409,18 +391,14 @@ __global__ __launch_bounds__(kThreads, 2) void FcInt4BlockwiseGemmKernel(GemmArg
       zp[i] = static_cast<float>(a.zero_points[m]);
       row_scale[i] = a.scaling_factors[m];
     }
+    const int n = ct * kTile + (lane & 15);
+    if (n >= a.out_depth) continue;
+    const float kfsum = a.kfsum[n];
+    const float bias = a.bias ? a.bias[n] : 0.0f;
 #pragma unroll
-    for (int cj = 0; cj < CT; ++cj) {
-      const int n = (ct0 + cj) * kTile + (lane & 15);
-      if (n >= a.out_depth) continue;
-      const float kfsum = a.kfsum[n];
-      const float bias = a.bias ? a.bias[n] : 0.0f;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float v = FinishOutput(out[cj][rj][i], zp[i], kfsum, row_scale[i], a.bias != nullptr,
-                                     bias);
-        if (m0 + i < a.batches) a.output[static_cast<size_t>(m0 + i) * a.out_depth + n] = v;
-      }
+    for (int i = 0; i < 4; ++i) {
+      const float v = FinishOutput(out[rj][i], zp[i], kfsum, row_scale[i], a.bias != nullptr, bias);
+      if (m0 + i < a.batches) a.output[static_cast<size_t>(m0 + i) * a.out_depth + n] = v;
     }
   }
 }
@@ -1334,8 +1312,8 @@ hipError_t LaunchFcInt4BlockwiseGemm(const float* input, int variant, float* sca
                                ((batches + kTile - 1) / kTile);
   const int64_t wide_tiles = static_cast<int64_t>((out_depth + kWide - 1) / kWide) *
                              ((batches + kWide - 1) / kWide);
-  if (narrow_tiles <= 1024) return launch(FcInt4BlockwiseGemmKernel<1, 1, 1, 8>, Narrow{}, 1, 1, 1);
-  if (narrow_tiles <= 2048) return launch(FcInt4BlockwiseGemmKernel<1, 2, 1, 4>, Narrow{}, 1, 2, 1);
+  if (narrow_tiles <= 1024) return launch(FcInt4BlockwiseGemmKernel<1, 8>, Narrow{}, 1, 1, 1);
+  if (narrow_tiles <= 2048) return launch(FcInt4BlockwiseGemmKernel<2, 4>, Narrow{}, 1, 2, 1);
   if (wide_tiles <= 2560) return launch(FcInt4BlockwiseGemmLargeKernel<1, 1, 1, 8>, Wide{}, 1, 1, 1);
   if (wide_tiles <= 6144) return launch(FcInt4BlockwiseGemmLargeKernel<1, 2, 1, 4>, Wide{}, 1, 2, 1);
   return launch(FcInt4BlockwiseGemmLargeKernel<2, 2, 2, 2>, Wide{}, 2, 2, 2);

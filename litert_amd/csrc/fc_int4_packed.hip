@@ -165,14 +165,15 @@ struct Int4Shared {
 };
 
 // GPT: groups of 8 depth positions each thread keeps in registers between the two passes of
-// the prologue; the register form covers depth <= GPT * 256 * 8.
+// the prologue; the register form covers depth <= GPT * THREADS * 8.
 // The work of one workgroup; `block` is its index among the workgroups of this filter.
 // gpw: consecutive channel groups one wavefront works through (ksplit == 1 only). Their
 // tiles are one contiguous stretch of the filter, so the ring of loads runs on across group
 // boundaries and the prologue (the row quantizer) is paid once for all of them.
-// ALL > 0: a wavefront has at most ALL tiles (ksplit == 1, gpw * chunks <= ALL) and requests
-// every one of them before it does anything else: no refills, one memory round trip per
-// wavefront, and straight-line code whose waits for each tile are exact.
+// ALL > 0: a wavefront has at most ALL tiles (ksplit == 1 and gpw * chunks <= ALL, or one tile of each
+// of ksplit == chunks wavefronts, WideDeep) and requests every one of them before it does anything
+// else: no refills, one memory round trip per wavefront, and straight-line code whose waits for
+// each tile are exact.
 template <int N, class F>
 __device__ __forceinline__ void StaticFor(F&& f) {
   if constexpr (N > 0) {
