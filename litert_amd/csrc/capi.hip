@@ -1314,12 +1314,13 @@ int lrtfc_fc_blockwise_int4(const float* input, const uint8_t* packed_filter,
   if (batches == 0 || out_depth == 0) return LRTFC_OK;
   LRTFC_REQUIRE(input && workspace, "null pointer");
   LRTFC_REQUIRE(depth > 0, "depth must be positive");
-  LRTFC_REQUIRE(workspace_bytes >= WorkspaceBytes(batches, depth),
-                "workspace too small: %zu < %zu bytes", workspace_bytes,
-                WorkspaceBytes(batches, depth));
+  // As in lrtfc_fc_hybrid, the rows need no padding on the model's layout.
+  const size_t need = lrtfc::ActivationWorkspaceBytes(batches, depth);
+  LRTFC_REQUIRE(workspace_bytes >= need, "workspace too small: %zu < %zu bytes", workspace_bytes,
+                need);
   LRTFC_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255) == 0,
                 "workspace must be 256-byte aligned");
-  const Workspace w = SplitWorkspace(workspace, batches, depth);
+  const Workspace w = lrtfc::SplitActivationWorkspace(workspace, batches, depth);
   // EvalBlockwise4Bit always quantizes asymmetrically (fully_connected.cc:1044-1047).
   int rc = lrtfc_batch_quantize_floats(input, batches, depth, w.q, w.sf, w.zp,
                                        /*do_asymmetric=*/1, quant_variant, stream);

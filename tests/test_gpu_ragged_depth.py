@@ -128,3 +128,35 @@ def test_int4_per_channel_nan_and_tiny_rows(fc, B, K):  # noqa: F811
     want = oracle.fc_hybrid_int4_per_channel(x, packed, 35, scales)
     got = fc.FullyConnectedHybridInt4PerChannel(packed, K, scales)(_cuda(x)).cpu().numpy()
     assert _bits_equal(got, want)
+
+
+def test_model_layout_entry_points_take_workspaces_without_padding(fc):  # noqa: F811
+    """What lrtfc_fc_blockwise_int4 and lrtfc_fc_hybrid need: rows of `depth` bytes, not of the padded
+    length that the re-tiled paths use and lrtfc_activation_workspace_bytes covers."""
+    import torch
+    B, K, N, bs = 40, 24, 10, 8
+    up = lambda v: (v + 255) // 256 * 256  # noqa: E731
+    exact = up(B * K) + 2 * up(4 * B)
+    lib = capi.load()
+    assert exact < lib.lrtfc_activation_workspace_bytes(B, K)
+    stream = torch.cuda.current_stream().cuda_stream
+    ptr = lambda t: t.data_ptr()  # noqa: E731
+    ws = torch.empty(exact, dtype=torch.uint8, device="cuda")
+    out = torch.empty((B, N), device="cuda")
+
+    c = wl.blockwise_int4_fc(B, K, N, blocksize=bs, seed=1, lo=-8, hi=7)
+    op = fc.FullyConnectedBlockwiseInt4(c["packed"], c["scales"], K, bs)
+    x = _cuda(c["x"])
+    capi.check(lib.lrtfc_fc_blockwise_int4(
+        ptr(x), ptr(op.filter), ptr(op.scales), ptr(op.kfsum), None, ptr(out), B, K, N, bs, 0, ptr(ws),
+        exact, stream))
+    want = oracle.fc_blockwise_int4(c["x"], c["packed"], N, c["scales"].view(np.uint16), bs)
+    assert _bits_equal(out.cpu().numpy(), want)
+
+    c = wl.hybrid_fc(B, K, N, seed=2)
+    op = fc.FullyConnectedHybrid(c["w"], c["pcs"], packed=False)
+    x = _cuda(c["x"])
+    capi.check(lib.lrtfc_fc_hybrid(
+        ptr(x), ptr(op.filter), ptr(op.pcs), 1.0, ptr(op.row_sums), None, ptr(out), B, K, N, 1, 0, 0,
+        ptr(ws), exact, stream))
+    assert _bits_equal(out.cpu().numpy(), oracle.fc_hybrid(c["x"], c["w"], c["pcs"]))
