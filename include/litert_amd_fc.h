@@ -237,8 +237,9 @@ int lrtfc_fc_hybrid_int8_packed(const int8_t* quantized_input, const float* scal
                                 void* stream);
 
 /* Bytes of device scratch for (batches, depth): quantized activations, in rows padded to a multiple of
- * 16 bytes, scaling factors and zero points. Enough for every entry point that asks for it;
- * lrtfc_fc_hybrid and lrtfc_fc_blockwise_int4 need the rows without the padding only. */
+ * 16 bytes, scaling factors and zero points. Enough for every entry point that asks for it. A
+ * workspace with the room of the rows without the padding is taken too, except by
+ * lrtfc_fc_blockwise_int4_gemm and its variants, which have a size of their own; results are the same. */
 size_t lrtfc_activation_workspace_bytes(int batches, int depth);
 
 /* EvalHybridDense end to end (tflite/kernels/fully_connected.cc:763-858):

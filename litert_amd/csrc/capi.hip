@@ -75,8 +75,12 @@ using Workspace = lrtfc::ActivationWorkspace;
 size_t WorkspaceBytes(int batches, int depth) {
   return lrtfc::ActivationWorkspaceBytes(batches, lrtfc::PaddedDepth(depth));
 }
-Workspace SplitWorkspace(void* base, int batches, int depth) {
-  return lrtfc::SplitActivationWorkspace(base, batches, lrtfc::PaddedDepth(depth));
+// How far apart the quantized rows lie in a workspace of workspace_bytes: PaddedDepth(depth), or depth
+// where it only has the room that rows without padding take (the kernels then shift each row's last
+// piece into place); 0 where it does not have that.
+int WorkspaceRowStride(int batches, int depth, size_t workspace_bytes) {
+  if (workspace_bytes >= WorkspaceBytes(batches, depth)) return lrtfc::PaddedDepth(depth);
+  return workspace_bytes >= lrtfc::ActivationWorkspaceBytes(batches, depth) ? depth : 0;
 }
 
 }  // namespace
@@ -519,12 +523,12 @@ int FcHybridInt8Packed(const int8_t* quantized_input, const float* scaling_facto
                  "packed hybrid GEMV");
 }
 
-// BatchQuantizeFloats into a workspace whose rows are padded (kernels.h).
-int BatchQuantizePadded(const float* values, int batches, int depth, const Workspace& w,
+// BatchQuantizeFloats into a workspace whose rows are `stride` bytes apart (kernels.h).
+int BatchQuantizePadded(const float* values, int batches, int depth, int stride, const Workspace& w,
                         int do_asymmetric, int variant, void* stream) {
   LRTFC_REQUIRE(variant >= 0 && variant <= LRTFC_QUANT_NEON_LEGACY, "unknown quantizer variant");
-  return FromHip(lrtfc::LaunchBatchQuantize(values, batches, depth, lrtfc::PaddedDepth(depth), w.q,
-                                            w.sf, w.zp, do_asymmetric, variant, AsStream(stream)),
+  return FromHip(lrtfc::LaunchBatchQuantize(values, batches, depth, stride, w.q, w.sf, w.zp,
+                                            do_asymmetric, variant, AsStream(stream)),
                  "batch quantize");
 }
 }  // namespace
@@ -551,19 +555,18 @@ int lrtfc_fc_hybrid_packed_workspace(const float* input, const int8_t* packed_fi
   LRTFC_REQUIRE(batches >= 0 && depth > 0 && out_depth >= 0, "bad dimension");
   if (batches == 0 || out_depth == 0) return LRTFC_OK;
   LRTFC_REQUIRE(input && workspace, "null pointer");
-  LRTFC_REQUIRE(workspace_bytes >= WorkspaceBytes(batches, depth),
-                "workspace too small: %zu < %zu bytes", workspace_bytes,
+  const int stride = WorkspaceRowStride(batches, depth, workspace_bytes);
+  LRTFC_REQUIRE(stride > 0, "workspace too small: %zu < %zu bytes", workspace_bytes,
                 WorkspaceBytes(batches, depth));
   LRTFC_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255) == 0,
                 "workspace must be 256-byte aligned");
-  const Workspace w = SplitWorkspace(workspace, batches, depth);
-  int rc = BatchQuantizePadded(input, batches, depth, w, asymmetric_quantize_inputs, quant_variant,
-                               stream);
+  const Workspace w = lrtfc::SplitActivationWorkspace(workspace, batches, stride);
+  int rc = BatchQuantizePadded(input, batches, depth, stride, w, asymmetric_quantize_inputs,
+                               quant_variant, stream);
   if (rc != LRTFC_OK) return rc;
   return FcHybridInt8Packed(w.q, w.sf, asymmetric_quantize_inputs ? w.zp : nullptr, packed_filter,
                             per_channel_scales, filter_scale, filter_row_sums, bias, output,
-                            batches, lrtfc::PaddedDepth(depth), out_depth, activation,
-                            /*zero_input_exit=*/1, stream);
+                            batches, stride, out_depth, activation, /*zero_input_exit=*/1, stream);
 }
 
 namespace {
@@ -609,15 +612,19 @@ int lrtfc_batch_matmul_hybrid_packed_nd(const float* lhs, const int* lhs_batch_d
   LRTFC_REQUIRE(lhs && packed_weights && row_sums && output && workspace, "null pointer");
   const size_t need =
       lrtfc_batch_matmul_workspace_bytes(static_cast<int>(lhs_matrices), rows, depth, adj_x);
-  LRTFC_REQUIRE(workspace_bytes >= need, "workspace too small: %zu < %zu bytes", workspace_bytes,
-                need);
+  const size_t transposed_bytes = adj_x ? TransposedBytes(lhs_matrices, rows, depth) : 0;
+  const int stride = workspace_bytes < transposed_bytes
+                         ? 0
+                         : WorkspaceRowStride(static_cast<int>(quant_rows), depth,
+                                              workspace_bytes - transposed_bytes);
+  LRTFC_REQUIRE(stride > 0, "workspace too small: %zu < %zu bytes", workspace_bytes, need);
   LRTFC_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255) == 0,
                 "workspace must be 256-byte aligned");
   void* quant_space = workspace;
   if (adj_x) {
     // The op's own first step (batch_matmul.cc:811-813): [.., depth, rows] -> [.., rows, depth].
     float* transposed = static_cast<float*>(workspace);
-    quant_space = static_cast<char*>(workspace) + TransposedBytes(lhs_matrices, rows, depth);
+    quant_space = static_cast<char*>(workspace) + transposed_bytes;
     int rc = FromHip(lrtfc::LaunchTransposeLastTwoF32(lhs, static_cast<int>(lhs_matrices), depth,
                                                       rows, transposed, AsStream(stream)),
                      "left operand transposition");
@@ -626,8 +633,9 @@ int lrtfc_batch_matmul_hybrid_packed_nd(const float* lhs, const int* lhs_batch_d
   }
   // BatchQuantizeFloats over every row of the float operand (batch_matmul.cc:472-497); symmetric
   // quantization leaves the offsets at zero (:487-489).
-  const Workspace w = SplitWorkspace(quant_space, static_cast<int>(quant_rows), depth);
-  int rc = BatchQuantizePadded(lhs, static_cast<int>(quant_rows), depth, w,
+  const Workspace w =
+      lrtfc::SplitActivationWorkspace(quant_space, static_cast<int>(quant_rows), stride);
+  int rc = BatchQuantizePadded(lhs, static_cast<int>(quant_rows), depth, stride, w,
                                asymmetric_quantize_inputs, quant_variant, stream);
   if (rc != LRTFC_OK) return rc;
   const int32_t* zp = asymmetric_quantize_inputs ? w.zp : nullptr;
@@ -655,13 +663,12 @@ int lrtfc_batch_matmul_hybrid_packed_nd(const float* lhs, const int* lhs_batch_d
       ++run;
     }
     const size_t row0 = static_cast<size_t>(l0) * rows;
-    rc = FcHybridInt8Packed(w.q + row0 * lrtfc::PaddedDepth(depth), w.sf + row0, zp ? zp + row0 : nullptr,
+    rc = FcHybridInt8Packed(w.q + row0 * stride, w.sf + row0, zp ? zp + row0 : nullptr,
                             packed_weights + static_cast<size_t>(w0) * matrix_bytes,
                             per_channel_scales, filter_scale,
                             row_sums + static_cast<size_t>(w0) * units, nullptr,
                             output + static_cast<size_t>(o) * rows * units,
-                            static_cast<int>(run * rows), lrtfc::PaddedDepth(depth), units,
-                            LRTFC_ACT_NONE, 0, stream,
+                            static_cast<int>(run * rows), stride, units, LRTFC_ACT_NONE, 0, stream,
                             /*batch_matmul=*/1);
     if (rc != LRTFC_OK) return rc;
     o += run;
@@ -946,23 +953,23 @@ int lrtfc_fc_hybrid_int4_per_channel_packed(const float* input, const int8_t* pa
   LRTFC_REQUIRE(input && packed_filter && output && workspace, "null pointer");
   LRTFC_REQUIRE(FloatActivationOk(activation),
                 "activation %d is not one of None/Relu/ReluN1To1/Relu6/SignBit", activation);
-  LRTFC_REQUIRE(workspace_bytes >= WorkspaceBytes(batches, depth),
-                "workspace too small: %zu < %zu bytes", workspace_bytes,
+  const int stride = WorkspaceRowStride(batches, depth, workspace_bytes);
+  LRTFC_REQUIRE(stride > 0, "workspace too small: %zu < %zu bytes", workspace_bytes,
                 WorkspaceBytes(batches, depth));
   LRTFC_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255) == 0,
                 "workspace must be 256-byte aligned");
   LRTFC_REQUIRE((reinterpret_cast<uintptr_t>(packed_filter) & 15) == 0,
                 "packed filter must be 16-byte aligned");
-  const Workspace w = SplitWorkspace(workspace, batches, depth);
-  int rc = FromHip(lrtfc::LaunchBatchQuantize4Bit(input, batches, depth, lrtfc::PaddedDepth(depth),
-                                                  w.q, w.sf, w.zp, AsStream(stream)),
+  const Workspace w = lrtfc::SplitActivationWorkspace(workspace, batches, stride);
+  int rc = FromHip(lrtfc::LaunchBatchQuantize4Bit(input, batches, depth, stride, w.q, w.sf, w.zp,
+                                                  AsStream(stream)),
                    "4-bit path row quantizer");
   if (rc != LRTFC_OK) return rc;
   lrtfc::FcInt8Args a{};
   a.input = w.q;
   a.filter = packed_filter;
   a.batches = batches;
-  a.depth = lrtfc::PaddedDepth(depth);
+  a.depth = stride;
   a.out_depth = out_depth;
   a.scaling_factors = w.sf;
   a.zero_points = w.zp;  // the rows' input offsets on this path
@@ -1015,7 +1022,7 @@ int lrtfc_fc_hybrid_int4_per_channel_nibbles(const float* input, const uint8_t* 
                 "activation %d is not one of None/Relu/ReluN1To1/Relu6/SignBit", activation);
   LRTFC_REQUIRE(lrtfc::FcInt4PerChannelGemvSupports(depth),
                 "depth %d is odd or too large for the nibble GEMV", depth);
-  LRTFC_REQUIRE(workspace_bytes >= WorkspaceBytes(batches, depth),
+  LRTFC_REQUIRE(WorkspaceRowStride(batches, depth, workspace_bytes) > 0,
                 "workspace too small: %zu < %zu bytes", workspace_bytes,
                 WorkspaceBytes(batches, depth));
   LRTFC_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255) == 0,
@@ -1029,16 +1036,26 @@ int lrtfc_fc_hybrid_int4_per_channel_nibbles(const float* input, const uint8_t* 
                                                      activation, AsStream(stream)),
                    "per-channel int4 hybrid GEMV (nibble layout, fused quantizer)");
   }
-  const Workspace w = SplitWorkspace(workspace, batches, depth);
-  int rc = FromHip(lrtfc::LaunchBatchQuantize4Bit(input, batches, depth, lrtfc::PaddedDepth(depth),
-                                                  w.q, w.sf, w.zp, AsStream(stream)),
-                   "4-bit path row quantizer");
-  if (rc != LRTFC_OK) return rc;
-  return FromHip(lrtfc::LaunchFcInt4PerChannelGemv(retiled_filter, nullptr, w.q, w.sf, w.zp,
-                                                   per_channel_scales, filter_scale, bias, output,
-                                                   batches, lrtfc::PaddedDepth(depth), out_depth,
-                                                   activation, AsStream(stream)),
+  // This kernel's rows are padded. A workspace with the room of rows without padding holds fewer of
+  // them, and always one (a region's size is rounded up to 256 bytes): as many at a time as fit.
+  int rows = batches;
+  while (rows > 1 && WorkspaceBytes(rows, depth) > workspace_bytes) --rows;
+  const Workspace w = lrtfc::SplitActivationWorkspace(workspace, rows, lrtfc::PaddedDepth(depth));
+  for (int row = 0; row < batches; row += rows) {
+    const int count = batches - row < rows ? batches - row : rows;
+    int rc = FromHip(lrtfc::LaunchBatchQuantize4Bit(input + static_cast<size_t>(row) * depth, count,
+                                                    depth, lrtfc::PaddedDepth(depth), w.q, w.sf, w.zp,
+                                                    AsStream(stream)),
+                     "4-bit path row quantizer");
+    if (rc != LRTFC_OK) return rc;
+    rc = FromHip(lrtfc::LaunchFcInt4PerChannelGemv(
+                     retiled_filter, nullptr, w.q, w.sf, w.zp, per_channel_scales, filter_scale, bias,
+                     output + static_cast<size_t>(row) * out_depth, count, lrtfc::PaddedDepth(depth),
+                     out_depth, activation, AsStream(stream)),
                  "per-channel int4 hybrid GEMV (nibble layout)");
+    if (rc != LRTFC_OK) return rc;
+  }
+  return LRTFC_OK;
 }
 
 size_t lrtfc_gemm_int4_blockwise_bytes(int out_depth, int depth) {

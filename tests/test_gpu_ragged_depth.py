@@ -160,3 +160,68 @@ def test_model_layout_entry_points_take_workspaces_without_padding(fc):  # noqa:
         ptr(x), ptr(op.filter), ptr(op.pcs), 1.0, ptr(op.row_sums), None, ptr(out), B, K, N, 1, 0, 0,
         ptr(ws), exact, stream))
     assert _bits_equal(out.cpu().numpy(), oracle.fc_hybrid(c["x"], c["w"], c["pcs"]))
+
+
+@pytest.mark.parametrize("B,K", [(1, 30), (5, 1030), (18, 2998), (40, 1030), (300, 1030)])
+def test_retiled_entry_points_take_workspaces_without_padding(fc, B, K):  # noqa: F811
+    """A workspace with the room that rows without padding take, as a caller's saved plan may have it:
+    the same bits as with the size that is asked for now, and one byte less is refused."""
+    import torch
+    N = 70
+    up = lambda v: (v + 255) // 256 * 256  # noqa: E731
+    exact = up(B * K) + 2 * up(4 * B)
+    assert exact <= capi.load().lrtfc_activation_workspace_bytes(B, K)
+    ws = torch.empty(exact, dtype=torch.uint8, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    ptr = lambda t: t.data_ptr()  # noqa: E731
+    lib = capi.load()
+
+    c = wl.hybrid_fc(B, K, N, seed=B)
+    op = fc.FullyConnectedHybrid(c["w"], c["pcs"])
+    x = _cuda(c["x"])
+    out = torch.empty((B, N), device="cuda")
+    args = (ptr(x), ptr(op.packed_filter), ptr(op.pcs), 1.0, ptr(op.row_sums), None, ptr(out), B, K, N,
+            1, 0, 0, ptr(ws))
+    capi.check(lib.lrtfc_fc_hybrid_packed_workspace(*args, exact, stream))
+    assert _bits_equal(out.cpu().numpy(), oracle.fc_hybrid(c["x"], c["w"], c["pcs"]))
+    assert lib.lrtfc_fc_hybrid_packed_workspace(*args, exact - 1, stream) == capi.INVALID_ARGUMENT
+
+    packed = wl.pack_int4(np.random.default_rng(B).integers(-7, 8, (N, K)).astype(np.int8))
+    scales = np.random.default_rng(K).uniform(0.01, 0.1, N).astype(np.float32)
+    want = oracle.fc_hybrid_int4_per_channel(c["x"], packed, N, scales)
+    op = fc.FullyConnectedHybridInt4PerChannel(packed, K, scales)
+    op(x), op(x, force_int8=True)  # packs both layouts
+    for entry, filter in ((lib.lrtfc_fc_hybrid_int4_per_channel_packed, op._packed_int8),
+                          (lib.lrtfc_fc_hybrid_int4_per_channel_nibbles, op._retiled_nibbles)):
+        if filter is None:  # more rows than the nibble layout is made for
+            continue
+        out.zero_()
+        args = (ptr(x), ptr(filter), ptr(op.pcs), 1.0, None, ptr(out), B, K, N, 0, ptr(ws))
+        capi.check(entry(*args, exact, stream))
+        assert _bits_equal(out.cpu().numpy(), want)
+        assert entry(*args, exact - 1, stream) == capi.INVALID_ARGUMENT
+
+
+@pytest.mark.parametrize("adj_x", [False, True])
+def test_batch_matmul_takes_a_workspace_without_padding(fc, monkeypatch, adj_x):  # noqa: F811
+    from litert_amd.batch_matmul import BatchMatMulHybrid
+    M, rows, K, units = 3, 7, 1030, 40
+    rng = np.random.default_rng(8)
+    lhs = rng.standard_normal((M, K, rows) if adj_x else (M, rows, K)).astype(np.float32)
+    weights = rng.integers(-127, 128, (M, units, K)).astype(np.int8)
+    op = BatchMatMulHybrid(weights, filter_scale=0.01, adj_x=adj_x, adj_y=True)
+    x = _cuda(lhs)
+    want = op(x).cpu().numpy()
+    up = lambda v: (v + 255) // 256 * 256  # noqa: E731
+    exact = up(M * rows * K) + 2 * up(4 * M * rows) + (up(4 * M * rows * K) if adj_x else 0)
+    assert exact < capi.load().lrtfc_batch_matmul_workspace_bytes(M, rows, K, int(adj_x))
+    lib = capi.load()
+
+    class Lib:  # as a caller that kept this size
+        def __getattr__(self, name):
+            return (lambda *args: exact) if name == "lrtfc_batch_matmul_workspace_bytes" else getattr(lib, name)
+    op._ws = None
+    monkeypatch.setattr(capi, "load", Lib)
+    got = op(x).cpu().numpy()
+    assert op._ws.numel() == exact
+    assert _bits_equal(got, want)
