@@ -684,7 +684,7 @@ struct NibbleGemmArgs {
 // A wavefront alone on its SIMD issues a vector operation every 8 cycles or so, and a block takes
 // 15 of them; with a branch per block, behind which each MFMA waited for the conversions and
 // additions of the one before, 14336 x 4096 at 16 rows took 16.9 us with the row quantizer, now
-// 14.1 us. One, two and four groups of 16 blocks in flight measure the same. Row tiles are
+// 13.5 us. One, two and four groups of 16 blocks in flight measure the same. Row tiles are
 // wavefronts of their own for the same reason (32 rows 19.0 us, as two tiles of one wavefront 22.3),
 // next to each other on one XCD, or the second fetches the filter from memory once more. Filters
 // that give every SIMD more than one wavefront by their channels alone (kPairedMinTiles) are bound
