@@ -1125,7 +1125,7 @@ int lrtfc_fc_blockwise_int4_preferred_form(int batches, int depth, int out_depth
   // Up to four rows the streaming kernel makes one pass over the filter. Beyond that the GEMMs
   // stream it once for the whole batch: the nibble-resident one where the filter stream is the
   // bound (up to 32 rows) and the filter is wide enough to give every SIMD a wavefront
-  // (14336 x 4096 takes 14.1 us at 5 to 16 rows against 24 us in two passes of the streaming kernel
+  // (14336 x 4096 takes 13.4 us at 5 to 16 rows against 23 us in two passes of the streaming kernel
   // and 20 us on the int8 copy), and where output tiles are so few that it gives each four
   // wavefronts (us, streaming or int8-expanded form -> here: 5 x 4096 -> 4096 13.2 -> 10.4,
   // 16 x 8192 -> 2048 20.8 -> 16.2, 64 x 4096 -> 1024 13.5 -> 10.5, 128 x 1024 -> 1024 8.0 -> 7.2);
