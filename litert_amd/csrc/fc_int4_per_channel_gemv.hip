@@ -444,7 +444,7 @@ void FcInt4PerChannelResidentKernel(const uint8_t* early_packed, const float* ea
       float scale_denom = fmaxf(fabsf(mn), fabsf(mx));
       if (scale_denom == 0.0f) scale_denom = 127.0f;
       const float mult = SymmetricMultiplier(scale_denom);
-      const float sf = static_cast<float>(static_cast<double>(scale_denom) / 127.0);
+      const float sf = Over127(scale_denom);
       int8_t* qrow = q + wave * qstride;
       int32_t sum = 0;
       // whole_c: a row that fills all pieces, in one straight line. A shorter one skips the pieces

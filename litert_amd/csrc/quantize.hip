@@ -101,7 +101,7 @@ __global__ __launch_bounds__(THREADS) void BatchQuantize4BitKernel(
     int32_t total = 0;
 #pragma unroll
     for (int w = 0; w < THREADS / kWaveSize; ++w) total += s_sum[w];
-    scaling_factors[row] = static_cast<float>(static_cast<double>(scale_denom) / 127.0);
+    scaling_factors[row] = Over127(scale_denom);
     input_offsets[row] = total * -7;
   }
 }

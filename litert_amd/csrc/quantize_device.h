@@ -7,55 +7,30 @@
 #define LITERT_AMD_CSRC_QUANTIZE_DEVICE_H_
 
 #include "device_utils.h"
+#include "row_params.h"
 #include "../../include/litert_amd_fc.h"
 
 namespace lrtfc {
 
-struct RowQuantParams {
-  float scale;     // scaling factor stored for the row
-  float inv;       // multiplier applied to each element
-  int32_t zero_point;
-  bool all_zero;   // the row quantizes to zeros with scale 1 / zero point 0
+// v_rcp_f64: 1 / x to 2^-24.
+struct HardwareReciprocal {
+  __device__ __forceinline__ double operator()(double x) const { return __builtin_amdgcn_rcp(x); }
 };
 
 // mn = min(0, min v), mx = max(0, max v) of the row.
 template <int VARIANT>
 __device__ __forceinline__ RowQuantParams AsymmetricRowParams(float mn, float mx) {
+  constexpr bool kPortable = VARIANT == LRTFC_QUANT_PORTABLE;
   RowQuantParams p;
-  p.zero_point = 0;
-  p.all_zero = false;
   if (mn == mx) {  // both 0
+    p.zero_point = 0;
     p.all_zero = true;
     p.scale = 1.0f;
     p.inv = 1.0f;
     return p;
   }
-  const double qmin = -128.0, qmax = 127.0;
-  const double rmin = static_cast<double>(mn);
-  const double rmax = static_cast<double>(mx);
-  // Portable widens to double before subtracting (portable_tensor_utils.cc:81-87); the
-  // NEON build subtracts in float (neon_tensor_utils.cc:2486).
-  const double span = (VARIANT == LRTFC_QUANT_PORTABLE)
-                          ? (rmax - rmin)
-                          : static_cast<double>(__fsub_rn(mx, mn));
-  const double scale = span / (qmax - qmin);
-  const double zp_from_min = qmin - rmin / scale;
-  const double zp_from_max = qmax - rmax / scale;
-  const double err_from_min = fabs(qmin) + fabs(rmin / scale);
-  const double err_from_max = fabs(qmax) + fabs(rmax / scale);
-  const double zp_double = err_from_min < err_from_max ? zp_from_min : zp_from_max;
-  if (zp_double <= qmin) {
-    p.zero_point = -128;
-  } else if (zp_double >= qmax) {
-    p.zero_point = 127;
-  } else {
-    p.zero_point = static_cast<int8_t>(round(zp_double));
-  }
-  p.scale = static_cast<float>(scale);
-  if (VARIANT == LRTFC_QUANT_PORTABLE) {
-    p.inv = __fdiv_rn(1.0f, p.scale);
-  } else {
-    p.inv = p.scale == 0.0f ? 0.0f : static_cast<float>(1.0 / static_cast<double>(p.scale));
+  if (!AsymmetricParamsFast<kPortable>(mn, mx, HardwareReciprocal{}, &p)) {
+    p = AsymmetricParamsDivided<kPortable>(mn, mx);
   }
   return p;
 }
@@ -189,7 +164,10 @@ __device__ __forceinline__ int32_t RoundHalfAwayToInt(float x) {
 // reference then multiplies by infinity and converts what comes out, infinities and (for a zero)
 // NaN, to int8, which gives 0 on x86. A NaN multiplier makes every value of the row such a 0.
 __device__ __forceinline__ float SymmetricMultiplier(float scale_denom) {
-  const float mult = static_cast<float>(127.0 / static_cast<double>(scale_denom));
+  float mult;
+  if (!Quotient127Fast(scale_denom, HardwareReciprocal{}, &mult)) {
+    mult = static_cast<float>(127.0 / static_cast<double>(scale_denom));
+  }
   return mult == __builtin_inff() ? __builtin_nanf("") : mult;
 }
 
