@@ -77,6 +77,33 @@ def build_python_calls():
     return out
 
 
+def torch_tensors_name(torch_version):
+    """File name of the extension that allocates output tensors: it is bound to one torch and one
+    interpreter."""
+    tag = "".join(c if c.isalnum() else "_" for c in torch_version)
+    return "litert_amd_tensors-torch" + tag + sysconfig.get_config_var("EXT_SUFFIX")
+
+
+def build_torch_tensors():
+    """Output tensors for the Python ops without torch.empty's argument parsing (host code only).
+    Without torch's or the interpreter's headers there is none, and the ops use torch.empty."""
+    import torch
+    root = os.path.dirname(torch.__file__)
+    python = sysconfig.get_paths()["include"]
+    if not (os.path.exists(os.path.join(python, "Python.h")) and
+            os.path.exists(os.path.join(root, "include", "ATen", "ATen.h"))):
+        print("no headers of torch or Python: litert_amd_tensors is not built", flush=True)
+        return None
+    out = os.path.join(LIB, torch_tensors_name(torch.__version__))
+    _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-w",
+          "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI,
+          "-I" + os.path.join(root, "include"),
+          "-I" + os.path.join(root, "include", "torch", "csrc", "api", "include"), "-I" + python,
+          "-o", out, os.path.join(CSRC, "host", "torch_tensors.cc"), "-L" + os.path.join(root, "lib"),
+          "-lc10", "-ltorch_cpu", "-ltorch_python"])
+    return out
+
+
 def build_delegate():
     src_dir = os.path.join(CSRC, "delegate")
     if not os.path.isdir(src_dir):
@@ -99,7 +126,8 @@ def build_bench_probes():
 
 
 def build_all():
-    outs = [build_fc(), build_python_calls(), build_bench_probes(), build_delegate()]
+    outs = [build_fc(), build_python_calls(), build_torch_tensors(), build_bench_probes(),
+            build_delegate()]
     return [out for out in outs if out]
 
 
@@ -110,6 +138,7 @@ if __name__ == "__main__":
     if args.only == "fc":
         build_fc()
         build_python_calls()
+        build_torch_tensors()
     elif args.only == "delegate":
         build_delegate()
     elif args.only == "probes":

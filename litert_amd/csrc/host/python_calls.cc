@@ -79,6 +79,8 @@ PyMethodDef kMethods[] = {
     LRTFC_METHOD(lrtfc_activation_workspace_bytes),
     LRTFC_METHOD(lrtfc_fc_blockwise_int4_preferred_form),
     LRTFC_METHOD(lrtfc_fc_blockwise_int4_packed),
+    LRTFC_METHOD(lrtfc_batch_quantize_floats),
+    LRTFC_METHOD(lrtfc_fc_blockwise_int4_packed_quantized),
     LRTFC_METHOD(lrtfc_fc_blockwise_int4_gemm_workspace_bytes),
     LRTFC_METHOD(lrtfc_fc_blockwise_int4_gemm),
     LRTFC_METHOD(lrtfc_fc_blockwise_int4_gemm_nibbles),

@@ -8,11 +8,14 @@ ABI on torch's current stream). Tensors handed to `__call__` are torch CUDA tens
 torch is used only for device memory and streams.
 """
 import ctypes as C
+import importlib.machinery
+import importlib.util
+import os
 
 import numpy as np
 import torch
 
-from . import capi
+from . import build, capi
 
 _ACT = {"none": capi.ACT_NONE, "relu": capi.ACT_RELU, "relu_n1_to_1": capi.ACT_RELU_N1_TO_1,
         "relu6": capi.ACT_RELU6, "sign_bit": capi.ACT_SIGN_BIT}
@@ -51,6 +54,25 @@ def _dev(a, dtype):
     if isinstance(a, torch.Tensor):
         return a.to(device="cuda", dtype=dtype).contiguous()
     return torch.from_numpy(np.ascontiguousarray(a)).to(device="cuda", dtype=dtype).contiguous()
+
+
+def _empty_functions():
+    """empty(like, rows, columns) for int8 and float32 outputs on like's device: native ones where
+    they have been built for this torch and interpreter (a small call's host part 6.0 -> 5.0 us)."""
+    path = os.path.join(os.path.dirname(capi.LIB_PATH), build.torch_tensors_name(torch.__version__))
+    if os.path.exists(path):
+        loader = importlib.machinery.ExtensionFileLoader("litert_amd_tensors", path)
+        spec = importlib.util.spec_from_file_location("litert_amd_tensors", path, loader=loader)
+        module = importlib.util.module_from_spec(spec)
+        loader.exec_module(module)
+        return module.empty_int8, module.empty_float32
+
+    def empty(dtype):
+        return lambda like, rows, columns: torch.empty((rows, columns), dtype=dtype, device=like.device)
+    return empty(torch.int8), empty(torch.float32)
+
+
+_empty_int8, _empty_float32 = _empty_functions()
 
 
 def _ensure_init():
@@ -174,7 +196,7 @@ class FullyConnectedInt8:
         x = x.contiguous()
         batches = x.numel() // self.depth if self.depth else 0
         if out is None:
-            out = torch.empty((batches, self.out_depth), dtype=torch.int8, device=x.device)
+            out = _empty_int8(x, batches, self.out_depth)
         if self.packed_filter is not None:
             capi.check(capi.calls().lrtfc_fc_int8_packed(
                 _addr(x), _addr(self.packed_filter), _addr(self.bias), _addr(self.multipliers),
@@ -255,7 +277,7 @@ class FullyConnectedHybrid:
         x = x.contiguous()
         batches = x.numel() // self.depth
         if out is None:
-            out = torch.empty((batches, self.out_depth), dtype=torch.float32, device=x.device)
+            out = _empty_float32(x, batches, self.out_depth)
         if self.packed_filter is not None and batches > self._fused_max():
             return self.call_split(x, out)
         if self.packed_filter is not None:
@@ -289,7 +311,7 @@ class FullyConnectedHybrid:
         x = x.contiguous()
         batches = x.numel() // self.depth
         if out is None:
-            out = torch.empty((batches, self.out_depth), dtype=torch.float32, device=x.device)
+            out = _empty_float32(x, batches, self.out_depth)
         ws = self._workspace(batches)
         capi.check(capi.calls().lrtfc_fc_hybrid_packed_workspace(
             _addr(x), _addr(self.packed_filter), _addr(self.pcs), self.filter_scale,
@@ -360,7 +382,7 @@ class FullyConnectedBlockwiseInt4:
         x = x.contiguous()
         batches = x.numel() // self.depth
         if out is None:
-            out = torch.empty((batches, self.out_depth), dtype=torch.float32, device=x.device)
+            out = _empty_float32(x, batches, self.out_depth)
         if self._gemm_filter is None:
             self._gemm_filter = torch.empty(
                 lib.lrtfc_gemm_int4_blockwise_bytes(self.out_depth, self.depth), dtype=torch.uint8,
@@ -400,7 +422,7 @@ class FullyConnectedBlockwiseInt4:
         x = x.contiguous()
         batches = x.numel() // self.depth
         if out is None:
-            out = torch.empty((batches, self.out_depth), dtype=torch.float32, device=x.device)
+            out = _empty_float32(x, batches, self.out_depth)
         self._nibble_filter_tensor()
         need = capi.calls().lrtfc_fc_blockwise_int4_gemm_workspace_bytes(batches, self.depth)
         if self._gemm_ws is None or self._gemm_ws.numel() < need:
@@ -422,7 +444,7 @@ class FullyConnectedBlockwiseInt4:
             if form == capi.INT4_FORM_GEMM_INT8:
                 return self.call_gemm(x, out)
         if out is None:
-            out = torch.empty((batches, self.out_depth), dtype=torch.float32, device=x.device)
+            out = _empty_float32(x, batches, self.out_depth)
         if (self.retiled is not None and self.depth > self.FUSED_MAX_DEPTH
                 and batches > self.DEEP_FUSED_MAX_BATCHES):
             return self.call_split(x, out)
@@ -451,7 +473,7 @@ class FullyConnectedBlockwiseInt4:
         x = x.contiguous()
         batches = x.numel() // self.depth
         if out is None:
-            out = torch.empty((batches, self.out_depth), dtype=torch.float32, device=x.device)
+            out = _empty_float32(x, batches, self.out_depth)
         key = (batches, str(x.device))
         if getattr(self, "_split_key", None) != key:
             self._split_q = torch.empty((batches, self.depth), dtype=torch.int8, device=x.device)
@@ -459,12 +481,12 @@ class FullyConnectedBlockwiseInt4:
             self._split_zp = torch.zeros(batches, dtype=torch.int32, device=x.device)
             self._split_key = key
         q, sf, zp = self._split_q, self._split_sf, self._split_zp
-        capi.check(capi.load().lrtfc_batch_quantize_floats(_ptr(x), batches, self.depth, _ptr(q),
-                                                           _ptr(sf), _ptr(zp), 1, self.variant,
-                                                           _stream()))
-        capi.check(capi.load().lrtfc_fc_blockwise_int4_packed_quantized(
-            _ptr(q), _ptr(sf), _ptr(zp), _ptr(self.retiled), _ptr(self.kfsum), _ptr(self.bias),
-            _ptr(out), batches, self.depth, self.out_depth, _stream()))
+        capi.check(capi.calls().lrtfc_batch_quantize_floats(
+            _addr(x), batches, self.depth, _addr(q), _addr(sf), _addr(zp), 1, self.variant,
+            _call_stream()))
+        capi.check(capi.calls().lrtfc_fc_blockwise_int4_packed_quantized(
+            _addr(q), _addr(sf), _addr(zp), _addr(self.retiled), _addr(self.kfsum), _addr(self.bias),
+            _addr(out), batches, self.depth, self.out_depth, _call_stream()))
         return out
 
 
@@ -500,7 +522,7 @@ class FullyConnectedHybridInt4PerChannel:
         x = x.contiguous()
         batches = x.numel() // self.depth
         if out is None:
-            out = torch.empty((batches, self.out_depth), dtype=torch.float32, device=x.device)
+            out = _empty_float32(x, batches, self.out_depth)
         need = capi.calls().lrtfc_activation_workspace_bytes(batches, self.depth)
         if self._ws is None or self._ws.numel() < need:
             self._ws = torch.empty(need, dtype=torch.uint8, device="cuda")

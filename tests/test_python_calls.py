@@ -43,3 +43,30 @@ def test_without_the_extension_calls_go_through_ctypes(monkeypatch):
     status = calls.lrtfc_fc_int8_packed(None, 4096, None, None, None, 0, None, None, -1, 16, 16, 0, 0,
                                         0, 0, 0)
     assert status != capi.OK
+
+
+def test_output_tensors_are_torch_empty_s(monkeypatch):
+    """The native allocation and the one without it: shape, type, device, strides, no gradient; what
+    is no tensor or no count is refused."""
+    import os
+    import torch
+    from litert_amd import build
+    from litert_amd import fully_connected as fc
+    native = fc._empty_functions()
+    monkeypatch.setattr(build, "torch_tensors_name", lambda version: "missing.so")
+    plain = fc._empty_functions()
+    like = torch.zeros((3, 2), dtype=torch.float64, requires_grad=True)
+    for functions in (native, plain):
+        for empty, dtype in zip(functions, (torch.int8, torch.float32)):
+            for shape in ((1, 2048), (0, 7), (5, 0), (77, 5003)):
+                out = empty(like, *shape)
+                want = torch.empty(shape, dtype=dtype, device=like.device)
+                assert (out.shape, out.dtype, out.device, out.stride(), out.requires_grad) == \
+                    (want.shape, want.dtype, want.device, want.stride(), False)
+            with pytest.raises((TypeError, AttributeError)):
+                empty(None, 1, 2)
+            with pytest.raises(RuntimeError):
+                empty(like, -1, 2)
+    monkeypatch.undo()
+    if os.path.exists(os.path.join(os.path.dirname(capi.LIB_PATH), build.torch_tensors_name(torch.__version__))):
+        assert native[0].__name__ == "empty_int8"
