@@ -57,7 +57,9 @@ __device__ __forceinline__ void ForEachConst(std::integer_sequence<int, Is...>, 
 // workgroups); kWaveTiles: 32-channel MFMA tiles per wavefront (2 or 1); kRagged: the depth is no
 // multiple of 16, so the last piece of every row is shifted into place on its way to LDS (a
 // form of its own: a test for it inside the steps would break their straight line).
-template <Int8Epilogue EPI, int BM, int kWaveTiles, bool kRagged>
+// kSlots: steps ahead at which weights are requested, one register set each (rows: one step less ahead
+// of their way to LDS).
+template <Int8Epilogue EPI, int BM, int kWaveTiles, bool kRagged, int kSlots>
 __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args a) {
   constexpr int BN = kWaves * kWaveTiles * 32;  // output channels per workgroup
   constexpr int kStageBytes = BM * kXStride;
@@ -167,11 +169,12 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
   const int ragged_skip = RowPieceSkip(ragged_step * kStep + ld_chunk * 16, K);
   const int half_step = (slabs & 1) ? steps - 1 : -1;
 
-  // Weights: wring[step % 2] holds a step's operands; a piece is requested again, for two steps
-  // later, right after the last MFMA that reads it. Rows: xr[step % 2], requested three steps
-  // before their use, staged two steps before it, read into fa during the step before it.
-  i32x4 wring[2][kWaveTiles][kSub];
-  i32x4 xr[2][kXChunks];
+  // Weights: wring[step % kSlots] holds a step's operands; a piece is requested again, for kSlots
+  // steps later, right after the last MFMA that reads it. Rows: xr[step % kSlots], requested
+  // kSlots + 1 steps before their use, staged two steps before it, read into fa during the step
+  // before it.
+  i32x4 wring[kSlots][kWaveTiles][kSub];
+  i32x4 xr[kSlots][kXChunks];
   auto load_w_piece = [&](int step, auto slot, auto tile, auto sub) {
     constexpr int i = decltype(tile)::value, h = decltype(sub)::value;
     const int slab = min(2 * step + h / 2, slabs - 1);
@@ -188,10 +191,10 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
   };
   auto store_x_piece = [&](int step, auto set, auto piece) {
     constexpr int p = decltype(piece)::value;
-    i32x4 v = xr[decltype(set)::value][p];
+    i32x4 v = xr[decltype(set)::value % kSlots][p];
     if (kRagged) v = ShiftBytesDown(v, step == ragged_step ? ragged_skip : 0);
     if (upper_chunk && step == half_step) v = i32x4{0, 0, 0, 0};
-    *reinterpret_cast<i32x4*>(smem + decltype(set)::value * kStageBytes + st_off +
+    *reinterpret_cast<i32x4*>(smem + decltype(set)::value % 2 * kStageBytes + st_off +
                               p * 32 * kXStride) = v;
   };
   // Operand of batch tile j, sub-step h: lane L reads row 32 j + L % 32, bytes
@@ -217,18 +220,27 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
     }
   }
 
-  // Prologue: rows of steps 0 and 1 staged, those of step 2 requested, weights of steps 0 and 1
-  // requested, operands of step 0 read.
+  // Prologue: rows of steps 0 and 1 staged, those of the steps up to kSlots requested, weights of the
+  // first kSlots steps requested, operands of step 0 read.
   ForEachConst(kChunks, [&](auto p) { load_x_piece(0, C0{}, p); });
   ForEachConst(kChunks, [&](auto p) { load_x_piece(1, C1{}, p); });
   asm volatile("" ::: "memory");
-  ForEachConst(kTiles, [&](auto i) { ForEachConst(kSubs, [&](auto h) { load_w_piece(0, C0{}, i, h); }); });
-  ForEachConst(kTiles, [&](auto i) { ForEachConst(kSubs, [&](auto h) { load_w_piece(1, C1{}, i, h); }); });
+  constexpr auto kTurn = std::make_integer_sequence<int, kSlots>{};
+  ForEachConst(kTurn, [&](auto slot) {
+    ForEachConst(kTiles, [&](auto i) {
+      ForEachConst(kSubs, [&](auto h) { load_w_piece(decltype(slot)::value, slot, i, h); });
+    });
+  });
   asm volatile("" ::: "memory");
   ForEachConst(kChunks, [&](auto p) { store_x_piece(0, C0{}, p); });
   ForEachConst(kChunks, [&](auto p) { store_x_piece(1, C1{}, p); });
   asm volatile("" ::: "memory");
-  ForEachConst(kChunks, [&](auto p) { load_x_piece(2, C0{}, p); });
+  ForEachConst(std::make_integer_sequence<int, kSlots - 1>{}, [&](auto n) {
+    constexpr int kStepAhead = decltype(n)::value + 2;
+    ForEachConst(kChunks, [&](auto p) {
+      load_x_piece(kStepAhead, std::integral_constant<int, kStepAhead % kSlots>{}, p);
+    });
+  });
   asm volatile("" ::: "memory");
   if (tid < BN) chan_params[tid] = chan_p;
   // The short requantization (RequantizeShort) needs every channel of the tile to shift right by
@@ -248,13 +260,13 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
     for (int h = 0; h < kSub; ++h) fa[j][h] = read_frag(C0{}, j, h);
   }
 
-  // One depth step s (slot = s % 2). MFMA number m works on sub-step h = m / kHalf, channel tile
+  // One depth step s (slot = s % kSlots). MFMA number m works on sub-step h = m / kHalf, channel tile
   // i = (m % kHalf) / kBatchTiles, batch tile j = m % kBatchTiles; what follows it:
   //   * after the first MFMA that frees an operand of the rows: the barrier that publishes the
   //     rows of step s + 1 (staged at the end of step s - 1);
   //   * after the last use of fa[j][h] (i = last tile): its LDS read for step s + 1;
-  //   * after the last use of weight piece (i, h) (j = last batch tile): its load for step s + 2;
-  //   * spread over the step: the loads of the rows of step s + 3;
+  //   * after the last use of weight piece (i, h) (j = last batch tile): its load for step s + kSlots;
+  //   * spread over the step: the loads of the rows of step s + kSlots + 1;
   //   * from the middle of the step on, one every few MFMAs: the LDS writes of the rows of step
   //     s + 2, into the buffer whose readers all passed this step's barrier (behind the last
   //     MFMAs instead they are still in the LDS queue when the next step's barrier waits for
@@ -268,7 +280,9 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
   auto step_body = [&](int s, auto slot) {
     constexpr int kSlot = decltype(slot)::value;
     using Slot = std::integral_constant<int, kSlot>;
-    using Other = std::integral_constant<int, 1 - kSlot>;
+    using Next = std::integral_constant<int, (kSlot + 1) % kSlots>;
+    using AfterNext = std::integral_constant<int, kSlot + 2>;
+    using Other = std::integral_constant<int, 1 - kSlot % 2>;
     ForEachConst(std::make_integer_sequence<int, kMfmas>{}, [&](auto index) {
       constexpr int m = decltype(index)::value;
       constexpr int h = m / kHalf, i = (m % kHalf) / kBatchTiles, j = m % kBatchTiles;
@@ -283,29 +297,30 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
         __builtin_amdgcn_sched_barrier(0);
       }
       if constexpr (j == kBatchTiles - 1) {
-        load_w_piece(s + 2, Slot{}, std::integral_constant<int, i>{}, std::integral_constant<int, h>{});
+        load_w_piece(s + kSlots, Slot{}, std::integral_constant<int, i>{}, std::integral_constant<int, h>{});
         __builtin_amdgcn_sched_barrier(0);
       }
       if constexpr (m % (kMfmas / kXChunks) == 1) {
-        load_x_piece(s + 3, Other{}, std::integral_constant<int, m / (kMfmas / kXChunks)>{});
+        load_x_piece(s + kSlots + 1, Next{}, std::integral_constant<int, m / (kMfmas / kXChunks)>{});
         __builtin_amdgcn_sched_barrier(0);
       }
       if constexpr (m >= kStoreAt && (m - kStoreAt) % kStoreEvery == 0 &&
                     (m - kStoreAt) / kStoreEvery < kXChunks) {
-        store_x_piece(s + 2, Slot{},
+        store_x_piece(s + 2, AfterNext{},
                       std::integral_constant<int, (m - kStoreAt) / kStoreEvery>{});
         __builtin_amdgcn_sched_barrier(0);
       }
     });
   };
 
-  // Pairs of steps run without branches so that the two slots stay fixed registers.
+  // Whole turns of the slots run without branches so that they stay fixed registers.
   int s0 = 0;
-  for (; s0 + 2 <= steps; s0 += 2) {
-    step_body(s0, C0{});
-    step_body(s0 + 1, C1{});
+  for (; s0 + kSlots <= steps; s0 += kSlots) {
+    ForEachConst(kTurn, [&](auto slot) { step_body(s0 + decltype(slot)::value, slot); });
   }
-  if (s0 < steps) step_body(s0, C0{});
+  ForEachConst(std::make_integer_sequence<int, kSlots - 1>{}, [&](auto slot) {
+    if (s0 + decltype(slot)::value < steps) step_body(s0 + decltype(slot)::value, slot);
+  });
 
   // Epilogue. Register e of acc[i][j] holds channel 32 i + 8 * (e / 4) + 4 * (L / 32) + e % 4 of
   // the wavefront's 64 and batch row 32 j + L % 32 of the workgroup's 128: four groups (g) of
@@ -473,25 +488,26 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
   }
 }
 
-template <int BM, int kWaveTiles, bool kRagged>
+template <int BM, int kWaveTiles, bool kRagged, int kSlots>
 hipError_t LaunchForm(const FcInt8Args& a, Int8Epilogue epilogue, int grid, hipStream_t stream) {
-  if (epilogue == Int8Epilogue::kRequantize) {
-    hipLaunchKernelGGL((FcInt8PackedGemmKernel<Int8Epilogue::kRequantize, BM, kWaveTiles, kRagged>),
-                       dim3(grid), dim3(kThreads), 0, stream, a);
-  } else if (epilogue == Int8Epilogue::kHybrid) {
-    hipLaunchKernelGGL((FcInt8PackedGemmKernel<Int8Epilogue::kHybrid, BM, kWaveTiles, kRagged>),
-                       dim3(grid), dim3(kThreads), 0, stream, a);
-  } else {
-    hipLaunchKernelGGL((FcInt8PackedGemmKernel<Int8Epilogue::kHybrid4Bit, BM, kWaveTiles, kRagged>),
-                       dim3(grid), dim3(kThreads), 0, stream, a);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), 0, stream, a);
+    return hipGetLastError();
+  };
+  switch (epilogue) {
+    case Int8Epilogue::kRequantize:
+      return launch(FcInt8PackedGemmKernel<Int8Epilogue::kRequantize, BM, kWaveTiles, kRagged, kSlots>);
+    case Int8Epilogue::kHybrid:
+      return launch(FcInt8PackedGemmKernel<Int8Epilogue::kHybrid, BM, kWaveTiles, kRagged, kSlots>);
+    default:
+      return launch(FcInt8PackedGemmKernel<Int8Epilogue::kHybrid4Bit, BM, kWaveTiles, kRagged, kSlots>);
   }
-  return hipGetLastError();
 }
 
-template <int BM, int kWaveTiles>
+template <int BM, int kWaveTiles, int kSlots>
 hipError_t LaunchShape(const FcInt8Args& a, Int8Epilogue epilogue, int grid, hipStream_t stream) {
-  return a.depth % 16 ? LaunchForm<BM, kWaveTiles, true>(a, epilogue, grid, stream)
-                      : LaunchForm<BM, kWaveTiles, false>(a, epilogue, grid, stream);
+  return a.depth % 16 ? LaunchForm<BM, kWaveTiles, true, kSlots>(a, epilogue, grid, stream)
+                      : LaunchForm<BM, kWaveTiles, false, kSlots>(a, epilogue, grid, stream);
 }
 
 constexpr int kMinLargeTiles = 128;
@@ -502,6 +518,17 @@ int LargeTiles(const FcInt8Args& a) {
 int SmallTiles(const FcInt8Args& a) {
   return ((a.batches + 63) / 64) * ((a.out_depth + 127) / 128);
 }
+
+// 64 x 128 tiles, a workgroup at most per CU: a wavefront alone on its SIMD waits out every load that
+// it asked for less than a memory latency before, and a step of this tile is 256 matrix-core
+// cycles. With two register sets rows had one step to arrive in (a step took 0.42 us); four sets cost
+// the second workgroup of a CU nothing where there is none. Two sets -> four, us, filters in the
+// cache / from memory: 300 x 4096 -> 4096 15.9 -> 12.9 / 20.3 -> 16.6, 400 x 11008 -> 4096 37.2 -> 29.5
+// / 49.6 -> 38.4, 256 x 8192 -> 6144 27.8 -> 23.0 / 40.0 -> 32.5, 300 x 3072 -> 5120 13.6 -> 12.2 /
+// 17.2 -> 14.7. A short walk gains only on filters from memory (400 x 2048 -> 4096 8.0 -> 8.5 /
+// 10.1 -> 9.1, 400 x 512 -> 4096 5.2 -> 5.4 / 5.9 -> 6.0), and in more than one workgroup per CU they
+// hide each other's waits (300 x 8192 -> 8192, 320 workgroups, 39.7 -> 44.0).
+bool DeepRing(const FcInt8Args& a) { return a.depth > 2048 && SmallTiles(a) <= 256; }
 
 }  // namespace
 
@@ -523,8 +550,10 @@ hipError_t LaunchFcInt8PackedGemm(const FcInt8Args& a, Int8Epilogue epilogue, hi
   if (!FcInt8PackedGemmSupports(a)) return hipErrorNotSupported;
   switch (FcInt8PackedGemmForm(a)) {
     case Int8GemmForm::kSplit: return LaunchFcInt8SplitGemm(a, epilogue, stream);
-    case Int8GemmForm::kTiles128x256: return LaunchShape<128, 2>(a, epilogue, LargeTiles(a), stream);
-    default: return LaunchShape<64, 1>(a, epilogue, SmallTiles(a), stream);
+    case Int8GemmForm::kTiles128x256: return LaunchShape<128, 2, 2>(a, epilogue, LargeTiles(a), stream);
+    default:
+      return DeepRing(a) ? LaunchShape<64, 1, 4>(a, epilogue, SmallTiles(a), stream)
+                         : LaunchShape<64, 1, 2>(a, epilogue, SmallTiles(a), stream);
   }
 }
 

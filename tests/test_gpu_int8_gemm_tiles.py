@@ -1,0 +1,54 @@
+"""Forms of the tiled int8 GEMM, whole batches against the same rows in pieces of at most 32 (other
+kernels, which have oracle tests of their own) and, at the first and last rows, against the oracle."""
+import numpy as np
+import pytest
+
+import oracle
+from litert_amd import capi
+from litert_amd import workloads as wl
+from tests.test_gpu_parity import _bits_equal, _cuda, fc  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(op, x, want_rows):
+    import torch
+    whole = op(x)
+    pieces = torch.cat([op(x[i:i + 32]) for i in range(0, len(x), 32)])
+    assert torch.equal(whole.view(torch.uint8), pieces.view(torch.uint8))
+    rows = [0, len(x) - 1]
+    assert _bits_equal(whole[rows].cpu().numpy(), want_rows(rows))
+
+
+def _int8(fc, B, K, N):  # noqa: F811
+    import torch
+    c = wl.int8_fc(B, K, N, in_zp=-3, seed=B + K + N)
+    op = fc.FullyConnectedInt8(c["w"], c["bias"], float(c["in_scale"]), c["in_zp"], c["w_scale"],
+                               float(c["out_scale"]), c["out_zp"], activation="relu6")
+    mult, shift = oracle.fc_prepare_per_channel(float(c["in_scale"]), c["w_scale"], float(c["out_scale"]))
+    lo, hi = oracle.activation_range_int8(fc._act("relu6"), float(c["out_scale"]), c["out_zp"])
+    whole = op(_cuda(c["x"]))
+    pieces = torch.cat([op(_cuda(c["x"][i:i + 32])) for i in range(0, B, 32)])
+    assert torch.equal(whole, pieces)
+    rows = [0, B - 1]
+    want = oracle.fc_int8_per_channel(c["x"][rows], c["w"], c["bias"], mult, shift, 3, c["out_zp"], lo, hi)
+    assert np.array_equal(whole.cpu().numpy()[rows], want)
+
+
+def _hybrid(fc, B, K, N):  # noqa: F811
+    c = wl.hybrid_fc(B, K, N, seed=B + K + N)
+    bias = np.random.default_rng(K).standard_normal(N).astype(np.float32)
+    bias[::5] = -0.0
+    op = fc.FullyConnectedHybrid(c["w"], c["pcs"], bias=bias, activation="relu" if N % 2 else "none")
+    _check(op, _cuda(c["x"]), lambda rows: oracle.fc_hybrid(
+        c["x"][rows], c["w"], c["pcs"], bias=bias, activation=fc._act("relu" if N % 2 else "none")))
+
+
+# 64 x 128 tiles with four steps of operands in flight: walks of 4 n to 4 n + 3 steps of 128, an odd
+# number of 64 deep slabs, rows that end inside a 16-byte piece; the last depth with two steps.
+@pytest.mark.parametrize("B,K,N", [(130, 2048, 8200), (130, 2049, 8200), (193, 2176, 7000), (257, 2200, 6130),
+                                   (130, 2304, 8200), (193, 2431, 7001), (257, 2432, 6130), (300, 4100, 4099)])
+def test_64x128_tiles_deep_walks(fc, B, K, N):  # noqa: F811
+    assert capi.load().lrtfc_fc_int8_packed_kernel(B, K, N) == capi.INT8_KERNEL_TILES_64X128
+    _int8(fc, B, K, N)
+    _hybrid(fc, B, K, N)
