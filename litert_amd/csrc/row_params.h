@@ -121,7 +121,8 @@ LRTFC_ROW_PARAMS bool Quotient127Fast(float d, Reciprocal reciprocal, float* quo
   return d > 1e-30f && d < 1e30f;
 }
 LRTFC_ROW_PARAMS float Over127(float d) {
-  return static_cast<float>(DivideByConstant(static_cast<double>(d), 127.0, 1.0 / 127.0));
+  const float q = static_cast<float>(DivideByConstant(static_cast<double>(d), 127.0, 1.0 / 127.0));
+  return d > 3.402823466e38f ? d : q;  // infinity has no remainder to correct by
 }
 
 }  // namespace lrtfc

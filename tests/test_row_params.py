@@ -87,7 +87,8 @@ def test_short_form_gives_the_divided_forms_bits(host, portable):
 
 
 def test_quotients_with_127(host):
-    bits = np.arange(1, 0x7F800000, 1511, dtype=np.uint32)  # every exponent, subnormals too
+    # every exponent, subnormals, the largest value and infinity
+    bits = np.append(np.arange(1, 0x7F800000, 1511), [0x7F7FFFFF, 0x7F800000]).astype(np.uint32)
     d = bits.view(np.float32)
     out = np.empty(d.size, np.uint8)
     eps = np.random.default_rng(3).uniform(-2.0 ** -20, 2.0 ** -20, d.size)
