@@ -150,7 +150,8 @@ int lrtfc_fc_hybrid_fused_max_batches(int depth, int out_depth);
  * of lrtfc_fc_hybrid_packed_workspace): for profiles, and for tests that are meant for one of them.
  * All give the same bits. The matrix-core GEMV takes 16 rows a pass, or up to 32 as two row tiles;
  * ROWS streams the filter once for up to 128; SPLIT deals the depth of small tiles to the wavefronts
- * of a workgroup; the rest are GEMM tiles of rows x channels. Pure host function. */
+ * of a workgroup; the rest are the GEMM on tiles of rows x channels, TILES_64X128 standing for all
+ * those smaller than 128 x 256 (64 x 128 and 128 x 128). Pure host function. */
 enum {
   LRTFC_INT8_KERNEL_GEMV = 0,
   LRTFC_INT8_KERNEL_GEMV_TWO_TILES = 1,

@@ -378,7 +378,7 @@ int lrtfc_fc_int8_packed_kernel(int batches, int depth, int out_depth) {
   }
   switch (lrtfc::FcInt8PackedGemmForm(a)) {
     case lrtfc::Int8GemmForm::kSplit: return LRTFC_INT8_KERNEL_SPLIT;
-    case lrtfc::Int8GemmForm::kTiles64x128: return LRTFC_INT8_KERNEL_TILES_64X128;
+    case lrtfc::Int8GemmForm::kSmallerTiles: return LRTFC_INT8_KERNEL_TILES_64X128;
     default: return LRTFC_INT8_KERNEL_TILES_128X256;
   }
 }

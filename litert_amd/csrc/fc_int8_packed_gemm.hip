@@ -19,8 +19,8 @@
 // and one barrier, all dealt out singly between the MFMAs: a wavefront is alone on its SIMD,
 // so whatever holds up its instruction stream idles the matrix pipe.
 // Launches that this 128 x 256 tile would cut into fewer workgroups than half the chip's CUs
-// (batches of a few dozen to a few hundred rows) run the same kernel with 64 rows x 128
-// channels per workgroup (32 channels per wavefront).
+// (batches of a few dozen to a few hundred rows), and short walks, run the same kernel with 64 or 128
+// rows x 128 channels per workgroup (32 channels per wavefront).
 //
 // The outputs of a tile are put together in LDS (the row buffers, free by then) and stored in
 // 16-byte pieces, whole cache lines per row.
@@ -511,9 +511,13 @@ hipError_t LaunchShape(const FcInt8Args& a, Int8Epilogue epilogue, int grid, hip
 }
 
 constexpr int kMinLargeTiles = 128;
+constexpr int kCus = 256;
 
 int LargeTiles(const FcInt8Args& a) {
   return ((a.batches + 127) / 128) * ((a.out_depth + 255) / 256);
+}
+int SquareTiles(const FcInt8Args& a) {
+  return ((a.batches + 127) / 128) * ((a.out_depth + 127) / 128);
 }
 int SmallTiles(const FcInt8Args& a) {
   return ((a.batches + 63) / 64) * ((a.out_depth + 127) / 128);
@@ -528,7 +532,19 @@ int SmallTiles(const FcInt8Args& a) {
 // 17.2 -> 14.7. A short walk gains only on filters from memory (400 x 2048 -> 4096 8.0 -> 8.5 /
 // 10.1 -> 9.1, 400 x 512 -> 4096 5.2 -> 5.4 / 5.9 -> 6.0), and in more than one workgroup per CU they
 // hide each other's waits (300 x 8192 -> 8192, 320 workgroups, 39.7 -> 44.0).
-bool DeepRing(const FcInt8Args& a) { return a.depth > 2048 && SmallTiles(a) <= 256; }
+bool DeepRing(const FcInt8Args& a) { return a.depth > 2048 && SmallTiles(a) <= kCus; }
+
+// Of the launches on smaller tiles: 128 x 128 moves two thirds of the bytes per product that 64 x 128
+// does. Among those that 128 x 256 would give half the chip or more, all but the short walks in one
+// round (see FcInt8PackedGemmForm). Below, where it makes one round of what 64 x 128 takes more than one
+// for (us, 64 x 128 -> 128 x 128, filters in the cache / from memory): 350 x 7792 -> 6425 50.6 -> 35.6
+// / 50.1 -> 47.6, 494 x 7376 -> 4530 36.5 -> 30.7 / 48.8 -> 43.5, 256 x 4096 -> 14336 22.8 -> 21.6 / 30.8
+// -> 28.1; least 1110 x 2240 -> 2805 14.9 -> 14.0 / 15.9 -> 15.3. (Shorter walks: 819 x 1392 -> 4231
+// 11.3 -> 12.2.)
+bool TakesSquareTiles(const FcInt8Args& a) {
+  if (LargeTiles(a) >= kMinLargeTiles) return LargeTiles(a) > kCus || a.depth > 2048;
+  return a.depth >= 2048 && SmallTiles(a) > kCus && SquareTiles(a) <= kCus;
+}
 
 }  // namespace
 
@@ -538,12 +554,31 @@ bool FcInt8PackedGemmSupports(const FcInt8Args& a) {
 }
 
 // 128 x 256 tiles move the fewest bytes per MFMA; a launch they would cut into fewer workgroups than
-// half the chip's CUs takes 64 x 128 tiles instead (four times as many), or, where those leave it
-// idle too, small tiles with the depth split over the wavefronts.
+// half the chip's CUs takes smaller tiles instead, or, where those leave it idle too, small tiles
+// with the depth split over the wavefronts. Above that line smaller tiles win where the walk is
+// short, because of a large tile's prologue and epilogue (9 us of a workgroup's time, and no second
+// workgroup on its CU to hide them), and where large tiles make exactly half a round.
+// 128 sizes between 100 x 2048 -> 320 and 2048 x 4096 -> 14336 measured on every form, filters in the
+// cache / from memory (us, 128 x 256 -> chosen):
+//   more than a round, depth 512 to 2048, to 128 x 128: 2048 x 1024 -> 14336 52.6 -> 47.5 / 57.5 -> 51.5,
+//     700 x 1024 -> 14336 24.7 -> 20.8 / 27.7 -> 23.3, 1715 x 560 -> 15924 52.4 -> 41.9 / 53.1 -> 42.3;
+//     least 1274 x 1712 -> 8524 35.1 -> 33.9 / 36.8 -> 36.0. Float outputs gain more: hybrid
+//     2048 x 1024 -> 14336 76 -> 63 / 83 -> 73. (Deeper: 769 x 2272 -> 14793 47 -> 50.)
+//   a round at most, depth 512 to 768, to 64 x 128: 1506 x 672 -> 2567 13.8 -> 8.5 / 14.5 -> 9.2,
+//     1806 x 608 -> 2575 13.4 -> 10.5 / 14.2 -> 11.3; least 1067 x 544 -> 6582 14.3 -> 12.9 / 15.3 -> 14.0.
+//     (Deeper: 750 x 912 -> 8538 16.5 -> 20.8.)
+//   half a round, depth above 2048, to one round of 128 x 128: 1000 x 4096 -> 4096 26.0 -> 22.4 / 30.2 -> 25.3.
+// Shallower launches than 512 are not in those figures and stay.
 Int8GemmForm FcInt8PackedGemmForm(const FcInt8Args& a) {
-  if (LargeTiles(a) >= kMinLargeTiles) return Int8GemmForm::kTiles128x256;
+  const int large = LargeTiles(a);
+  if (large >= kMinLargeTiles) {
+    const bool smaller = large > kCus ? a.depth >= 512 && a.depth <= 2048
+                                      : (a.depth >= 512 && a.depth <= 768) ||
+                                            (a.depth > 2048 && SquareTiles(a) <= kCus);
+    return smaller ? Int8GemmForm::kSmallerTiles : Int8GemmForm::kTiles128x256;
+  }
   return FcInt8SplitGemmBeatsTiles(a, SmallTiles(a)) ? Int8GemmForm::kSplit
-                                                     : Int8GemmForm::kTiles64x128;
+                                                     : Int8GemmForm::kSmallerTiles;
 }
 
 hipError_t LaunchFcInt8PackedGemm(const FcInt8Args& a, Int8Epilogue epilogue, hipStream_t stream) {
@@ -552,6 +587,7 @@ hipError_t LaunchFcInt8PackedGemm(const FcInt8Args& a, Int8Epilogue epilogue, hi
     case Int8GemmForm::kSplit: return LaunchFcInt8SplitGemm(a, epilogue, stream);
     case Int8GemmForm::kTiles128x256: return LaunchShape<128, 2, 2>(a, epilogue, LargeTiles(a), stream);
     default:
+      if (TakesSquareTiles(a)) return LaunchShape<128, 1, 2>(a, epilogue, SquareTiles(a), stream);
       return DeepRing(a) ? LaunchShape<64, 1, 4>(a, epilogue, SmallTiles(a), stream)
                          : LaunchShape<64, 1, 2>(a, epilogue, SmallTiles(a), stream);
   }

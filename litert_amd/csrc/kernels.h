@@ -146,7 +146,7 @@ bool FcInt8PackedGemvTakesRowsInOnePass(const FcInt8Args& a);
 bool FcInt8RowsGemvTakes(const FcInt8Args& a);
 hipError_t LaunchFcInt8RowsGemv(const FcInt8Args& a, Int8Epilogue epilogue, hipStream_t stream);
 bool FcInt8PackedGemmSupports(const FcInt8Args& a);
-enum class Int8GemmForm { kSplit, kTiles64x128, kTiles128x256 };
+enum class Int8GemmForm { kSplit, kSmallerTiles, kTiles128x256 };
 Int8GemmForm FcInt8PackedGemmForm(const FcInt8Args& a);
 hipError_t LaunchFcInt8PackedGemm(const FcInt8Args& a, Int8Epilogue epilogue, hipStream_t stream);
 // The same for launches that leave the chip idle in those tiles (fc_int8_split_gemm.hip): small tiles,

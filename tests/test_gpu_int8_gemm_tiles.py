@@ -52,3 +52,23 @@ def test_64x128_tiles_deep_walks(fc, B, K, N):  # noqa: F811
     assert capi.load().lrtfc_fc_int8_packed_kernel(B, K, N) == capi.INT8_KERNEL_TILES_64X128
     _int8(fc, B, K, N)
     _hybrid(fc, B, K, N)
+
+
+# 128 x 128 tiles: in place of 64 x 128 in more than a round (even and odd numbers of steps and slabs, rows
+# that end inside a piece), at the edge of what one round of them holds, in short walks of more than a
+# round of 128 x 256, and where those make half a round; and 64 x 128 in short walks within a round.
+@pytest.mark.parametrize("B,K,N", [(130, 2048, 11300), (192, 2049, 11300), (300, 2176, 6600), (200, 2200, 16383),
+                                   (1100, 512, 7300), (1100, 515, 7299), (1025, 2048, 8190),
+                                   (1000, 2100, 4001), (1100, 512, 4000), (1100, 760, 4003)])
+def test_tiles_between(fc, B, K, N):  # noqa: F811
+    assert capi.load().lrtfc_fc_int8_packed_kernel(B, K, N) == capi.INT8_KERNEL_TILES_64X128
+    _int8(fc, B, K, N)
+    if B * K * N < 6e9:
+        _hybrid(fc, B, K, N)
+
+
+# The other side of each line: 128 x 256 tiles.
+@pytest.mark.parametrize("B,K,N", [(1100, 511, 7300), (1100, 2049, 7400), (1100, 769, 4000), (1000, 2048, 4001)])
+def test_tiles_between_other_side(fc, B, K, N):  # noqa: F811
+    assert capi.load().lrtfc_fc_int8_packed_kernel(B, K, N) == capi.INT8_KERNEL_TILES_128X256
+    _int8(fc, B, K, N)
