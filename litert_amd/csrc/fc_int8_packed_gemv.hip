@@ -1174,8 +1174,12 @@ hipError_t LaunchPackInt8Filter(const int8_t* filter, int out_depth, int depth, 
 
 int FcInt8PackedGemvFusedMaxRows(int depth) {
   // Eight rows where a wavefront can hold a whole row (the register-resident form: one wavefront
-  // of eight per row); four on deeper rows, which every wavefront of a workgroup quantizes.
-  return (depth >= 4 && depth <= kFusedRowMaxDepth) ? kFusedMaxRows : 4;
+  // of eight per row). Deeper rows are quantized by every workgroup, one after the other: two of up
+  // to 8192, one beyond (us fused / quantizer and product in two launches: 5120 -> 2048 at 2 / 3 / 4
+  // rows 7.6, 11.7, 13.7 / 8.0, 8.1, 8.9; 8192 -> 4096 at 2 / 4 10.0, 19.5 / 9.7, 10.5, the second launch
+  // 3 us of the host's time; 16384 -> 2048 at 1 / 2 / 4 11.0, 20.8, 32.6 / 13.0, 13.6, 14.9).
+  if (depth >= 4 && depth <= kFusedRowMaxDepth) return kFusedMaxRows;
+  return depth < 4 ? 4 : depth <= 8192 ? 2 : 1;
 }
 
 bool FcInt8PackedGemvTakesRowsInOnePass(const FcInt8Args& a) {
