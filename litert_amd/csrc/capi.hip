@@ -1129,13 +1129,15 @@ int lrtfc_fc_blockwise_int4_preferred_form(int batches, int depth, int out_depth
   // and 20 us on the int8 copy), and where output tiles are so few that it gives each four
   // wavefronts (us, streaming or int8-expanded form -> here: 5 x 4096 -> 4096 13.2 -> 10.4,
   // 16 x 8192 -> 2048 20.8 -> 16.2, 64 x 4096 -> 1024 13.5 -> 10.5, 128 x 1024 -> 1024 8.0 -> 7.2);
-  // the int8-expanded one from 16 rows on otherwise. Depths beyond 8192 keep the answer they had
-  // before the four-wavefront tiles: callers re-tile their filters for it, and it is part of what the
-  // tests of this function fix (16 x 16384 -> 2048: 26.8 us there, 48.8 on the int8 copy).
+  // the int8-expanded one from 16 rows on otherwise. Deeper than 8192 the streaming kernel in passes is
+  // worse still (us, there -> here: 5 x 8448 -> 4096 22.3 -> 17.4, 12 x 11008 -> 4096 59 -> 20.7) and
+  // the int8 copy no better (16 x 14336 -> 2048 31.4 -> 23.9, from memory 42.1 -> 24.7). Beyond 14336
+  // five to eight rows are faster streamed (8 x 16352 -> 2048 24.3, here 26.8), and the answers
+  // there are as they were: callers re-tile their filters for them (16 x 16384 -> 2048: 26.8 us here).
   const int channel_tiles = (out_depth + 15) / 16;
   if (batches <= 4) return LRTFC_INT4_FORM_DECODE;
-  if (depth <= 8192 && ((batches <= 32 && channel_tiles >= 512) ||
-                        lrtfc::FcInt4NibbleGemmFewTiles(batches, out_depth))) {
+  if (depth <= 14336 && ((batches <= 32 && channel_tiles >= 512) ||
+                         lrtfc::FcInt4NibbleGemmFewTiles(batches, out_depth))) {
     return LRTFC_INT4_FORM_GEMM_NIBBLES;
   }
   return batches >= 16 ? LRTFC_INT4_FORM_GEMM_INT8 : LRTFC_INT4_FORM_DECODE;

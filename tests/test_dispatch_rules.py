@@ -24,3 +24,30 @@ def test_deep_hybrid_rows_fused_and_in_two_launches(rows, depth, channels, monke
     assert np.array_equal(op(x).cpu().numpy().view(np.uint32), want)
     monkeypatch.setattr(fc.FullyConnectedHybrid, "FUSED_MAX_BATCHES", 100)
     assert np.array_equal(op(x).cpu().numpy().view(np.uint32), want)
+
+
+D, N, I = capi.INT4_FORM_DECODE, capi.INT4_FORM_GEMM_NIBBLES, capi.INT4_FORM_GEMM_INT8
+
+
+@pytest.mark.parametrize("rows,depth,channels,form", [
+    (4, 8224, 1000, D), (5, 8224, 1000, N), (32, 14336, 8192, N), (33, 14336, 8192, I), (64, 11008, 2048, N),
+    (65, 11008, 2048, I), (5, 14368, 1000, D), (16, 14368, 1000, I), (5, 8224, 8200, N)])
+def test_blockwise_int4_form_of_deep_filters(rows, depth, channels, form):
+    assert capi.load().lrtfc_fc_blockwise_int4_preferred_form(rows, depth, channels) == form
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,depth,channels", [(5, 8224, 40), (12, 11008, 50), (33, 8960, 100), (16, 14336, 33),
+                                                 (7, 8224, 8200), (17, 9216, 8193)])
+def test_blockwise_int4_deep_filters_on_the_resident_form(rows, depth, channels):
+    import numpy as np
+    import torch
+    import oracle
+    from litert_amd import fully_connected as fc
+    from litert_amd import workloads as wl
+    assert capi.load().lrtfc_fc_blockwise_int4_preferred_form(rows, depth, channels) == N
+    c = wl.blockwise_int4_fc(rows, depth, channels, seed=depth, lo=-8, hi=7)
+    op = fc.FullyConnectedBlockwiseInt4(c["packed"], c["scales"], depth, 32)
+    want = oracle.fc_blockwise_int4(c["x"], c["packed"], channels, c["scales"].view(np.uint16), 32)
+    got = op(torch.from_numpy(c["x"]).cuda()).cpu().numpy()
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
