@@ -400,7 +400,9 @@ int lrtfc_fc_hybrid_int4_per_channel_packed(const float* input, const int8_t* pa
  * ([out_depth, depth / 2] bytes, low nibble first; even depth) into
  * lrtfc_packed_int4_per_channel_bytes(out_depth, depth) bytes, 16-byte aligned. Meant for
  * decode batches (it makes one pass over the filter per 16 rows); prefill batches are faster on
- * the int8 copy above. Results are identical bit for bit. */
+ * the int8 copy above, from one more than lrtfc_fc_hybrid_int4_per_channel_nibbles_max_batches on (a
+ * pure host function). Results are identical bit for bit. */
+int lrtfc_fc_hybrid_int4_per_channel_nibbles_max_batches(int depth, int out_depth);
 size_t lrtfc_packed_int4_per_channel_bytes(int out_depth, int depth);
 int lrtfc_pack_int4_per_channel(const uint8_t* packed_filter, int out_depth, int depth,
                                 uint8_t* retiled_filter, void* stream);

@@ -1008,6 +1008,19 @@ int lrtfc_pack_int4_per_channel(const uint8_t* packed_filter, int out_depth, int
                  "per-channel int4 filter re-tiling");
 }
 
+int lrtfc_fc_hybrid_int4_per_channel_nibbles_max_batches(int depth, int out_depth) {
+  // One pass of the nibble kernel takes 16 rows, as long as 64 KB of LDS hold them; beyond either it
+  // walks a ring of loads or the filter again, and the int8 copy wins though twice the bytes (us,
+  // nibbles / int8, filters in the cache): 17 x 4096 -> 4096 13.0 / 8.0, 17 x 4096 -> 14336 17.1 / 14.7,
+  // 32 x 1024 -> 1024 9.7 / 6.3, 16 x 5120 -> 2048 17.8 / 8.9, 10 x 8192 -> 4096 15.6 / 10.7, 16 x 11008 ->
+  // 4096 29.9 / 13.7, 32 x 16384 -> 2048 64.5 / 17.7; within both, 16 x 4096 -> 14336 11.0 / 13.5,
+  // 12 x 5120 -> 8192 11.1 / 12.4, 8 x 8192 -> 1024 9.4 / 10.0. From memory the line is the same. Filters
+  // of fewer than 128 channels, a handful of workgroups on either, keep to the one layout they had.
+  if (out_depth < 128 || depth <= 0) return 32;
+  const int fit = 65536 / depth;
+  return fit > 16 ? 16 : fit < 4 ? 4 : fit;
+}
+
 int lrtfc_fc_hybrid_int4_per_channel_nibbles(const float* input, const uint8_t* retiled_filter,
                                              const float* per_channel_scales, float filter_scale,
                                              const float* bias, float* output, int batches,

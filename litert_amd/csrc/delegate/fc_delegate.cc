@@ -568,9 +568,6 @@ struct FcNode {
 constexpr int kInt4FusedMaxDepth = 4096;
 constexpr int kInt4DeepFusedMaxBatches = 2;
 constexpr int kInt4GroupedMaxOutDepth = 511 * 16;  // wider ones fill the chip by themselves from five rows on
-// Up to this many rows a per-channel int4 node streams its filter as nibbles (one pass per 16
-// rows); above, the MFMA GEMM on the int8 expansion streams it once.
-constexpr int kInt4PerChannelNibbleMaxBatches = 32;
 
 // Up to this many bytes of host outputs per partition are written by the kernels directly into
 // page-locked host memory instead of being copied there afterwards. The invariant this rests on:
@@ -1097,7 +1094,8 @@ TfLiteStatus PrepareNode(TfLiteContext* ctx, PartitionKernel* k, FcNode* n) {
     n->per_channel = fq->scale->size > 1;
     n->filter_scale = fq->scale->data[0];
     n->use_retiled = true;
-    n->nibble_layout = n->batches <= kInt4PerChannelNibbleMaxBatches;
+    n->nibble_layout =
+        n->batches <= lrtfc_fc_hybrid_int4_per_channel_nibbles_max_batches(n->depth, n->out_depth);
     if (weights > 0 && !(n->nibble_layout ? n->have_nibbles : n->have_retiled)) {
       DeviceBuffer nibbles;
       RETURN_IF_HIP(ctx, nibbles.Upload(filter.data.raw, (weights + 1) / 2, s));

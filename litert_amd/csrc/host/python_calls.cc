@@ -84,6 +84,7 @@ PyMethodDef kMethods[] = {
     LRTFC_METHOD(lrtfc_fc_blockwise_int4_gemm_workspace_bytes),
     LRTFC_METHOD(lrtfc_fc_blockwise_int4_gemm),
     LRTFC_METHOD(lrtfc_fc_blockwise_int4_gemm_nibbles),
+    LRTFC_METHOD(lrtfc_fc_hybrid_int4_per_channel_nibbles_max_batches),
     LRTFC_METHOD(lrtfc_fc_hybrid_int4_per_channel_nibbles),
     LRTFC_METHOD(lrtfc_fc_hybrid_int4_per_channel_packed),
     {nullptr, nullptr, 0, nullptr},

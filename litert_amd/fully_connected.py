@@ -516,7 +516,14 @@ class FullyConnectedHybridInt4PerChannel:
         self.activation = _act(activation)
         self._ws = None
 
-    NIBBLE_MAX_BATCHES = 32  # above: one pass of the MFMA GEMM over the int8 copy is cheaper
+    # Above this many rows one pass of a matrix-core kernel over the int8 copy is cheaper: None = what
+    # the library says for the shape (lrtfc_fc_hybrid_int4_per_channel_nibbles_max_batches).
+    NIBBLE_MAX_BATCHES = None
+
+    def _nibble_max(self):
+        if self.NIBBLE_MAX_BATCHES is not None:
+            return self.NIBBLE_MAX_BATCHES
+        return capi.calls().lrtfc_fc_hybrid_int4_per_channel_nibbles_max_batches(self.depth, self.out_depth)
 
     def __call__(self, x, out=None, force_int8=False):
         x = x.contiguous()
@@ -527,7 +534,7 @@ class FullyConnectedHybridInt4PerChannel:
         if self._ws is None or self._ws.numel() < need:
             self._ws = torch.empty(need, dtype=torch.uint8, device="cuda")
         lib = capi.load()
-        if batches <= self.NIBBLE_MAX_BATCHES and not force_int8:
+        if not force_int8 and batches <= self._nibble_max():
             if self._retiled_nibbles is None:
                 self._retiled_nibbles = torch.empty(
                     lib.lrtfc_packed_int4_per_channel_bytes(self.out_depth, self.depth),

@@ -51,3 +51,29 @@ def test_blockwise_int4_deep_filters_on_the_resident_form(rows, depth, channels)
     want = oracle.fc_blockwise_int4(c["x"], c["packed"], channels, c["scales"].view(np.uint16), 32)
     got = op(torch.from_numpy(c["x"]).cuda()).cpu().numpy()
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("depth,rows", [(2, 16), (4096, 16), (4098, 15), (5120, 12), (8192, 8), (8194, 7), (16384, 4),
+                                        (16386, 4), (60000, 4)])
+def test_per_channel_int4_rows_on_nibbles(depth, rows):
+    assert capi.load().lrtfc_fc_hybrid_int4_per_channel_nibbles_max_batches(depth, 128) == rows
+    assert capi.load().lrtfc_fc_hybrid_int4_per_channel_nibbles_max_batches(depth, 127) == 32
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("depth,channels", [(34, 20), (1030, 131), (4096, 300), (5122, 128), (11010, 129)])
+def test_per_channel_int4_rows_around_the_line(depth, channels):
+    import numpy as np
+    import torch
+    import oracle
+    from litert_amd import fully_connected as fc
+    rng = np.random.default_rng(depth)
+    packed = rng.integers(0, 256, (channels, depth // 2), dtype=np.uint8)
+    scales = rng.uniform(0.01, 0.1, channels).astype(np.float32)
+    x = rng.standard_normal((33, depth)).astype(np.float32)
+    want = oracle.fc_hybrid_int4_per_channel(x, packed, channels, scales).view(np.uint32)
+    op = fc.FullyConnectedHybridInt4PerChannel(packed, depth, scales)
+    line = op._nibble_max()
+    for rows in (line, line + 1, 16, 17, 32, 33):
+        xs = torch.from_numpy(x[:rows]).cuda()
+        assert np.array_equal(op(xs).cpu().numpy().view(np.uint32), want[:rows])
