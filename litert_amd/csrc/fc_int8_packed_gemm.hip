@@ -121,7 +121,9 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
     const bool mine = tid < BN && n0 + tid < N && a.bias_f32 != nullptr &&
                       IsNegativeZero(__int_as_float(chan_p[1]));
     if (__syncthreads_or(mine)) {
-      zero_input = WorkgroupAllZeroInt8(a.input, static_cast<size_t>(M) * K);
+      zero_input = a.whole_input
+                       ? WorkgroupAllZeroInt8(a.whole_input, static_cast<size_t>(a.whole_batches) * K)
+                       : WorkgroupAllZeroInt8(a.input, static_cast<size_t>(M) * K);
     }
   }
 
@@ -581,8 +583,44 @@ Int8GemmForm FcInt8PackedGemmForm(const FcInt8Args& a) {
                                                      : Int8GemmForm::kSmallerTiles;
 }
 
+namespace {
+
+// A few tiles more than one per CU cost a second round, nearly all of it on an idle chip. The rows of that
+// tail go in a launch of their own then, on the tiles that suit them: the number of rows the first
+// launch keeps. For tails up to a quarter of a round and walks deeper than 2048 (shorter ones are on
+// smaller tiles), us, one launch -> two: 2048 x 7808 -> 4352, 272 tiles, 103 -> 84-92; 2048 x 4096 -> 4352
+// 59.4 -> 50.8; 1100 x 4096 -> 8192, 288 tiles, 60.8 -> 50.2; 1800 x 4096 -> 5120, 300 tiles, 58.9 -> 50.2;
+// least 1614 x 5680 -> 5909, 312 tiles, 83 -> 81. A larger tail gains less (800 x 4096 -> 12288, 336
+// tiles, 61.8 -> 59.6), one behind two or three rounds loses (2048 x 4096 -> 8448 96.6 -> 104, 2048 x 2560 ->
+// 12800 93 -> 107: the last tiles of a round overlap the first of the next).
+int RowsOfWholeRound(const FcInt8Args& a) {
+  const int tiles = LargeTiles(a);
+  if (a.depth <= 2048 || tiles <= kCus || tiles > kCus + kCus / 4) return a.batches;
+  const int tiles_n = (a.out_depth + 255) / 256;
+  const int kept = kCus / tiles_n;  // rows of tiles
+  if (kept * tiles_n < kCus - kCus / 16) return a.batches;
+  return min(kept * 128, a.batches);
+}
+
+}  // namespace
+
 hipError_t LaunchFcInt8PackedGemm(const FcInt8Args& a, Int8Epilogue epilogue, hipStream_t stream) {
   if (!FcInt8PackedGemmSupports(a)) return hipErrorNotSupported;
+  if (const int kept = RowsOfWholeRound(a); kept < a.batches) {
+    FcInt8Args part = a;
+    part.whole_input = a.whole_input ? a.whole_input : a.input;
+    part.whole_batches = a.whole_input ? a.whole_batches : a.batches;
+    part.batches = kept;
+    if (hipError_t err = LaunchShape<128, 2, 2>(part, epilogue, LargeTiles(part), stream)) return err;
+    const size_t rows = kept, out = rows * a.out_depth;
+    part.batches = a.batches - kept;
+    part.input += rows * a.depth;
+    if (part.output_i8) part.output_i8 += out;
+    if (part.output_f32) part.output_f32 += out;
+    if (part.scaling_factors) part.scaling_factors += rows;
+    if (part.zero_points) part.zero_points += rows;
+    return LaunchFcInt8PackedGemm(part, epilogue, stream);
+  }
   switch (FcInt8PackedGemmForm(a)) {
     case Int8GemmForm::kSplit: return LaunchFcInt8SplitGemm(a, epilogue, stream);
     case Int8GemmForm::kTiles128x256: return LaunchShape<128, 2, 2>(a, epilogue, LargeTiles(a), stream);

@@ -156,7 +156,9 @@ void FcInt8SplitGemmKernel(FcInt8Args a, int tiles, bool rows_inner, int total, 
   bool zero_input = false;
   if (EPI == Int8Epilogue::kHybrid && a.zero_input_exit && a.bias_f32 != nullptr) {
     if (__syncthreads_or(n0 + local_n < N && IsNegativeZero(__int_as_float(p1)))) {
-      zero_input = WorkgroupAllZeroInt8(a.input, static_cast<size_t>(M) * K);
+      zero_input = a.whole_input
+                       ? WorkgroupAllZeroInt8(a.whole_input, static_cast<size_t>(a.whole_batches) * K)
+                       : WorkgroupAllZeroInt8(a.input, static_cast<size_t>(M) * K);
     }
   }
   for (int i = tid; i < BM * kSumStride; i += kThreads) sums[i] = 0;

@@ -68,6 +68,10 @@ struct FcInt8Args {
   // Non-zero: EvalHybridDense semantics for a whole-zero input (output = activation(bias), no
   // product added; fully_connected.cc:789-795). Zero: MatrixBatchVectorMultiplyAccumulate as is.
   int zero_input_exit;
+  // The rows that decide this where a launch computes a part of them (null: its own). Set by
+  // LaunchFcInt8PackedGemm for itself and the split tiles; no other kernel reads them.
+  const int8_t* whole_input;
+  int whole_batches;
   // Non-zero: the arithmetic of the hybrid BATCH_MATMUL kernel (reference/batch_matmul.h:
   // 190-206) instead of MatrixBatchVectorMultiplyAccumulate's; no bias, no activation.
   int batch_matmul;

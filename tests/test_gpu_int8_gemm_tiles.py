@@ -72,3 +72,30 @@ def test_tiles_between(fc, B, K, N):  # noqa: F811
 def test_tiles_between_other_side(fc, B, K, N):  # noqa: F811
     assert capi.load().lrtfc_fc_int8_packed_kernel(B, K, N) == capi.INT8_KERNEL_TILES_128X256
     _int8(fc, B, K, N)
+
+
+# A tail of up to 64 tiles of 128 x 256 over one per CU: its rows in a launch of their own; rows that end
+# inside a piece; the largest tail, and a launch of two rounds that stays whole.
+@pytest.mark.parametrize("B,K,N", [(2000, 2064, 4200), (2040, 2049, 4350), (1153, 2177, 8192), (1100, 2177, 16200)])
+def test_tail_rows_in_their_own_launch(fc, B, K, N):  # noqa: F811
+    _int8(fc, B, K, N)
+    _hybrid(fc, B, K, N)
+
+
+@pytest.mark.parametrize("zero_rows", ["first", "tail", "all"])
+def test_tail_rows_and_the_whole_zero_exit(fc, zero_rows):  # noqa: F811
+    """A whole-zero input keeps the sign of a bias of -0.0f; zeros in one of the two launches do not."""
+    B, K, N = 2000, 2064, 4200
+    rng = np.random.default_rng(4)
+    w = rng.integers(-127, 128, (N, K)).astype(np.int8)
+    pcs = rng.uniform(1e-3, 1e-2, N).astype(np.float32)
+    bias = np.full(N, -0.0, np.float32)
+    x = rng.standard_normal((B, K)).astype(np.float32)
+    if zero_rows != "tail":
+        x[:1920] = 0
+    if zero_rows != "first":
+        x[1920:] = 0
+    got = fc.FullyConnectedHybrid(w, pcs, bias=bias)(_cuda(x)).cpu().numpy()[:, :8]
+    want = oracle.fc_hybrid(x, w[:8], pcs[:8], bias=bias[:8])
+    assert np.array_equal(got.view(np.uint32), np.ascontiguousarray(want).view(np.uint32))
+    assert (np.signbit(got[0, 0]) == (zero_rows == "all")) or zero_rows == "tail"
