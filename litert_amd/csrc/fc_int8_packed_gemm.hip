@@ -412,6 +412,23 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
     constexpr int kRowBytes = BN * 4 + 16;
     static_assert(32 * kRowBytes <= 2 * kStageBytes, "a batch tile of floats does not fit");
     constexpr int kPiecesPerRow = BN / 4;
+    // The lane's channels, read from LDS once for all batch tiles (the registers of the loop's operands
+    // are free by now).
+    float chan_scale[kWaveTiles][4][4], chan_bias[kWaveTiles][4][4];
+    int32_t chan_sum[kWaveTiles][4][4];
+#pragma unroll
+    for (int i = 0; i < kWaveTiles; ++i) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const i32x4 p = chan_params[(wave * kWaveTiles + i) * 32 + 8 * g + 4 * (lane >> 5) + r];
+          chan_scale[i][g][r] = __int_as_float(p[0]);
+          chan_bias[i][g][r] = __int_as_float(p[1]);
+          chan_sum[i][g][r] = p[2];
+        }
+      }
+    }
 #pragma unroll
     for (int j = 0; j < kBatchTiles; ++j) {
       const float bscale = row_scale[j];
@@ -425,20 +442,18 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
           float v[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const i32x4 p = chan_params[local + r];
+            const float scale = chan_scale[i][g][r], bias = chan_bias[i][g][r];
+            const int32_t row_sum = chan_sum[i][g][r];
             const int32_t dot = acc[i][j][4 * g + r];
             if (EPI == Int8Epilogue::kHybrid4Bit) {
-              v[r] = activate(Hybrid4BitCore(dot, bscale, __int_as_float(p[0]), bzp,
-                                             __int_as_float(p[1]), a.bias_f32 != nullptr, 0));
+              v[r] = activate(Hybrid4BitCore(dot, bscale, scale, bzp, bias, a.bias_f32 != nullptr, 0));
             } else if (kForm != 0) {
               v[r] = activate(__fadd_rn(
-                  __int_as_float(p[1]),
-                  __fmul_rn(static_cast<float>(dot - __mul24(p[2], bzp)),
-                            __fmul_rn(bscale, __int_as_float(p[0])))));
+                  bias, __fmul_rn(static_cast<float>(dot - __mul24(row_sum, bzp)),
+                                  __fmul_rn(bscale, scale))));
             } else {
-              v[r] = HybridCoreSelect(dot, bscale, __int_as_float(p[0]), bzp, p[2],
-                                      __int_as_float(p[1]), a.activation, a.batch_matmul != 0,
-                                      zero_input);
+              v[r] = HybridCoreSelect(dot, bscale, scale, bzp, row_sum, bias, a.activation,
+                                      a.batch_matmul != 0, zero_input);
             }
           }
           *reinterpret_cast<float4*>(smem + row_in_tile * kRowBytes + local * 4) =
