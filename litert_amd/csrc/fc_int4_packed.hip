@@ -676,6 +676,267 @@ __global__ __launch_bounds__(THREADS) void FcInt4PackedKernel(
       min(bt, batches - first_row), ksplit, gpw, smem);
 }
 
+// One channel group per workgroup on deep rows (DeepNode). Bound by latency: the additions of an output
+// are a chain of one every 8 cycles, 1.8 us at 512 blocks, and behind the loads quantizing 16384 values
+// and multiplying them takes as long again. Here eight wavefronts quantize and multiply in steps of two
+// tiles, and a ninth adds a step's products while the others work on the next; in a step a wavefront has
+// one tile's blocks of two channels, and everything is requested at the start. Filters not in the caches,
+// us at 1 / 2 / 4 rows (4: int8 rows in, with their quantizer), FcInt4PackedKernel -> this one: 16384 ->
+// 2048 8.7 / 10.7 / 14.1 -> 8.2 / 10.4 / 13.6, 11008 -> 2048 10.1 / 12.1 / 23.8 -> 7.5 / 9.7 / 16.6,
+// 8192 -> 2048 6.4 / 8.1 / 11.2 -> 6.1 / 7.6 / 10.1, 4608 -> 1000 7.9 -> 5.0 at one row. A lane reads its
+// two channels' scales alone: 92 registers at one row, with the whole plane 104 and 0.2 us more.
+constexpr int kDeepWorkers = 8;
+constexpr int kDeepThreads = (kDeepWorkers + 1) * kWaveSize;
+constexpr int kDeepSteps = 4;  // of two tiles: depth up to 16384
+constexpr int kStepTiles = 2;
+constexpr int kWorkerThreads = kDeepWorkers * kWaveSize;  // eight values of a step each
+static_assert(kWorkerThreads * 8 == kStepTiles * kTileBlocks * kBlock, "a step's values");
+
+template <int BT>
+size_t DeepLds(int chunks) {
+  return static_cast<size_t>(BT) * chunks * kTileBlocks * kBlock +
+         static_cast<size_t>(chunks) * kTileRows * BT * kPStride * 4 + BT * kDeepWorkers * 2 * 4;
+}
+
+template <int BT, bool FUSED, int VARIANT>
+__global__ __launch_bounds__(kDeepThreads, 1) void FcInt4DeepKernel(
+    const uint8_t* packed, const void* rows, int depth, int out_depth, int chunks, int batches,
+    int batch0, int bt, Int4PackedArgs rest) {
+  extern __shared__ __align__(16) int8_t smem[];
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWaveSize - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWaveSize);
+  const int padded = chunks * kTileBlocks * kBlock;
+  const int steps = (chunks + kStepTiles - 1) / kStepTiles;
+  const int group = blockIdx.x;
+  int32_t* const q = reinterpret_cast<int32_t*>(smem);  // as in Int4Shared
+  float* const p = reinterpret_cast<float*>(smem + static_cast<size_t>(BT) * padded);
+  float* const mm = p + static_cast<size_t>(chunks) * kTileRows * BT * kPStride;  // [BT][workers][2]
+  const int rows_here = min(bt, batches - batch0);
+  const int b_here = lane & (BT - 1);  // the row whose parameters and outputs this lane has
+  const int groups8 = depth / 8;
+
+  // Every wavefront derives every row's parameters from the workers' ranges; lane L has row L % BT's.
+  auto row_params = [&] {
+    const int row = min(b_here, rows_here - 1);
+    float mn = mm[row * kDeepWorkers * 2], mx = mm[row * kDeepWorkers * 2 + 1];
+#pragma unroll
+    for (int w = 1; w < kDeepWorkers; ++w) {
+      mn = fminf(mn, mm[(row * kDeepWorkers + w) * 2]);
+      mx = fmaxf(mx, mm[(row * kDeepWorkers + w) * 2 + 1]);
+    }
+    return AsymmetricRowParams<VARIANT>(mn, mx);
+  };
+
+  if (wave < kDeepWorkers) {
+    // Rows, then (behind a barrier, see FcInt4PackedBody) weights.
+    float4 xr[BT][kDeepSteps][2];
+    i32x2 qr[BT][kDeepSteps];
+#pragma unroll
+    for (int b = 0; b < BT; ++b) {
+      const size_t row = static_cast<size_t>(batch0 + min(b, rows_here - 1)) * depth;
+#pragma unroll
+      for (int j = 0; j < kDeepSteps; ++j) {
+        const int g = min(j * kWorkerThreads + tid, groups8 - 1);
+        if (FUSED) {
+          const LRTFC_GLOBAL float* x = (const LRTFC_GLOBAL float*)rows + row + g * 8;
+          const f32x4 lo = *reinterpret_cast<const LRTFC_GLOBAL f32x4*>(x);
+          const f32x4 hi = *reinterpret_cast<const LRTFC_GLOBAL f32x4*>(x + 4);
+          xr[b][j][0] = make_float4(lo.x, lo.y, lo.z, lo.w);
+          xr[b][j][1] = make_float4(hi.x, hi.y, hi.z, hi.w);
+        } else {
+          qr[b][j] = *reinterpret_cast<const LRTFC_GLOBAL i32x2*>(
+              (const LRTFC_GLOBAL int8_t*)rows + row + g * 8);
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    const int half = wave >> 2, channel0 = 2 * (wave & 3);
+    const LRTFC_GLOBAL i32x4* const tiles = (const LRTFC_GLOBAL i32x4*)packed +
+                                            static_cast<size_t>(group) * chunks * kTileVecs + lane;
+    i32x4 w[kDeepSteps][2];
+    uint32_t sc[kDeepSteps];  // the two channels' scales, of the tile's last plane (eight a block)
+#pragma unroll
+    for (int j = 0; j < kDeepSteps; ++j) {
+      const LRTFC_GLOBAL i32x4* tile = tiles + static_cast<size_t>(min(kStepTiles * j + half, chunks - 1)) * kTileVecs;
+      sc[j] = ((const LRTFC_GLOBAL uint32_t*)(tile + kTileRows * 64))[channel0 / 2];
+      w[j][0] = __builtin_nontemporal_load(tile + channel0 * 64);
+      w[j][1] = __builtin_nontemporal_load(tile + (channel0 + 1) * 64);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    float inv = 0.0f;
+    int32_t zero_point = 0;
+    if (FUSED) {
+#pragma unroll
+      for (int b = 0; b < BT; ++b) {
+        float mn = 0.0f, mx = 0.0f;
+#pragma unroll
+        for (int j = 0; j < kDeepSteps; ++j) {
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const float4 t = xr[b][j][h];  // clamped duplicates past the row are harmless here
+            mn = fminf(fminf(mn, t.x), fminf(fminf(t.y, t.z), t.w));
+            mx = fmaxf(fmaxf(mx, t.x), fmaxf(fmaxf(t.y, t.z), t.w));
+          }
+        }
+        mn = WaveMinF32(mn);
+        mx = WaveMaxF32(mx);
+        if (lane == 0) {
+          mm[(b * kDeepWorkers + wave) * 2] = mn;
+          mm[(b * kDeepWorkers + wave) * 2 + 1] = mx;
+        }
+      }
+      __syncthreads();
+      const RowQuantParams qp = row_params();
+      inv = ElementwiseInv(qp);
+      zero_point = qp.zero_point;
+    }
+    const int vector_end = depth - (depth % 8);
+#pragma unroll
+    for (int j = 0; j < kDeepSteps; ++j) {
+      if (j >= steps) break;
+      const int g = j * kWorkerThreads + tid;
+      if (g < padded / 8) {
+#pragma unroll
+        for (int b = 0; b < BT; ++b) {
+          int32_t high = 0, low = 0;
+          if (g < groups8) {
+            uint32_t lo, hi;
+            if (FUSED) {
+              RowQuantParams qp;
+              qp.inv = ReadLaneF32(inv, b);
+              qp.zero_point = __builtin_amdgcn_readlane(zero_point, b);
+              const float4 x0 = xr[b][j][0], x1 = xr[b][j][1];
+              const bool tail = g * 8 >= vector_end;
+              lo = static_cast<uint32_t>(QuantizePack4<VARIANT>(x0.x, x0.y, x0.z, x0.w, qp, tail));
+              hi = static_cast<uint32_t>(QuantizePack4<VARIANT>(x1.x, x1.y, x1.z, x1.w, qp, tail));
+            } else {
+              lo = static_cast<uint32_t>(qr[b][j].x);
+              hi = static_cast<uint32_t>(qr[b][j].y);
+            }
+            NibblePlanes(lo, hi, &high, &low);
+          }
+          q[b * (padded / 4) + (g >> 2) * 8 + (g & 3)] = high;
+          q[b * (padded / 4) + (g >> 2) * 8 + 4 + (g & 3)] = low;
+        }
+      }
+      __syncthreads();  // the step's rows are there, and the step before's products
+      const int tile = kStepTiles * j + half;
+      if (tile < chunks) {
+        const int blk = tile * kTileBlocks + lane;
+        const float scale[2] = {HalfBitsToFloatFast(static_cast<uint16_t>(sc[j] & 0xFFFF)),
+                                HalfBitsToFloatFast(static_cast<uint16_t>(sc[j] >> 16))};
+        i32x4 ws[2];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+#pragma unroll
+          for (int d = 0; d < 4; ++d) ws[c][d] = w[j][c][d] ^ static_cast<int32_t>(0x88888888u);
+        }
+#pragma unroll
+        for (int b = 0; b < BT; ++b) {
+          const i32x4* at = reinterpret_cast<const i32x4*>(q + b * (padded / 4) + blk * 8);
+          const i32x4 qh = at[0], ql = at[1];
+          uint32_t t = 0;
+#pragma unroll
+          for (int d = 0; d < 4; ++d) t = UDot8(static_cast<uint32_t>(ql[d]), 0x11111111u, t);
+          const uint32_t seed = 0u - 8u * t;
+#pragma unroll
+          for (int c = 0; c < 2; ++c) {
+            int32_t sd = 0;
+            uint32_t ud = seed;
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+              sd = SDot8(ws[c][d], qh[d], sd);
+              ud = UDot8(static_cast<uint32_t>(w[j][c][d]), static_cast<uint32_t>(ql[d]), ud);
+            }
+            const int32_t acc = (sd << 4) + static_cast<int32_t>(ud);
+            p[((tile * kTileRows + channel0 + c) * BT + b) * kPStride + lane] =
+                __fmul_rn(static_cast<float>(acc), scale[c]);
+          }
+        }
+      }
+    }
+    __syncthreads();  // the last step's products
+    return;
+  }
+
+  // The ninth wavefront: lane = channel * BT + row.
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_s_setprio(3);  // a chain of one addition at a time, the others fill what it leaves
+  const int channel = min(group * kTileRows + lane / BT, out_depth - 1);
+  const float kfsum = ((const LRTFC_GLOBAL float*)rest.kfsum)[channel];
+  const float bias = rest.bias ? ((const LRTFC_GLOBAL float*)rest.bias)[channel] : 0.0f;
+  float row_scale = 0.0f;
+  int32_t row_zero_point = 0;
+  if (FUSED) {
+    __syncthreads();
+    const RowQuantParams qp = row_params();
+    row_scale = qp.scale;
+    row_zero_point = qp.zero_point;
+  } else {
+    const int b = batch0 + min(b_here, rows_here - 1);
+    row_scale = ((const LRTFC_GLOBAL float*)rest.scaling_factors)[b];
+    row_zero_point = ((const LRTFC_GLOBAL int32_t*)rest.zero_points)[b];
+  }
+  const bool chain_lane = lane < kTileRows * BT;
+  const int nblk = depth / kBlock;
+  float out = 0.0f;
+  // The products of `count` tiles from `tile` on, half a tile read ahead of the additions.
+  auto add_tiles = [&](int tile, int count) {
+    const float* line = p + static_cast<size_t>(tile) * kTileRows * BT * kPStride + lane * kPStride;
+    constexpr int kAhead = kTileBlocks / 8;  // float4 per half tile
+    constexpr int kTileFloats = kTileRows * BT * kPStride;
+    const int blocks = min(count * kTileBlocks, nblk - tile * kTileBlocks);
+    if (blocks == count * kTileBlocks) {
+      auto read_half = [&](int half, float4* v) {
+        const float4* from = reinterpret_cast<const float4*>(
+            line + static_cast<size_t>(half >> 1) * kTileFloats + (half & 1) * (kTileBlocks / 2));
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) v[i] = from[i];
+      };
+      auto add_half = [&](const float4* v) {
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+          out = __fadd_rn(out, v[i].x);
+          out = __fadd_rn(out, v[i].y);
+          out = __fadd_rn(out, v[i].z);
+          out = __fadd_rn(out, v[i].w);
+        }
+      };
+      float4 even[kAhead], odd[kAhead];
+      read_half(0, even);
+      for (int half = 0; half < 2 * count; half += 2) {
+        read_half(half + 1, odd);
+        add_half(even);
+        read_half(min(half + 2, 2 * count - 1), even);
+        add_half(odd);
+      }
+    } else {
+      for (int i = 0; i < blocks; ++i) {
+        out = __fadd_rn(out, line[static_cast<size_t>(i / kTileBlocks) * kTileFloats + i % kTileBlocks]);
+      }
+    }
+  };
+  for (int j = 0; j < steps; ++j) {
+    __syncthreads();
+    if (j > 0 && chain_lane) add_tiles(kStepTiles * (j - 1), kStepTiles);
+  }
+  __syncthreads();
+  if (chain_lane) {
+    add_tiles(kStepTiles * (steps - 1), chunks - kStepTiles * (steps - 1));
+    // fully_connected.cc:1078-1082
+    float o = __fsub_rn(out, __fmul_rn(static_cast<float>(row_zero_point), kfsum));
+    o = __fmul_rn(o, row_scale);
+    if (rest.bias) o = __fadd_rn(o, bias);
+    const int n = group * kTileRows + lane / BT;
+    if (b_here < rows_here && n < out_depth) {
+      ((LRTFC_GLOBAL float*)rest.output)[static_cast<size_t>(batch0 + b_here) * out_depth + n] = o;
+    }
+  }
+}
+
 // Several filters of the same depth in one launch (nodes of a graph that do not depend on
 // each other: the q/k/v or gate/up projections of a decoder layer). The table lives in device
 // memory: per node its arguments and the index of its first workgroup. One launch instead of
@@ -773,18 +1034,31 @@ int ChooseKsplit(int out_depth, int chunks) {
 }
 
 // Single nodes of deep rows whose tiles make about one workgroup of eight wavefronts per CU, one tile
-// each: a wavefront alone on its SIMD issues a vector operation every 8 cycles or so, and the
-// prologue (16384 values quantized and split into nibble planes by every workgroup) is the larger
-// part of such a launch. Four wavefronts -> eight, us at 1 / 2 / 4 rows (4: int8 rows in, with
-// their quantizer): 16384 -> 2048 10.1 / 12.3 / 16.5 -> 9.5 / 11.0 / 14.1, 8192 -> 2048 8.3 / 9.7 /
-// 13.4 -> 7.0 / 8.3 / 11.5. With two tiles each it is no gain (11008 -> 4096 11.1 -> 11.5 at one
-// row), in more than one round a loss (4608 -> 12000 13.0 -> 17.3, 16384 -> 2050 14.4 -> 16.5).
+// each, beyond the groups of FcInt4DeepKernel (and unaligned rows within them): a wavefront alone on its
+// SIMD issues a vector operation every 8 cycles or so, and the prologue (the row quantized and split into
+// nibble planes by every workgroup) is the larger part of such a launch. Four wavefronts -> eight, us at
+// 1 / 2 / 4 rows: 8192 -> 2048 8.3 / 9.7 / 13.4 -> 7.0 / 8.3 / 11.5. With two tiles each it is no gain
+// (11008 -> 4096 11.1 -> 11.5 at one row), in more than one round a loss (4608 -> 12000 13.0 -> 17.3,
+// 16384 -> 2050 14.4 -> 16.5).
 bool WideDeep(int depth, int out_depth, int chunks) {
   constexpr int kWideWaves = kWideThreads / kWaveSize;
   if (depth <= kShallowDepth || depth > kDeepDepth) return false;
   if (chunks > kWideWaves || kWideWaves % chunks != 0) return false;
   const int groups = (out_depth + kTileRows - 1) / kTileRows;
   return groups <= kWideWaves / chunks * 256;
+}
+
+// Single nodes of deep rows with at most one channel group per CU: FcInt4DeepKernel. The rows have to
+// lie on 16 bytes (8, as int8): the kernel has no other way to read them. Beyond one round of its
+// workgroups every row is quantized once more per channel group than there: at one row 9216 -> 3072 9.5 ->
+// 10.5 us, 8192 -> 4096 7.3 -> 10.0, 16384 -> 4096 13.3 -> 14.7.
+constexpr int kDeepMaxGroups = 256;
+
+bool DeepNode(const Int4PackedArgs& a, bool fused) {
+  const auto at = reinterpret_cast<uintptr_t>(fused ? static_cast<const void*>(a.input_f32)
+                                                    : static_cast<const void*>(a.input_q));
+  return a.depth > kShallowDepth && a.depth <= kDeepDepth && a.depth % 8 == 0 &&
+         (at & (fused ? 15 : 7)) == 0 && (a.out_depth + kTileRows - 1) / kTileRows <= kDeepMaxGroups;
 }
 
 // Channel groups per wavefront. Measured on launches from 7 MB to 340 MB: a wavefront should
@@ -824,6 +1098,15 @@ constexpr int kStraightTiles = 2;
 template <int BT, bool FUSED, int VARIANT, int GPT>
 hipError_t LaunchOne(const Int4PackedArgs& a, int batch0, int bt, int slices, hipStream_t stream) {
   if constexpr (GPT > kShallowGpt) {
+    if (DeepNode(a, FUSED)) {
+      const size_t lds = DeepLds<BT>(a.chunks);
+      auto kernel = FcInt4DeepKernel<BT, FUSED, VARIANT>;
+      if (hipError_t err = EnsureDynamicLds(reinterpret_cast<const void*>(kernel), lds)) return err;
+      const void* rows = FUSED ? static_cast<const void*>(a.input_f32) : static_cast<const void*>(a.input_q);
+      hipLaunchKernelGGL(kernel, dim3((a.out_depth + kTileRows - 1) / kTileRows), dim3(kDeepThreads), lds,
+                         stream, a.packed, rows, a.depth, a.out_depth, a.chunks, a.batches, batch0, bt, a);
+      return hipGetLastError();
+    }
     if (WideDeep(a.depth, a.out_depth, a.chunks)) {
       return LaunchSized<BT, FUSED, VARIANT, GPT * kThreads / kWideThreads, 1, 1, kWideThreads>(
           a, batch0, bt, slices, /*ksplit=*/a.chunks, 1, stream);

@@ -1,6 +1,6 @@
 """Blockwise-int4 decode launches around their dispatch rules: eight wavefronts per workgroup on deep
 rows of four and eight tiles (whole and partial), one round of workgroups and one past it; three
-and four rows as two pairs side by side. Bit-identical to the CPU oracle."""
+and four rows as two pairs side by side; deep rows of one channel group per workgroup. Bit-identical to the CPU oracle."""
 import numpy as np
 import pytest
 
@@ -32,3 +32,20 @@ def test_int4_decode_forms_match_oracle(fc, B, K, N):  # noqa: F811
     if B <= 4:
         assert _bits_equal(op(x).cpu().numpy(), want)
     assert _bits_equal(op.call_split(x).cpu().numpy(), want)  # ... and those on quantized rows
+
+
+@pytest.mark.parametrize("variant", [oracle.QUANT_PORTABLE, oracle.QUANT_NEON_V8, oracle.QUANT_NEON_LEGACY])
+@pytest.mark.parametrize("B,K,N", [
+    (1, 4128, 8), (2, 6176, 2041), (1, 10208, 2048), (2, 12320, 15), (1, 14336, 257), (2, 16352, 1),
+    (2, 11008, 2049),  # one group past it
+])
+def test_int4_deep_rows_variants_and_alignment(fc, B, K, N, variant):  # noqa: F811
+    c = wl.blockwise_int4_fc(B, K, N, seed=K + N, lo=-8, hi=7)
+    c["x"][0, K - 1] = 30.0  # the range comes from the last partial step
+    want = oracle.fc_blockwise_int4(c["x"], c["packed"], N, c["scales"].view(np.uint16), 32, variant=variant)
+    op = fc.FullyConnectedBlockwiseInt4(c["packed"], c["scales"], K, 32, quant_variant=variant)
+    op.FUSED_MAX_DEPTH = 1 << 30
+    x = _cuda(c["x"])
+    shifted = _cuda(np.concatenate([[0.0], c["x"].ravel()]).astype(np.float32))[1:].view(B, K)
+    for rows in (x, shifted):  # on 16 bytes, and 4 past them
+        assert _bits_equal(op(rows).cpu().numpy(), want)
