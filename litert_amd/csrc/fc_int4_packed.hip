@@ -955,8 +955,8 @@ struct Int4GroupTable {
   Int4PackedArgs node[kMaxGroupNodes];
 };
 
-template <int BT, bool FUSED, int VARIANT, int GPT>
-__global__ __launch_bounds__(kThreads) void FcInt4PackedGroupedKernel(
+template <int BT, bool FUSED, int VARIANT, int GPT, int ALL = 0, int PRE = 0, int THREADS = kThreads>
+__global__ __launch_bounds__(THREADS) void FcInt4PackedGroupedKernel(
     const Int4GroupTable* __restrict__ table, int count, int depth, int chunks, int batches,
     int batch0, int bt, int ksplit, int gpw) {
   extern __shared__ __align__(16) int8_t smem[];
@@ -998,8 +998,8 @@ __global__ __launch_bounds__(kThreads) void FcInt4PackedGroupedKernel(
   }
   // Row tiles side by side (gridDim.y > 1): slice y of the grid takes rows batch0 + y * bt on.
   const int first_row = batch0 + static_cast<int>(blockIdx.y) * bt;
-  FcInt4PackedBody<BT, FUSED, VARIANT, GPT>(start, table->node[node], block - first, first_row,
-                                            min(bt, batches - first_row), ksplit, gpw, smem);
+  FcInt4PackedBody<BT, FUSED, VARIANT, GPT, ALL, PRE, THREADS>(
+      start, table->node[node], block - first, first_row, min(bt, batches - first_row), ksplit, gpw, smem);
 }
 
 // The row quantizer for a whole group: workgroup r quantizes row r % batches of node
@@ -1356,33 +1356,33 @@ size_t Int4GroupTableBytes() {
 }
 
 namespace {
-template <int BT, bool FUSED, int VARIANT, int GPT>
+template <int BT, bool FUSED, int VARIANT, int GPT, int ALL = 0, int PRE = 0, int THREADS = kThreads>
 hipError_t LaunchGroupedOne(const void* table, const lrtfc_int4_group_launch& l, int batch0,
                             int bt, hipStream_t stream, int row_tiles = 1) {
   const int chunks = (l.depth / kBlock + kTileBlocks - 1) / kTileBlocks;
   const int padded = chunks * kTileBlocks * kBlock;
-  const size_t lds = Int4Shared<BT>::Bytes(padded, l.ksplit);
-  auto kernel = FcInt4PackedGroupedKernel<BT, FUSED, VARIANT, GPT>;
+  const size_t lds = Int4Shared<BT, THREADS>::Bytes(padded, l.ksplit);
+  auto kernel = FcInt4PackedGroupedKernel<BT, FUSED, VARIANT, GPT, ALL, PRE, THREADS>;
   if (hipError_t err = EnsureDynamicLds(reinterpret_cast<const void*>(kernel), lds)) return err;
-  hipLaunchKernelGGL(kernel, dim3(l.grid_blocks, row_tiles), dim3(kThreads), lds, stream,
+  hipLaunchKernelGGL(kernel, dim3(l.grid_blocks, row_tiles), dim3(THREADS), lds, stream,
                      static_cast<const Int4GroupTable*>(table), l.count, l.depth, chunks, l.batches,
-                     batch0, bt, l.ksplit, l.groups_per_wave);
+                     batch0, bt, l.ksplit, l.groups_per_wave * kThreads / THREADS);
   return hipGetLastError();
 }
 
-template <int BT, int GPT>
+template <int BT, int GPT, int ALL = 0, int PRE = 0, int THREADS = kThreads>
 hipError_t LaunchGroupedVariant(const void* table, const lrtfc_int4_group_launch& l, int variant,
                                 int batch0, int bt, hipStream_t stream, int row_tiles = 1) {
   switch (variant) {
     case LRTFC_QUANT_NEON_V8:
-      return LaunchGroupedOne<BT, true, LRTFC_QUANT_NEON_V8, GPT>(table, l, batch0, bt, stream,
-                                                                  row_tiles);
+      return LaunchGroupedOne<BT, true, LRTFC_QUANT_NEON_V8, GPT, ALL, PRE, THREADS>(
+          table, l, batch0, bt, stream, row_tiles);
     case LRTFC_QUANT_NEON_LEGACY:
-      return LaunchGroupedOne<BT, true, LRTFC_QUANT_NEON_LEGACY, GPT>(table, l, batch0, bt, stream,
-                                                                      row_tiles);
+      return LaunchGroupedOne<BT, true, LRTFC_QUANT_NEON_LEGACY, GPT, ALL, PRE, THREADS>(
+          table, l, batch0, bt, stream, row_tiles);
     default:
-      return LaunchGroupedOne<BT, true, LRTFC_QUANT_PORTABLE, GPT>(table, l, batch0, bt, stream,
-                                                                   row_tiles);
+      return LaunchGroupedOne<BT, true, LRTFC_QUANT_PORTABLE, GPT, ALL, PRE, THREADS>(
+          table, l, batch0, bt, stream, row_tiles);
   }
 }
 
@@ -1449,6 +1449,21 @@ hipError_t LaunchFcInt4PackedGrouped(const void* table, const lrtfc_int4_group_l
     // Three or four rows of a small group: two slices of the grid, two fused rows each.
     return deep ? LaunchGroupedVariant<2, 8>(table, l, variant, 0, 2, stream, 2)
                 : LaunchGroupedVariant<2, 2>(table, l, variant, 0, 2, stream, 2);
+  }
+  // One row, and the tiles of a wavefront known: straight-line code, as for single nodes. One tile each:
+  // 2048 -> 2048 + 256 + 256 4.75 -> 4.2 us, 1152 -> 6912 + 6912 8.7 -> 7.2. Four each (beyond that a group
+  // fills the ring's turns): eight wavefronts a workgroup with two each, one ahead of the prologue: 2048 ->
+  // 2 x 16384 9.45 -> 9.0 us, 4096 -> 2 x 11008 13.9 -> 13.4, 2048 -> 18 x 2048 13.4 -> 12.5 (both ahead, or
+  // both behind: 10). Two each stay with the ring, which requests both ahead: straight-line 2 % slower. So
+  // do two and more rows, where neither form is a gain (6 layers of 2048 / 12288 at two rows 175.5 us a
+  // token, with both 176.5).
+  if (l.batches == 1 && l.depth <= kShallowDepth && l.ksplit == 1) {
+    const int tiles = l.groups_per_wave * chunks;
+    if (tiles == 1) return LaunchGroupedVariant<1, kShallowGpt, 1, 1>(table, l, variant, 0, 1, stream);
+    if (tiles == 2 * kStraightTiles && l.groups_per_wave % 2 == 0) {
+      return LaunchGroupedVariant<1, kShallowGpt * kThreads / kWideThreads, kStraightTiles, 1, kWideThreads>(
+          table, l, variant, 0, 1, stream);
+    }
   }
   const int tile = FitBatchTile(MaxBatchTile<true>(l.depth), padded, l.ksplit);
   for (int batch0 = 0; batch0 < l.batches; batch0 += tile) {  // more rows: one launch per tile

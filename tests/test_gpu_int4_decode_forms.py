@@ -3,6 +3,7 @@ rows of four and eight tiles (whole and partial), one round of workgroups and on
 and four rows as two pairs side by side; deep rows of one channel group per workgroup. Bit-identical to the CPU oracle."""
 import numpy as np
 import pytest
+import torch
 
 import oracle
 from litert_amd import workloads as wl
@@ -49,3 +50,18 @@ def test_int4_deep_rows_variants_and_alignment(fc, B, K, N, variant):  # noqa: F
     shifted = _cuda(np.concatenate([[0.0], c["x"].ravel()]).astype(np.float32))[1:].view(B, K)
     for rows in (x, shifted):  # on 16 bytes, and 4 past them
         assert _bits_equal(op(rows).cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("K,outs", [
+    (96, (33, 7, 120)), (2048, (40, 8)),              # a tile per wavefront
+    (96, (20011, 9001)), (2112, (7001, 7400)),        # four
+    (2048, (9000, 5500)), (96, (20011, 20011, 20011)),  # two, and eight
+])
+def test_int4_groups_of_one_row(fc, K, outs):  # noqa: F811
+    cases = [wl.blockwise_int4_fc(1, K, n, seed=n, lo=-8, hi=7) for n in outs]
+    ops = [fc.FullyConnectedBlockwiseInt4(c["packed"], c["scales"], K, 32) for c in cases]
+    out = [torch.full((1, n), np.nan, device="cuda") for n in outs]
+    fc.GroupedBlockwiseInt4(ops).bind([_cuda(c["x"]) for c in cases], out)()
+    for c, n, y in zip(cases, outs, out):
+        want = oracle.fc_blockwise_int4(c["x"], c["packed"], n, c["scales"].view(np.uint16), 32)
+        assert _bits_equal(y.cpu().numpy(), want)
