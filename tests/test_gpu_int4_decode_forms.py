@@ -65,3 +65,17 @@ def test_int4_groups_of_one_row(fc, K, outs):  # noqa: F811
     for c, n, y in zip(cases, outs, out):
         want = oracle.fc_blockwise_int4(c["x"], c["packed"], n, c["scales"].view(np.uint16), 32)
         assert _bits_equal(y.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("B", [1, 2, 4])
+@pytest.mark.parametrize("blocks", [1, 4, 15, 16, 17, 31, 33, 48, 49, 63, 65, 81, 127, 129, 143, 191, 257])
+def test_int4_partial_tiles(fc, B, blocks):  # noqa: F811
+    K, N = 32 * blocks, 35
+    c = wl.blockwise_int4_fc(B, K, N, seed=blocks, lo=-8, hi=7)
+    c["packed"][3] = 0        # weights 0: products of -0 where the scale is negative
+    c["scales"][3] = -c["scales"][3]
+    op = fc.FullyConnectedBlockwiseInt4(c["packed"], c["scales"], K, 32)
+    op.FUSED_MAX_DEPTH = 1 << 30
+    want = oracle.fc_blockwise_int4(c["x"], c["packed"], N, c["scales"].view(np.uint16), 32)
+    assert _bits_equal(op(_cuda(c["x"])).cpu().numpy(), want)
+    assert _bits_equal(op.call_split(_cuda(c["x"])).cpu().numpy(), want)
