@@ -65,7 +65,9 @@ __global__ __launch_bounds__(THREADS) void BatchQuantize4BitKernel(
   const RowRange range = BlockMinMax<THREADS>(mn, mx);
   float scale_denom = fmaxf(fabsf(range.mn), fabsf(range.mx));
   if (scale_denom == 0.0f) scale_denom = 127.0f;
-  const float multiplier = SymmetricMultiplier(scale_denom);
+  // Divided: the reciprocal's form is no gain among a workgroup's 16 wavefronts (with the product, 362 x
+  // 4764 -> 899: 15.0 us, divided 14.8).
+  const float multiplier = SymmetricMultiplierDivided(scale_denom);
   int32_t sum = 0;
   auto emit4 = [&](int i, const float4& t) {
     uint32_t word = QuantizeSymmetricPack4(t.x, t.y, t.z, t.w, multiplier);
@@ -101,7 +103,7 @@ __global__ __launch_bounds__(THREADS) void BatchQuantize4BitKernel(
     int32_t total = 0;
 #pragma unroll
     for (int w = 0; w < THREADS / kWaveSize; ++w) total += s_sum[w];
-    scaling_factors[row] = Over127(scale_denom);
+    scaling_factors[row] = static_cast<float>(static_cast<double>(scale_denom) / 127.0);
     input_offsets[row] = total * -7;
   }
 }

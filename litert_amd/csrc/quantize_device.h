@@ -163,12 +163,16 @@ __device__ __forceinline__ int32_t RoundHalfAwayToInt(float x) {
 // 127 / the row's largest magnitude, divided in double. Below 3.8e-37 that is no float32: the
 // reference then multiplies by infinity and converts what comes out, infinities and (for a zero)
 // NaN, to int8, which gives 0 on x86. A NaN multiplier makes every value of the row such a 0.
+__device__ __forceinline__ float SymmetricMultiplierDivided(float scale_denom) {
+  const float mult = static_cast<float>(127.0 / static_cast<double>(scale_denom));
+  return mult == __builtin_inff() ? __builtin_nanf("") : mult;
+}
 __device__ __forceinline__ float SymmetricMultiplier(float scale_denom) {
   float mult;
-  if (!Quotient127Fast(scale_denom, HardwareReciprocal{}, &mult)) {
-    mult = static_cast<float>(127.0 / static_cast<double>(scale_denom));
+  if (Quotient127Fast(scale_denom, HardwareReciprocal{}, &mult)) {
+    return mult == __builtin_inff() ? __builtin_nanf("") : mult;
   }
-  return mult == __builtin_inff() ? __builtin_nanf("") : mult;
+  return SymmetricMultiplierDivided(scale_denom);
 }
 
 // Four values of a row times its multiplier, rounded half away from zero, as four bytes. With
