@@ -35,9 +35,12 @@ _current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device
 
 
 def _call_stream():
-    if _raw_stream is None:
-        return torch.cuda.current_stream().cuda_stream
     return _raw_stream(_current_device())
+
+
+if _raw_stream is None:
+    def _call_stream():  # noqa: F811
+        return torch.cuda.current_stream().cuda_stream
 
 
 def _addr(t):
@@ -57,22 +60,34 @@ def _dev(a, dtype):
 
 
 def _empty_functions():
-    """empty(like, rows, columns) for int8 and float32 outputs on like's device: native ones where
-    they have been built for this torch and interpreter (a small call's host part 6.0 -> 5.0 us)."""
+    """empty(like, rows, columns) for int8 and float32 outputs on like's device, and scratch(like, bytes):
+    native ones where they have been built for this torch and interpreter (a small call's host part 6.0 ->
+    5.0 us).
+
+    scratch is memory for the launches of one call, as its address and what holds it. Torch's allocator hands
+    it to later work of the same stream only, and keeps it for a graph that captured the call; an op that used
+    it again would share it between its calls on several streams and threads. Ops hold the last call's until
+    the next one is through: the allocator then alternates, and a quantizer does not write what the product
+    before it has left in every XCD's L2 (three hybrid 2999 -> 5003 in turn at 77 rows: 9.83 us each in one
+    piece of memory, 9.68 in several)."""
     path = os.path.join(os.path.dirname(capi.LIB_PATH), build.torch_tensors_name(torch.__version__))
     if os.path.exists(path):
         loader = importlib.machinery.ExtensionFileLoader("litert_amd_tensors", path)
         spec = importlib.util.spec_from_file_location("litert_amd_tensors", path, loader=loader)
         module = importlib.util.module_from_spec(spec)
         loader.exec_module(module)
-        return module.empty_int8, module.empty_float32
+        return module.empty_int8, module.empty_float32, module.scratch
 
     def empty(dtype):
         return lambda like, rows, columns: torch.empty((rows, columns), dtype=dtype, device=like.device)
-    return empty(torch.int8), empty(torch.float32)
+
+    def scratch(like, size):
+        memory = torch.empty(size, dtype=torch.uint8, device=like.device)
+        return memory.data_ptr(), memory
+    return empty(torch.int8), empty(torch.float32), scratch
 
 
-_empty_int8, _empty_float32 = _empty_functions()
+_empty_int8, _empty_float32, _scratch = _empty_functions()
 
 
 def _ensure_init():
@@ -262,16 +277,11 @@ class FullyConnectedHybrid:
         self.row_sums = torch.empty(self.out_depth, dtype=torch.int32, device="cuda")
         capi.check(capi.load().lrtfc_row_sums_int8(_ptr(self.filter), self.out_depth, self.depth,
                                                    _ptr(self.row_sums), _stream()))
-        self._ws = None
         # packed: one fused kernel (quantize in the prologue, matrix-core GEMV);
         # otherwise the two-kernel form on the row-major filter.
         self.packed_filter = _pack_int8(self.filter) if packed else None
-
-    def _workspace(self, batches):
-        need = capi.calls().lrtfc_activation_workspace_bytes(batches, self.depth)
-        if self._ws is None or self._ws.numel() < need:
-            self._ws = torch.empty(need, dtype=torch.uint8, device="cuda")
-        return self._ws
+        self._library_fused_max = capi.load().lrtfc_fc_hybrid_fused_max_batches(self.depth, self.out_depth)
+        self._need = (0, 0)  # rows of the last split call and what their scratch takes
 
     def __call__(self, x, out=None):
         x = x.contiguous()
@@ -279,18 +289,20 @@ class FullyConnectedHybrid:
         if out is None:
             out = _empty_float32(x, batches, self.out_depth)
         if self.packed_filter is not None and batches > self._fused_max():
-            return self.call_split(x, out)
+            return self._call_split(x, batches, out)
         if self.packed_filter is not None:
             capi.check(capi.calls().lrtfc_fc_hybrid_packed(
                 _addr(x), _addr(self.packed_filter), _addr(self.pcs), self.filter_scale,
                 _addr(self.row_sums), _addr(self.bias), _addr(out), batches, self.depth,
                 self.out_depth, int(self.asymmetric), self.activation, self.variant, _call_stream()))
             return out
-        ws = self._workspace(batches)
+        need = capi.calls().lrtfc_activation_workspace_bytes(batches, self.depth)
+        ws, held = _scratch(x, need)
         capi.check(capi.calls().lrtfc_fc_hybrid(
             _addr(x), _addr(self.filter), _addr(self.pcs), self.filter_scale, _addr(self.row_sums),
             _addr(self.bias), _addr(out), batches, self.depth, self.out_depth, int(self.asymmetric),
-            self.activation, self.variant, _addr(ws), ws.numel(), _call_stream()))
+            self.activation, self.variant, ws, need, _call_stream()))
+        self._held = held
         return out
 
 
@@ -299,9 +311,8 @@ class FullyConnectedHybrid:
     FUSED_MAX_BATCHES = None
 
     def _fused_max(self):
-        if self.FUSED_MAX_BATCHES is not None:
-            return self.FUSED_MAX_BATCHES
-        return capi.calls().lrtfc_fc_hybrid_fused_max_batches(self.depth, self.out_depth)
+        limit = self.FUSED_MAX_BATCHES
+        return self._library_fused_max if limit is None else limit
 
     def call_split(self, x, out=None):
         """Two launches on the packed filter: the standalone row quantizer, then the
@@ -309,14 +320,26 @@ class FullyConnectedHybrid:
         if self.packed_filter is None:
             raise RuntimeError("call_split needs the packed filter (packed=True)")
         x = x.contiguous()
-        batches = x.numel() // self.depth
+        return self._call_split(x, x.numel() // self.depth, out)
+
+    def _call_split(self, x, batches, out):
+        # Two small launches, of which the host's part takes as long: nothing is called here that need not be.
+        calls, pcs, bias = capi.calls(), self.pcs, self.bias
         if out is None:
             out = _empty_float32(x, batches, self.out_depth)
-        ws = self._workspace(batches)
-        capi.check(capi.calls().lrtfc_fc_hybrid_packed_workspace(
-            _addr(x), _addr(self.packed_filter), _addr(self.pcs), self.filter_scale,
-            _addr(self.row_sums), _addr(self.bias), _addr(out), batches, self.depth, self.out_depth,
-            int(self.asymmetric), self.activation, self.variant, _addr(ws), ws.numel(), _call_stream()))
+        rows, need = self._need
+        if rows != batches:
+            need = calls.lrtfc_activation_workspace_bytes(batches, self.depth)
+            self._need = (batches, need)
+        ws, held = _scratch(x, need)
+        status = calls.lrtfc_fc_hybrid_packed_workspace(
+            x.data_ptr(), self.packed_filter.data_ptr(), pcs if pcs is None else pcs.data_ptr(),
+            self.filter_scale, self.row_sums.data_ptr(), bias if bias is None else bias.data_ptr(),
+            out.data_ptr(), batches, self.depth, self.out_depth, self.asymmetric, self.activation,
+            self.variant, ws, need, _call_stream())
+        if status:
+            capi.check(status)
+        self._held = held
         return out
 
 
@@ -347,10 +370,8 @@ class FullyConnectedBlockwiseInt4:
         capi.check(capi.load().lrtfc_blockwise_int4_kfsum(
             _ptr(self.filter), _ptr(self.scales), self.out_depth, self.depth, self.blocksize,
             _ptr(self.kfsum), _stream()))
-        self._ws = None
         self._gemm_filter = None
         self._nibble_filter = None
-        self._gemm_ws = None
         # packed: one fused kernel on the re-tiled filter (block size 32 only); otherwise the
         # two-kernel form on the reference layout.
         self.retiled = None
@@ -362,12 +383,6 @@ class FullyConnectedBlockwiseInt4:
             capi.check(lib.lrtfc_pack_int4_blockwise(_ptr(self.filter), _ptr(self.scales),
                                                      self.out_depth, self.depth, 32,
                                                      _ptr(self.retiled), _stream()))
-
-    def _workspace(self, batches):
-        need = capi.calls().lrtfc_activation_workspace_bytes(batches, self.depth)
-        if self._ws is None or self._ws.numel() < need:
-            self._ws = torch.empty(need, dtype=torch.uint8, device="cuda")
-        return self._ws
 
     # From this many rows on a matrix-core GEMM streams the filter once for the whole batch,
     # whatever the shape (lrtfc_fc_blockwise_int4_preferred_form picks the form per shape).
@@ -391,12 +406,11 @@ class FullyConnectedBlockwiseInt4:
                 _ptr(self.filter), _ptr(self.scales), self.out_depth, self.depth, 32,
                 _ptr(self._gemm_filter), _stream()))
         need = capi.calls().lrtfc_fc_blockwise_int4_gemm_workspace_bytes(batches, self.depth)
-        if self._gemm_ws is None or self._gemm_ws.numel() < need:
-            self._gemm_ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+        ws, held = _scratch(x, need)
         capi.check(capi.calls().lrtfc_fc_blockwise_int4_gemm(
             _addr(x), _addr(self._gemm_filter), _addr(self.kfsum), _addr(self.bias), _addr(out), batches,
-            self.depth, self.out_depth, self.variant, _addr(self._gemm_ws), self._gemm_ws.numel(),
-            _call_stream()))
+            self.depth, self.out_depth, self.variant, ws, need, _call_stream()))
+        self._held = held
         return out
 
     def _nibble_filter_tensor(self):
@@ -418,19 +432,18 @@ class FullyConnectedBlockwiseInt4:
         the form for batches between decode and prefill. Same results as the other forms."""
         if self.blocksize != 32 or self.depth % 32:
             raise RuntimeError("call_gemm_nibbles needs block size 32")
-        lib = capi.load()
         x = x.contiguous()
         batches = x.numel() // self.depth
+        calls = capi.calls()
         if out is None:
             out = _empty_float32(x, batches, self.out_depth)
-        self._nibble_filter_tensor()
-        need = capi.calls().lrtfc_fc_blockwise_int4_gemm_workspace_bytes(batches, self.depth)
-        if self._gemm_ws is None or self._gemm_ws.numel() < need:
-            self._gemm_ws = torch.empty(need, dtype=torch.uint8, device="cuda")
-        capi.check(capi.calls().lrtfc_fc_blockwise_int4_gemm_nibbles(
-            _addr(x), _addr(self._nibble_filter), _addr(self.kfsum), _addr(self.bias), _addr(out),
-            batches, self.depth, self.out_depth, self.variant, _addr(self._gemm_ws),
-            self._gemm_ws.numel(), _call_stream()))
+        nibbles = self._nibble_filter_tensor()
+        need = calls.lrtfc_fc_blockwise_int4_gemm_workspace_bytes(batches, self.depth)
+        ws, held = _scratch(x, need)
+        capi.check(calls.lrtfc_fc_blockwise_int4_gemm_nibbles(
+            x.data_ptr(), nibbles.data_ptr(), self.kfsum.data_ptr(), _addr(self.bias), out.data_ptr(), batches,
+            self.depth, self.out_depth, self.variant, ws, need, _call_stream()))
+        self._held = held
         return out
 
     def __call__(self, x, out=None):
@@ -453,11 +466,13 @@ class FullyConnectedBlockwiseInt4:
                 _addr(x), _addr(self.retiled), _addr(self.kfsum), _addr(self.bias), _addr(out), batches,
                 self.depth, self.out_depth, self.variant, _call_stream()))
             return out
-        ws = self._workspace(batches)
+        need = capi.calls().lrtfc_activation_workspace_bytes(batches, self.depth)
+        ws, held = _scratch(x, need)
         capi.check(capi.load().lrtfc_fc_blockwise_int4(
             _ptr(x), _ptr(self.filter), _ptr(self.scales), _ptr(self.kfsum), _ptr(self.bias),
             _ptr(out), batches, self.depth, self.out_depth, self.blocksize, self.variant,
-            _ptr(ws), ws.numel(), _stream()))
+            ws, need, _stream()))
+        self._held = held
         return out
 
     # Rows deeper than FUSED_MAX_DEPTH fuse the quantizer for at most DEEP_FUSED_MAX_BATCHES
@@ -474,19 +489,16 @@ class FullyConnectedBlockwiseInt4:
         batches = x.numel() // self.depth
         if out is None:
             out = _empty_float32(x, batches, self.out_depth)
-        key = (batches, str(x.device))
-        if getattr(self, "_split_key", None) != key:
-            self._split_q = torch.empty((batches, self.depth), dtype=torch.int8, device=x.device)
-            self._split_sf = torch.empty(batches, dtype=torch.float32, device=x.device)
-            self._split_zp = torch.zeros(batches, dtype=torch.int32, device=x.device)
-            self._split_key = key
-        q, sf, zp = self._split_q, self._split_sf, self._split_zp
+        # Rows, scales and zero points, each on 256 bytes.
+        q_bytes, row_bytes = -(-batches * self.depth // 256) * 256, -(-batches * 4 // 256) * 256
+        q, held = _scratch(x, q_bytes + 2 * row_bytes)
+        sf, zp = q + q_bytes, q + q_bytes + row_bytes
         capi.check(capi.calls().lrtfc_batch_quantize_floats(
-            _addr(x), batches, self.depth, _addr(q), _addr(sf), _addr(zp), 1, self.variant,
-            _call_stream()))
+            _addr(x), batches, self.depth, q, sf, zp, 1, self.variant, _call_stream()))
         capi.check(capi.calls().lrtfc_fc_blockwise_int4_packed_quantized(
-            _addr(q), _addr(sf), _addr(zp), _addr(self.retiled), _addr(self.kfsum), _addr(self.bias),
-            _addr(out), batches, self.depth, self.out_depth, _call_stream()))
+            q, sf, zp, _addr(self.retiled), _addr(self.kfsum), _addr(self.bias), _addr(out), batches, self.depth,
+            self.out_depth, _call_stream()))
+        self._held = held
         return out
 
 
@@ -514,7 +526,6 @@ class FullyConnectedHybridInt4PerChannel:
         self.filter_scale = float(fs[0])
         self.bias = _dev(bias, torch.float32)
         self.activation = _act(activation)
-        self._ws = None
 
     # Above this many rows one pass of a matrix-core kernel over the int8 copy is cheaper: None = what
     # the library says for the shape (lrtfc_fc_hybrid_int4_per_channel_nibbles_max_batches).
@@ -528,34 +539,37 @@ class FullyConnectedHybridInt4PerChannel:
     def __call__(self, x, out=None, force_int8=False):
         x = x.contiguous()
         batches = x.numel() // self.depth
+        calls = capi.calls()
         if out is None:
             out = _empty_float32(x, batches, self.out_depth)
-        need = capi.calls().lrtfc_activation_workspace_bytes(batches, self.depth)
-        if self._ws is None or self._ws.numel() < need:
-            self._ws = torch.empty(need, dtype=torch.uint8, device="cuda")
-        lib = capi.load()
+        need = calls.lrtfc_activation_workspace_bytes(batches, self.depth)
+        ws, held = _scratch(x, need)
         if not force_int8 and batches <= self._nibble_max():
             if self._retiled_nibbles is None:
+                lib = capi.load()
                 self._retiled_nibbles = torch.empty(
                     lib.lrtfc_packed_int4_per_channel_bytes(self.out_depth, self.depth),
                     dtype=torch.uint8, device="cuda")
                 capi.check(lib.lrtfc_pack_int4_per_channel(
                     _ptr(self._nibbles), self.out_depth, self.depth, _ptr(self._retiled_nibbles),
                     _stream()))
-            capi.check(capi.calls().lrtfc_fc_hybrid_int4_per_channel_nibbles(
-                _addr(x), _addr(self._retiled_nibbles), _addr(self.pcs), self.filter_scale,
-                _addr(self.bias), _addr(out), batches, self.depth, self.out_depth, self.activation,
-                _addr(self._ws), self._ws.numel(), _call_stream()))
+            capi.check(calls.lrtfc_fc_hybrid_int4_per_channel_nibbles(
+                x.data_ptr(), self._retiled_nibbles.data_ptr(), _addr(self.pcs), self.filter_scale,
+                _addr(self.bias), out.data_ptr(), batches, self.depth, self.out_depth, self.activation,
+                ws, need, _call_stream()))
+            self._held = held
             return out
         if self._packed_int8 is None:
+            lib = capi.load()
             unpacked = torch.empty((self.out_depth, self.depth), dtype=torch.int8, device="cuda")
             capi.check(lib.lrtfc_unpack_int4(_ptr(self._nibbles), self.out_depth * self.depth,
                                              _ptr(unpacked), _stream()))
             self._packed_int8 = _pack_int8(unpacked)
-        capi.check(capi.calls().lrtfc_fc_hybrid_int4_per_channel_packed(
-            _addr(x), _addr(self._packed_int8), _addr(self.pcs), self.filter_scale, _addr(self.bias),
-            _addr(out), batches, self.depth, self.out_depth, self.activation, _addr(self._ws),
-            self._ws.numel(), _call_stream()))
+        capi.check(calls.lrtfc_fc_hybrid_int4_per_channel_packed(
+            x.data_ptr(), self._packed_int8.data_ptr(), _addr(self.pcs), self.filter_scale, _addr(self.bias),
+            out.data_ptr(), batches, self.depth, self.out_depth, self.activation, ws, need,
+            _call_stream()))
+        self._held = held
         return out
 
 

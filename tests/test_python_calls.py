@@ -1,4 +1,6 @@
 """The entry points without ctypes in between: same values, and arguments that do not fit are errors."""
+import ctypes as C
+
 import pytest
 
 from litert_amd import capi
@@ -70,3 +72,26 @@ def test_output_tensors_are_torch_empty_s(monkeypatch):
     monkeypatch.undo()
     if os.path.exists(os.path.join(os.path.dirname(capi.LIB_PATH), build.torch_tensors_name(torch.__version__))):
         assert native[0].__name__ == "empty_int8"
+
+
+def test_scratch_lives_as_long_as_it_is_held(monkeypatch):
+    """Native and plain: distinct memory while both are held, of any size; what is no tensor or no size is
+    refused."""
+    import torch
+    from litert_amd import build
+    from litert_amd import fully_connected as fc
+    native = fc._empty_functions()[2]
+    monkeypatch.setattr(build, "torch_tensors_name", lambda version: "missing.so")
+    plain = fc._empty_functions()[2]
+    like = torch.zeros(3)
+    for scratch in (native, plain):
+        held = [scratch(like, size) for size in (1, 1 << 20, 1 << 20, 0)]
+        assert len({address for address, _ in held[:3]}) == 3 and held[3][0] == 0
+        address, memory = held[1]
+        C.memset(address, 7, 1 << 20)
+        assert C.string_at(address + (1 << 20) - 1, 1) == b"\x07"
+        del held, memory
+        with pytest.raises((TypeError, AttributeError)):
+            scratch(None, 1)
+        with pytest.raises((OverflowError, RuntimeError)):
+            scratch(like, -1)
