@@ -11,6 +11,7 @@ import ctypes as C
 import importlib.machinery
 import importlib.util
 import os
+import threading
 
 import numpy as np
 import torch
@@ -101,6 +102,31 @@ def _pack_int8(filter_dev):
     packed = torch.empty(lib.lrtfc_packed_int8_filter_bytes(n, k), dtype=torch.int8, device="cuda")
     capi.check(lib.lrtfc_pack_int8_filter(_ptr(filter_dev), n, k, _ptr(packed), _stream()))
     return packed
+
+
+_layout_lock = threading.Lock()
+
+
+def _laid_out(op, name, make, stream):
+    """op.<name>: a layout of its filter, made on first use by launches on the current stream, and kept. The
+    first call on any other stream waits for the one that made it. A capture keeps nothing (what it launches
+    runs with the graph, not now): its graph has a layout of its own."""
+    layout = getattr(op, name)
+    if layout is not None and stream in op._behind[name][1]:
+        return layout
+    if torch.cuda.is_current_stream_capturing():
+        return make() if layout is None else layout
+    with _layout_lock:
+        layout = getattr(op, name)
+        if layout is None:
+            layout = make()
+            op._behind[name] = (torch.cuda.current_stream(), {stream})
+            setattr(op, name, layout)
+            return layout
+    maker, streams = op._behind[name]
+    torch.cuda.current_stream().wait_stream(maker)
+    streams.add(stream)
+    return layout
 
 
 def quantize_multiplier(m):
@@ -372,6 +398,8 @@ class FullyConnectedBlockwiseInt4:
             _ptr(self.kfsum), _stream()))
         self._gemm_filter = None
         self._nibble_filter = None
+        self._behind = {}  # see _laid_out
+        self._gemm_need = (0, 0)  # rows of the last call of call_gemm_nibbles and what their scratch takes
         # packed: one fused kernel on the re-tiled filter (block size 32 only); otherwise the
         # two-kernel form on the reference layout.
         self.retiled = None
@@ -393,39 +421,41 @@ class FullyConnectedBlockwiseInt4:
         re-tiled for it (made on first use and kept). Same results as the other forms."""
         if self.blocksize != 32 or self.depth % 32:
             raise RuntimeError("call_gemm needs block size 32")
-        lib = capi.load()
         x = x.contiguous()
         batches = x.numel() // self.depth
         if out is None:
             out = _empty_float32(x, batches, self.out_depth)
-        if self._gemm_filter is None:
-            self._gemm_filter = torch.empty(
-                lib.lrtfc_gemm_int4_blockwise_bytes(self.out_depth, self.depth), dtype=torch.uint8,
-                device="cuda")
-            capi.check(lib.lrtfc_pack_int4_blockwise_gemm(
-                _ptr(self.filter), _ptr(self.scales), self.out_depth, self.depth, 32,
-                _ptr(self._gemm_filter), _stream()))
+        stream = _call_stream()
+        gemm_filter = _laid_out(self, "_gemm_filter", self._pack_gemm_filter, stream)
         need = capi.calls().lrtfc_fc_blockwise_int4_gemm_workspace_bytes(batches, self.depth)
         ws, held = _scratch(x, need)
         capi.check(capi.calls().lrtfc_fc_blockwise_int4_gemm(
-            _addr(x), _addr(self._gemm_filter), _addr(self.kfsum), _addr(self.bias), _addr(out), batches,
-            self.depth, self.out_depth, self.variant, ws, need, _call_stream()))
+            _addr(x), _addr(gemm_filter), _addr(self.kfsum), _addr(self.bias), _addr(out), batches,
+            self.depth, self.out_depth, self.variant, ws, need, stream))
         self._held = held
         return out
+
+    def _pack_gemm_filter(self):
+        lib = capi.load()
+        packed = torch.empty(lib.lrtfc_gemm_int4_blockwise_bytes(self.out_depth, self.depth), dtype=torch.uint8,
+                             device="cuda")
+        capi.check(lib.lrtfc_pack_int4_blockwise_gemm(
+            _ptr(self.filter), _ptr(self.scales), self.out_depth, self.depth, 32, _ptr(packed), _stream()))
+        return packed
 
     def _nibble_filter_tensor(self):
         """The filter re-tiled at 4 bits per weight for the matrix cores (made once)."""
         if self.blocksize != 32 or self.depth % 32:
             raise RuntimeError("the 4-bit-resident matrix-core form needs block size 32")
-        if self._nibble_filter is None:
-            lib = capi.load()
-            self._nibble_filter = torch.empty(
-                lib.lrtfc_gemm_int4_blockwise_nibble_bytes(self.out_depth, self.depth),
-                dtype=torch.uint8, device="cuda")
-            capi.check(lib.lrtfc_pack_int4_blockwise_gemm_nibbles(
-                _ptr(self.filter), _ptr(self.scales), self.out_depth, self.depth, 32,
-                _ptr(self._nibble_filter), _stream()))
-        return self._nibble_filter
+        return _laid_out(self, "_nibble_filter", self._pack_nibble_filter, _call_stream())
+
+    def _pack_nibble_filter(self):
+        lib = capi.load()
+        packed = torch.empty(lib.lrtfc_gemm_int4_blockwise_nibble_bytes(self.out_depth, self.depth),
+                             dtype=torch.uint8, device="cuda")
+        capi.check(lib.lrtfc_pack_int4_blockwise_gemm_nibbles(
+            _ptr(self.filter), _ptr(self.scales), self.out_depth, self.depth, 32, _ptr(packed), _stream()))
+        return packed
 
     def call_gemm_nibbles(self, x, out=None):
         """The same GEMM on the filter kept at 4 bits per weight (made on first use and kept):
@@ -433,16 +463,21 @@ class FullyConnectedBlockwiseInt4:
         if self.blocksize != 32 or self.depth % 32:
             raise RuntimeError("call_gemm_nibbles needs block size 32")
         x = x.contiguous()
-        batches = x.numel() // self.depth
-        calls = capi.calls()
+        return self._call_gemm_nibbles(x, x.numel() // self.depth, out)
+
+    def _call_gemm_nibbles(self, x, batches, out):
+        calls, stream, bias = capi.calls(), _call_stream(), self.bias
         if out is None:
             out = _empty_float32(x, batches, self.out_depth)
-        nibbles = self._nibble_filter_tensor()
-        need = calls.lrtfc_fc_blockwise_int4_gemm_workspace_bytes(batches, self.depth)
+        nibbles = _laid_out(self, "_nibble_filter", self._pack_nibble_filter, stream)
+        rows, need = self._gemm_need
+        if rows != batches:
+            need = calls.lrtfc_fc_blockwise_int4_gemm_workspace_bytes(batches, self.depth)
+            self._gemm_need = (batches, need)
         ws, held = _scratch(x, need)
         capi.check(calls.lrtfc_fc_blockwise_int4_gemm_nibbles(
-            x.data_ptr(), nibbles.data_ptr(), self.kfsum.data_ptr(), _addr(self.bias), out.data_ptr(), batches,
-            self.depth, self.out_depth, self.variant, ws, need, _call_stream()))
+            x.data_ptr(), nibbles.data_ptr(), self.kfsum.data_ptr(), bias if bias is None else bias.data_ptr(),
+            out.data_ptr(), batches, self.depth, self.out_depth, self.variant, ws, need, stream))
         self._held = held
         return out
 
@@ -453,7 +488,7 @@ class FullyConnectedBlockwiseInt4:
             form = capi.calls().lrtfc_fc_blockwise_int4_preferred_form(batches, self.depth,
                                                                        self.out_depth)
             if form == capi.INT4_FORM_GEMM_NIBBLES:
-                return self.call_gemm_nibbles(x, out)
+                return self._call_gemm_nibbles(x, batches, out)
             if form == capi.INT4_FORM_GEMM_INT8:
                 return self.call_gemm(x, out)
         if out is None:
@@ -521,54 +556,64 @@ class FullyConnectedHybridInt4PerChannel:
         self._nibbles = nibbles
         self._retiled_nibbles = None
         self._packed_int8 = None
+        self._behind = {}  # see _laid_out
         fs = np.atleast_1d(np.asarray(filter_scales, dtype=np.float32))
         self.pcs = _dev(fs, torch.float32) if fs.size > 1 else None
         self.filter_scale = float(fs[0])
         self.bias = _dev(bias, torch.float32)
         self.activation = _act(activation)
+        self._library_nibble_max = lib.lrtfc_fc_hybrid_int4_per_channel_nibbles_max_batches(self.depth, self.out_depth)
+        self._need = (0, 0)  # rows of the last call and what their scratch takes
 
     # Above this many rows one pass of a matrix-core kernel over the int8 copy is cheaper: None = what
     # the library says for the shape (lrtfc_fc_hybrid_int4_per_channel_nibbles_max_batches).
     NIBBLE_MAX_BATCHES = None
 
     def _nibble_max(self):
-        if self.NIBBLE_MAX_BATCHES is not None:
-            return self.NIBBLE_MAX_BATCHES
-        return capi.calls().lrtfc_fc_hybrid_int4_per_channel_nibbles_max_batches(self.depth, self.out_depth)
+        limit = self.NIBBLE_MAX_BATCHES
+        return self._library_nibble_max if limit is None else limit
+
+    def _pack_nibbles(self):
+        lib = capi.load()
+        packed = torch.empty(lib.lrtfc_packed_int4_per_channel_bytes(self.out_depth, self.depth), dtype=torch.uint8,
+                             device="cuda")
+        capi.check(lib.lrtfc_pack_int4_per_channel(_ptr(self._nibbles), self.out_depth, self.depth, _ptr(packed),
+                                                   _stream()))
+        return packed
+
+    def _expand_int8(self):
+        unpacked = torch.empty((self.out_depth, self.depth), dtype=torch.int8, device="cuda")
+        capi.check(capi.load().lrtfc_unpack_int4(_ptr(self._nibbles), self.out_depth * self.depth, _ptr(unpacked),
+                                                 _stream()))
+        return _pack_int8(unpacked)
 
     def __call__(self, x, out=None, force_int8=False):
         x = x.contiguous()
         batches = x.numel() // self.depth
-        calls = capi.calls()
+        calls, stream = capi.calls(), _call_stream()
         if out is None:
             out = _empty_float32(x, batches, self.out_depth)
-        need = calls.lrtfc_activation_workspace_bytes(batches, self.depth)
+        rows, need = self._need
+        if rows != batches:
+            need = calls.lrtfc_activation_workspace_bytes(batches, self.depth)
+            self._need = (batches, need)
         ws, held = _scratch(x, need)
         if not force_int8 and batches <= self._nibble_max():
-            if self._retiled_nibbles is None:
-                lib = capi.load()
-                self._retiled_nibbles = torch.empty(
-                    lib.lrtfc_packed_int4_per_channel_bytes(self.out_depth, self.depth),
-                    dtype=torch.uint8, device="cuda")
-                capi.check(lib.lrtfc_pack_int4_per_channel(
-                    _ptr(self._nibbles), self.out_depth, self.depth, _ptr(self._retiled_nibbles),
-                    _stream()))
-            capi.check(calls.lrtfc_fc_hybrid_int4_per_channel_nibbles(
-                x.data_ptr(), self._retiled_nibbles.data_ptr(), _addr(self.pcs), self.filter_scale,
-                _addr(self.bias), out.data_ptr(), batches, self.depth, self.out_depth, self.activation,
-                ws, need, _call_stream()))
+            nibbles, pcs, bias = self._retiled_nibbles, self.pcs, self.bias
+            if nibbles is None or stream not in self._behind["_retiled_nibbles"][1]:
+                nibbles = _laid_out(self, "_retiled_nibbles", self._pack_nibbles, stream)
+            status = calls.lrtfc_fc_hybrid_int4_per_channel_nibbles(
+                x.data_ptr(), nibbles.data_ptr(), pcs if pcs is None else pcs.data_ptr(), self.filter_scale,
+                bias if bias is None else bias.data_ptr(), out.data_ptr(), batches, self.depth, self.out_depth,
+                self.activation, ws, need, stream)
+            if status:
+                capi.check(status)
             self._held = held
             return out
-        if self._packed_int8 is None:
-            lib = capi.load()
-            unpacked = torch.empty((self.out_depth, self.depth), dtype=torch.int8, device="cuda")
-            capi.check(lib.lrtfc_unpack_int4(_ptr(self._nibbles), self.out_depth * self.depth,
-                                             _ptr(unpacked), _stream()))
-            self._packed_int8 = _pack_int8(unpacked)
+        packed = _laid_out(self, "_packed_int8", self._expand_int8, stream)
         capi.check(calls.lrtfc_fc_hybrid_int4_per_channel_packed(
-            x.data_ptr(), self._packed_int8.data_ptr(), _addr(self.pcs), self.filter_scale, _addr(self.bias),
-            out.data_ptr(), batches, self.depth, self.out_depth, self.activation, ws, need,
-            _call_stream()))
+            x.data_ptr(), packed.data_ptr(), _addr(self.pcs), self.filter_scale, _addr(self.bias),
+            out.data_ptr(), batches, self.depth, self.out_depth, self.activation, ws, need, stream))
         self._held = held
         return out
 

@@ -37,8 +37,9 @@ def _op(cls, fields):
     tensors = ("filter", "scales", "pcs", "bias", "row_sums", "kfsum", "packed_filter", "retiled", "_gemm_filter",
                "_nibble_filter", "_nibbles", "_retiled_nibbles", "_packed_int8")
     vars(op).update({name: t for name in tensors}, depth=8192, out_depth=256, filter_scale=1.0, asymmetric=True,
-                    activation=0, variant=0, blocksize=32, _library_fused_max=2,
-                    _need=(0, 0))
+                    activation=0, variant=0, blocksize=32, _library_fused_max=2, _library_nibble_max=8, _gemm_need=(0, 0),
+                    _need=(0, 0), 
+                    _behind={name: (None, {0}) for name in tensors})
     vars(op).update(fields)
     return op
 
@@ -87,6 +88,61 @@ def test_two_calls_at_once_have_their_own_scratch(name, monkeypatch):
     assert mine and [entry for entry, _ in mine] == [entry for entry, _ in other]
     for (_, a), (_, b) in zip(mine, other):
         assert None not in a and not set(a) & set(b)
+
+
+def test_a_layout_in_the_making(monkeypatch):
+    """A layout that a call makes on first use: kept, and the first call on another stream waits for it; not
+    kept by a capture, which does not run what makes it."""
+    from litert_amd import fully_connected as fc
+    current, capturing, made, waits = ["a"], [True], [], []
+
+    class Stream:
+        def __init__(self, name):
+            self.name = name
+
+        def wait_stream(self, other):
+            waits.append((self.name, other.name))
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: Stream(current[0]))
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    op = _op("FullyConnectedHybridInt4PerChannel", {"_packed_int8": None, "_behind": {}})
+    op._expand_int8 = lambda: made.append(torch.zeros(1)) or made[-1]
+
+    def layout(stream):
+        current[0] = stream
+        return fc._laid_out(op, "_packed_int8", op._expand_int8, stream)
+    assert layout("a") is made[0] and layout("a") is made[1] and op._packed_int8 is None
+    capturing[0] = False
+    kept = layout("a")
+    assert kept is made[2] and op._packed_int8 is kept
+    assert layout("a") is kept and not waits
+    assert layout("b") is kept and layout("b") is kept and waits == [("b", "a")]
+    assert layout("c") is kept and waits == [("b", "a"), ("c", "a")]
+    capturing[0] = True
+    assert layout("d") is kept and layout("a") is kept and len(made) == 3 and len(waits) == 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 20])
+def test_a_layout_first_made_in_a_capture(rows):
+    from litert_amd import fully_connected as fc
+    rng = np.random.default_rng(rows)
+    packed = rng.integers(0, 256, (300, 320), dtype=np.uint8)
+    scales = rng.uniform(0.01, 0.1, 300).astype(np.float32)
+    x = rng.standard_normal((rows, 640)).astype(np.float32)
+    want = oracle.fc_hybrid_int4_per_channel(x, packed, 300, scales).view(np.uint32)
+    op = fc.FullyConnectedHybridInt4PerChannel(packed, 640, scales)
+    xs, out = torch.from_numpy(x).cuda(), torch.empty((rows, 300), device="cuda")
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        op(xs, out=out)
+    assert np.array_equal(op(xs).cpu().numpy().view(np.uint32), want)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy().view(np.uint32), want)
+        assert np.array_equal(op(xs).cpu().numpy().view(np.uint32), want)
 
 
 @pytest.mark.gpu
