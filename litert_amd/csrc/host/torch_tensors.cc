@@ -10,6 +10,7 @@
 #include <pybind11/pybind11.h>
 
 #include <memory>
+#include <utility>
 
 namespace {
 
@@ -23,7 +24,13 @@ PyObject* Empty(PyObject*, PyObject* const* args, Py_ssize_t count) {
   const long long columns = PyLong_AsLongLong(args[2]);
   if (PyErr_Occurred()) return nullptr;
   const c10::Device device = THPVariable_Unpack(args[0]).device();
-  return THPVariable_Wrap(at::empty({rows, columns}, at::TensorOptions().dtype(kType).device(device)));
+  at::Tensor out;
+  {
+    // As torch.empty does: an allocation that has to ask the device, or wait for it, stops no other thread.
+    pybind11::gil_scoped_release unlocked;
+    out = at::empty({rows, columns}, at::TensorOptions().dtype(kType).device(device));
+  }
+  return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }
 

@@ -38,7 +38,7 @@ def _op(cls, fields):
                "_nibble_filter", "_nibbles", "_retiled_nibbles", "_packed_int8")
     vars(op).update({name: t for name in tensors}, depth=8192, out_depth=256, filter_scale=1.0, asymmetric=True,
                     activation=0, variant=0, blocksize=32, _library_fused_max=2, _library_nibble_max=8, _gemm_need=(0, 0),
-                    _need=(0, 0), 
+                    _need=(0, 0),
                     _behind={name: (None, {0}) for name in tensors})
     vars(op).update(fields)
     return op

@@ -95,3 +95,31 @@ def test_scratch_lives_as_long_as_it_is_held(monkeypatch):
             scratch(None, 1)
         with pytest.raises((OverflowError, RuntimeError)):
             scratch(like, -1)
+
+
+def test_output_allocation_lets_other_threads_run():
+    """An allocation that takes its time (here: one that is filled) does not hold the interpreter's lock."""
+    import threading
+    import time
+    import torch
+    from litert_amd import fully_connected as fc
+    ticks, stop = [], threading.Event()
+
+    def tick():
+        while not stop.is_set():
+            ticks.append(time.perf_counter())
+            time.sleep(0.001)
+    like = torch.zeros(1)
+    torch.use_deterministic_algorithms(True)
+    thread = threading.Thread(target=tick)
+    thread.start()
+    try:
+        for empty, columns in zip(fc._empty_functions(), (1 << 30, 1 << 28)):
+            start = time.perf_counter()
+            empty(like, 1, columns)
+            took = time.perf_counter() - start
+            assert any(start + 0.3 * took < t < start + 0.7 * took for t in ticks), took
+    finally:
+        torch.use_deterministic_algorithms(False)
+        stop.set()
+        thread.join()
