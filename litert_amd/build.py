@@ -85,9 +85,14 @@ def torch_tensors_name(torch_version):
 
 
 def build_torch_tensors():
-    """Output tensors for the Python ops without torch.empty's argument parsing (host code only).
-    Without torch's or the interpreter's headers there is none, and the ops use torch.empty."""
-    import torch
+    """Output tensors and scratch for the Python ops without torch.empty's argument parsing (host code
+    only). Without torch or the interpreter's headers, or where they do not compile, there is none, and the
+    ops use torch.empty; nothing else needs it."""
+    try:
+        import torch
+    except (ImportError, OSError) as e:
+        print("no torch (%s): litert_amd_tensors is not built" % e, flush=True)
+        return None
     root = os.path.dirname(torch.__file__)
     python = sysconfig.get_paths()["include"]
     if not (os.path.exists(os.path.join(python, "Python.h")) and
@@ -95,12 +100,18 @@ def build_torch_tensors():
         print("no headers of torch or Python: litert_amd_tensors is not built", flush=True)
         return None
     out = os.path.join(LIB, torch_tensors_name(torch.__version__))
-    _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-w",
-          "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI,
-          "-I" + os.path.join(root, "include"),
-          "-I" + os.path.join(root, "include", "torch", "csrc", "api", "include"), "-I" + python,
-          "-o", out, os.path.join(CSRC, "host", "torch_tensors.cc"), "-L" + os.path.join(root, "lib"),
-          "-lc10", "-ltorch_cpu", "-ltorch_python"])
+    try:
+        _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-w",
+              "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI,
+              "-I" + os.path.join(root, "include"),
+              "-I" + os.path.join(root, "include", "torch", "csrc", "api", "include"), "-I" + python,
+              "-o", out, os.path.join(CSRC, "host", "torch_tensors.cc"), "-L" + os.path.join(root, "lib"),
+              "-lc10", "-ltorch_cpu", "-ltorch_python"])
+    except (subprocess.CalledProcessError, OSError) as e:
+        print("%s: litert_amd_tensors is not built" % e, flush=True)
+        if os.path.exists(out):
+            os.remove(out)  # an earlier build's, which the ops would load
+        return None
     return out
 
 
@@ -126,8 +137,8 @@ def build_bench_probes():
 
 
 def build_all():
-    outs = [build_fc(), build_python_calls(), build_torch_tensors(), build_bench_probes(),
-            build_delegate()]
+    outs = [build_fc(), build_python_calls(), build_bench_probes(), build_delegate(),
+            build_torch_tensors()]
     return [out for out in outs if out]
 
 
