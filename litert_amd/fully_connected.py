@@ -12,6 +12,7 @@ import importlib.machinery
 import importlib.util
 import os
 import threading
+import warnings
 
 import numpy as np
 import torch
@@ -75,9 +76,13 @@ def _empty_functions():
     if os.path.exists(path):
         loader = importlib.machinery.ExtensionFileLoader("litert_amd_tensors", path)
         spec = importlib.util.spec_from_file_location("litert_amd_tensors", path, loader=loader)
-        module = importlib.util.module_from_spec(spec)
-        loader.exec_module(module)
-        return module.empty_int8, module.empty_float32, module.scratch
+        try:
+            module = importlib.util.module_from_spec(spec)
+            loader.exec_module(module)
+            return module.empty_int8, module.empty_float32, module.scratch
+        except (ImportError, AttributeError) as e:  # (of another torch, or an older build)
+            warnings.warn("%s does not load (%s; `python -m litert_amd.build` makes it again): ops allocate "
+                          "through torch.empty, 1 us more each" % (path, e))
 
     def empty(dtype):
         return lambda like, rows, columns: torch.empty((rows, columns), dtype=dtype, device=like.device)

@@ -123,3 +123,18 @@ def test_output_allocation_lets_other_threads_run():
         torch.use_deterministic_algorithms(False)
         stop.set()
         thread.join()
+
+
+def test_a_helper_that_does_not_load_is_done_without(monkeypatch, tmp_path):
+    """A file of the right name that this torch cannot load (one rebuilt under the same version)."""
+    import torch
+    from litert_amd import build
+    from litert_amd import fully_connected as fc
+    broken = tmp_path / "broken.so"
+    broken.write_bytes(b"no library")
+    monkeypatch.setattr(build, "torch_tensors_name", lambda version: str(broken))
+    with pytest.warns(UserWarning, match="torch.empty"):
+        empty_int8, empty_float32, scratch = fc._empty_functions()
+    like = torch.zeros(1)
+    assert empty_int8(like, 2, 3).dtype == torch.int8 and empty_float32(like, 2, 3).dtype == torch.float32
+    assert scratch(like, 16)[0] != 0
