@@ -73,11 +73,26 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
   const int steps = (slabs + 1) / 2;
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   const int total = tiles_m * tiles_n;
+  // The arguments that the first loads need, in registers ahead of the tile's arithmetic: the compiler reads
+  // them behind it otherwise, and the workgroup waits once more (2048 x 4096 -> 4096 33.8 us, so 33.5).
+  if (EPI == Int8Epilogue::kRequantize) {
+    asm volatile("" ::"s"(a.multipliers), "s"(a.shifts), "s"(a.bias_i32), "s"(a.filter_row_sums),
+                 "s"(a.per_channel), "s"(a.input_offset), "s"(a.output_offset), "s"(a.act_min),
+                 "s"(a.act_max));
+  } else {
+    asm volatile("" ::"s"(a.per_channel_scales), "s"(a.bias_f32), "s"(a.zero_points), "s"(a.filter_row_sums));
+  }
+  asm volatile("" ::"s"(a.input), "s"(a.filter));
 
   // Workgroups are dealt round-robin to the 8 XCDs; give each XCD a contiguous range of tile
-  // ids, ordered so that a range is a compact rectangle whose operands stay in that XCD's L2.
-  int id = blockIdx.x;
-  if (total % 8 == 0) id = (blockIdx.x % 8) * (total / 8) + blockIdx.x / 8;
+  // ids, ordered so that a range is a compact rectangle whose operands stay in that XCD's L2. The first
+  // total % 8 XCDs have a tile more than the others. (Grids that are no multiple of 8 went unsorted: 5000
+  // launches of 65 to 3000 rows, of which two thirds are such grids, us unsorted -> sorted: 64 x 128 tiles
+  // 0.92 of the time in the mean, 128 x 128 0.95, 128 x 256 0.97; where 128 x 128 tiles had taken the place
+  // of a sorted grid of 128 x 256, 1778 x 1949 -> 6928 55.6 -> 50.3, 44.5 before, 640 x 7256 -> 3511 from
+  // memory 46.0 -> 40.4, 39.9 before.)
+  const int xcd = static_cast<int>(blockIdx.x % 8);
+  const int id = xcd * (total / 8) + min(xcd, total % 8) + static_cast<int>(blockIdx.x / 8);
   const int width = kGroupM * tiles_n;
   const int group = id / width;
   const int first_m = group * kGroupM;

@@ -99,3 +99,11 @@ def test_tail_rows_and_the_whole_zero_exit(fc, zero_rows):  # noqa: F811
     want = oracle.fc_hybrid(x, w[:8], pcs[:8], bias=bias[:8])
     assert np.array_equal(got.view(np.uint32), np.ascontiguousarray(want).view(np.uint32))
     assert (np.signbit(got[0, 0]) == (zero_rows == "all")) or zero_rows == "tail"
+
+
+# Grids of every remainder by the eight XCDs, to each of which a contiguous range of tiles is dealt: 513 to
+# 534 tiles of 64 x 128, and 129 to 150 of 128 x 256.
+@pytest.mark.parametrize("B,K,N", [(129, 512, 128 * n) for n in range(171, 179)] +
+                         [(257, 96, 256 * n) for n in range(43, 51)])
+def test_grids_of_any_remainder(fc, B, K, N):  # noqa: F811
+    _int8(fc, B, K, N)
