@@ -88,9 +88,8 @@ __global__ __launch_bounds__(kThreads, 1) void FcInt8PackedGemmKernel(FcInt8Args
   // ids, ordered so that a range is a compact rectangle whose operands stay in that XCD's L2. The first
   // total % 8 XCDs have a tile more than the others. (Grids that are no multiple of 8 went unsorted: 5000
   // launches of 65 to 3000 rows, of which two thirds are such grids, us unsorted -> sorted: 64 x 128 tiles
-  // 0.92 of the time in the mean, 128 x 128 0.95, 128 x 256 0.97; where 128 x 128 tiles had taken the place
-  // of a sorted grid of 128 x 256, 1778 x 1949 -> 6928 55.6 -> 50.3, 44.5 before, 640 x 7256 -> 3511 from
-  // memory 46.0 -> 40.4, 39.9 before.)
+  // 0.92 of the time in the mean, 128 x 128 0.95, 128 x 256 0.97; 1485 x 768 -> 9536, where 900 of the second
+  // had taken the place of 456 of the third, 29.3 -> 23.8, with those 24.7.)
   const int xcd = static_cast<int>(blockIdx.x % 8);
   const int id = xcd * (total / 8) + min(xcd, total % 8) + static_cast<int>(blockIdx.x / 8);
   const int width = kGroupM * tiles_n;
@@ -572,7 +571,9 @@ bool DeepRing(const FcInt8Args& a) { return a.depth > 2048 && SmallTiles(a) <= k
 // for (us, 64 x 128 -> 128 x 128, filters in the cache / from memory): 350 x 7792 -> 6425 50.6 -> 35.6
 // / 50.1 -> 47.6, 494 x 7376 -> 4530 36.5 -> 30.7 / 48.8 -> 43.5, 256 x 4096 -> 14336 22.8 -> 21.6 / 30.8
 // -> 28.1; least 1110 x 2240 -> 2805 14.9 -> 14.0 / 15.9 -> 15.3. (Shorter walks: 819 x 1392 -> 4231
-// 11.3 -> 12.2.)
+// 11.3 -> 12.2.) Of 370 such sizes with 156 tiles and more it takes 0.90 / 0.93 of the time of 64 x 128, float
+// outputs 0.94 / 0.97; of 100 with fewer 0.89 / 1.04 and 0.93 / 1.08 (640 x 7256 -> 3511, 140 tiles: 41.5 ->
+// 39.8 / 40.7 -> 45.6): half the CUs ask for the whole filter.
 bool TakesSquareTiles(const FcInt8Args& a) {
   if (LargeTiles(a) >= kMinLargeTiles) return LargeTiles(a) > kCus || a.depth > 2048;
   return a.depth >= 2048 && SmallTiles(a) > kCus && SquareTiles(a) <= kCus;
@@ -590,23 +591,31 @@ bool FcInt8PackedGemmSupports(const FcInt8Args& a) {
 // with the depth split over the wavefronts. Above that line smaller tiles win where the walk is
 // short, because of a large tile's prologue and epilogue (9 us of a workgroup's time, and no second
 // workgroup on its CU to hide them), and where large tiles make exactly half a round.
-// 128 sizes between 100 x 2048 -> 320 and 2048 x 4096 -> 14336 measured on every form, filters in the
-// cache / from memory (us, 128 x 256 -> chosen):
+// (us, 128 x 256 -> chosen, filters in the cache / from memory:)
 //   more than a round, depth 512 to 2048, to 128 x 128: 2048 x 1024 -> 14336 52.6 -> 47.5 / 57.5 -> 51.5,
-//     700 x 1024 -> 14336 24.7 -> 20.8 / 27.7 -> 23.3, 1715 x 560 -> 15924 52.4 -> 41.9 / 53.1 -> 42.3;
-//     least 1274 x 1712 -> 8524 35.1 -> 33.9 / 36.8 -> 36.0. Float outputs gain more: hybrid
-//     2048 x 1024 -> 14336 76 -> 63 / 83 -> 73. (Deeper: 769 x 2272 -> 14793 47 -> 50.)
-//   a round at most, depth 512 to 768, to 64 x 128: 1506 x 672 -> 2567 13.8 -> 8.5 / 14.5 -> 9.2,
-//     1806 x 608 -> 2575 13.4 -> 10.5 / 14.2 -> 11.3; least 1067 x 544 -> 6582 14.3 -> 12.9 / 15.3 -> 14.0.
-//     (Deeper: 750 x 912 -> 8538 16.5 -> 20.8.)
-//   half a round, depth above 2048, to one round of 128 x 128: 1000 x 4096 -> 4096 26.0 -> 22.4 / 30.2 -> 25.3.
+//     700 x 1024 -> 14336 24.7 -> 20.8 / 27.7 -> 23.3, 1715 x 560 -> 15924 52.4 -> 41.9 / 53.1 -> 42.3. Float
+//     outputs gain more: hybrid 2048 x 1024 -> 14336 76 -> 63 / 83 -> 73. Of 220 such sizes where they fill
+//     less than two rounds for one of 128 x 256 0.85 of the time in the mean (least 1.03), of 100 where they fill
+//     two 0.96 (least 1.04). Rows that end inside a 16-byte piece are read twice as often from addresses that are no
+//     multiple of 16: deeper than 1024 and in two rounds for one they lose (1.05 of the time in the mean,
+//     1778 x 1949 -> 6928 46.9 -> 60 / 44.5 -> 53, 1600 x 1434 -> 7948 38.6 -> 46 / 38.2 -> 42) and stay.
+//   a round at most, depth 512 to 768, to 64 x 128 as long as those are three rounds: 1506 x 672 -> 2567 13.8 ->
+//     8.5 / 14.5 -> 9.2, 1806 x 608 -> 2575 13.4 -> 10.5 / 14.2 -> 11.3; of 66 such sizes 0.86 of the time in the
+//     mean, least 1.01. (In a fourth round: 392 x 704 -> 14656 14.3 -> 17.7 / 13.2 -> 17.1, 652 x 576 -> 9024
+//     12.4 -> 15.9 / 12.0 -> 14.3. Deeper: 750 x 912 -> 8538 16.5 -> 20.8.)
+//   half a round, depth above 2048, to one round of 128 x 128: 1000 x 4096 -> 4096 26.0 -> 22.4 / 30.2 -> 25.3; 17
+//     sizes, least 0.83 of the time.
 // Shallower launches than 512 are not in those figures and stay.
 Int8GemmForm FcInt8PackedGemmForm(const FcInt8Args& a) {
   const int large = LargeTiles(a);
   if (large >= kMinLargeTiles) {
-    const bool smaller = large > kCus ? a.depth >= 512 && a.depth <= 2048
-                                      : (a.depth >= 512 && a.depth <= 768) ||
-                                            (a.depth > 2048 && SquareTiles(a) <= kCus);
+    const int square = SquareTiles(a);
+    const auto rounds = [](int tiles) { return (tiles + kCus - 1) / kCus; };
+    const bool two_for_one = rounds(square) >= 2 * rounds(large);
+    const bool smaller = large > kCus ? a.depth >= 512 && a.depth <= 2048 &&
+                                            !(a.depth % 16 && a.depth > 1024 && two_for_one)
+                                      : (a.depth >= 512 && a.depth <= 768 && SmallTiles(a) <= 3 * kCus) ||
+                                            (a.depth > 2048 && square <= kCus);
     return smaller ? Int8GemmForm::kSmallerTiles : Int8GemmForm::kTiles128x256;
   }
   return FcInt8SplitGemmBeatsTiles(a, SmallTiles(a)) ? Int8GemmForm::kSplit

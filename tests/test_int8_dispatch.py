@@ -63,3 +63,19 @@ def test_no_row_count_falls_between_the_rules():
     (4, 16384, 256, capi.INT8_KERNEL_GEMV), (5, 16384, 256, capi.INT8_KERNEL_SPLIT)])
 def test_up_to_sixteen_rows(rows, depth, channels, kernel):
     assert _kernel(rows, depth, channels) == kernel
+
+
+@pytest.mark.parametrize("rows,depth,channels,kernel", [
+    (768, 512, 8192, capi.INT8_KERNEL_TILES_64X128), (768, 512, 8193, capi.INT8_KERNEL_TILES_128X256),  # 768 tiles
+    (392, 704, 14656, capi.INT8_KERNEL_TILES_128X256), (652, 576, 9024, capi.INT8_KERNEL_TILES_128X256)])
+def test_short_walks_in_up_to_three_rounds_of_64x128(rows, depth, channels, kernel):
+    assert _kernel(rows, depth, channels) == kernel
+
+
+@pytest.mark.parametrize("rows,depth,channels,kernel", [
+    (1778, 1949, 6928, capi.INT8_KERNEL_TILES_128X256), (1600, 1434, 7948, capi.INT8_KERNEL_TILES_128X256),
+    (1778, 1952, 6928, capi.INT8_KERNEL_TILES_64X128),  # whole pieces
+    (1778, 1023, 6928, capi.INT8_KERNEL_TILES_64X128),  # shallow
+    (1536, 1949, 8192, capi.INT8_KERNEL_TILES_64X128)])  # 768 tiles: three rounds for two
+def test_ragged_rows_read_twice_in_two_rounds_for_one(rows, depth, channels, kernel):
+    assert _kernel(rows, depth, channels) == kernel
