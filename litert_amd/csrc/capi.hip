@@ -1009,14 +1009,25 @@ int lrtfc_pack_int4_per_channel(const uint8_t* packed_filter, int out_depth, int
 }
 
 int lrtfc_fc_hybrid_int4_per_channel_nibbles_max_batches(int depth, int out_depth) {
+  // (us, nibbles / int8, filters in the cache; over 36,000 launches of up to 32 rows. From memory the line is
+  // the same but where it is said.)
   // One pass of the nibble kernel takes 16 rows, as long as 64 KB of LDS hold them; beyond either it
-  // walks a ring of loads or the filter again, and the int8 copy wins though twice the bytes (us,
-  // nibbles / int8, filters in the cache): 17 x 4096 -> 4096 13.0 / 8.0, 17 x 4096 -> 14336 17.1 / 14.7,
-  // 32 x 1024 -> 1024 9.7 / 6.3, 16 x 5120 -> 2048 17.8 / 8.9, 10 x 8192 -> 4096 15.6 / 10.7, 16 x 11008 ->
-  // 4096 29.9 / 13.7, 32 x 16384 -> 2048 64.5 / 17.7; within both, 16 x 4096 -> 14336 11.0 / 13.5,
-  // 12 x 5120 -> 8192 11.1 / 12.4, 8 x 8192 -> 1024 9.4 / 10.0. From memory the line is the same. Filters
-  // of fewer than 128 channels, a handful of workgroups on either, keep to the one layout they had.
+  // walks a ring of loads or the filter again, and the int8 copy wins though twice the bytes:
+  // 17 x 4096 -> 4096 13.0 / 8.0, 17 x 4096 -> 14336 17.1 / 14.7, 32 x 1024 -> 1024 9.7 / 6.3,
+  // 16 x 5120 -> 2048 17.8 / 8.9, 10 x 8192 -> 4096 15.6 / 10.7, 16 x 11008 -> 4096 29.9 / 13.7, 32 x 16384 -> 2048
+  // 64.5 / 17.7; within both, 16 x 4096 -> 14336 11.0 / 13.5, 12 x 5120 -> 8192 11.1 / 12.4, 8 x 8192 -> 1024 9.4 /
+  // 10.0. (Five and six rows deeper than 12288 on more than 3000 channels: 0.90 of the time, from memory 1.15.)
+  // More than 8192 channels: the int8 copy's rows up to 16 go to a GEMV that has no other way for deep ones
+  // either, and reads twice the bytes: 13 x 7488 -> 9344 21.4 / 36.1, 16 x 5312 -> 12160 21.0 / 34.5, 5 x 16384 ->
+  // 16384 33.5 / 66.9, 16 x 16384 -> 16384 70.1 / 145; 17 rows there 70.4 / 47.6. And of 17 to 32 rows two
+  // stretches gain nothing: 20 x 3072 -> 9280 15.8 / 17.2, 17 x 3584 -> 10224 17.5 / 18.4; 17 x 900 -> 16400 11.5 /
+  // 13.9 (16384 channels 11.2 / 8.7).
+  // Filters of fewer than 128 channels, a handful of workgroups on either, keep to the one layout they had.
   if (out_depth < 128 || depth <= 0) return 32;
+  if (out_depth > 8192) {
+    const bool two_passes = out_depth <= 10224 ? depth > 2048 && depth <= 4096 : out_depth > 16384 && depth < 1024;
+    return two_passes ? 32 : 16;
+  }
   const int fit = 65536 / depth;
   return fit > 16 ? 16 : fit < 4 ? 4 : fit;
 }

@@ -60,6 +60,33 @@ def test_per_channel_int4_rows_on_nibbles(depth, rows):
     assert capi.load().lrtfc_fc_hybrid_int4_per_channel_nibbles_max_batches(depth, 127) == 32
 
 
+@pytest.mark.parametrize("depth,channels,rows", [
+    (7488, 8192, 8), (7488, 8193, 16), (16384, 16384, 16), (16384, 4096, 4), (4096, 14336, 16), (60000, 9000, 16),
+    (2048, 9000, 16), (2050, 9000, 32), (4096, 10224, 32), (4098, 10224, 16), (4096, 10225, 16), (3072, 8192, 16),
+    (1022, 16385, 32), (1024, 16385, 16), (1022, 16384, 16)])
+def test_per_channel_int4_rows_on_nibbles_of_wide_filters(depth, channels, rows):
+    assert capi.load().lrtfc_fc_hybrid_int4_per_channel_nibbles_max_batches(depth, channels) == rows
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("depth,channels", [(5122, 8200), (2050, 8200), (514, 16390)])
+def test_per_channel_int4_rows_of_wide_filters(depth, channels):
+    import numpy as np
+    import torch
+    import oracle
+    from litert_amd import fully_connected as fc
+    rng = np.random.default_rng(depth)
+    packed = rng.integers(0, 256, (channels, depth // 2), dtype=np.uint8)
+    scales = rng.uniform(0.01, 0.1, channels).astype(np.float32)
+    x = rng.standard_normal((33, depth)).astype(np.float32)
+    some = np.r_[0:40, channels - 40:channels]
+    want = oracle.fc_hybrid_int4_per_channel(x, packed[some], some.size, scales[some]).view(np.uint32)
+    op = fc.FullyConnectedHybridInt4PerChannel(packed, depth, scales)
+    for rows in (5, 13, 16, 17, 32, 33):
+        got = op(torch.from_numpy(x[:rows]).cuda()).cpu().numpy()[:, some]
+        assert np.array_equal(got.view(np.uint32), want[:rows])
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("depth,channels", [(34, 20), (1030, 131), (4096, 300), (5122, 128), (11010, 129)])
 def test_per_channel_int4_rows_around_the_line(depth, channels):
