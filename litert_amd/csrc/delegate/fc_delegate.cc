@@ -568,6 +568,7 @@ struct FcNode {
 constexpr int kInt4FusedMaxDepth = 4096;
 constexpr int kInt4DeepFusedMaxBatches = 2;
 constexpr int kInt4GroupedMaxOutDepth = 511 * 16;  // wider ones fill the chip by themselves from five rows on
+constexpr int kInt4PerChannelNibbleMaxBatches = 32;  // of a node that holds nibbles already
 
 // Up to this many bytes of host outputs per partition are written by the kernels directly into
 // page-locked host memory instead of being copied there afterwards. The invariant this rests on:
@@ -1094,8 +1095,12 @@ TfLiteStatus PrepareNode(TfLiteContext* ctx, PartitionKernel* k, FcNode* n) {
     n->per_channel = fq->scale->size > 1;
     n->filter_scale = fq->scale->data[0];
     n->use_retiled = true;
+    // A node that holds its filter as nibbles keeps them up to kInt4PerChannelNibbleMaxBatches rows: the
+    // int8 copy saves it 5 us a launch (17 x 4096 -> 4096 13.0 -> 8.0) or more of deep rows, but every
+    // resize across the line would upload the model's filter again, expand and re-tile it.
     n->nibble_layout =
-        n->batches <= lrtfc_fc_hybrid_int4_per_channel_nibbles_max_batches(n->depth, n->out_depth);
+        n->batches <= lrtfc_fc_hybrid_int4_per_channel_nibbles_max_batches(n->depth, n->out_depth) ||
+        (n->have_nibbles && n->batches <= kInt4PerChannelNibbleMaxBatches);
     if (weights > 0 && !(n->nibble_layout ? n->have_nibbles : n->have_retiled)) {
       DeviceBuffer nibbles;
       RETURN_IF_HIP(ctx, nibbles.Upload(filter.data.raw, (weights + 1) / 2, s));
@@ -2191,6 +2196,8 @@ int litert_amd_describe_partition(const void* user_data, char* out, size_t out_s
     }
     // "m4" / "m8": blockwise int4 on the matrix-core GEMM, weights of 4 bits or expanded to 8
     if (n.gemm_layout) text += n.gemm_nibbles ? "/m4" : "/m8";
+    // "p4" / "p8": per-channel int4 on nibbles or their int8 copy
+    if (n.kind == FcKind::kHybridInt4) text += n.nibble_layout ? "/p4" : "/p8";
   }
   std::snprintf(out, out_size, "%s", text.c_str());
   return static_cast<int>(k->groups.size());

@@ -1031,3 +1031,35 @@ def test_completion_mark_follows_the_work_enqueued_before_it():
     torch.cuda.synchronize()
     assert lib.lrtfc_mark_completion(None, 1, stream) != 0
     assert lib.lrtfc_mark_completion(word.data_ptr() + 2, 1, stream) != 0
+
+
+def test_per_channel_int4_resized_around_its_line_keeps_its_nibbles():
+    """A fresh node takes the int8 copy from 17 rows on (K <= 4096); one that holds nibbles keeps them up to
+    32 rows, so that resizes between decode and short batches re-tile nothing."""
+    K, N, most = 64, 256, 40
+    rng = np.random.default_rng(11)
+    packed = rng.integers(0, 256, (N, K // 2), dtype=np.uint8)
+    fs = rng.uniform(0.01, 0.1, N).astype(np.float32)
+    xs = rng.standard_normal((most, K)).astype(np.float32)
+    want = oracle.fc_hybrid_int4_per_channel(xs, packed, N, fs, None, 0)
+    cases = [((1, 20, 32, 1, 33, 20, 17, 16, 20), ["p4", "p4", "p4", "p4", "p8", "p8", "p8", "p4", "p4"]),
+             ((20, 17, 1, 20), ["p8", "p8", "p4", "p4"])]
+    for sizes, expected in cases:
+        with FakeHost() as h:
+            x = h.tensor(FLOAT32, (sizes[0], K), data=xs[:sizes[0]])
+            w = h.tensor(INT4, (N, K), data=packed, const=True)
+            h.affine(w, fs)
+            y = h.tensor(FLOAT32, (sizes[0], N))
+            h.fc(x, w, None, y)
+            assert h.load_delegate() == 0, h.errors()
+            assert h.modify_graph_with_delegate() == OK and h.allocate_tensors() == OK, h.errors()
+            forms = []
+            for rows in sizes:
+                h.resize(x, (rows, K))
+                h.resize(y, (rows, N))
+                h.write(x, xs[:rows])
+                assert h.allocate_tensors() == OK, h.errors()
+                forms.append(h.describe_partition(h.plan()[0][2])[1].split("/")[-1])
+                assert h.invoke() == OK, h.errors()
+                assert np.array_equal(h.read(y).view(np.uint32), want[:rows].view(np.uint32)), rows
+            assert forms == expected
