@@ -511,6 +511,10 @@ int lrtfc_fc_blockwise_int4_gemm(const float* input, const uint8_t* gemm_filter,
  * this nibble-resident GEMM, or the int8-expanded GEMM. All three give the same bits; a caller
  * keeps the filter in the one layout its batch size asks for. Pure host function. */
 int lrtfc_fc_blockwise_int4_preferred_form(int batches, int depth, int out_depth);
+/* Rows per pass over the filter of the streaming kernel on a single node: of float rows (quantized == 0,
+ * lrtfc_fc_blockwise_int4_packed) or of int8 rows (lrtfc_fc_blockwise_int4_packed_quantized) that lie on 16
+ * bytes. More rows are further launches. For tests and profiles. Pure host function. */
+int lrtfc_fc_blockwise_int4_rows_per_launch(int depth, int out_depth, int quantized);
 size_t lrtfc_gemm_int4_blockwise_nibble_bytes(int out_depth, int depth);
 int lrtfc_pack_int4_blockwise_gemm_nibbles(const uint8_t* packed_filter,
                                            const uint16_t* scales_f16, int out_depth, int depth,

@@ -91,6 +91,7 @@ SYMBOLS = [
     ("lrtfc_fc_blockwise_int4_gemm_workspace_bytes", _sz, [_i, _i]),
     ("lrtfc_fc_blockwise_int4_gemm", _i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp, _sz, _vp]),
     ("lrtfc_fc_blockwise_int4_preferred_form", _i, [_i, _i, _i]),
+    ("lrtfc_fc_blockwise_int4_rows_per_launch", _i, [_i, _i, _i]),
     ("lrtfc_gemm_int4_blockwise_nibble_bytes", _sz, [_i, _i]),
     ("lrtfc_pack_int4_blockwise_gemm_nibbles", _i, [_vp, _vp, _i, _i, _i, _vp, _vp]),
     ("lrtfc_fc_blockwise_int4_gemm_nibbles", _i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp, _sz,

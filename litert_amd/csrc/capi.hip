@@ -1167,6 +1167,11 @@ int lrtfc_fc_blockwise_int4_preferred_form(int batches, int depth, int out_depth
   return batches >= 16 ? LRTFC_INT4_FORM_GEMM_INT8 : LRTFC_INT4_FORM_DECODE;
 }
 
+int lrtfc_fc_blockwise_int4_rows_per_launch(int depth, int out_depth, int quantized) {
+  if (!lrtfc::FcInt4PackedSupports(depth, 32) || out_depth <= 0) return 0;
+  return lrtfc::FcInt4PackedRowsPerLaunch(depth, out_depth, /*fused=*/quantized == 0);
+}
+
 size_t lrtfc_gemm_int4_blockwise_nibble_bytes(int out_depth, int depth) {
   if (out_depth <= 0 || depth <= 0) return 0;
   return lrtfc::GemmInt4BlockwiseNibbleBytes(out_depth, depth);

@@ -711,7 +711,7 @@ __global__ __launch_bounds__(THREADS) void FcInt4PackedKernel(
 // tiles, and a ninth adds a step's products while the others work on the next; in a step a wavefront has
 // one tile's blocks of two channels, and everything is requested at the start. Filters not in the caches,
 // us at 1 / 2 / 4 rows (4: int8 rows in, with their quantizer), FcInt4PackedKernel -> this one: 16384 ->
-// 2048 8.7 / 10.7 / 14.1 -> 8.2 / 10.4 / 13.6, 11008 -> 2048 10.1 / 12.1 / 23.8 -> 7.5 / 9.7 / 16.6,
+// 2048 8.7 / 10.7 / 14.1 -> 8.2 / 10.4 / 13.6, 11008 -> 2048 10.1 / 12.1 / 23.8 -> 7.5 / 9.7 / 12.0,
 // 8192 -> 2048 6.4 / 8.1 / 11.2 -> 6.1 / 7.6 / 10.1, 4608 -> 1000 7.9 -> 5.0 at one row. A lane reads its
 // two channels' scales alone: 92 registers at one row, with the whole plane 104 and 0.2 us more.
 constexpr int kDeepWorkers = 8;
@@ -722,7 +722,7 @@ constexpr int kWorkerThreads = kDeepWorkers * kWaveSize;  // eight values of a s
 static_assert(kWorkerThreads * 8 == kStepTiles * kTileBlocks * kBlock, "a step's values");
 
 template <int BT>
-size_t DeepLds(int chunks) {
+constexpr size_t DeepLds(int chunks) {
   return static_cast<size_t>(BT) * chunks * kTileBlocks * kBlock +
          static_cast<size_t>(chunks) * kTileRows * BT * kPStride * 4 + BT * kDeepWorkers * 2 * 4;
 }
@@ -1171,6 +1171,17 @@ int FitBatchTile(int want, int padded, int ksplit, bool wide = false) {
   return bt;
 }
 
+static_assert(DeepLds<4>(kDeepSteps * kStepTiles) <= kLdsBudget, "four deep rows fit whatever their depth");
+
+// Rows of a launch of a single node, by the LDS map of the kernel that LaunchOne takes.
+int RowsPerLaunch(const Int4PackedArgs& a, bool fused) {
+  const int most = fused ? MaxBatchTile<true>(a.depth) : MaxBatchTile<false>(a.depth);
+  if (DeepNode(a, fused)) return most;
+  const bool wide = WideDeep(a.depth, a.out_depth, a.chunks);
+  return FitBatchTile(most, a.chunks * kTileBlocks * kBlock,
+                      wide ? a.chunks : ChooseKsplit(a.out_depth, a.chunks), wide);
+}
+
 template <bool FUSED>
 hipError_t LaunchTile(const Int4PackedArgs& a, int variant, int batch0, int bt, int slices,
                       hipStream_t stream) {
@@ -1227,9 +1238,6 @@ hipError_t LaunchFcInt4Packed(const FcInt4Args& q, const uint8_t* packed, const 
   a.depth = q.depth;
   a.out_depth = q.out_depth;
   a.chunks = (q.depth / kBlock + kTileBlocks - 1) / kTileBlocks;
-  const int padded = a.chunks * kTileBlocks * kBlock;
-  const bool wide = WideDeep(q.depth, q.out_depth, a.chunks);
-  const int ksplit = wide ? a.chunks : ChooseKsplit(q.out_depth, a.chunks);
   // Three or four fused rows of a small filter: two pairs side by side in one launch, as in small
   // groups (PrepareInt4Group); us at four rows, one tile of four -> pairs: 2048 -> 2048 6.8 -> 4.8,
   // 4096 -> 4096 8.7 -> 6.0. Both slices together are one round of a workgroup per CU; in two they read
@@ -1237,12 +1245,11 @@ hipError_t LaunchFcInt4Packed(const FcInt4Args& q, const uint8_t* packed, const 
   // 9.2 -> 9.9, 4096 -> 7700 9.2 -> 9.9; in it, 2048 -> 8192 6.9 -> 6.3).
   if (input_f32 && (q.batches == 3 || q.batches == 4) && q.depth <= kShallowDepth &&
       static_cast<int64_t>(q.out_depth) * q.depth / 2 <= kSideBySideMaxFilterBytes) {
-    const int groups_per_wg = kWaves / ksplit;  // (shallow rows: ksplit is at most kWaves)
+    const int groups_per_wg = kWaves / ChooseKsplit(q.out_depth, a.chunks);
     const int blocks = ((q.out_depth + kTileRows - 1) / kTileRows + groups_per_wg - 1) / groups_per_wg;
     if (2 * blocks <= kPairRound) return LaunchTile<true>(a, variant, 0, 2, 2, stream);
   }
-  const int tile = FitBatchTile(input_f32 ? MaxBatchTile<true>(q.depth) : MaxBatchTile<false>(q.depth),
-                                padded, ksplit, wide);
+  const int tile = RowsPerLaunch(a, input_f32 != nullptr);
   int batch0 = 0;
   while (batch0 < q.batches) {
     const int bt = min(tile, q.batches - batch0);
@@ -1254,6 +1261,13 @@ hipError_t LaunchFcInt4Packed(const FcInt4Args& q, const uint8_t* packed, const 
   return hipSuccess;
 }
 
+int FcInt4PackedRowsPerLaunch(int depth, int out_depth, bool fused) {
+  Int4PackedArgs a{};  // null pointers: aligned ones
+  a.depth = depth;
+  a.out_depth = out_depth;
+  a.chunks = (depth / kBlock + kTileBlocks - 1) / kTileBlocks;
+  return RowsPerLaunch(a, fused);
+}
 
 hipError_t PrepareInt4Group(const lrtfc_int4_group_node* nodes, int count, int batches, int depth,
                             void* device_table, lrtfc_int4_group_launch* launch,

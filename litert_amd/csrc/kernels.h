@@ -201,6 +201,7 @@ hipError_t PrepareInt4NibbleGroup(const lrtfc_int4_group_node* nodes, int count,
                                   hipStream_t stream);
 hipError_t LaunchFcInt4NibbleGrouped(const void* table, const lrtfc_int4_group_launch& launch,
                                      int variant, hipStream_t stream);
+int FcInt4PackedRowsPerLaunch(int depth, int out_depth, bool fused);
 hipError_t LaunchFcInt4Packed(const FcInt4Args& q, const uint8_t* packed, const float* input_f32,
                               int variant, hipStream_t stream);
 

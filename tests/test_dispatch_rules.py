@@ -104,3 +104,29 @@ def test_per_channel_int4_rows_around_the_line(depth, channels):
     for rows in (line, line + 1, 16, 17, 32, 33):
         xs = torch.from_numpy(x[:rows]).cuda()
         assert np.array_equal(op(xs).cpu().numpy().view(np.uint32), want[:rows])
+
+
+@pytest.mark.parametrize("depth,channels,fused,quantized", [
+    (4096, 2048, 4, 4), (4128, 2048, 2, 4), (10240, 2048, 2, 4), (10272, 2048, 2, 4), (11008, 2048, 2, 4),
+    (14336, 2048, 2, 4), (16384, 2048, 2, 4), (11008, 2049, 2, 2), (14336, 2056, 2, 2), (16384, 2056, 2, 4)])
+def test_blockwise_int4_rows_per_launch(depth, channels, fused, quantized):
+    """Deep single nodes of up to 256 channel groups take as many rows as their kernel holds (257 groups: as the
+    other one does)."""
+    rows = capi.load().lrtfc_fc_blockwise_int4_rows_per_launch
+    assert (rows(depth, channels, 0), rows(depth, channels, 1)) == (fused, quantized)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [3, 4, 7])
+@pytest.mark.parametrize("depth,channels", [(10272, 40), (11008, 2048), (14336, 50)])
+def test_blockwise_int4_deep_rows_in_one_launch(rows, depth, channels):
+    import numpy as np
+    import torch
+    import oracle
+    from litert_amd import fully_connected as fc
+    from litert_amd import workloads as wl
+    c = wl.blockwise_int4_fc(rows, depth, channels, seed=depth, lo=-8, hi=7)
+    op = fc.FullyConnectedBlockwiseInt4(c["packed"], c["scales"], depth, 32)
+    want = oracle.fc_blockwise_int4(c["x"], c["packed"], channels, c["scales"].view(np.uint16), 32)
+    got = op.call_split(torch.from_numpy(c["x"]).cuda()).cpu().numpy()
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
