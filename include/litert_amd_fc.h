@@ -162,6 +162,20 @@ enum {
 };
 int lrtfc_fc_int8_packed_kernel(int batches, int depth, int out_depth);
 
+/* The GEMM among them by its tiles: rows x channels of a workgroup, _AHEAD with operands requested four
+ * steps ahead instead of two; NONE where the launch is one of the GEMVs'. *rows (null: not asked) is how many
+ * rows go in that launch: the others, a tail over one round of tiles, follow in one of their own, whose
+ * form is that of their count. Pure host function. */
+enum {
+  LRTFC_INT8_TILES_NONE = 0,
+  LRTFC_INT8_TILES_SPLIT = 1,
+  LRTFC_INT8_TILES_64X128 = 2,
+  LRTFC_INT8_TILES_64X128_AHEAD = 3,
+  LRTFC_INT8_TILES_128X128 = 4,
+  LRTFC_INT8_TILES_128X256 = 5
+};
+int lrtfc_fc_int8_packed_tiles(int batches, int depth, int out_depth, int* rows);
+
 /* Re-tiles a row-major int8 filter [out_depth, depth] for the matrix-core GEMV: tiles of
  * 16 output channels x 64 depth (1 KiB each, zero-padded at the edges), the 16 bytes of
  * lane L inside a tile being channel L % 16, depth 16 * (L / 16) .. +16; tiles of one

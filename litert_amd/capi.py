@@ -23,6 +23,8 @@ OUT_FLOAT32, OUT_FLOAT16 = range(2)
 INT4_FORM_DECODE, INT4_FORM_GEMM_NIBBLES, INT4_FORM_GEMM_INT8 = range(3)
 (INT8_KERNEL_GEMV, INT8_KERNEL_GEMV_TWO_TILES, INT8_KERNEL_ROWS, INT8_KERNEL_SPLIT,
  INT8_KERNEL_TILES_64X128, INT8_KERNEL_TILES_128X256) = range(6)
+(INT8_TILES_NONE, INT8_TILES_SPLIT, INT8_TILES_64X128, INT8_TILES_64X128_AHEAD, INT8_TILES_128X128,
+ INT8_TILES_128X256) = range(6)
 
 # Every symbol include/litert_amd_fc.h declares: (name, restype, argtypes).
 _vp, _i, _i32, _i64, _f, _d, _sz = (C.c_void_p, C.c_int, C.c_int32, C.c_int64, C.c_float,
@@ -45,6 +47,7 @@ SYMBOLS = [
     ("lrtfc_fc_blockwise_int4_preferred_layout", _i, [_i, _i]),
     ("lrtfc_fc_hybrid_fused_max_batches", _i, [_i, _i]),
     ("lrtfc_fc_int8_packed_kernel", _i, [_i, _i, _i]),
+    ("lrtfc_fc_int8_packed_tiles", _i, [_i, _i, _i, _pint]),
     ("lrtfc_packed_int8_filter_bytes", _sz, [_i, _i]),
     ("lrtfc_pack_int8_filter", _i, [_vp, _i, _i, _vp, _vp]),
     ("lrtfc_fc_int8_packed", _i, [_vp, _vp, _vp, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _i32, _i32,

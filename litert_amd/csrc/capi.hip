@@ -378,9 +378,28 @@ int lrtfc_fc_int8_packed_kernel(int batches, int depth, int out_depth) {
   }
   switch (lrtfc::FcInt8PackedGemmForm(a)) {
     case lrtfc::Int8GemmForm::kSplit: return LRTFC_INT8_KERNEL_SPLIT;
-    case lrtfc::Int8GemmForm::kSmallerTiles: return LRTFC_INT8_KERNEL_TILES_64X128;
-    default: return LRTFC_INT8_KERNEL_TILES_128X256;
+    case lrtfc::Int8GemmForm::kTiles128x256: return LRTFC_INT8_KERNEL_TILES_128X256;
+    default: return LRTFC_INT8_KERNEL_TILES_64X128;
   }
+}
+
+int lrtfc_fc_int8_packed_tiles(int batches, int depth, int out_depth, int* rows) {
+  const int kernel = lrtfc_fc_int8_packed_kernel(batches, depth, out_depth);
+  if (rows) *rows = batches;
+  if (kernel < LRTFC_INT8_KERNEL_SPLIT) return LRTFC_INT8_TILES_NONE;
+  lrtfc::FcInt8Args a{};
+  a.batches = batches;
+  a.depth = depth;
+  a.out_depth = out_depth;
+  if (rows) *rows = lrtfc::FcInt8PackedGemmFirstRows(a);
+  switch (lrtfc::FcInt8PackedGemmForm(a)) {
+    case lrtfc::Int8GemmForm::kSplit: return LRTFC_INT8_TILES_SPLIT;
+    case lrtfc::Int8GemmForm::kTiles64x128: return LRTFC_INT8_TILES_64X128;
+    case lrtfc::Int8GemmForm::kTiles64x128Ahead: return LRTFC_INT8_TILES_64X128_AHEAD;
+    case lrtfc::Int8GemmForm::kTiles128x128: return LRTFC_INT8_TILES_128X128;
+    case lrtfc::Int8GemmForm::kTiles128x256: return LRTFC_INT8_TILES_128X256;
+  }
+  return LRTFC_INT8_TILES_NONE;
 }
 
 int lrtfc_fc_blockwise_int4_preferred_layout(int depth, int blocksize) {

@@ -595,10 +595,10 @@ bool FcInt8PackedGemmSupports(const FcInt8Args& a) {
 //   more than a round, depth 512 to 2048, to 128 x 128: 2048 x 1024 -> 14336 52.6 -> 47.5 / 57.5 -> 51.5,
 //     700 x 1024 -> 14336 24.7 -> 20.8 / 27.7 -> 23.3, 1715 x 560 -> 15924 52.4 -> 41.9 / 53.1 -> 42.3. Float
 //     outputs gain more: hybrid 2048 x 1024 -> 14336 76 -> 63 / 83 -> 73. Of 220 such sizes where they fill
-//     less than two rounds for one of 128 x 256 0.85 of the time in the mean (least 1.03), of 100 where they fill
-//     two 0.96 (least 1.04). Rows that end inside a 16-byte piece are read twice as often from addresses that are no
-//     multiple of 16: deeper than 1024 and in two rounds for one they lose (1.05 of the time in the mean,
-//     1778 x 1949 -> 6928 46.9 -> 60 / 44.5 -> 53, 1600 x 1434 -> 7948 38.6 -> 46 / 38.2 -> 42) and stay.
+//     less than two rounds for one of 128 x 256 0.85 of the time in the mean (least 1.03), of 100 where they
+//     fill two 0.96 (least 1.04). Rows that end inside a 16-byte piece are read twice as often from addresses
+//     that are no multiple of 16: deeper than 1024 and in two rounds for one they lose (1.05 of the time in
+//     the mean, 1778 x 1949 -> 6928 46.9 -> 60 / 44.5 -> 53, 1600 x 1434 -> 7948 38.6 -> 46 / 38.2 -> 42) and stay.
 //   a round at most, depth 512 to 768, to 64 x 128 as long as those are three rounds: 1506 x 672 -> 2567 13.8 ->
 //     8.5 / 14.5 -> 9.2, 1806 x 608 -> 2575 13.4 -> 10.5 / 14.2 -> 11.3; of 66 such sizes 0.86 of the time in the
 //     mean, least 1.01. (In a fourth round: 392 x 704 -> 14656 14.3 -> 17.7 / 13.2 -> 17.1, 652 x 576 -> 9024
@@ -616,13 +616,13 @@ Int8GemmForm FcInt8PackedGemmForm(const FcInt8Args& a) {
                                             !(a.depth % 16 && a.depth > 1024 && two_for_one)
                                       : (a.depth >= 512 && a.depth <= 768 && SmallTiles(a) <= 3 * kCus) ||
                                             (a.depth > 2048 && square <= kCus);
-    return smaller ? Int8GemmForm::kSmallerTiles : Int8GemmForm::kTiles128x256;
+    if (!smaller) return Int8GemmForm::kTiles128x256;
+  } else if (FcInt8SplitGemmBeatsTiles(a, SmallTiles(a))) {
+    return Int8GemmForm::kSplit;
   }
-  return FcInt8SplitGemmBeatsTiles(a, SmallTiles(a)) ? Int8GemmForm::kSplit
-                                                     : Int8GemmForm::kSmallerTiles;
+  if (TakesSquareTiles(a)) return Int8GemmForm::kTiles128x128;
+  return DeepRing(a) ? Int8GemmForm::kTiles64x128Ahead : Int8GemmForm::kTiles64x128;
 }
-
-namespace {
 
 // A few tiles more than one per CU cost a second round, nearly all of it on an idle chip. The rows of that
 // tail go in a launch of their own then, on the tiles that suit them: the number of rows the first
@@ -632,7 +632,7 @@ namespace {
 // least 1614 x 5680 -> 5909, 312 tiles, 83 -> 81. A larger tail gains less (800 x 4096 -> 12288, 336
 // tiles, 61.8 -> 59.6), one behind two or three rounds loses (2048 x 4096 -> 8448 96.6 -> 104, 2048 x 2560 ->
 // 12800 93 -> 107: the last tiles of a round overlap the first of the next).
-int RowsOfWholeRound(const FcInt8Args& a) {
+int FcInt8PackedGemmFirstRows(const FcInt8Args& a) {
   const int tiles = LargeTiles(a);
   if (a.depth <= 2048 || tiles <= kCus || tiles > kCus + kCus / 4) return a.batches;
   const int tiles_n = (a.out_depth + 255) / 256;
@@ -641,11 +641,9 @@ int RowsOfWholeRound(const FcInt8Args& a) {
   return min(kept * 128, a.batches);
 }
 
-}  // namespace
-
 hipError_t LaunchFcInt8PackedGemm(const FcInt8Args& a, Int8Epilogue epilogue, hipStream_t stream) {
   if (!FcInt8PackedGemmSupports(a)) return hipErrorNotSupported;
-  if (const int kept = RowsOfWholeRound(a); kept < a.batches) {
+  if (const int kept = FcInt8PackedGemmFirstRows(a); kept < a.batches) {
     FcInt8Args part = a;
     part.whole_input = a.whole_input ? a.whole_input : a.input;
     part.whole_batches = a.whole_input ? a.whole_batches : a.batches;
@@ -662,12 +660,12 @@ hipError_t LaunchFcInt8PackedGemm(const FcInt8Args& a, Int8Epilogue epilogue, hi
   }
   switch (FcInt8PackedGemmForm(a)) {
     case Int8GemmForm::kSplit: return LaunchFcInt8SplitGemm(a, epilogue, stream);
+    case Int8GemmForm::kTiles64x128: return LaunchShape<64, 1, 2>(a, epilogue, SmallTiles(a), stream);
+    case Int8GemmForm::kTiles64x128Ahead: return LaunchShape<64, 1, 4>(a, epilogue, SmallTiles(a), stream);
+    case Int8GemmForm::kTiles128x128: return LaunchShape<128, 1, 2>(a, epilogue, SquareTiles(a), stream);
     case Int8GemmForm::kTiles128x256: return LaunchShape<128, 2, 2>(a, epilogue, LargeTiles(a), stream);
-    default:
-      if (TakesSquareTiles(a)) return LaunchShape<128, 1, 2>(a, epilogue, SquareTiles(a), stream);
-      return DeepRing(a) ? LaunchShape<64, 1, 4>(a, epilogue, SmallTiles(a), stream)
-                         : LaunchShape<64, 1, 2>(a, epilogue, SmallTiles(a), stream);
   }
+  return hipErrorInvalidValue;
 }
 
 }  // namespace lrtfc

@@ -150,8 +150,11 @@ bool FcInt8PackedGemvTakesRowsInOnePass(const FcInt8Args& a);
 bool FcInt8RowsGemvTakes(const FcInt8Args& a);
 hipError_t LaunchFcInt8RowsGemv(const FcInt8Args& a, Int8Epilogue epilogue, hipStream_t stream);
 bool FcInt8PackedGemmSupports(const FcInt8Args& a);
-enum class Int8GemmForm { kSplit, kSmallerTiles, kTiles128x256 };
+// Tiles of rows x channels; kTiles64x128Ahead requests operands four steps ahead instead of two.
+enum class Int8GemmForm { kSplit, kTiles64x128, kTiles64x128Ahead, kTiles128x128, kTiles128x256 };
 Int8GemmForm FcInt8PackedGemmForm(const FcInt8Args& a);
+// Rows of the launch, where the others go in one of their own (a.batches: all in one).
+int FcInt8PackedGemmFirstRows(const FcInt8Args& a);
 hipError_t LaunchFcInt8PackedGemm(const FcInt8Args& a, Int8Epilogue epilogue, hipStream_t stream);
 // The same for launches that leave the chip idle in those tiles (fc_int8_split_gemm.hip): small tiles,
 // the depth dealt to the wavefronts of a workgroup. LaunchFcInt8PackedGemm takes it by itself.

@@ -1,5 +1,7 @@
 """Forms of the tiled int8 GEMM, whole batches against the same rows in pieces of at most 32 (other
 kernels, which have oracle tests of their own) and, at the first and last rows, against the oracle."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -44,12 +46,20 @@ def _hybrid(fc, B, K, N):  # noqa: F811
         c["x"][rows], c["w"], c["pcs"], bias=bias, activation=fc._act("relu" if N % 2 else "none")))
 
 
-# 64 x 128 tiles with four steps of operands in flight: walks of 4 n to 4 n + 3 steps of 128, an odd
-# number of 64 deep slabs, rows that end inside a 16-byte piece; the last depth with two steps.
+def _tiles(B, K, N):
+    """The launch's tiles and how many of its rows they take."""
+    rows = C.c_int()
+    return capi.load().lrtfc_fc_int8_packed_tiles(B, K, N, C.byref(rows)), rows.value
+
+
+# 64 x 128 tiles with four steps of operands in flight: walks of 4 n to 4 n + 3 steps of 128 (20; 17, 33; 18; 19),
+# odd and even numbers of 64 deep slabs, rows that end inside a 16-byte piece; 2048 deep with two steps.
 @pytest.mark.parametrize("B,K,N", [(130, 2048, 8200), (130, 2049, 8200), (193, 2176, 7000), (257, 2200, 6130),
-                                   (130, 2304, 8200), (193, 2431, 7001), (257, 2432, 6130), (300, 4100, 4099)])
+                                   (130, 2304, 8200), (193, 2431, 7001), (257, 2432, 6130), (300, 4100, 4099),
+                                   (130, 2560, 8200), (193, 2496, 7000), (130, 2555, 8200)])
 def test_64x128_tiles_deep_walks(fc, B, K, N):  # noqa: F811
     assert capi.load().lrtfc_fc_int8_packed_kernel(B, K, N) == capi.INT8_KERNEL_TILES_64X128
+    assert _tiles(B, K, N) == (capi.INT8_TILES_64X128_AHEAD if K > 2048 else capi.INT8_TILES_64X128, B)
     _int8(fc, B, K, N)
     _hybrid(fc, B, K, N)
 
@@ -62,6 +72,7 @@ def test_64x128_tiles_deep_walks(fc, B, K, N):  # noqa: F811
                                    (1000, 2100, 4001), (1100, 512, 4000), (1100, 760, 4003)])
 def test_tiles_between(fc, B, K, N):  # noqa: F811
     assert capi.load().lrtfc_fc_int8_packed_kernel(B, K, N) == capi.INT8_KERNEL_TILES_64X128
+    assert _tiles(B, K, N) == (capi.INT8_TILES_64X128 if (B, N // 10) == (1100, 400) else capi.INT8_TILES_128X128, B)
     _int8(fc, B, K, N)
     if B * K * N < 6e9:
         _hybrid(fc, B, K, N)
@@ -71,13 +82,20 @@ def test_tiles_between(fc, B, K, N):  # noqa: F811
 @pytest.mark.parametrize("B,K,N", [(1100, 511, 7300), (1100, 2049, 7400), (1100, 769, 4000), (1000, 2048, 4001)])
 def test_tiles_between_other_side(fc, B, K, N):  # noqa: F811
     assert capi.load().lrtfc_fc_int8_packed_kernel(B, K, N) == capi.INT8_KERNEL_TILES_128X256
+    assert _tiles(B, K, N) == (capi.INT8_TILES_128X256, B)
     _int8(fc, B, K, N)
 
 
 # A tail of up to 64 tiles of 128 x 256 over one per CU: its rows in a launch of their own; rows that end
-# inside a piece; the largest tail, and a launch of two rounds that stays whole.
+# inside a piece; tails on split tiles and on 64 x 128; and 320 tiles whose whole rows leave too much of the
+# round (192 of 256), which stay one launch.
 @pytest.mark.parametrize("B,K,N", [(2000, 2064, 4200), (2040, 2049, 4350), (1153, 2177, 8192), (1100, 2177, 16200)])
 def test_tail_rows_in_their_own_launch(fc, B, K, N):  # noqa: F811
+    kept = {4200: 1920, 4350: 1920, 8192: 1024, 16200: B}[N]
+    assert _tiles(B, K, N) == (capi.INT8_TILES_128X256, kept)
+    if kept < B:
+        tail = capi.INT8_TILES_64X128_AHEAD if N == 8192 else capi.INT8_TILES_SPLIT
+        assert _tiles(B - kept, K, N) == (tail, B - kept)
     _int8(fc, B, K, N)
     _hybrid(fc, B, K, N)
 
@@ -106,4 +124,5 @@ def test_tail_rows_and_the_whole_zero_exit(fc, zero_rows):  # noqa: F811
 @pytest.mark.parametrize("B,K,N", [(129, 512, 128 * n) for n in range(171, 179)] +
                          [(257, 96, 256 * n) for n in range(43, 51)])
 def test_grids_of_any_remainder(fc, B, K, N):  # noqa: F811
+    assert _tiles(B, K, N) == (capi.INT8_TILES_64X128 if K == 512 else capi.INT8_TILES_128X256, B)
     _int8(fc, B, K, N)

@@ -1,5 +1,7 @@
 """Which kernel int8 rows on a re-tiled filter go to (lrtfc_fc_int8_packed_kernel, a host function):
 each line of the rule at sizes on both its sides, as measured."""
+import ctypes as C
+
 import pytest
 
 from litert_amd import capi
@@ -79,3 +81,23 @@ def test_short_walks_in_up_to_three_rounds_of_64x128(rows, depth, channels, kern
     (1536, 1949, 8192, capi.INT8_KERNEL_TILES_64X128)])  # 768 tiles: three rounds for two
 def test_ragged_rows_read_twice_in_two_rounds_for_one(rows, depth, channels, kernel):
     assert _kernel(rows, depth, channels) == kernel
+
+
+S, T, A, Q, L = (capi.INT8_TILES_SPLIT, capi.INT8_TILES_64X128, capi.INT8_TILES_64X128_AHEAD,
+                 capi.INT8_TILES_128X128, capi.INT8_TILES_128X256)
+
+
+@pytest.mark.parametrize("rows,depth,channels,tiles,first", [
+    (1, 2048, 2048, capi.INT8_TILES_NONE, 1), (77, 3008, 5003, S, 77),
+    (130, 2048, 8200, T, 130), (130, 2049, 8200, A, 130),  # four steps ahead from there on ...
+    (300, 2049, 6528, A, 300), (300, 2049, 6529, Q, 300),  # ... in one round of 64 x 128; 128 x 128 beyond it
+    (300, 2048, 6529, Q, 300), (300, 2047, 6529, T, 300),
+    (1000, 2048, 4096, L, 1000), (1000, 2049, 4096, Q, 1000), (1000, 2049, 4097, L, 1000),  # half a round
+    (1100, 511, 7300, L, 1100), (1100, 512, 7300, Q, 1100), (1100, 2048, 7300, Q, 1100), (1100, 2049, 8192, L, 1024),
+    (1024, 4096, 8192, L, 1024), (1025, 4096, 8192, L, 1024), (1280, 4096, 8192, L, 1024),  # 256, 288, 320 tiles
+    (1281, 4096, 8192, L, 1281), (1025, 2048, 8192, Q, 1025), (640, 4096, 15616, L, 512),
+    (1152, 4096, 8448, L, 1152)])  # 231 tiles in the rows of a round: too few
+def test_tiles_of_the_gemm(rows, depth, channels, tiles, first):
+    n = C.c_int()
+    assert (capi.load().lrtfc_fc_int8_packed_tiles(rows, depth, channels, C.byref(n)), n.value) == (tiles, first)
+    assert capi.load().lrtfc_fc_int8_packed_tiles(rows, depth, channels, None) == tiles
