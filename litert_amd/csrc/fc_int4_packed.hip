@@ -106,7 +106,6 @@ struct Int4Start {
   int depth, out_depth, chunks;
 };
 
-
 // Nibble planes of eight consecutive int8 activations (lo = q0..q3, hi = q4..q7 as packed
 // bytes): `high` holds (q >> 4) & 15 and `low` holds q & 15 of element i in bits 4i .. 4i + 3,
 // the order in which a dword of the filter holds its eight weights. With q = 16 * qh + ql
@@ -140,10 +139,10 @@ struct Int4Shared {
   float* mm;    // [BT][waves][2]
   float* kb;    // [waves][2][64]: kfsum and bias of the channels a wavefront covers
   float* ob;    // [waves][64 * BT]: finished outputs of those channels
-  // ksplit is a power of two everywhere (a division by it cost every wavefront some 30 scalar and vector
-  // instructions ahead of its first load). Floats of parked products: one tile per wavefront when a wavefront owns a channel group
-  // alone; every tile of the group when `ksplit` wavefronts share it (the ordered walk then
-  // needs them all).
+  // Floats of parked products: one tile per wavefront when a wavefront owns a channel group alone; every
+  // tile of the group when `ksplit` wavefronts share it (the ordered walk then needs them all). ksplit is
+  // a power of two everywhere: a division by it cost every wavefront some 30 scalar and vector
+  // instructions ahead of its first load.
   __host__ __device__ static size_t ProductFloats(int chunks, int ksplit) {
     constexpr int waves = THREADS / kWaveSize;
     const size_t tile = static_cast<size_t>(8) * BT * kPStride;
@@ -822,7 +821,6 @@ __global__ __launch_bounds__(kDeepThreads, 1) void FcInt4DeepKernel(
       inv = ElementwiseInv(qp);
       zero_point = qp.zero_point;
     }
-    const int vector_end = depth - (depth % 8);
 #pragma unroll
     for (int j = 0; j < kDeepSteps; ++j) {
       if (j >= steps) break;
@@ -838,9 +836,8 @@ __global__ __launch_bounds__(kDeepThreads, 1) void FcInt4DeepKernel(
               qp.inv = ReadLaneF32(inv, b);
               qp.zero_point = __builtin_amdgcn_readlane(zero_point, b);
               const float4 x0 = xr[b][j][0], x1 = xr[b][j][1];
-              const bool tail = g * 8 >= vector_end;
-              lo = static_cast<uint32_t>(QuantizePack4<VARIANT>(x0.x, x0.y, x0.z, x0.w, qp, tail));
-              hi = static_cast<uint32_t>(QuantizePack4<VARIANT>(x1.x, x1.y, x1.z, x1.w, qp, tail));
+              lo = static_cast<uint32_t>(QuantizePack4<VARIANT>(x0.x, x0.y, x0.z, x0.w, qp, /*tail=*/false));
+              hi = static_cast<uint32_t>(QuantizePack4<VARIANT>(x1.x, x1.y, x1.z, x1.w, qp, /*tail=*/false));
             } else {
               lo = static_cast<uint32_t>(qr[b][j].x);
               hi = static_cast<uint32_t>(qr[b][j].y);
@@ -1064,8 +1061,8 @@ constexpr int kDeepMaxGroups = 256;
 bool DeepNode(const Int4PackedArgs& a, bool fused) {
   const auto at = reinterpret_cast<uintptr_t>(fused ? static_cast<const void*>(a.input_f32)
                                                     : static_cast<const void*>(a.input_q));
-  return a.depth > kShallowDepth && a.depth <= kDeepDepth && a.depth % 8 == 0 &&
-         (at & (fused ? 15 : 7)) == 0 && (a.out_depth + kTileRows - 1) / kTileRows <= kDeepMaxGroups;
+  return a.depth > kShallowDepth && a.depth <= kDeepDepth && (at & (fused ? 15 : 7)) == 0 &&
+         (a.out_depth + kTileRows - 1) / kTileRows <= kDeepMaxGroups;
 }
 
 // Channel groups per wavefront. Measured on launches from 7 MB to 340 MB: a wavefront should
