@@ -9,8 +9,9 @@
 // added to the accumulator unfused, the reference's own order of float operations (:1069-1077),
 // so the results are bit-identical to the decode kernel's and the oracle's.
 //
-// The vector operations per output and block draw as much on the power cap as the matrix cores (the MFMA
-// of a block takes 16 cycles of its SIMD, three operations on its 4 outputs per lane 29 to 48). Two suffice:
+// The vector operations per output and block take longer than the matrix cores, and their time adds to the
+// MFMAs' (of a block and 16 x 16 tile: 16 cycles of its SIMD, and three operations on its 4 outputs per
+// lane 27 from two wavefronts on). Two suffice:
 //   * The accumulator input of every MFMA is the bit pattern of 1.5 * 2^23, so its integer result
 //     READ AS A FLOAT is 1.5 * 2^23 + sum, exactly (|sum| <= 32 * 8 * 128 < 2^22): no conversion.
 //   * fma(that, scale, -1.5 * 2^23 * scale) rounds the exact product sum * scale once, which is
@@ -19,9 +20,11 @@
 //   * The batch rows are the A operand and the channels the B operand, so that a lane's four results
 //     are four rows of ONE channel: one scale per lane and block (and its product with -1.5 * 2^23)
 //     serves every row tile, where four channels per lane took four broadcasts per block.
-// Bound by the power cap: 2048 x 4096 -> 14336 has 2 x 4 x 14.7 M wavefront operations, about 100 us of
-// issue at 2.4 cycles each; they and the MFMAs take 192 to 213 us on registers alone, at the 1.5 to 1.8 GHz
-// that the cap leaves, the launch without operand loads 235, with them 263.
+// Bound by issue, at the clock that the power cap leaves: 2048 x 4096 -> 14336 is 3584 tiles of 32 x 32 and
+// blocks a SIMD, each 32 cycles of MFMA and 72 of vector operations, 107 for both: 383 thousand cycles, 159 us
+// at 2.4 GHz, 193 at the 1.98 GHz that this loop holds on random bits. The launch takes 544 thousand (259 us
+// at 2.1 GHz; on constant operands 529 at 2.39), 480 thousand without operand loads, of which the last
+// half round of workgroups is 25.
 //
 // Layouts, made once at prepare (filter) or per call (activations):
 //   filter `tile32x32s`: for channel tile t (32 channels) and block b, 1 KiB: lane L's 16 bytes are
@@ -407,7 +410,7 @@ __global__ __launch_bounds__(kThreads, 2) void FcInt4BlockwiseGemmKernel(GemmArg
 
 // The large form: CT x RT tiles of 32 channels x 32 rows per wavefront, four wavefronts in WROWS x
 // 4 / WROWS; BLOCKS blocks in flight. Per tile and block one MFMA (32 cycles of the matrix core) and
-// 32 vector operations on its 16 results per lane (77 cycles of the SIMD from two wavefronts on).
+// 32 vector operations on its 16 results per lane (72 cycles of the SIMD from two wavefronts on).
 template <int CT, int RT, int WROWS, int BLOCKS>
 __global__ __launch_bounds__(kThreads, 2) void FcInt4BlockwiseGemmLargeKernel(GemmArgs a, int wgs_c,
                                                                               int wgs_r) {
