@@ -1175,8 +1175,9 @@ int lrtfc_fc_blockwise_int4_preferred_form(int batches, int depth, int out_depth
   // the int8-expanded one from 16 rows on otherwise. Deeper than 8192 the streaming kernel in passes is
   // worse still (us, there -> here: 5 x 8448 -> 4096 22.3 -> 17.4, 12 x 11008 -> 4096 59 -> 20.7) and
   // the int8 copy no better (16 x 14336 -> 2048 31.4 -> 23.9, from memory 42.1 -> 24.7). Beyond 14336
-  // five to eight rows are faster streamed (8 x 16352 -> 2048 24.3, here 26.8), and the answers
-  // there are as they were: callers re-tile their filters for them (16 x 16384 -> 2048: 26.8 us here).
+  // five to eight rows are faster streamed (8 x 16352 -> 2048 24.3, here 26.8). From 16 rows on this form
+  // would be the faster one there too (16 x 16384 -> 2048 26.8 us, 48.8 on the int8 copy); the answer is
+  // still the int8 copy, as callers and tests have it from before this form reached that deep.
   const int channel_tiles = (out_depth + 15) / 16;
   if (batches <= 4) return LRTFC_INT4_FORM_DECODE;
   if (depth <= 14336 && ((batches <= 32 && channel_tiles >= 512) ||
